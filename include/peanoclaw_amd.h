@@ -304,7 +304,8 @@ int pc_set_prune_slack(pc_pool *pool, double slack);
 /* Row segments of the batched update (no reference counterpart): 0 =
  * automatic (a step with fewer tasks than the GPU holds splits the rows of
  * each patch into 2 or 4 segments of at least 8 rows, each marched by its
- * own wavefront), 1 = whole patches, 2 or 4 = that many segments where the
+ * own wavefront; with still fewer, into segments of at most 4 rows whose
+ * speeds are exact in every launch mode), 1 = whole patches, 2 or 4 = that many segments where the
  * patch has at least 8 rows per segment.  Results do not depend on it. */
 int pc_set_row_segments(pc_pool *pool, int segments);
 /* Run k global-dt steps of every scenario that has patches. */
@@ -312,7 +313,9 @@ int pc_step_all(pc_pool *pool, int k);
 /* Plain per-patch-launch form of the same step (reference call pattern:
  * ghost fill, per-patch CFL estimate, per-patch update, one launch each). */
 int pc_step_all_per_patch(pc_pool *pool, int k);
-/* Capture one step as a hipGraph and replay it k times. */
+/* Capture one step as a hipGraph and replay it k times (steps of so few
+ * patches that they run on short row segments: their two kernels are
+ * launched again instead, which leaves no gap between steps). */
 int pc_graph_capture(pc_pool *pool);
 int pc_graph_replay(pc_pool *pool, int k);
 /* Refinement flags of all patches (1 refine, 0 coarsening allowed, 2 keep),
@@ -329,7 +332,8 @@ int pc_scenario_mass(pc_pool *pool, int scenario, double *out);
 /* Device time (ms) of the last pc_step_all / pc_graph_replay call measured
  * with HIP events on the pool stream, and (pc_step_all only) the mean
  * duration of one update-kernel launch over that call's steps, from an
- * event pair recorded around every update launch. */
+ * event pair recorded around every update launch (steps of so few patches
+ * that they run on short row segments: around the last one). */
 int pc_last_timing(pc_pool *pool, double *total_ms, double *update_ms);
 
 /* Diagnostic: run the pool's device edge solver on n host edges

@@ -15,7 +15,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 SRC = os.path.join(PKG, "csrc", "pc_abi.hip")
 DEPS = [os.path.join(PKG, "csrc", f) for f in
-        ("pc_abi.hip", "pc_kernels.hpp", "pc_patch_kernels.hpp", "pc_server.hpp",
+        ("pc_abi.hip", "pc_kernels.hpp", "pc_patch_kernels.hpp", "pc_seg_kernels.hpp", "pc_server.hpp",
          "pc_amr.hpp", "pc_vtu.hpp", "swe_device.hpp")] + \
        [os.path.join(ROOT, "include", "peanoclaw_amd.h")]
 LIB = os.path.join(PKG, "libpeanoclaw_amd.so")

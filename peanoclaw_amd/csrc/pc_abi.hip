@@ -19,6 +19,7 @@
 #include "../../include/peanoclaw_amd.h"
 #include "pc_kernels.hpp"
 #include "pc_patch_kernels.hpp"
+#include "pc_seg_kernels.hpp"
 
 using namespace pcamd;
 
@@ -88,6 +89,7 @@ struct pc_pool {
   bool sides_any = false;
   bool edges_dirty = true;
   bool fused_ready = false;
+  bool uploaded = true;  // state changed from outside since the last batched step
   int* d_scn_of = nullptr;
   int nentries = 0;
   ScnDev* d_scn = nullptr;
@@ -101,6 +103,25 @@ struct pc_pool {
   int nutasks = 0;
   int row_segments = 0;  // 0 automatic, 1 off, 2 or 4 forced
   std::vector<int> h_rseg;  // row segments per slot of the current list
+  // steps with too few patches to fill the GPU run on short row segments
+  // (pc_seg_kernels.hpp) of at most seg_rows rows; 0: the row march
+  int seg_rows = 0;
+  int seg_solver = -1;  // the solver seg_rows was chosen for
+  Task* d_stasks = nullptr;
+  int nstasks = 0;
+  size_t stasks_cap = 0;
+  SegDesc* d_segdesc = nullptr;  // per entry of the task patch list
+  size_t segdesc_cap = 0;
+  int nsegdesc = 0;
+  double* d_smax_seg = nullptr;  // kSegSlots per slot
+  size_t smax_seg_cap = 0;
+  double* d_cfl_block = nullptr;  // smallest CFL step of every workgroup
+  size_t cfl_block_cap = 0;
+  SegRange* d_ranges = nullptr;  // workgroups per scenario
+  size_t ranges_cap = 0;
+  ScnDev* d_scn_alt = nullptr;  // the clocks a segment update writes
+  size_t scn_alt_cap = 0;
+  bool est_in_segments = false;  // the patches' estimates: from d_smax_seg
   int* d_plist = nullptr;
   int* d_plist_scn = nullptr;
   size_t plist_cap = 0;
@@ -333,6 +354,7 @@ bool valid_slot(pc_pool* p, int s) {
 void mark_state_changed(pc_pool* p) {
   p->edges_dirty = true;
   p->fused_ready = false;
+  p->uploaded = true;
 }
 
 int sync_scn_host(pc_pool* p) {
@@ -346,6 +368,7 @@ int sync_scn_host(pc_pool* p) {
 
 int upload_scn(pc_pool* p) {
   CHK(ensure_dev(&p->d_scn, &p->scn_cap, std::max<size_t>(p->scn.size(), 1)));
+  CHK(ensure_dev(&p->d_scn_alt, &p->scn_alt_cap, std::max<size_t>(p->scn.size(), 1)));
   if (!p->scn.empty())
     HIPCHK(hipMemcpyAsync(p->d_scn, p->scn.data(), p->scn.size() * sizeof(ScnDev),
                           hipMemcpyHostToDevice, p->stream));
@@ -398,9 +421,140 @@ PatchDev make_patchdev(const Slot& s) {
   return d;
 }
 
+// The patches' own estimates after a step on short row segments, from their
+// segments' speed maxima (only when someone asks, or before the lists they
+// belong to are rebuilt).
+int segment_estimates(pc_pool* p) {
+  if (!p->est_in_segments) return PC_OK;
+  p->est_in_segments = false;
+  hipLaunchKernelGGL(k_seg_estimates, dim3((p->nsegdesc + 63) / 64), dim3(64), 0, p->stream,
+                     p->d_segdesc, p->nsegdesc, p->seg_rows, p->d_smax_seg, p->d_est);
+  HIPCHK(hipGetLastError());
+  return PC_OK;
+}
+
+// Rows per segment of a step on short row segments, 0 for the row march.
+//
+// Fewer rows shorten the chain of a wavefront, more rows save work (R rows
+// read R + 2 and solve R + 1 x-edges per column).  The lines are where the
+// measured times cross, us a step of n x n grids of 32^2 patches (9, 16, 24,
+// 32, 40 a side; wavefronts at R = 2: 656, 2048, 4608, 8192, 12800):
+//   f-wave    R = 2: 14.9 19.7 35.7 52.6  83.2   R = 4: 17.0 19.2 30.3 41.4 63.1
+//             row march (pruned speeds): 35.0 36.3 40.6 44.6 57.1
+//   augmented R = 1: 41 66 129 220 343   R = 2: 43 57 108 165 250
+//             R = 4: 62 63 107 149 227   row march: 180 182 202 215 283
+// and 9 x 9 patches of 16^2: f-wave 14.1 (R = 2), 17.0 (R = 4), 34.7 (march);
+// augmented 31.9 (R = 1), 41.8, 64.1, 128 (march).  The augmented solver's
+// edges cost about six times the f-wave's, so its lines lie further out; at
+// 40 x 40 patches of 64^2 (25,600 wavefronts) R = 4 still takes 794 us, the
+// march 923 us.
+int choose_seg_rows(const pc_pool* p) {
+  if (p->row_segments != 0 || p->h_tasks.empty()) return 0;
+  auto waves = [&](int R) {
+    long long n = 0;
+    for (const Task& t : p->h_tasks) n += seg_count(t.nx, R);
+    return n;
+  };
+  if (p->solver) {
+    if (waves(1) <= 1536) return 1;
+    if (waves(2) <= 4096) return 2;
+    return waves(4) <= 32768 ? 4 : 0;
+  }
+  if (waves(2) <= 1536) return 2;
+  return waves(4) <= 4608 ? 4 : 0;
+}
+
+// The work list and patch records of a step on short row segments.
+int build_segments(pc_pool* p) {
+  CHK(segment_estimates(p));
+  p->seg_solver = p->solver;
+  p->seg_rows = choose_seg_rows(p);
+  p->nstasks = 0;
+  if (!p->seg_rows) return PC_OK;
+  std::vector<PatchDev> pd(p->slots.size());
+  for (int i : p->h_live) pd[i] = make_patchdev(p->slots[i]);
+  // segments by scenario, each scenario's list padded to whole workgroups
+  const int nscn = (int)p->scn.size();
+  std::vector<std::vector<int>> by_scn(nscn);
+  for (size_t k = 0; k < p->h_tasks.size(); ++k)
+    by_scn[pd[p->h_plist[p->h_tasks[k].first]].scn].push_back((int)k);
+  std::vector<Task> st;
+  std::vector<SegRange> ranges(std::max(nscn, 1));
+  std::vector<SegDesc> desc(p->h_plist.size());
+  for (int s = 0; s < nscn; ++s) {
+    ranges[s].first = (int)st.size() / kSegWaves;
+    for (int ti : by_scn[s]) {
+      const Task& t = p->h_tasks[ti];
+      const int n = seg_count(t.nx, p->seg_rows);
+      for (int k = 0; k < n; ++k) {
+        Task u = t;
+        u.r0 = seg_first_row(k, t.nx, n);
+        u.r1 = seg_first_row(k + 1, t.nx, n) - 1;
+        u.sidx = k;
+        u.scn = s;
+        st.push_back(u);
+      }
+    }
+    while (st.size() % kSegWaves) {
+      Task u = st.back();
+      u.nseg = 0;
+      st.push_back(u);
+    }
+    ranges[s].last = (int)st.size() / kSegWaves;
+  }
+  for (size_t k = 0; k < desc.size(); ++k) {
+    const int i = p->h_plist[k];
+    const PatchDev& P = pd[i];
+    const SideDev& sd = p->h_sides[i];
+    SegDesc& D = desc[k];
+    D.off = P.off;
+    D.nx = P.nx;
+    D.ny = P.ny;
+    D.stride = P.stride;
+    D.neg = 0;
+    D.slot = i;
+    D.scn = P.scn;
+    D.dx = P.dx; D.dy = P.dy; D.dxinv = P.dxinv; D.dyinv = P.dyinv;
+    for (int side = 0; side < 4; ++side) {
+      const int upper = side & 1;
+      // the row or column whose cells are the ghosts, and its tile (a
+      // neighbour has the same size and stride)
+      long long off = P.off;
+      int at = side < 2 ? (upper ? P.nx + 1 : 0) : (upper ? P.ny + 1 : 0);
+      if (sd.kind[side] == kSideNeighbour) {
+        off = pd[sd.src[side]].off;
+        at = upper ? 1 : (side < 2 ? P.nx : P.ny);
+      } else if (sd.kind[side] == kSideWall) {
+        at = upper ? (side < 2 ? P.nx : P.ny) : 1;
+        D.neg |= 1 << side;
+      }
+      if (side < 2)
+        D.gx[upper] = off + (long long)at * P.stride;
+      else
+        D.gy[upper] = off + at;
+    }
+  }
+  p->nstasks = (int)st.size();
+  p->nsegdesc = (int)desc.size();
+  CHK(ensure_dev(&p->d_stasks, &p->stasks_cap, st.size()));
+  CHK(ensure_dev(&p->d_segdesc, &p->segdesc_cap, desc.size()));
+  CHK(ensure_dev(&p->d_ranges, &p->ranges_cap, ranges.size()));
+  CHK(ensure_dev(&p->d_cfl_block, &p->cfl_block_cap, st.size() / kSegWaves));
+  CHK(ensure_dev(&p->d_smax_seg, &p->smax_seg_cap, p->slots.size() * kSegSlots));
+  HIPCHK(hipMemcpyAsync(p->d_stasks, st.data(), st.size() * sizeof(Task), hipMemcpyHostToDevice,
+                        p->stream));
+  HIPCHK(hipMemcpyAsync(p->d_segdesc, desc.data(), desc.size() * sizeof(SegDesc),
+                        hipMemcpyHostToDevice, p->stream));
+  HIPCHK(hipMemcpyAsync(p->d_ranges, ranges.data(), ranges.size() * sizeof(SegRange),
+                        hipMemcpyHostToDevice, p->stream));
+  HIPCHK(hipStreamSynchronize(p->stream));  // the host vectors end here
+  return PC_OK;
+}
+
 // Work list: tasks of same-size patches of one scenario, large sizes first.
 int rebuild_topology(pc_pool* p) {
   if (!p->topo_dirty) return PC_OK;
+  CHK(segment_estimates(p));  // from the old lists
   const int ns = (int)p->slots.size();
   std::vector<PatchDev> pd(std::max(ns, 1));
   for (int i = 0; i < ns; ++i)
@@ -641,6 +795,7 @@ int rebuild_topology(pc_pool* p) {
       HIPCHK(hipMemcpyAsync(p->d_bdesc, bdv.data(), bdv.size() * sizeof(BoundaryDesc),
                             hipMemcpyHostToDevice, p->stream));
   }
+  CHK(build_segments(p));
   CHK(ensure_dev(&p->d_live, &p->live_cap, std::max<size_t>(live.size(), 1)));
   if (!live.empty())
     HIPCHK(hipMemcpyAsync(p->d_live, live.data(), live.size() * sizeof(int),
@@ -659,6 +814,7 @@ int rebuild_topology(pc_pool* p) {
 int prepare(pc_pool* p) {
   CHK(sync_scn_host(p));
   CHK(rebuild_topology(p));
+  if (p->seg_solver != p->solver) CHK(build_segments(p));  // its line is the solver's
   if (p->scn_dev_dirty) CHK(upload_scn(p));
   return PC_OK;
 }
@@ -674,8 +830,11 @@ EdgeBufs edges_of(pc_pool* p) {
 // Everything the batched step needs that is derived from the current
 // state: edge buffers (after uploads / per-patch calls), and in fused mode
 // the interior speed maxima of the current state.
-int prepare_batched(pc_pool* p) {
+int prepare_batched(pc_pool* p, bool march = false) {
   CHK(prepare(p));
+  p->uploaded = false;
+  // a step on short row segments reads the tiles alone
+  if (p->seg_rows && !march) return PC_OK;
   if (p->sides_any && p->edges_dirty && !p->h_live.empty()) {
     hipLaunchKernelGGL(k_edges_init, dim3((unsigned)p->h_live.size()), dim3(64), 0, p->stream,
                        p->d_live, (int)p->h_live.size(), p->d_pd, fields_of(p), p->d_scn,
@@ -697,9 +856,56 @@ int prepare_batched(pc_pool* p) {
   return PC_OK;
 }
 
+template <int R, int SOLVER>
+void launch_segments(pc_pool* p, Fields F, hipEvent_t eb, hipEvent_t ee) {
+  const unsigned g = (unsigned)(p->nstasks / kSegWaves);
+  hipLaunchKernelGGL((k_seg_speed<R, SOLVER>), dim3(g), dim3(64 * kSegWaves), 0, p->stream,
+                     p->d_stasks, p->d_segdesc, F, p->d_scn, p->d_smax_seg, p->d_cfl_block);
+  if (eb) hipEventRecord(eb, p->stream);
+  hipLaunchKernelGGL((k_seg_update<R, SOLVER>), dim3(g + 1), dim3(64 * kSegWaves), 0,
+                     p->stream, p->d_stasks, p->d_segdesc, F, p->d_scn, p->d_scn_alt,
+                     (int)p->scn.size(), p->d_ranges, p->d_cfl_block);
+  if (ee) hipEventRecord(ee, p->stream);
+  std::swap(p->d_scn, p->d_scn_alt);
+  std::swap(p->scn_cap, p->scn_alt_cap);
+}
+
+template <int R>
+void launch_segments(pc_pool* p, Fields F, hipEvent_t eb, hipEvent_t ee) {
+  if (p->solver)
+    launch_segments<R, 1>(p, F, eb, ee);
+  else
+    launch_segments<R, 0>(p, F, eb, ee);
+}
+
+// A step on short row segments: exact speeds, then dt and update, straight
+// from the tiles.  The edge buffers and interior maxima of the row march are left
+// behind.
+int launch_seg_step(pc_pool* p, hipEvent_t eb, hipEvent_t ee) {
+  const Fields F = fields_of(p);
+  if (p->nstrips > 0)
+    hipLaunchKernelGGL(k_gather, dim3((p->nstrips + 3) / 4), dim3(256), 0, p->stream,
+                       p->d_strips, p->nstrips, p->d_pd, F, p->d_scn);
+  if (p->seg_rows == 1)
+    launch_segments<1>(p, F, eb, ee);
+  else if (p->seg_rows == 2)
+    launch_segments<2>(p, F, eb, ee);
+  else
+    launch_segments<4>(p, F, eb, ee);
+  HIPCHK(hipGetLastError());
+  p->edges_dirty = true;
+  p->fused_ready = false;
+  p->est_in_segments = true;
+  return PC_OK;
+}
+
 // One step: [ghost strips] -> CFL speeds -> dt -> update.
 int launch_step(pc_pool* p, bool timed_update, hipEvent_t eb = nullptr,
                 hipEvent_t ee = nullptr) {
+  if (p->seg_rows)
+    return launch_seg_step(p, timed_update ? (eb ? eb : p->ev2) : nullptr,
+                           timed_update ? (ee ? ee : p->ev3) : nullptr);
+  p->est_in_segments = false;
   Fields F = fields_of(p);
   EdgeBufs E = edges_of(p);
   const SideDev* sides = p->sides_any ? p->d_sides : nullptr;
@@ -873,7 +1079,9 @@ int pc_pool_destroy(pc_pool* p) {
                   p->d_plist, p->d_plist_scn, p->d_scn_of, p->d_live, p->d_bdesc, p->d_strips,
                   p->d_counter, p->d_iota, p->d_segmax, p->d_keep, p->d_result, p->d_aux, p->d_flags, p->d_ebuf[0],
                   p->d_ebuf[1], p->d_bcol, p->d_sides, p->d_single, p->d_single_slot,
-                  p->d_edge_io, p->d_flux, p->d_batch, p->amr_tables};
+                  p->d_edge_io, p->d_flux, p->d_batch, p->amr_tables, p->d_stasks,
+                  p->d_segdesc, p->d_smax_seg, p->d_cfl_block, p->d_ranges,
+                  p->d_scn_alt};
   for (void* q : ptrs)
     if (q) hipFree(q);
   if (p->h_result) hipHostFree(p->h_result);
@@ -1001,6 +1209,7 @@ int pc_patch_get_description(pc_pool* p, int slot, pc_cell_description* out) {
       // pruned speeds: only the scenario minimum is exact
       e = S.est;
     } else if (p->d_est && !p->topo_dirty) {
+      CHK(segment_estimates(p));
       HIPCHK(hipMemcpyAsync(&e, p->d_est + slot, sizeof(double), hipMemcpyDeviceToHost,
                             p->stream));
       HIPCHK(hipStreamSynchronize(p->stream));
@@ -2394,6 +2603,15 @@ int pc_set_row_segments(pc_pool* p, int segments) {
   return PC_OK;
 }
 
+// The captured step still describes the pool: its lists, the clocks on the
+// device and (row march) what the march derives from the state.
+static bool graph_usable(const pc_pool* p) {
+  if (p->topo_dirty || !p->graph_valid || p->scn_dev_dirty) return false;
+  if (p->seg_rows) return !(p->sides_any && p->uploaded);
+  return !(p->sides_any && p->edges_dirty) &&
+         !(fused_mode(p) && p->sides_any && !p->fused_ready);
+}
+
 static void mark_batched_clock(pc_pool* p) {
   for (int s : p->h_live) p->slots[s].clock_from_scenario = true;
 }
@@ -2403,26 +2621,31 @@ int pc_step_all(pc_pool* p, int k) {
   hipSetDevice(p->device);
   CHK(prepare_batched(p));
   // one event pair around every update launch: the update kernel's mean
-  // duration over exactly these k steps
-  while (p->upd_ev.size() < 2 * (size_t)k) {
+  // duration over exactly these k steps.  On short row segments around the
+  // last one only: a pair leaves the GPU idle for about 8 us, half of such a
+  // step.
+  const int first = p->seg_rows && k > 0 ? k - 1 : 0;
+  while (p->upd_ev.size() < 2 * (size_t)(k - first)) {
     hipEvent_t e;
     HIPCHK(hipEventCreate(&e));
     p->upd_ev.push_back(e);
   }
   HIPCHK(hipEventRecord(p->ev0, p->stream));
-  for (int i = 0; i < k; ++i) CHK(launch_step(p, true, p->upd_ev[2 * i], p->upd_ev[2 * i + 1]));
+  for (int i = 0; i < first; ++i) CHK(launch_step(p, false));
+  for (int i = 0; i < k - first; ++i)
+    CHK(launch_step(p, true, p->upd_ev[2 * i], p->upd_ev[2 * i + 1]));
   HIPCHK(hipEventRecord(p->ev1, p->stream));
   HIPCHK(hipEventSynchronize(p->ev1));
   HIPCHK(hipEventElapsedTime(&p->last_total_ms, p->ev0, p->ev1));
   p->last_update_ms = 0.f;
   if (k > 0 && p->ntasks > 0) {
     double sum = 0.0;
-    for (int i = 0; i < k; ++i) {
+    for (int i = 0; i < k - first; ++i) {
       float ms = 0.f;
       HIPCHK(hipEventElapsedTime(&ms, p->upd_ev[2 * i], p->upd_ev[2 * i + 1]));
       sum += ms;
     }
-    p->last_update_ms = (float)(sum / k);
+    p->last_update_ms = (float)(sum / (k - first));
   }
   p->scn_host_stale = true;
   mark_batched_clock(p);
@@ -2434,7 +2657,7 @@ int pc_step_all_per_patch(pc_pool* p, int k) {
   hipSetDevice(p->device);
   const int fused = p->fused;
   p->fused = 0;  // the plain form computes every patch's CFL step separately
-  int rc = prepare_batched(p);
+  int rc = prepare_batched(p, true);
   p->fused = fused;
   if (rc != PC_OK) return rc;
   // per-patch tasks (one patch per launch)
@@ -2459,6 +2682,7 @@ int pc_step_all_per_patch(pc_pool* p, int k) {
   EdgeBufs E = edges_of(p);
   const SideDev* sides = p->sides_any ? p->d_sides : nullptr;
   const int nscn = (int)p->scn.size();
+  p->est_in_segments = false;
   HIPCHK(hipEventRecord(p->ev0, p->stream));
   for (int it = 0; it < k; ++it) {
     // ghost fill of tile-side patches, one launch per destination patch
@@ -2491,6 +2715,7 @@ int pc_step_all_per_patch(pc_pool* p, int k) {
   p->last_update_ms = 0.f;
   p->scn_host_stale = true;
   p->fused_ready = false;
+  p->uploaded = fused_mode(p) != 0;  // a captured fused step needs a fresh start
   mark_batched_clock(p);
   return PC_OK;
 }
@@ -2543,6 +2768,13 @@ int pc_graph_capture(pc_pool* p) {
   hipSetDevice(p->device);
   CHK(prepare_batched(p));
   CHK(invalidate_graph(p));
+  if (p->seg_rows) {
+    // nothing to capture: the two kernels of such a step are launched again
+    // by the replay.  Between two graph launches the GPU idles 5-8 us, more
+    // than half of a small step; between two kernel launches it does not.
+    p->graph_valid = true;
+    return PC_OK;
+  }
   HIPCHK(hipStreamSynchronize(p->stream));
   HIPCHK(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
   int rc = launch_step(p, false);
@@ -2559,12 +2791,14 @@ int pc_graph_capture(pc_pool* p) {
 int pc_graph_replay(pc_pool* p, int k) {
   if (!p || k < 0) return fail(PC_E_INVALID, "invalid argument");
   hipSetDevice(p->device);
-  if (p->topo_dirty || !p->graph_valid || p->scn_dev_dirty ||
-      (p->sides_any && p->edges_dirty) || (fused_mode(p) && p->sides_any && !p->fused_ready))
+  if (!graph_usable(p))
     return fail(PC_E_INVALID, "no valid captured graph (grid, scenarios or state changed)");
   CHK(sync_scn_host(p));
   HIPCHK(hipEventRecord(p->ev0, p->stream));
-  for (int i = 0; i < k; ++i) HIPCHK(hipGraphLaunch(p->gexec, p->stream));
+  if (p->seg_rows)
+    for (int i = 0; i < k; ++i) CHK(launch_step(p, false));
+  else
+    for (int i = 0; i < k; ++i) HIPCHK(hipGraphLaunch(p->gexec, p->stream));
   HIPCHK(hipEventRecord(p->ev1, p->stream));
   HIPCHK(hipEventSynchronize(p->ev1));
   HIPCHK(hipEventElapsedTime(&p->last_total_ms, p->ev0, p->ev1));

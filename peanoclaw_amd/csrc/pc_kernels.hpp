@@ -142,6 +142,7 @@ struct Task {
   // row segment: the task finalises interior rows r0..r1 (r1 = 0: nx) of its
   // patches; segment sidx of the patch's row segments (see seg_first_row)
   int r0 = 1, r1 = 0, sidx = 0;
+  int scn = 0;  // scenario of its patches (short row segments only)
 };
 
 // Row segments of a patch: a launch with fewer tasks than the GPU holds

@@ -1,0 +1,463 @@
+// Short row segments of the batched step: the speed pass and the update of a
+// step with too few patches to fill the GPU by marching.
+//
+// Such a step is bound by latency, not by HBM: a wavefront of the row march
+// (pc_kernels.hpp) walks at least 8 rows one after another, a dependent chain
+// of FP64 operations per row and one row of loads in flight, after a chain of
+// about ten dependent descriptor loads.  Here a wavefront takes at most R
+// rows of its patches (R a template parameter), issues the loads of all its
+// rows at once, and does all its edges as straight-line code, so the chains
+// of the rows overlap; everything a patch needs besides its cells is in one
+// record (SegDesc).  The x-edges between two segments are solved by both
+// (the same operands, so the same bits).  The step is two launches, exact
+// speeds and update; the update takes its dt from the speed pass's block
+// minima itself, so there is no reduction launch and none for a fallback.
+// 9 x 9 patches of 16^2, f-wave: 34.7 -> 14.1 us a step (speeds 5.4, update
+// 5.6, the rest launches; five launches before, update 16.9); 24 x 24 of
+// 32^2: 40.6 -> 30.3 us; 16 x 16 of 32^2, augmented: 182 -> 57 us.
+//
+// Results are those of the row march bit for bit: the same operations per
+// edge and the same order of accumulation per cell (x-left, x-right, y-up,
+// y-down).
+#pragma once
+
+#include "pc_kernels.hpp"
+
+namespace pcamd {
+
+// Everything the segment kernels read of a patch besides its cells.
+//   gx[s]: index of column 0 of the row across x side s: the neighbour's
+//          boundary row, the own boundary row (wall) or the own ghost row;
+//   gy[s]: index, in row 0, of the cell across y side s (row r: + r stride);
+//   neg:   bit k set: side k (x-, x+, y-, y+) is a wall, its normal momentum
+//          negated.
+struct SegDesc {
+  long long off;
+  long long gx[2];
+  long long gy[2];
+  int nx, ny, stride, neg;
+  int slot, scn;
+  double dx, dy, dxinv, dyinv;
+};
+
+// Slots per patch of the segments' speed maxima (nx <= 64 rows).
+constexpr int kSegSlots = 64;
+constexpr int kSegWaves = 4;  // wavefronts (independent tasks) per workgroup
+constexpr double kNoLimit = 1.7976931348623157e308;
+
+// Segments of a patch with nx rows, at most R rows each.
+__host__ __device__ __forceinline__ int seg_count(int nx, int R) { return (nx + R - 1) / R; }
+
+// Net updates of one f-wave edge of two wet cells before they are handed to
+// the cells on its sides.
+struct WetEdge {
+  double s1, s2, b1, b2;
+};
+
+__device__ __forceinline__ WetEdge wet_edge(const CellQ& L, const CellQ& R) {
+  WetEdge e;
+  wave_speeds_wet(L, R, e.s1, e.s2);
+  const double d0 = R.q - L.q;
+  const double d1 = (R.f - L.f) + (kHalfG * (L.h + R.h)) * (R.b - L.b);
+  const double inv = div_nr(1.0, e.s2 - e.s1);
+  e.b1 = (e.s2 * d0 - d1) * inv;
+  e.b2 = (d1 - e.s1 * d0) * inv;
+  return e;
+}
+
+// The edge's four shares.  `sub`: every edge of the wavefront is subsonic
+// (wave 1 goes left, wave 2 right); the signs of zeros that may differ from
+// the general sums do not reach a cell (see edge_solve_wet).
+__device__ __forceinline__ void wet_shares(const WetEdge& e, bool sub, double& dhL, double& dhR,
+                                           double& dqL, double& dqR) {
+  const double z1 = e.b1 * e.s1, z2 = e.b2 * e.s2;
+  if (sub) {
+    dhL = e.b1; dqL = z1; dhR = e.b2; dqR = z2;
+    return;
+  }
+  double a = 0.0, b = 0.0, c = 0.0, d = 0.0;
+  if (e.s1 < -kZeroTol) {
+    a += e.b1; c += z1;
+  } else if (e.s1 > kZeroTol) {
+    b += e.b1; d += z1;
+  } else {
+    a += 0.5 * e.b1; c += 0.5 * z1;
+    b += 0.5 * e.b1; d += 0.5 * z1;
+  }
+  if (e.s2 < -kZeroTol) {
+    a += e.b2; c += z2;
+  } else if (e.s2 > kZeroTol) {
+    b += e.b2; d += z2;
+  } else {
+    a += 0.5 * e.b2; c += 0.5 * z2;
+    b += 0.5 * e.b2; d += 0.5 * z2;
+  }
+  dhL = a; dhR = b; dqL = c; dqR = d;
+}
+
+__device__ __forceinline__ CellQ left_cell(const CellQ& c) {
+  CellQ l;
+  l.h = from_left(c.h); l.q = from_left(c.q); l.b = from_left(c.b);
+  l.u = from_left(c.u); l.sq = from_left(c.sq); l.c = from_left(c.c);
+  l.f = from_left(c.f);
+  return l;
+}
+
+// The rows of one wavefront and the lanes' places in them.
+struct SegLane {
+  int ra, rb, rows;      // interior rows ra..rb of the patch
+  int seg, col;          // patch of the task, 1-based interior column
+  bool segok, active;
+};
+
+__device__ __forceinline__ SegLane seg_lane(const Task& t) {
+  SegLane g;
+  const int lane = threadIdx.x & 63;
+  const int W = pow2ceil(t.ny);
+  g.ra = t.r0;
+  g.rb = t.r1;
+  g.rows = t.r1 - t.r0 + 1;
+  g.seg = lane / W;
+  g.col = lane - g.seg * W + 1;
+  g.segok = g.seg < t.nseg;
+  g.active = g.segok && g.col <= t.ny;
+  return g;
+}
+
+// Cells of rows ra-1 .. ra+R of the lane's column (rows past rb+1 and lanes
+// without a cell: a wet cell at rest).  hv of a ghost row is not used.
+template <int R, bool B>
+struct SegRows {
+  double h[R + 2], hu[R + 2], hv[R + 2], b[R + 2];
+  __device__ __forceinline__ void load(const SegDesc& D, const SegLane& g, const double* H,
+                                       const double* HU, const double* HV, const double* Bf,
+                                       int last) {
+#pragma unroll
+    for (int k = 0; k < R + 2; ++k) {
+      h[k] = 1.0; hu[k] = 0.0; hv[k] = 0.0; b[k] = 0.0;
+      const int r = g.ra - 1 + k;
+      if (!g.active || r > last) continue;
+      const long long i = D.off + (long long)r * D.stride + g.col;
+      const long long j = r == 0 ? D.gx[0] + g.col : (r == D.nx + 1 ? D.gx[1] + g.col : i);
+      h[k] = gl(H + j);
+      hu[k] = gl(HU + j);
+      hv[k] = gl(HV + j);
+      if (B) b[k] = gl(Bf + i);
+    }
+#pragma unroll
+    for (int k = 0; k < R + 2; ++k) {
+      const int r = g.ra - 1 + k;
+      if ((r == 0 && (D.neg & 1)) || (r == D.nx + 1 && (D.neg & 2))) hu[k] = -hu[k];
+    }
+  }
+};
+
+// The y-edges that touch the ghost columns, two per row and patch, one per
+// lane: entry e is side e & 1 of row ra + (e >> 1) % rows of patch
+// (e >> 1) / rows.
+struct SegSide {
+  int slot, side;
+  double hL, hvL, bL, hR, hvR, bR, dyinv;
+  template <bool B>
+  __device__ __forceinline__ void load(const SegDesc* __restrict__ desc, const Task& t,
+                                       const SegLane& g, int e, const double* H,
+                                       const double* HV, const double* Bf) {
+    side = e & 1;
+    const int s = (e >> 1) / g.rows;
+    const int row = g.ra + (e >> 1) - s * g.rows;
+    slot = e >> 1;
+    const SegDesc Q = gl(desc + t.first + s);
+    dyinv = Q.dyinv;
+    const long long at = Q.off + (long long)row * Q.stride;
+    const long long io = at + (side ? Q.ny : 1);
+    const long long ig = (side ? Q.gy[1] : Q.gy[0]) + (long long)row * Q.stride;
+    const double ho = gl(H + io), hvo = gl(HV + io);
+    double hg = gl(H + ig), hvg = gl(HV + ig);
+    if (Q.neg & (side ? 8 : 4)) hvg = -hvg;
+    const double bo = B ? gl(Bf + io) : 0.0;
+    const double bg = B ? gl(Bf + at + (side ? Q.ny + 1 : 0)) : 0.0;
+    hL = side ? ho : hg; hvL = side ? hvo : hvg; bL = side ? bo : bg;
+    hR = side ? hg : ho; hvR = side ? hvg : hvo; bR = side ? bg : bo;
+  }
+};
+
+// Minimum of v over the workgroup (every thread calls it), in thread 0.
+__device__ __forceinline__ double block_min(double v, double* red) {
+  for (int o = 32; o >= 1; o >>= 1) v = dmin(v, __shfl_xor(v, o));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int k = 1; k < (int)blockDim.x / 64; ++k) v = dmin(v, red[k]);
+  return v;
+}
+
+// Exact edge speeds of the current state: one maximum per row segment in
+// smax_seg[slot * kSegSlots + segment] (for the patches' own estimates), and
+// per workgroup the smallest CFL step of its segments.  The CFL step falls
+// with the speed, so the minimum over segments is the minimum over patches.
+template <int R, int SOLVER>
+__global__ void __launch_bounds__(64 * kSegWaves)
+k_seg_speed(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
+            const ScnDev* __restrict__ scn, double* __restrict__ smax_seg,
+            double* __restrict__ cfl_block) {
+  using ES = EdgeSolver<SOLVER>;
+  constexpr bool B = SOLVER != 0;  // the f-wave's speeds do not depend on b
+  __shared__ double pre[kSegWaves][2][64];
+  __shared__ double red[kSegWaves];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
+  const SegLane g = seg_lane(t);
+  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
+  const int par = gl(&scn[t.scn].stepc) & 1;
+  const double *H = F.H(par), *HU = F.HU(par), *HV = F.HV(par);
+  // the edge below the last row belongs to the next segment
+  const int last = g.rb == t.nx ? g.rb + 1 : g.rb;
+  SegRows<R, B> q;
+  q.load(D, g, H, HU, HV, F.b, last);
+  const int npre = t.nseg * g.rows * 2;
+  for (int e = lane; e < npre; e += 64) {
+    SegSide s;
+    s.load<B>(desc, t, g, e, H, HV, F.b);
+    const CellQ cl = cell_dir(cell_base(s.hL, s.bL), s.hvL);
+    const CellQ cr = cell_dir(cell_base(s.hR, s.bR), s.hvR);
+    pre[w][s.side][s.slot] = ES::speed(cl, cr);
+  }
+  CellBase cb[R + 2];
+  CellQ cx[R + 2];
+  bool wet = true;
+#pragma unroll
+  for (int k = 0; k < R + 2; ++k) {
+    cb[k] = cell_base(q.h[k], q.b[k]);
+    cx[k] = cell_dir(cb[k], q.hu[k]);
+    wet = wet && q.h[k] >= kDryTol;
+  }
+  double sm = 0.0;
+  if (SOLVER == 0 && wave_all(wet)) {
+#pragma unroll
+    for (int k = 1; k < R + 2; ++k) {
+      const double sx = edge_speed_wet(cx[k - 1], cx[k]);
+      if (g.ra - 1 + k <= last) sm = dmax(sm, sx);
+      if (k > R) break;
+      const CellQ cy = cell_dir(cb[k], q.hv[k]);
+      const double sy = edge_speed_wet(left_cell(cy), cy);
+      if (g.col >= 2 && k <= g.rows) sm = dmax(sm, sy);
+    }
+  } else {
+#pragma unroll
+    for (int k = 1; k < R + 2; ++k) {
+      if (g.ra - 1 + k <= last) sm = dmax(sm, ES::speed(cx[k - 1], cx[k]));
+      if (k > R || k > g.rows) continue;
+      const CellQ cy = cell_dir(cb[k], q.hv[k]);
+      const double sy = ES::speed(left_cell(cy), cy);
+      if (g.col >= 2) sm = dmax(sm, sy);
+    }
+  }
+  wave_sync();
+  if (g.active && (g.col == 1 || g.col == t.ny))
+    for (int k = 0; k < g.rows; ++k) {
+      if (g.col == 1) sm = dmax(sm, pre[w][0][g.seg * g.rows + k]);
+      if (g.col == t.ny) sm = dmax(sm, pre[w][1][g.seg * g.rows + k]);
+    }
+  double v = g.active ? sm : 0.0;
+  for (int m = pow2ceil(t.ny) >> 1; m >= 1; m >>= 1) v = dmax(v, __shfl_xor(v, m));
+  if (g.segok && g.col == 1) gs(smax_seg + (long long)D.slot * kSegSlots + t.sidx, v);
+  const double c = block_min(g.segok ? max_timestep(v, D.dx, D.dy) : kNoLimit, red);
+  if (threadIdx.x == 0) gs(cfl_block + blockIdx.x, c);
+}
+
+// Every patch's own CFL step from its segments' speed maxima.
+__global__ void __launch_bounds__(64)
+k_seg_estimates(const SegDesc* __restrict__ desc, int n, int R,
+                const double* __restrict__ smax_seg, double* __restrict__ est) {
+  const int k = blockIdx.x * 64 + threadIdx.x;
+  if (k >= n) return;
+  const SegDesc D = gl(desc + k);
+  double s = 0.0;
+  for (int j = 0; j < seg_count(D.nx, R); ++j)
+    s = dmax(s, gl(smax_seg + (long long)D.slot * kSegSlots + j));
+  est[D.slot] = max_timestep(s, D.dx, D.dy);
+}
+
+// Blocks [first, last) of the segment kernels hold the tasks of a scenario.
+struct SegRange {
+  int first, last;
+};
+
+// This thread's share of a scenario's CFL step: the minimum over every
+// `stride`-th of its blocks from the `at`-th on.
+__device__ __forceinline__ double cfl_share(const SegRange& r,
+                                            const double* __restrict__ cfl_block, int at,
+                                            int stride) {
+  double v = kNoLimit;
+  for (int k = r.first + at; k < r.last; k += stride) v = dmin(v, gl(cfl_block + k));
+  for (int o = 32; o >= 1; o >>= 1) v = dmin(v, __shfl_xor(v, o));
+  return v;
+}
+
+// The update of the same segments, current state -> other state.  Every
+// workgroup takes its scenario's step from the blocks' minima and the clock
+// `in`; the last workgroup advances the clocks of all scenarios into `out`
+// (the next step's `in`), so no launch is needed between the speeds and the
+// update.
+template <int R, int SOLVER>
+__global__ void __launch_bounds__(64 * kSegWaves)
+__attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
+k_seg_update(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
+             const ScnDev* __restrict__ in, ScnDev* __restrict__ out, int nscn,
+             const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block) {
+  using ES = EdgeSolver<SOLVER>;
+  __shared__ double pre[kSegWaves][4][64];
+  __shared__ double red[kSegWaves];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (blockIdx.x == gridDim.x - 1) {
+    for (int s = w; s < nscn; s += kSegWaves) {
+      const double cfl = cfl_share(gl(ranges + s), cfl_block, lane, 64);
+      if (lane == 0) {
+        ScnDev S = in[s];
+        dt_final_one(S, cfl, 0, nullptr, 1.0);
+        out[s] = S;
+      }
+    }
+    return;
+  }
+  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
+  const SegLane g = seg_lane(t);
+  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
+  const ScnDev* S = in + t.scn;  // one scenario per workgroup
+  const double max_dt = gl(&S->end_time) - (gl(&S->time) + gl(&S->dt));
+  if (!(max_dt - 0.0 > kLaEps)) return;
+  const int par = gl(&S->stepc) & 1;
+  const double *H = F.H(par), *HU = F.HU(par), *HV = F.HV(par);
+  SegRows<R, true> q;
+  q.load(D, g, H, HU, HV, F.b, g.rb + 1);
+  const double share = cfl_share(gl(ranges + t.scn), cfl_block, (int)threadIdx.x,
+                                 64 * kSegWaves);
+  if (lane == 0) red[w] = share;
+  const int npre = t.nseg * g.rows * 2;
+  for (int e = lane; e < npre; e += 64) {
+    SegSide s;
+    s.load<true>(desc, t, g, e, H, HV, F.b);
+    const CellQ cl = cell_dir(cell_base(s.hL, s.bL), s.hvL);
+    const CellQ cr = cell_dir(cell_base(s.hR, s.bR), s.hvR);
+    double dhL, dhR, dqL, dqR;
+    ES::solve(cl, cr, dhL, dhR, dqL, dqR);
+    // side 0: the right cell (row,1) takes the "upwards" part;
+    // side 1: the left cell (row,ny) takes the "downwards" part.
+    pre[w][s.side * 2 + 0][s.slot] = s.dyinv * (s.side ? dhL : dhR);
+    pre[w][s.side * 2 + 1][s.slot] = s.dyinv * (s.side ? dqL : dqR);
+  }
+  __syncthreads();
+  double dt = max_dt;
+  for (int k = 0; k < kSegWaves; ++k) dt = fmin(red[k], dt);
+  if (t.nseg == 0) return;
+  bool wet = true;
+#pragma unroll
+  for (int k = 0; k < R + 2; ++k) wet = wet && q.h[k] >= kDryTol;
+  const bool fast = SOLVER == 0 && wave_all(wet);
+  const unsigned long long col1 = __builtin_amdgcn_ballot_w64(g.col == 1);
+  const double dxinv = D.dxinv, dyinv = D.dyinv;
+  double* const Hd = F.H(1 - par);
+  double* const HUd = F.HU(1 - par);
+  double* const HVd = F.HV(1 - par);
+  // Chunks of rows: the edges below the chunk's rows (x-edge k | k+1, y-edges
+  // of row k+1) in straight-line code, one vote, then the rows they complete.
+  // Few rows go in one chunk (most overlap); with more, two by two, for the
+  // registers.
+  constexpr int C = R <= 2 ? R + 1 : 1;
+  CellBase cb = cell_base(q.h[0], q.b[0]);
+  CellQ cx = cell_dir(cb, q.hu[0]);
+  double accH = 0.0, accHu = 0.0, uph = 0.0, upq = 0.0, dnh = 0.0, dnq = 0.0;
+#pragma unroll
+  for (int k0 = 0; k0 <= R; k0 += C) {
+    if (k0 > g.rows) break;
+    double xhL[C], xhR[C], xqL[C], xqR[C], yhL[C], yhR[C], yqL[C], yqR[C];
+    if (fast) {
+      WetEdge ex[C], ey[C];
+      bool sub = true, suby = true;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int k = k0 + c;
+        const CellBase nb = cell_base(q.h[k + 1], q.b[k + 1]);
+        const CellQ nx = cell_dir(nb, q.hu[k + 1]);
+        ex[c] = wet_edge(cx, nx);
+        sub = sub && ex[c].s1 < -kZeroTol && ex[c].s2 > kZeroTol;
+        if (k < R) {
+          const CellQ cy = cell_dir(nb, q.hv[k + 1]);
+          ey[c] = wet_edge(left_cell(cy), cy);
+          suby = suby && ey[c].s1 < -kZeroTol && ey[c].s2 > kZeroTol;
+        }
+        cx = nx;
+      }
+      const bool all = (__builtin_amdgcn_ballot_w64(sub) &
+                        (__builtin_amdgcn_ballot_w64(suby) | col1)) ==
+                       __builtin_amdgcn_read_exec();
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        wet_shares(ex[c], all, xhL[c], xhR[c], xqL[c], xqR[c]);
+        if (k0 + c < R) wet_shares(ey[c], all, yhL[c], yhR[c], yqL[c], yqR[c]);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int k = k0 + c;
+        xhL[c] = xhR[c] = xqL[c] = xqR[c] = 0.0;
+        yhL[c] = yhR[c] = yqL[c] = yqR[c] = 0.0;
+        if (k > g.rows) continue;
+        const CellBase nb = cell_base(q.h[k + 1], q.b[k + 1]);
+        const CellQ nx = cell_dir(nb, q.hu[k + 1]);
+        ES::solve(cx, nx, xhL[c], xhR[c], xqL[c], xqR[c]);
+        if (k < R) {
+          const CellQ cy = cell_dir(nb, q.hv[k + 1]);
+          ES::solve(left_cell(cy), cy, yhL[c], yhR[c], yqL[c], yqR[c]);
+        }
+        cx = nx;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int k = k0 + c;
+      if (k > g.rows) break;
+      if (k >= 1) {
+        // row k: x-left (in acc), x-right, y-up, y-down
+        double nH = accH + dxinv * xhL[c];
+        double nHu = accHu + dxinv * xqL[c];
+        nH = nH + uph;
+        nH = nH + dnh;
+        double nHv = 0.0 + upq;
+        nHv = nHv + dnq;
+        double h1 = q.h[k] - dt * nH;
+        double hu1 = q.hu[k] - dt * nHu;
+        double hv1 = q.hv[k] - dt * nHv;
+        if (h1 < kClampH) { hu1 = 0.0; hv1 = 0.0; }
+        if (h1 < 0.0) h1 = 0.0;
+        if (g.active) {
+          const long long o = D.off + (long long)(g.ra - 1 + k) * D.stride + g.col;
+          gs(Hd + o, h1);
+          gs(HUd + o, hu1);
+          gs(HVd + o, hv1);
+        }
+      }
+      accH = 0.0 + dxinv * xhR[c];
+      accHu = 0.0 + dxinv * xqR[c];
+      if (k < R) {
+        // shares of the y-edges of row k + 1; the lower neighbour's is
+        // handed down one lane
+        uph = dyinv * yhR[c];
+        upq = dyinv * yqR[c];
+        dnh = from_right(dyinv * yhL[c]);
+        dnq = from_right(dyinv * yqL[c]);
+        const int slot = g.seg * g.rows + k;
+        if (k < g.rows && g.active && g.col == 1) {
+          uph = pre[w][0][slot];
+          upq = pre[w][1][slot];
+        }
+        if (k < g.rows && g.active && g.col == t.ny) {
+          dnh = pre[w][2][slot];
+          dnq = pre[w][3][slot];
+        }
+      }
+    }
+  }
+}
+
+}  // namespace pcamd

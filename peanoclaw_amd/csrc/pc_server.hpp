@@ -341,10 +341,7 @@ int pc_server_round(pc_server* s, int steps, int* active_out, int* queued_out) {
     // sequence: replay it as a captured graph (state read on the device);
     // after a change, one plain step applies it and the graph is captured
     // again.
-    const bool replay = !p->topo_dirty && p->graph_valid && !p->scn_dev_dirty &&
-                        !(p->sides_any && p->edges_dirty) &&
-                        !(fused_mode(p) && p->sides_any && !p->fused_ready);
-    if (replay) {
+    if (graph_usable(p)) {
       CHK(pc_graph_replay(p, steps));
     } else {
       CHK(pc_step_all(p, 1));
