@@ -11,22 +11,23 @@
 // (GhostlayerCompositorFunctors.cpp:59-69; SWEKernel.cpp:239-286), walls
 // (SolveTimestep.cpp:87-142), the global CFL minimum and solveTimestep of
 // every leaf.  Here the host hands over that plan once (a device-side
-// table rebuilt only when the grid changes) and every step is seven
-// launches, each phase over all patches at once, replayed from a captured
-// graph:
+// table rebuilt only when the grid changes) and every step is three
+// launches over all patches at once:
 //
-//   restrict one thread per virtual-patch cell: the contributions of the
-//            leaves covering it (a per-cell list, in plan order), then
-//            h+b -> h
-//   copy     uNew -> uOld of every leaf
-//   ghosts   one wavefront per face: copy with time factor, or d-linear
-//            interpolation from the coarser leaf (h+b, back to h with the
-//            destination's b)
-//   walls    one workgroup per leaf with domain walls, in call order
-//   speed    exact edge speeds of every leaf (row march over uOld)
-//   dt       global CFL minimum, bounded by the end time
-//   solve    update of every leaf with that step (row march, uOld -> uNew),
-//            then the leaves' clock
+//   restrict the contributions of the leaves covering every virtual-patch
+//            cell, then h+b -> h
+//   fill     one workgroup per task of leaves: uNew -> uOld, the ghost
+//            layer of every face (copy with time factor, or d-linear
+//            interpolation from the coarser leaf: h+b, back to h with the
+//            destination's b), the walls in call order, then the exact edge
+//            speeds of the leaves and the smallest CFL step of the workgroup
+//   update   of every leaf, uOld -> uNew, with the smallest of those steps
+//            bounded by the end time; one workgroup advances the clock
+//
+// These grids hold a few hundred thousand cells, so latency bounds them: the
+// fill loads a leaf's cells once for the copy and the speeds, and neither
+// the copy, the walls nor the reduction of dt is a launch of its own.  The
+// launches are issued one by one: graph launches left 5-8 us between steps.
 //
 // Every phase first checks the step bound end_time - (time + dt); a step
 // past the end time does nothing.
@@ -41,13 +42,15 @@
 
 #include <unordered_map>
 
+#include "pc_seg_kernels.hpp"
+
 namespace {
 
 struct AmrClock {
   double time, dt;  // the leaves' clock (time, timestep_size)
   double end_time;
   double bound;     // dt of the step being run
-  int advance;      // the step runs (set by the dt phase for the solve)
+  int advance;      // the last step ran
   int pad;
   long long steps;
 };
@@ -108,12 +111,24 @@ struct AmrGhost {
   int kind, src, dst;
   int sx, sy, sox, soy, dox, doy;
   int sn[2];
-  int pad;
+  int cell0;  // its first cell among the ghost cells of its task's leaves
   double spos[2], ssub[2], sinv[2], dpos[2], dsub[2];
 };
 
+// walls[first .. first + count) of a leaf as (dim, upper) pairs
 struct AmrWalls {
-  int slot, first, count, pad;  // walls[first .. first+count) as (dim, upper) pairs
+  int first, count;
+};
+
+// One task of leaves in the fill: its row segments tasks[first .. first +
+// nwaves), its leaves at plist positions [leaf0, leaf0 + nseg), its ghost
+// cells (entry of each in gmap[cell0 .. cell0 + ncells)).
+struct AmrBlock {
+  int first, nwaves, leaf0, nseg;
+  int nx, ny;
+  int cell0, ncells;
+  int nwalls;  // most walls of one of its leaves
+  int pad;
 };
 
 // Restriction time factors of a leaf source on the [0, 1] basis
@@ -241,57 +256,37 @@ k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ cpt
   }
 }
 
-__global__ void __launch_bounds__(256)
-k_amr_copy(const int* __restrict__ leaves, const PatchDev* __restrict__ pd, Fields F, int cur,
-           const AmrClock* clock) {
-  if (!amr_advance(*clock)) return;
-  const PatchDev P = pd[leaves[blockIdx.x]];
-  for (int k = threadIdx.x; k < P.nx * P.ny; k += blockDim.x) {
-    const long long i = tile_index(P, k / P.ny, k - (k / P.ny) * P.ny);
-    F.H(1 - cur)[i] = F.H(cur)[i];
-    F.HU(1 - cur)[i] = F.HU(cur)[i];
-    F.HV(1 - cur)[i] = F.HV(cur)[i];
-  }
-}
-
-// One wavefront per face entry (4 per workgroup).
+// Cell k of a ghost entry.  LTS: every leaf runs on its own clock.  Else all
+// leaves run on (time, dt), and a leaf's uOld is its uNew (copied in the same
+// launch, so not read here).
 template <bool LTS>
-__global__ void __launch_bounds__(256)
-k_amr_ghosts(const AmrGhost* __restrict__ ghosts, int nghosts, const PatchDev* __restrict__ pd,
-             Fields F, int cur, const AmrClock* clock, AmrLts L) {
-  const AmrClock c = *clock;
-  if (!amr_phase_runs<LTS>(clock, L)) return;
-  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (e >= nghosts) return;
-  const int lane = threadIdx.x & 63;
-  const AmrGhost g = ghosts[e];
-  if (LTS && !L.adv[g.dst]) return;
+__device__ __forceinline__ void amr_ghost_cell(const AmrGhost& g, int k,
+                                               const PatchDev* __restrict__ pd, const Fields& F,
+                                               int cur, const AmrClock& c, const AmrLts& L) {
   const PatchDev S = pd[g.src], D = pd[g.dst];
   const int oldSt = 1 - cur;
-  // global steps: every leaf runs on the clock (time, dt); local time
-  // stepping: each leaf on its own
+  const int kind = g.kind;
   const double dTime = LTS ? L.t[g.dst] : c.time, dDt = LTS ? L.dt[g.dst] : c.dt;
-  const double sTime = (LTS && g.kind != kAmrTransferVirtual) ? L.t[g.src] : c.time;
-  const double sDt = (LTS && g.kind != kAmrTransferVirtual) ? L.dt[g.src] : c.dt;
+  const double sTime = (LTS && kind != kAmrTransferVirtual) ? L.t[g.src] : c.time;
+  const double sDt = (LTS && kind != kAmrTransferVirtual) ? L.dt[g.src] : c.dt;
   const double dstTimeUNew = dTime + dDt;
-  if (g.kind != kAmrInterpolate) {
+  const int x = k / g.sy, y = k - (k / g.sy) * g.sy;
+  const long long di = tile_index(D, g.dox + x, g.doy + y);
+  const int srcOld = LTS || kind == kAmrTransferVirtual ? oldSt : cur;
+  if (kind != kAmrInterpolate) {
     // DefaultTransfer.cpph:27-51
     double tf;
-    if (g.kind == kAmrTransferVirtual) {
+    if (kind == kAmrTransferVirtual) {
       tf = (dstTimeUNew - 0.0) / 1.0;
     } else {
       const double sNew = sTime + sDt, sOld = sTime;
       tf = (sNew - sOld - 0.0 > kLaEps) ? (dstTimeUNew - sOld) / (sNew - sOld) : 1.0;
     }
     const double inv = 1.0 - tf;
-    for (int k = lane; k < g.sx * g.sy; k += 64) {
-      const int x = k / g.sy, y = k - (k / g.sy) * g.sy;
-      const long long si = tile_index(S, g.sox + x, g.soy + y);
-      const long long di = tile_index(D, g.dox + x, g.doy + y);
-      F.H(oldSt)[di] = F.H(cur)[si] * tf + F.H(oldSt)[si] * inv;
-      F.HU(oldSt)[di] = F.HU(cur)[si] * tf + F.HU(oldSt)[si] * inv;
-      F.HV(oldSt)[di] = F.HV(cur)[si] * tf + F.HV(oldSt)[si] * inv;
-    }
+    const long long si = tile_index(S, g.sox + x, g.soy + y);
+    F.H(oldSt)[di] = F.H(cur)[si] * tf + F.H(srcOld)[si] * inv;
+    F.HU(oldSt)[di] = F.HU(cur)[si] * tf + F.HU(srcOld)[si] * inv;
+    F.HV(oldSt)[di] = F.HV(cur)[si] * tf + F.HV(srcOld)[si] * inv;
     return;
   }
   // DefaultInterpolation.cpph:45-67 (toCurrentTime = 0, useTimeUNewOrUOld = 1)
@@ -303,58 +298,73 @@ k_amr_ghosts(const AmrGhost* __restrict__ ghosts, int nghosts, const PatchDev* _
     tf = (dstTimeUNew - sOld) / (sNew - sOld);
   }
   tf = dmax(0.0, dmin(1.0, tf));
-  for (int k = lane; k < g.sx * g.sy; k += 64) {
-    const int x = g.dox + k / g.sy, y = g.doy + (k - (k / g.sy) * g.sy);
-    const long long di = tile_index(D, x, y);
-    double acc[3] = {0.0, 0.0, 0.0};
-    double cc[2];
-    cc[0] = g.dpos[0] + g.dsub[0] * (double)x + g.dsub[0] * 0.5;
-    cc[1] = g.dpos[1] + g.dsub[1] * (double)y + g.dsub[1] * 0.5;
-    int si[2];
-    for (int d = 0; d < 2; ++d) {
-      const double base = g.spos[d] + g.ssub[d] * 0.5;
-      const double loc = cc[d] - base;
-      int v = (int)floor(loc * g.sinv[d]);
-      v = v < g.sn[d] - 2 ? v : g.sn[d] - 2;
-      v = v > 0 ? v : 0;
-      si[d] = v;
-    }
-    for (int o = 0; o < 4; ++o) {
-      const int off[2] = {o & 1, (o >> 1) & 1};
-      const int nb[2] = {si[0] + off[0], si[1] + off[1]};
-      double np[2];
-      np[0] = g.spos[0] + g.ssub[0] * (double)nb[0] + g.ssub[0] * 0.5;
-      np[1] = g.spos[1] + g.ssub[1] * (double)nb[1] + g.ssub[1] * 0.5;
-      double sf = 1.0;
-      for (int d = 0; d < 2; ++d) {
-        const double sign = (double)(1 - 2 * off[d]);
-        sf *= 1.0 - (sign * (cc[d] - np[d])) * g.sinv[d];
-      }
-      const long long sidx = tile_index(S, nb[0], nb[1]);
-      const double bv = F.b[sidx];
-      const double vo[3] = {F.H(oldSt)[sidx] + 1.0 * bv, F.HU(oldSt)[sidx], F.HV(oldSt)[sidx]};
-      const double vn[3] = {F.H(cur)[sidx] + 1.0 * bv, F.HU(cur)[sidx], F.HV(cur)[sidx]};
-      for (int q = 0; q < 3; ++q) acc[q] = acc[q] + sf * (vo[q] * (1.0 - tf) + vn[q] * tf);
-    }
-    F.H(oldSt)[di] = acc[0] + (-1.0) * F.b[di];
-    F.HU(oldSt)[di] = acc[1];
-    F.HV(oldSt)[di] = acc[2];
+  double acc[3] = {0.0, 0.0, 0.0};
+  double cc[2];
+  cc[0] = g.dpos[0] + g.dsub[0] * (double)(g.dox + x) + g.dsub[0] * 0.5;
+  cc[1] = g.dpos[1] + g.dsub[1] * (double)(g.doy + y) + g.dsub[1] * 0.5;
+  int si[2];
+  for (int d = 0; d < 2; ++d) {
+    const double base = g.spos[d] + g.ssub[d] * 0.5;
+    const double loc = cc[d] - base;
+    int v = (int)floor(loc * g.sinv[d]);
+    v = v < g.sn[d] - 2 ? v : g.sn[d] - 2;
+    v = v > 0 ? v : 0;
+    si[d] = v;
   }
+  for (int o = 0; o < 4; ++o) {
+    const int off[2] = {o & 1, (o >> 1) & 1};
+    const int nb[2] = {si[0] + off[0], si[1] + off[1]};
+    double np[2];
+    np[0] = g.spos[0] + g.ssub[0] * (double)nb[0] + g.ssub[0] * 0.5;
+    np[1] = g.spos[1] + g.ssub[1] * (double)nb[1] + g.ssub[1] * 0.5;
+    double sf = 1.0;
+    for (int d = 0; d < 2; ++d) {
+      const double sign = (double)(1 - 2 * off[d]);
+      sf *= 1.0 - (sign * (cc[d] - np[d])) * g.sinv[d];
+    }
+    const long long sidx = tile_index(S, nb[0], nb[1]);
+    const double bv = F.b[sidx];
+    const double vo[3] = {F.H(srcOld)[sidx] + 1.0 * bv, F.HU(srcOld)[sidx], F.HV(srcOld)[sidx]};
+    const double vn[3] = {F.H(cur)[sidx] + 1.0 * bv, F.HU(cur)[sidx], F.HV(cur)[sidx]};
+    for (int q = 0; q < 3; ++q) acc[q] = acc[q] + sf * (vo[q] * (1.0 - tf) + vn[q] * tf);
+  }
+  F.H(oldSt)[di] = acc[0] + (-1.0) * F.b[di];
+  F.HU(oldSt)[di] = acc[1];
+  F.HV(oldSt)[di] = acc[2];
 }
 
-// SWEKernel::fillBoundaryLayer (SWEKernel.cpp:176-237) of one leaf, its
-// walls in call order (corner cells read what the previous wall wrote).
-__global__ void __launch_bounds__(64)
-k_amr_walls(const AmrWalls* __restrict__ walls, const int* __restrict__ dims,
-            const PatchDev* __restrict__ pd, Fields F, int cur, const AmrClock* clock) {
-  if (!amr_advance(*clock)) return;
-  const AmrWalls W = walls[blockIdx.x];
-  const PatchDev P = pd[W.slot];
-  const int st = 1 - cur;
-  for (int w = 0; w < W.count; ++w) {
-    const int dim = dims[2 * (W.first + w)], upper = dims[2 * (W.first + w) + 1];
-    const int n_other = dim == 0 ? P.ny : P.nx;
-    for (int k = -1 + (int)threadIdx.x; k < n_other + 1; k += blockDim.x) {
+// Local time stepping: the ghost cells of the advancing leaves, before any
+// leaf changes (one thread per ghost cell of the plan).
+__global__ void __launch_bounds__(256)
+k_lts_ghosts(const unsigned* __restrict__ gmap, const int* __restrict__ gcell0, int ncells,
+             const AmrGhost* __restrict__ ghosts, const PatchDev* __restrict__ pd, Fields F,
+             int cur, const AmrClock* clock, AmrLts L) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= ncells || *L.iter == 0) return;
+  const unsigned e = gmap[c];
+  const AmrGhost& g = ghosts[e];
+  if (!L.adv[g.dst]) return;
+  amr_ghost_cell<true>(g, c - gcell0[e], pd, F, cur, *clock, L);
+}
+
+// SWEKernel::fillBoundaryLayer (SWEKernel.cpp:176-237) of the leaves of a
+// task, their walls in call order (corner cells read what the previous wall
+// wrote); `adv` null: all of them.
+__device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegDesc* __restrict__ desc,
+                                          const AmrWalls* __restrict__ walls,
+                                          const int* __restrict__ dims,
+                                          const PatchDev* __restrict__ pd, const Fields& F,
+                                          int st, const int* adv) {
+  const int len = (K.nx > K.ny ? K.nx : K.ny) + 2;
+  for (int w = 0; w < K.nwalls; ++w) {
+    for (int i = threadIdx.x; i < K.nseg * len; i += blockDim.x) {
+      const int s = i / len, k = i - s * len - 1;
+      const AmrWalls W = walls[K.leaf0 + s];
+      if (w >= W.count) continue;
+      const int dim = dims[2 * (W.first + w)], upper = dims[2 * (W.first + w) + 1];
+      const int slot = desc[K.leaf0 + s].slot;
+      const PatchDev P = pd[slot];
+      if (k >= (dim == 0 ? P.ny : P.nx) + 1 || (adv && !adv[slot])) continue;
       int dx, dy, sx, sy;
       if (dim == 0) {
         dx = upper ? P.nx : -1;
@@ -365,8 +375,8 @@ k_amr_walls(const AmrWalls* __restrict__ walls, const int* __restrict__ dims,
         sy = dy + (upper ? -1 : 1);
         dx = sx = k;
       }
-      const long long d = tile_index(P, dx, dy), s = tile_index(P, sx, sy);
-      const double h = F.H(st)[s], hu = F.HU(st)[s], hv = F.HV(st)[s];
+      const long long d = tile_index(P, dx, dy), q = tile_index(P, sx, sy);
+      const double h = F.H(st)[q], hu = F.HU(st)[q], hv = F.HV(st)[q];
       F.H(st)[d] = h;
       F.HU(st)[d] = dim == 0 ? -hu : hu;
       F.HV(st)[d] = dim == 1 ? -hv : hv;
@@ -375,53 +385,174 @@ k_amr_walls(const AmrWalls* __restrict__ walls, const int* __restrict__ dims,
   }
 }
 
-template <int SOLVER>
-__global__ void __launch_bounds__(64)
-k_amr_speed(const Task* __restrict__ tasks, const int* __restrict__ plist,
-            const PatchDev* __restrict__ pd, Fields F, int cur, double* __restrict__ smax,
-            const AmrClock* clock) {
-  __shared__ MarchLds L;
-  if (!amr_advance(*clock)) return;
-  const Task t = tasks[blockIdx.x];
-  EdgeBufs none{{nullptr, nullptr}, nullptr};
-  MarchArgs A{plist, pd, F, nullptr, none, 1 - cur, 0.0, smax, nullptr, 1.0};
-  // one slot per row segment (tasks may be row segments of their leaves)
-  A.smax_stride = kMaxRowSeg;
-  march_task<kSpeed, false, 0, SOLVER>(t, A, L);
-}
+// What the fill and the update read of the plan.
+struct AmrPlanDev {
+  const AmrBlock* blocks;
+  const Task* tasks;
+  const SegDesc* desc;  // per leaf in task order, ghosts in the own tile
+  const unsigned* gmap;
+  const AmrGhost* ghosts;
+  const AmrWalls* walls;  // per leaf in task order
+  const int* dims;
+};
 
-// Global CFL minimum over the leaves (one workgroup), bounded by the step
-// left to the end time (AMR driver: min(min over leaves, maxdt)).
-__global__ void __launch_bounds__(256)
-k_amr_dt(const int* __restrict__ leaves, int nleaves, const PatchDev* __restrict__ pd,
-         const double* __restrict__ smax, const int* __restrict__ rseg, AmrClock* clock) {
-  __shared__ double red[256];
-  const bool adv = amr_advance(*clock);
-  if (!adv) {
-    if (threadIdx.x == 0) clock->advance = 0;
+// The fill of one task of leaves (see the top of this file), one wavefront
+// per row segment.  Global steps: the workgroup's smallest CFL step goes to
+// cfl_block.  Local time stepping: the leaves that advance only, their ghost
+// cells filled before (k_lts_ghosts), and each leaf's step fmin(own CFL step,
+// end - (t + dt)) (SWEKernel.cpp:60-68) to L.stepdt.
+// MAXT: most threads of a workgroup (the register budget).
+template <int R, int SOLVER, bool LTS, int MAXT>
+__global__ void __launch_bounds__(MAXT)
+k_amr_fill(AmrPlanDev A, const PatchDev* __restrict__ pd, Fields F, int cur,
+           const AmrClock* clock, double* __restrict__ cfl_block, AmrLts L) {
+  __shared__ double pre[MAXT / 64][2][64];
+  __shared__ double red[MAXT / 64];
+  __shared__ double leaf_max[LTS ? MAXT / 64 : 1][64];
+  const AmrClock c = *clock;
+  if (!amr_phase_runs<LTS>(clock, L)) return;
+  const AmrBlock K = A.blocks[blockIdx.x];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (LTS) {
+    const bool go = lane < K.nseg && L.adv[A.desc[K.leaf0 + lane].slot] != 0;
+    if (__builtin_amdgcn_ballot_w64(go) == 0) return;  // the same in every wavefront
+  }
+  Task t = gl(A.tasks + K.first + (w < K.nwaves ? w : 0));
+  if (w >= K.nwaves) t.nseg = 0;
+  SegLane g = seg_lane(t);
+  const SegDesc D = gl(A.desc + t.first + (g.segok ? g.seg : 0));
+  if (LTS && g.segok && !L.adv[D.slot]) g.active = false;
+  const State N = state_of(F, cur), O = state_of(F, 1 - cur);
+  const int last = g.rb == t.nx ? g.rb + 1 : g.rb;
+  SegRows<R, SOLVER != 0> q;
+  q.template load<kRowsInterior>(D, g, N, F.b, last);
+  if (!LTS)
+    for (int i = threadIdx.x; i < K.ncells; i += blockDim.x) {
+      const AmrGhost& e = A.ghosts[A.gmap[K.cell0 + i]];
+      amr_ghost_cell<false>(e, i - e.cell0, pd, F, cur, c, L);
+    }
+  // uNew -> uOld (DefaultTransfer::copyUNewToUOld)
+#pragma unroll
+  for (int k = 1; k <= R; ++k) {
+    if (!g.active || k > g.rows) continue;
+    const long long o = D.off + (long long)(g.ra - 1 + k) * D.stride + g.col;
+    gs(F.H(1 - cur) + o, q.h[k]);
+    gs(F.HU(1 - cur) + o, q.hu[k]);
+    gs(F.HV(1 - cur) + o, q.hv[k]);
+  }
+  __syncthreads();
+  amr_walls(K, A.desc, A.walls, A.dims, pd, F, 1 - cur, LTS ? L.adv : nullptr);
+  q.template load<kRowsGhost>(D, g, O, F.b, last);
+  const double v = seg_speeds<R, SOLVER>(t, g, A.desc, q, last, N, O, F.b, pre[w]);
+  if (!LTS) {
+    const double m = block_min(g.segok ? max_timestep(v, D.dx, D.dy) : kNoLimit, red);
+    if (threadIdx.x == 0) gs(cfl_block + blockIdx.x, m);
     return;
   }
-  double m = 1.7976931348623157e308;
-  for (int k = threadIdx.x; k < nleaves; k += blockDim.x) {
-    const int s = leaves[k];
-    const PatchDev P = pd[s];
-    // the speed maximum of the leaf: over its row segments' slots
-    const double* sm = smax + (long long)s * kMaxRowSeg;
-    double v = sm[0];
-    for (int j = 1; j < rseg[k]; ++j) v = dmax(v, sm[j]);
-    m = dmin(m, max_timestep(v, P.dx, P.dy));
-  }
-  red[threadIdx.x] = m;
+  if (g.segok && g.col == 1) leaf_max[w][g.seg] = v;
   __syncthreads();
-  for (int w = 128; w >= 1; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = dmin(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
+  if ((int)threadIdx.x < K.nseg) {
+    const SegDesc P = gl(A.desc + K.leaf0 + threadIdx.x);
+    if (L.adv[P.slot]) {
+      double m = leaf_max[0][threadIdx.x];
+      for (int k = 1; k < K.nwaves; ++k) m = dmax(m, leaf_max[k][threadIdx.x]);
+      const double md = c.end_time - (L.t[P.slot] + L.dt[P.slot]);
+      L.stepdt[P.slot] = fmin(max_timestep(m, P.dx, P.dy), md);
+    }
   }
-  if (threadIdx.x == 0) {
-    const double cfl = red[0];
-    const double md = clock->end_time - (clock->time + clock->dt);
-    clock->bound = md < cfl ? md : cfl;
-    clock->advance = 1;
+}
+
+// The smallest of many workgroups' CFL steps, where the update's workgroups
+// would otherwise each read more than kCflFold of them.
+constexpr int kCflFold = 1024;
+__global__ void __launch_bounds__(1024)
+k_cfl_fold(const double* __restrict__ cfl_block, int n, double* __restrict__ out) {
+  __shared__ double red[16];
+  double v = kNoLimit;
+  for (int k = threadIdx.x; k < n; k += 1024) v = dmin(v, gl(cfl_block + k));
+  v = block_min(v, red);
+  if (threadIdx.x == 0) *out = v;
+}
+
+// The update of every leaf, uOld -> uNew, after the fill; the last workgroup
+// does the clocks.  Global steps: the step is the smallest of cfl[0 .. ncfl)
+// bounded by the step left to the end time (every leaf's fmin(own CFL step,
+// bound) equals it), the clock goes from `in` to `out`.  Local time stepping:
+// the advancing leaves by their own steps, their clocks (SWEKernel.cpp:83-87)
+// by their first segment.
+template <int R, int SOLVER, bool LTS>
+__global__ void __launch_bounds__(64 * kSegWaves)
+__attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
+k_amr_update(AmrPlanDev A, Fields F, int cur, const AmrClock* in, AmrClock* out,
+             const double* __restrict__ cfl, int ncfl, AmrLts L) {
+  __shared__ double pre[kSegWaves][4][64];
+  __shared__ double red[kSegWaves];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const bool tail = blockIdx.x == gridDim.x - 1;
+  double dt = 0.0;
+  if (LTS) {
+    if (tail) {  // no other workgroup of this launch reads them
+      if (threadIdx.x == 0) {
+        *L.iter = 0;
+        *L.itn = *L.itn + 1;
+      }
+      return;
+    }
+  } else {
+    const AmrClock c = *in;
+    const bool adv = amr_advance(c);
+    if (!adv && !tail) return;
+    const SegRange all{0, ncfl};
+    if (tail) {
+      if (w) return;
+      const double m = cfl_share(all, cfl, lane, 64);
+      if (lane) return;
+      AmrClock n = c;
+      n.advance = adv ? 1 : 0;
+      if (adv) {
+        const double md = c.end_time - (c.time + c.dt);
+        n.bound = md < m ? md : m;
+        // SWEKernel.cpp:83-87 for every leaf
+        if (n.bound - 0.0 > kLaEps) {
+          n.time = c.time + c.dt;
+          n.dt = n.bound;
+        }
+        n.steps = c.steps + 1;
+      }
+      *out = n;
+      return;
+    }
+    dt = c.end_time - (c.time + c.dt);
+    const double m = cfl_share(all, cfl, (int)threadIdx.x, 64 * kSegWaves);
+    if (lane == 0) red[w] = m;
+  }
+  const Task t = gl(A.tasks + blockIdx.x * kSegWaves + w);
+  SegLane g = seg_lane(t);
+  const SegDesc D = gl(A.desc + t.first + (g.segok ? g.seg : 0));
+  const State O = state_of(F, 1 - cur);
+  if (LTS) {
+    const bool go = g.segok && L.adv[D.slot] != 0;
+    g.active = g.active && go;
+    if (__builtin_amdgcn_ballot_w64(go) == 0) return;  // LTS has no workgroup barrier
+    dt = go ? L.stepdt[D.slot] : 0.0;
+  }
+  SegRows<R, true> q;
+  q.template load<kRowsAll>(D, g, O, F.b, g.rb + 1);
+  seg_side_shares<SOLVER>(t, g, A.desc, O, F.b, pre[w]);
+  if (LTS) {
+    wave_sync();
+  } else {
+    __syncthreads();
+    for (int k = 0; k < kSegWaves; ++k) dt = red[k] < dt ? red[k] : dt;
+    if (t.nseg == 0) return;
+  }
+  seg_update_rows<R, SOLVER>(t, g, D, q, dt, pre[w], F.H(cur), F.HU(cur), F.HV(cur));
+  if (LTS && g.active && g.col == 1 && t.sidx == 0) {
+    if (dt - 0.0 > kLaEps) {
+      L.t[D.slot] = L.t[D.slot] + L.dt[D.slot];
+      L.dt[D.slot] = dt;
+    }
+    atomicAdd(L.steps, 1ull);
   }
 }
 
@@ -514,231 +645,32 @@ k_lts_flags_block(const int* __restrict__ leaves, int nleaves, const int* __rest
   }
 }
 
-// uNew -> uOld and the walls (in call order) of one advancing leaf
-// (DefaultTransfer::copyUNewToUOld; SWEKernel::fillBoundaryLayer,
-// SWEKernel.cpp:176-237); widx[slot] = its entry in `walls`, -1 for none.
-__global__ void __launch_bounds__(256)
-k_lts_prep(const int* __restrict__ leaves, const int* __restrict__ widx,
-           const AmrWalls* __restrict__ walls, const int* __restrict__ dims,
-           const PatchDev* __restrict__ pd, Fields F, int cur, AmrLts L) {
-  if (*L.iter == 0) return;
-  const int s = leaves[blockIdx.x];
-  if (!L.adv[s]) return;
-  const PatchDev P = pd[s];
-  for (int k = threadIdx.x; k < P.nx * P.ny; k += blockDim.x) {
-    const long long i = tile_index(P, k / P.ny, k - (k / P.ny) * P.ny);
-    F.H(1 - cur)[i] = F.H(cur)[i];
-    F.HU(1 - cur)[i] = F.HU(cur)[i];
-    F.HV(1 - cur)[i] = F.HV(cur)[i];
-  }
-  const int w = widx[s];
-  if (w < 0) return;
-  __syncthreads();
-  const AmrWalls W = walls[w];
-  const int st = 1 - cur;
-  for (int q = 0; q < W.count; ++q) {
-    const int dim = dims[2 * (W.first + q)], upper = dims[2 * (W.first + q) + 1];
-    const int n_other = dim == 0 ? P.ny : P.nx;
-    for (int k = -1 + (int)threadIdx.x; k < n_other + 1; k += blockDim.x) {
-      int dx, dy, sx, sy;
-      if (dim == 0) {
-        dx = upper ? P.nx : -1;
-        sx = dx + (upper ? -1 : 1);
-        dy = sy = k;
-      } else {
-        dy = upper ? P.ny : -1;
-        sy = dy + (upper ? -1 : 1);
-        dx = sx = k;
-      }
-      const long long d = tile_index(P, dx, dy), sidx = tile_index(P, sx, sy);
-      const double h = F.H(st)[sidx], hu = F.HU(st)[sidx], hv = F.HV(st)[sidx];
-      F.H(st)[d] = h;
-      F.HU(st)[d] = dim == 0 ? -hu : hu;
-      F.HV(st)[d] = dim == 1 ? -hv : hv;
-    }
-    __syncthreads();
-  }
-}
-
-// One task of leaves: CFL speeds from uOld with its ghost layer, each
-// advancing leaf's step dt = fmin(CFL step, end - (t + dt))
-// (SWEKernel.cpp:60-68), the update of the advancing leaves with their own
-// steps, then their clocks (:83-87).  Zeroes *iter for the next iteration
-// (no block of this launch reads it).
-template <int SOLVER>
-__global__ void __launch_bounds__(64)
-k_lts_task(const Task* __restrict__ tasks, const int* __restrict__ plist,
-           const PatchDev* __restrict__ pd, Fields F, int cur, double* __restrict__ smax,
-           const AmrClock* clock, AmrLts T) {
-  __shared__ MarchLds L;
-  const Task t = tasks[blockIdx.x];
-  const int lane = threadIdx.x & 63;
-  const int W = pow2ceil(t.ny);
-  const int seg = lane / W;
-  const int col = lane - seg * W + 1;
-  const bool segok = seg < t.nseg;
-  const int p = plist[t.first + (segok ? seg : 0)];
-  const bool lead = segok && col == 1 && T.adv[p] != 0;
-  if (__any(lead ? 1 : 0)) {
-    EdgeBufs none{{nullptr, nullptr}, nullptr};
-    MarchArgs A{plist, pd, F, nullptr, none, 1 - cur, 0.0, smax, nullptr, 1.0};
-    march_task<kSpeed, false, 0, SOLVER>(t, A, L);
-    __syncthreads();
-    if (lead) {
-      const PatchDev P = pd[p];
-      const double md = clock->end_time - (T.t[p] + T.dt[p]);
-      T.stepdt[p] = fmin(max_timestep(smax[p], P.dx, P.dy), md);
-    }
-    __syncthreads();
-    MarchArgs B{plist, pd, F, nullptr, none, cur, 0.0, nullptr, nullptr, 1.0};
-    B.seg_dt = T.stepdt;
-    B.seg_adv = T.adv;
-    march_task<kUpdateSwap, false, 0, SOLVER, true>(t, B, L);
-    if (lead) {
-      const double dt = T.stepdt[p];
-      if (dt - 0.0 > kLaEps) {
-        T.t[p] = T.t[p] + T.dt[p];
-        T.dt[p] = dt;
-      }
-      atomicAdd(T.steps, 1ull);
-    }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *T.iter = 0;
-    *T.itn = *T.itn + 1;
-  }
-}
-
-// The same iteration in row segments (the global step's segmented tasks):
-// exact speeds of every task with an advancing leaf into one slot per row
-// segment; the step of every advancing leaf, fmin(own CFL step, end - (t +
-// dt)), from its segments' slots; the update of the advancing leaves (their
-// uNew -> uOld ran in k_lts_prep, so it reads uOld and writes uNew) and
-// their clocks.
-template <int SOLVER>
-__global__ void __launch_bounds__(64)
-k_lts_speed(const Task* __restrict__ tasks, const int* __restrict__ plist,
-            const PatchDev* __restrict__ pd, Fields F, int cur, double* __restrict__ smax,
-            AmrLts T) {
-  __shared__ MarchLds L;
-  const Task t = tasks[blockIdx.x];
-  const int lane = threadIdx.x & 63;
-  const int W = pow2ceil(t.ny);
-  const int seg = lane / W;
-  const int col = lane - seg * W + 1;
-  const bool segok = seg < t.nseg;
-  const int p = plist[t.first + (segok ? seg : 0)];
-  const bool lead = segok && col == 1 && T.adv[p] != 0;
-  if (!__any(lead ? 1 : 0)) return;
-  EdgeBufs none{{nullptr, nullptr}, nullptr};
-  MarchArgs A{plist, pd, F, nullptr, none, 1 - cur, 0.0, smax, nullptr, 1.0};
-  A.smax_stride = kMaxRowSeg;
-  march_task<kSpeed, false, 0, SOLVER>(t, A, L);
-}
-
-__global__ void __launch_bounds__(256)
-k_lts_dt(const int* __restrict__ leaves, int nleaves, const int* __restrict__ rseg,
-         const PatchDev* __restrict__ pd, const double* __restrict__ smax,
-         const AmrClock* clock, AmrLts T) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nleaves) return;
-  const int p = leaves[k];
-  if (!T.adv[p]) return;
-  const double* sm = smax + (long long)p * kMaxRowSeg;
-  double v = sm[0];
-  for (int j = 1; j < rseg[k]; ++j) v = dmax(v, sm[j]);
-  const PatchDev P = pd[p];
-  const double md = clock->end_time - (T.t[p] + T.dt[p]);
-  T.stepdt[p] = fmin(max_timestep(v, P.dx, P.dy), md);
-}
-
-template <int SOLVER>
-__global__ void __launch_bounds__(64)
-k_lts_update(const Task* __restrict__ tasks, const int* __restrict__ plist,
-             const PatchDev* __restrict__ pd, Fields F, int cur, AmrLts T) {
-  __shared__ MarchLds L;
-  const Task t = tasks[blockIdx.x];
-  const int lane = threadIdx.x & 63;
-  const int W = pow2ceil(t.ny);
-  const int seg = lane / W;
-  const int col = lane - seg * W + 1;
-  const bool segok = seg < t.nseg;
-  const int p = plist[t.first + (segok ? seg : 0)];
-  const bool lead = segok && col == 1 && T.adv[p] != 0;
-  if (__any(lead ? 1 : 0)) {
-    EdgeBufs none{{nullptr, nullptr}, nullptr};
-    MarchArgs B{plist, pd, F, nullptr, none, cur, 0.0, nullptr, nullptr, 1.0};
-    B.seg_dt = T.stepdt;
-    B.seg_adv = T.adv;
-    march_task<kUpdateFromOld, false, 0, SOLVER, true>(t, B, L);
-    if (lead && t.sidx == 0) {
-      // SWEKernel.cpp:83-87 for the leaf (once, by its first row segment)
-      const double dt = T.stepdt[p];
-      if (dt - 0.0 > kLaEps) {
-        T.t[p] = T.t[p] + T.dt[p];
-        T.dt[p] = dt;
-      }
-      atomicAdd(T.steps, 1ull);
-    }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *T.iter = 0;
-    *T.itn = *T.itn + 1;
-  }
-}
-
-template <int SOLVER>
-__global__ void __launch_bounds__(64)
-k_amr_solve(const Task* __restrict__ tasks, const int* __restrict__ plist,
-            const PatchDev* __restrict__ pd, Fields F, int cur, AmrClock* clock) {
-  __shared__ MarchLds L;
-  // the dt phase decided; this launch's blocks read only advance and bound
-  if (!clock->advance) return;
-  const Task t = tasks[blockIdx.x];
-  const double dt = clock->bound;
-  EdgeBufs none{{nullptr, nullptr}, nullptr};
-  // every leaf's step fmin(own CFL step, bound) equals the bound, which is
-  // at most the minimum of the CFL steps.  uNew -> uOld ran before (k_amr_copy),
-  // so the update reads uOld and writes uNew without the swap's uOld store
-  // (the swap of SWEKernel.cpp:72-73 would store the values already there).
-  MarchArgs A{plist, pd, F, nullptr, none, cur, dt, nullptr, nullptr, 1.0};
-  march_task<kUpdateFromOld, false, 0, SOLVER>(t, A, L);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    // SWEKernel.cpp:83-87 for every leaf
-    if (dt - 0.0 > kLaEps) {
-      clock->time = clock->time + clock->dt;
-      clock->dt = dt;
-    }
-    clock->steps += 1;
-  }
-}
-
 }  // namespace
 
 struct pc_amr {
   pc_pool* pool = nullptr;
   std::vector<int> leaves, virtuals, plan_slots;
   std::vector<int> leaf_nx, leaf_ny;
-  int ntasks = 0, nvblocks = 0, nghosts = 0, nwall_leaves = 0;
+  int nvblocks = 0, nghosts = 0;
+  // tasks of leaves, their row segments (at most seg_rows rows), and what
+  // the fill reads (AmrPlanDev)
+  int seg_rows = 4, nblocks = 0, nsegs = 0, nseg_cells = 0, max_waves = 1;
+  AmrBlock* d_blocks = nullptr;
   Task* d_tasks = nullptr;
-  // the global step's speed and update tasks: d_tasks with the rows of
-  // every leaf split into row segments when the plan has few tasks; per
-  // leaf (plan order) its number of row segments
-  int nutasks = 0;
-  Task* d_utasks = nullptr;
-  int* d_rseg = nullptr;
-  double* d_smax_seg = nullptr;
-  int* d_plist = nullptr;
+  SegDesc* d_desc = nullptr;
+  unsigned* d_gmap = nullptr;
+  int* d_gcell0 = nullptr;  // per ghost entry: its first cell in gmap
+  double* d_cfl = nullptr;  // per block, then the folded one
   int* d_leaves = nullptr;
   AmrVBlock* d_vblocks = nullptr;
   int* d_cptr = nullptr;
   int* d_cpairs = nullptr;
   AmrRestrict* d_pairs = nullptr;
   AmrGhost* d_ghosts = nullptr;
-  AmrWalls* d_walls = nullptr;
+  AmrWalls* d_walls = nullptr;  // per leaf in task order
   int* d_wall_dims = nullptr;
-  double* d_smax = nullptr;
   AmrClock* d_clock = nullptr;
+  AmrClock* d_clock_next = nullptr;  // the clock a global step writes
   char* d_tables = nullptr;  // one allocation holding every d_* table above
   size_t tables_cap = 0;
   double last_dt = 0.0;
@@ -753,23 +685,10 @@ struct pc_amr {
   int* d_rptr = nullptr;   // per leaf (plan order): the virtual patches its faces read
   int* d_rsrc = nullptr;
   std::vector<AmrGhost> h_ghosts;
-  int* d_widx = nullptr;   // per slot: entry of the leaf's walls, -1 for none
-  std::vector<AmrWalls> h_walls;
   int* d_vptr = nullptr;
   int* d_vleaf = nullptr;
   int* d_nptr = nullptr;
   int* d_nbr = nullptr;
-  hipGraph_t lgraph = nullptr;
-  hipGraphExec_t lgexec = nullptr;
-  const PatchDev* lg_pd = nullptr;
-  Fields lg_F{};
-  int lg_solver = -1, lg_cur = -1;
-  // captured step and what it was captured with
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
-  const PatchDev* g_pd = nullptr;
-  Fields g_F{};
-  int g_solver = -1, g_cur = -1;
 };
 
 namespace {
@@ -791,14 +710,27 @@ void amr_free(pc_amr* a) {
     hipFree(a->d_tables);
   }
   a->d_tables = nullptr;
-  if (a->gexec) hipGraphExecDestroy(a->gexec);
-  if (a->graph) hipGraphDestroy(a->graph);
-  void* lts[] = {a->lts.t,    a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
-                 a->lts.itn,  a->lts.need, a->d_vidx,  a->d_widx,     a->d_vptr,   a->d_vleaf,
-                 a->d_nptr,   a->d_nbr,    a->d_rptr,  a->d_rsrc};
+  void* lts[] = {a->lts.t,   a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
+                 a->lts.itn, a->lts.need, a->d_vidx,  a->d_vptr,     a->d_vleaf,  a->d_nptr,
+                 a->d_nbr,   a->d_rptr,   a->d_rsrc};
   for (void* q : lts) hipFree(q);
-  if (a->lgexec) hipGraphExecDestroy(a->lgexec);
-  if (a->lgraph) hipGraphDestroy(a->lgraph);
+}
+
+// Leaves per task: their ghost-column edges (two per row) fit the segments'
+// LDS at 4 rows.
+constexpr int kAmrTaskLeaves = 16;
+
+// Rows per segment of the plan's leaves: 2 while that gives at most 2.5
+// wavefronts a SIMD (2-level grid of 1129 16^2 leaves, 2264 wavefronts: 63 us
+// a step against 65 with 4 rows), else 4 (3-level grid of 729 27^2 leaves,
+// 5110 wavefronts: 92 us against 94).
+int amr_seg_rows(const std::vector<Task>& tasks) {
+  long long n = 0;
+  for (const Task& t : tasks) {
+    n += seg_count(t.nx, 2);
+    if (t.nx > 32) return 4;  // at most 16 wavefronts per workgroup
+  }
+  return n <= 2560 ? 2 : 4;
 }
 
 // The plan's slots must still be live with the same role and size.
@@ -886,7 +818,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     const int nx = a->leaf_nx[i], ny = a->leaf_ny[i];
     int w = 1;
     while (w < ny) w <<= 1;
-    const int per = 64 / w;
+    const int per = std::min(64 / w, kAmrTaskLeaves);
     Task t{(int)plist.size(), 0, nx, ny};
     while (i < a->leaves.size() && t.nseg < per && a->leaf_nx[i] == nx && a->leaf_ny[i] == ny) {
       plist.push_back(a->leaves[i]);
@@ -895,31 +827,53 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     }
     tasks.push_back(t);
   }
-  a->ntasks = (int)tasks.size();
-  // row segments of the global step's tasks: as in the pool's batched step,
-  // a plan with fewer tasks than the GPU holds splits each leaf's rows into
-  // 2 or 4 segments of at least 8 rows
-  std::vector<Task> utasks;
-  std::vector<int> rseg_slot(p->slots.size(), 1), rseg;
-  {
-    constexpr int kFill = 3 * 1024;
-    int want = 1;
-    while (want < kMaxRowSeg && (long long)a->ntasks * want * 2 <= kFill) want *= 2;
-    for (const Task& t : tasks) {
-      int r = want;
-      while (r > 1 && t.nx / r < 8) r /= 2;
-      for (int k = 0; k < r; ++k) {
-        Task u = t;
-        u.r0 = seg_first_row(k, t.nx, r);
-        u.r1 = seg_first_row(k + 1, t.nx, r) - 1;
-        u.sidx = k;
-        utasks.push_back(u);
-      }
-      for (int k = 0; k < t.nseg; ++k) rseg_slot[plist[t.first + k]] = r;
-    }
-    for (int s : a->leaves) rseg.push_back(rseg_slot[s]);
+  // row segments: short ones while they are few (latency), else longer ones
+  // (work); per task a workgroup of the fill
+  a->seg_rows = amr_seg_rows(tasks);
+  std::vector<Task> segs;
+  std::vector<AmrBlock> blocks;
+  std::vector<SegDesc> desc;
+  std::vector<int> pos(p->slots.size(), -1);  // place of a leaf in plist
+  for (size_t k = 0; k < plist.size(); ++k) {
+    const PatchDev P = make_patchdev(p->slots[plist[k]]);
+    SegDesc d{};
+    d.off = P.off;
+    d.gx[0] = P.off;
+    d.gx[1] = P.off + (long long)(P.nx + 1) * P.stride;
+    d.gy[0] = P.off;
+    d.gy[1] = P.off + P.ny + 1;
+    d.nx = P.nx; d.ny = P.ny; d.stride = P.stride;
+    d.slot = plist[k];
+    d.scn = P.scn;
+    d.dx = P.dx; d.dy = P.dy; d.dxinv = P.dxinv; d.dyinv = P.dyinv;
+    desc.push_back(d);
+    pos[plist[k]] = (int)k;
   }
-  a->nutasks = (int)utasks.size();
+  for (const Task& t : tasks) {
+    AmrBlock B{};
+    B.first = (int)segs.size();
+    B.nwaves = seg_count(t.nx, a->seg_rows);
+    B.leaf0 = t.first;
+    B.nseg = t.nseg;
+    B.nx = t.nx;
+    B.ny = t.ny;
+    for (int k = 0; k < B.nwaves; ++k) {
+      Task u = t;
+      u.r0 = seg_first_row(k, t.nx, B.nwaves);
+      u.r1 = seg_first_row(k + 1, t.nx, B.nwaves) - 1;
+      u.sidx = k;
+      segs.push_back(u);
+    }
+    a->max_waves = std::max(a->max_waves, B.nwaves);
+    blocks.push_back(B);
+  }
+  while (segs.size() % kSegWaves) {
+    Task u = segs.back();
+    u.nseg = 0;
+    segs.push_back(u);
+  }
+  a->nblocks = (int)blocks.size();
+  a->nsegs = (int)segs.size();
   // restriction pairs grouped by virtual patch, in the given order; per
   // virtual cell the list of pairs covering it
   std::vector<AmrVBlock> vblocks;
@@ -1073,26 +1027,54 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   }
   a->nghosts = (int)gh.size();
   a->h_ghosts = gh;
+  // the ghost cells of every task, one after another
+  std::vector<int> block_of(plist.size());
+  for (size_t b = 0; b < blocks.size(); ++b)
+    for (int k = 0; k < blocks[b].nseg; ++k) block_of[blocks[b].leaf0 + k] = (int)b;
+  std::vector<int> gcell0(gh.size());
+  std::vector<unsigned> gmap;
+  {
+    std::vector<int> b_of(gh.size());
+    for (size_t e = 0; e < gh.size(); ++e) {
+      b_of[e] = block_of[pos[gh[e].dst]];
+      AmrBlock& B = blocks[b_of[e]];
+      gh[e].cell0 = B.ncells;
+      B.ncells += gh[e].sx * gh[e].sy;
+    }
+    int top = 0;
+    for (AmrBlock& B : blocks) {
+      B.cell0 = top;
+      top += B.ncells;
+    }
+    gmap.resize(top);
+    for (size_t e = 0; e < gh.size(); ++e) {
+      gcell0[e] = blocks[b_of[e]].cell0 + gh[e].cell0;
+      std::fill_n(gmap.begin() + gcell0[e], gh[e].sx * gh[e].sy, (unsigned)e);
+    }
+  }
+  a->nseg_cells = (int)gmap.size();
   // walls grouped per leaf in call order
-  std::vector<AmrWalls> wl;
-  std::vector<int> wdims;
-  for (int i = 0; i < nwalls;) {
+  std::vector<AmrWalls> wl(plist.size(), AmrWalls{0, 0});
+  for (int i = 0; i < nwalls; ++i) {
     const int s = walls[i].slot;
     if (s < 0 || s >= (int)role.size() || role[s] != 1) return bail("walls belong to leaves");
-    AmrWalls W{s, (int)(wdims.size() / 2), 0, 0};
-    while (i < nwalls && walls[i].slot == s) {
-      if ((walls[i].dimension != 0 && walls[i].dimension != 1) ||
-          (walls[i].upper != 0 && walls[i].upper != 1))
-        return bail("wall dimension and side must be 0 or 1");
-      wdims.push_back(walls[i].dimension);
-      wdims.push_back(walls[i].upper);
-      ++W.count;
-      ++i;
-    }
-    wl.push_back(W);
+    if ((walls[i].dimension != 0 && walls[i].dimension != 1) ||
+        (walls[i].upper != 0 && walls[i].upper != 1))
+      return bail("wall dimension and side must be 0 or 1");
+    ++wl[pos[s]].count;
   }
-  a->nwall_leaves = (int)wl.size();
-  a->h_walls = wl;
+  std::vector<int> wdims(2 * (size_t)nwalls), wnext(plist.size());
+  for (size_t k = 0, top = 0; k < wl.size(); ++k) {
+    wl[k].first = wnext[k] = (int)top;
+    top += wl[k].count;
+    AmrBlock& B = blocks[block_of[k]];
+    B.nwalls = std::max(B.nwalls, wl[k].count);
+  }
+  for (int i = 0; i < nwalls; ++i) {
+    const int w = wnext[pos[walls[i].slot]]++;
+    wdims[2 * w] = walls[i].dimension;
+    wdims[2 * w + 1] = walls[i].upper;
+  }
   AmrClock c{};
   c.time = t0;
   c.dt = dt0;
@@ -1100,15 +1082,15 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   // makes a new plan: one allocation, usually the previous plan's, and one
   // DMA instead of fifteen of each)
   PinnedTables st;
-  const size_t o_tasks = st.add(tasks), o_utasks = st.add(utasks), o_rseg = st.add(rseg);
-  const size_t o_smax_seg = st.add(nullptr, p->slots.size() * kMaxRowSeg * sizeof(double));
-  const size_t o_plist = st.add(plist), o_leaves = st.add(a->leaves);
+  const size_t o_blocks = st.add(blocks), o_tasks = st.add(segs), o_desc = st.add(desc);
+  const size_t o_gmap = st.add(gmap), o_gcell0 = st.add(gcell0);
+  const size_t o_cfl = st.add(nullptr, (blocks.size() + 1) * sizeof(double));
+  const size_t o_leaves = st.add(a->leaves);
   const size_t o_vblocks = st.add(vblocks), o_cptr = st.add(cptr), o_cpairs = st.add(cpairs);
   const size_t o_pairs = st.add(pairs), o_ghosts = st.add(gh), o_walls = st.add(wl);
   const size_t o_wall_dims = st.add(wdims);
-  const size_t o_smax = st.add(nullptr, p->slots.size() * sizeof(double));
   const std::vector<AmrClock> clk{c};
-  const size_t o_clock = st.add(clk);
+  const size_t o_clock = st.add(clk), o_next = st.add(clk);
   hipError_t e = hipSuccess;
   if (p->amr_tables && p->amr_tables_cap >= st.total) {
     a->d_tables = p->amr_tables;  // idle: its plan was destroyed after a sync
@@ -1131,11 +1113,12 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     return urc;
   }
   char* const base = a->d_tables;
+  a->d_blocks = reinterpret_cast<AmrBlock*>(base + o_blocks);
   a->d_tasks = reinterpret_cast<Task*>(base + o_tasks);
-  a->d_utasks = reinterpret_cast<Task*>(base + o_utasks);
-  a->d_rseg = reinterpret_cast<int*>(base + o_rseg);
-  a->d_smax_seg = reinterpret_cast<double*>(base + o_smax_seg);
-  a->d_plist = reinterpret_cast<int*>(base + o_plist);
+  a->d_desc = reinterpret_cast<SegDesc*>(base + o_desc);
+  a->d_gmap = reinterpret_cast<unsigned*>(base + o_gmap);
+  a->d_gcell0 = reinterpret_cast<int*>(base + o_gcell0);
+  a->d_cfl = reinterpret_cast<double*>(base + o_cfl);
   a->d_leaves = reinterpret_cast<int*>(base + o_leaves);
   a->d_vblocks = reinterpret_cast<AmrVBlock*>(base + o_vblocks);
   a->d_cptr = reinterpret_cast<int*>(base + o_cptr);
@@ -1144,8 +1127,8 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->d_ghosts = reinterpret_cast<AmrGhost*>(base + o_ghosts);
   a->d_walls = reinterpret_cast<AmrWalls*>(base + o_walls);
   a->d_wall_dims = reinterpret_cast<int*>(base + o_wall_dims);
-  a->d_smax = reinterpret_cast<double*>(base + o_smax);
   a->d_clock = reinterpret_cast<AmrClock*>(base + o_clock);
+  a->d_clock_next = reinterpret_cast<AmrClock*>(base + o_next);
   *out = a;
   return PC_OK;
 }
@@ -1154,44 +1137,67 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
 
 namespace {
 
-void amr_launch_step(pc_amr* a, Fields F, int cur) {
+AmrPlanDev amr_plan(const pc_amr* a) {
+  return AmrPlanDev{a->d_blocks, a->d_tasks, a->d_desc,     a->d_gmap,
+                    a->d_ghosts, a->d_walls, a->d_wall_dims};
+}
+
+template <int R, int SOLVER, bool LTS>
+void amr_launch_segments(pc_amr* a, Fields F, int cur) {
   pc_pool* p = a->pool;
-  const int nl = (int)a->leaves.size();
-  const AmrLts none{};  // unused by the global phases
+  const AmrPlanDev A = amr_plan(a);
+  const dim3 b(64 * a->max_waves);
+  if (a->max_waves <= 8)
+    hipLaunchKernelGGL((k_amr_fill<R, SOLVER, LTS, 512>), dim3(a->nblocks), b, 0, p->stream, A,
+                       p->d_pd, F, cur, a->d_clock, a->d_cfl, a->lts);
+  else
+    hipLaunchKernelGGL((k_amr_fill<R, SOLVER, LTS, 1024>), dim3(a->nblocks), b, 0, p->stream, A,
+                       p->d_pd, F, cur, a->d_clock, a->d_cfl, a->lts);
+  const double* cfl = a->d_cfl;
+  int ncfl = a->nblocks;
+  if (!LTS && ncfl > kCflFold) {
+    hipLaunchKernelGGL(k_cfl_fold, dim3(1), dim3(1024), 0, p->stream, a->d_cfl, ncfl,
+                       a->d_cfl + a->nblocks);
+    cfl = a->d_cfl + a->nblocks;
+    ncfl = 1;
+  }
+  hipLaunchKernelGGL((k_amr_update<R, SOLVER, LTS>), dim3(a->nsegs / kSegWaves + 1),
+                     dim3(64 * kSegWaves), 0, p->stream, A, F, cur, a->d_clock, a->d_clock_next,
+                     cfl, ncfl, a->lts);
+}
+
+template <bool LTS>
+void amr_launch_leaves(pc_amr* a, Fields F, int cur) {
+  if (a->pool->solver) {
+    if (a->seg_rows == 2)
+      amr_launch_segments<2, 1, LTS>(a, F, cur);
+    else
+      amr_launch_segments<4, 1, LTS>(a, F, cur);
+  } else {
+    if (a->seg_rows == 2)
+      amr_launch_segments<2, 0, LTS>(a, F, cur);
+    else
+      amr_launch_segments<4, 0, LTS>(a, F, cur);
+  }
+}
+
+int amr_launch_step(pc_amr* a, Fields F, int cur) {
+  pc_pool* p = a->pool;
   if (a->nvblocks > 0)
     hipLaunchKernelGGL(k_amr_restrict<false>, dim3(a->nvblocks), dim3(64), 0, p->stream,
                        a->d_vblocks, a->d_cptr, a->d_cpairs, a->d_pairs, p->d_pd, F, cur,
-                       a->d_clock, none);
-  hipLaunchKernelGGL(k_amr_copy, dim3(nl), dim3(256), 0, p->stream, a->d_leaves, p->d_pd, F,
-                     cur, a->d_clock);
-  if (a->nghosts > 0)
-    hipLaunchKernelGGL(k_amr_ghosts<false>, dim3((a->nghosts + 3) / 4), dim3(256), 0, p->stream,
-                       a->d_ghosts, a->nghosts, p->d_pd, F, cur, a->d_clock, none);
-  if (a->nwall_leaves > 0)
-    hipLaunchKernelGGL(k_amr_walls, dim3(a->nwall_leaves), dim3(64), 0, p->stream, a->d_walls,
-                       a->d_wall_dims, p->d_pd, F, cur, a->d_clock);
-  if (p->solver)
-    hipLaunchKernelGGL(k_amr_speed<1>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, a->d_smax_seg, a->d_clock);
-  else
-    hipLaunchKernelGGL(k_amr_speed<0>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, a->d_smax_seg, a->d_clock);
-  hipLaunchKernelGGL(k_amr_dt, dim3(1), dim3(256), 0, p->stream, a->d_leaves, nl, p->d_pd,
-                     a->d_smax_seg, a->d_rseg, a->d_clock);
-  if (p->solver)
-    hipLaunchKernelGGL(k_amr_solve<1>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, a->d_clock);
-  else
-    hipLaunchKernelGGL(k_amr_solve<0>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, a->d_clock);
+                       a->d_clock, a->lts);
+  amr_launch_leaves<false>(a, F, cur);
+  HIPCHK(hipGetLastError());
+  std::swap(a->d_clock, a->d_clock_next);
+  return PC_OK;
 }
 
 // One grid iteration with local time stepping: advance flags from the
 // clocks at its start; restriction of every leaf on its own interval; the
 // ghost faces of the advancing leaves (every neighbour read before any leaf
-// changes); uNew -> uOld and walls; then CFL speeds, steps, update and
-// clocks, in three launches over row segments or one over whole leaves.
-void amr_launch_lts(pc_amr* a, Fields F, int cur) {
+// changes); their uNew -> uOld, walls, speeds and steps; update and clocks.
+int amr_launch_lts(pc_amr* a, Fields F, int cur) {
   pc_pool* p = a->pool;
   const int nl = (int)a->leaves.size();
   const AmrLts& L = a->lts;
@@ -1208,89 +1214,12 @@ void amr_launch_lts(pc_amr* a, Fields F, int cur) {
     hipLaunchKernelGGL(k_amr_restrict<true>, dim3(a->nvblocks), dim3(64), 0, p->stream,
                        a->d_vblocks, a->d_cptr, a->d_cpairs, a->d_pairs, p->d_pd, F, cur,
                        a->d_clock, L);
-  if (a->nghosts > 0)
-    hipLaunchKernelGGL(k_amr_ghosts<true>, dim3((a->nghosts + 3) / 4), dim3(256), 0, p->stream,
-                       a->d_ghosts, a->nghosts, p->d_pd, F, cur, a->d_clock, L);
-  hipLaunchKernelGGL(k_lts_prep, dim3(nl), dim3(256), 0, p->stream, a->d_leaves, a->d_widx,
-                     a->d_walls, a->d_wall_dims, p->d_pd, F, cur, L);
-  if (a->nutasks == a->ntasks) {
-    // whole leaves: speeds, steps, update and clocks in one launch
-    if (p->solver)
-      hipLaunchKernelGGL(k_lts_task<1>, dim3(a->ntasks), dim3(64), 0, p->stream, a->d_tasks,
-                         a->d_plist, p->d_pd, F, cur, a->d_smax, a->d_clock, L);
-    else
-      hipLaunchKernelGGL(k_lts_task<0>, dim3(a->ntasks), dim3(64), 0, p->stream, a->d_tasks,
-                         a->d_plist, p->d_pd, F, cur, a->d_smax, a->d_clock, L);
-    return;
-  }
-  if (p->solver)
-    hipLaunchKernelGGL(k_lts_speed<1>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, a->d_smax_seg, L);
-  else
-    hipLaunchKernelGGL(k_lts_speed<0>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, a->d_smax_seg, L);
-  hipLaunchKernelGGL(k_lts_dt, dim3((nl + 255) / 256), dim3(256), 0, p->stream, a->d_leaves, nl,
-                     a->d_rseg, p->d_pd, a->d_smax_seg, a->d_clock, L);
-  if (p->solver)
-    hipLaunchKernelGGL(k_lts_update<1>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, L);
-  else
-    hipLaunchKernelGGL(k_lts_update<0>, dim3(a->nutasks), dim3(64), 0, p->stream, a->d_utasks,
-                       a->d_plist, p->d_pd, F, cur, L);
-}
-
-bool same_fields(const Fields& x, const Fields& y) {
-  return x.h[0] == y.h[0] && x.h[1] == y.h[1] && x.hu[0] == y.hu[0] && x.hu[1] == y.hu[1] &&
-         x.hv[0] == y.hv[0] && x.hv[1] == y.hv[1] && x.b == y.b;
-}
-
-// (Re)capture the step graph when the pool's arrays, the solver or the
-// state parity differ from those it was captured with.
-int amr_graph(pc_amr* a, Fields F, int cur) {
-  pc_pool* p = a->pool;
-  if (a->gexec && a->g_pd == p->d_pd && same_fields(a->g_F, F) && a->g_solver == p->solver &&
-      a->g_cur == cur)
-    return PC_OK;
-  if (a->gexec) HIPCHK(hipGraphExecDestroy(a->gexec));
-  if (a->graph) HIPCHK(hipGraphDestroy(a->graph));
-  a->gexec = nullptr;
-  a->graph = nullptr;
-  HIPCHK(hipStreamSynchronize(p->stream));
-  HIPCHK(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
-  amr_launch_step(a, F, cur);
-  hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(p->stream, &g);
-  if (e != hipSuccess) return fail(PC_E_HIP, std::string("capture: ") + hipGetErrorString(e));
-  a->graph = g;
-  HIPCHK(hipGraphInstantiate(&a->gexec, g, nullptr, nullptr, 0));
-  a->g_pd = p->d_pd;
-  a->g_F = F;
-  a->g_solver = p->solver;
-  a->g_cur = cur;
-  return PC_OK;
-}
-
-int amr_lts_graph(pc_amr* a, Fields F, int cur) {
-  pc_pool* p = a->pool;
-  if (a->lgexec && a->lg_pd == p->d_pd && same_fields(a->lg_F, F) &&
-      a->lg_solver == p->solver && a->lg_cur == cur)
-    return PC_OK;
-  if (a->lgexec) HIPCHK(hipGraphExecDestroy(a->lgexec));
-  if (a->lgraph) HIPCHK(hipGraphDestroy(a->lgraph));
-  a->lgexec = nullptr;
-  a->lgraph = nullptr;
-  HIPCHK(hipStreamSynchronize(p->stream));
-  HIPCHK(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
-  amr_launch_lts(a, F, cur);
-  hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(p->stream, &g);
-  if (e != hipSuccess) return fail(PC_E_HIP, std::string("capture: ") + hipGetErrorString(e));
-  a->lgraph = g;
-  HIPCHK(hipGraphInstantiate(&a->lgexec, g, nullptr, nullptr, 0));
-  a->lg_pd = p->d_pd;
-  a->lg_F = F;
-  a->lg_solver = p->solver;
-  a->lg_cur = cur;
+  if (a->nseg_cells > 0)
+    hipLaunchKernelGGL(k_lts_ghosts, dim3((a->nseg_cells + 255) / 256), dim3(256), 0, p->stream,
+                       a->d_gmap, a->d_gcell0, a->nseg_cells, a->d_ghosts, p->d_pd, F, cur,
+                       a->d_clock, L);
+  amr_launch_leaves<true>(a, F, cur);
+  HIPCHK(hipGetLastError());
   return PC_OK;
 }
 
@@ -1328,26 +1257,21 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   const size_t ns = p->slots.size();
   std::vector<double> t(ns, 0.0), dt(ns, 0.0);
   for (int s : a->leaves) slot_clock(p, s, &t[s], &dt[s]);
-  void* old[] = {a->lts.t,    a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
-                 a->lts.itn,  a->lts.need, a->d_vidx,  a->d_widx,     a->d_vptr,   a->d_vleaf,
-                 a->d_nptr,   a->d_nbr,    a->d_rptr,  a->d_rsrc};
+  void* old[] = {a->lts.t,   a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
+                 a->lts.itn, a->lts.need, a->d_vidx,  a->d_vptr,     a->d_vleaf,  a->d_nptr,
+                 a->d_nbr,   a->d_rptr,   a->d_rsrc};
   for (void* q : old) hipFree(q);
   a->lts = AmrLts{};
-  a->d_vidx = a->d_widx = a->d_vptr = a->d_vleaf = a->d_nptr = a->d_nbr = nullptr;
+  a->d_vidx = a->d_vptr = a->d_vleaf = a->d_nptr = a->d_nbr = nullptr;
   a->d_rptr = a->d_rsrc = nullptr;
-  if (a->lgexec) hipGraphExecDestroy(a->lgexec);
-  if (a->lgraph) hipGraphDestroy(a->lgraph);
-  a->lgexec = nullptr;
-  a->lgraph = nullptr;
   CHK(amr_upload(&a->lts.t, t));
   CHK(amr_upload(&a->lts.dt, dt));
   CHK(amr_upload(&a->lts.adv, std::vector<int>(ns, 0)));
   CHK(amr_upload(&a->lts.stepdt, std::vector<double>(ns, 0.0)));
   CHK(amr_upload(&a->lts.iter, std::vector<int>(1, 0)));
   CHK(amr_upload(&a->lts.steps, std::vector<unsigned long long>(1, 0)));
-  std::vector<int> vidx(ns, -1), widx(ns, -1);
+  std::vector<int> vidx(ns, -1);
   for (size_t v = 0; v < a->virtuals.size(); ++v) vidx[a->virtuals[v]] = (int)v;
-  for (size_t w = 0; w < a->h_walls.size(); ++w) widx[a->h_walls[w].slot] = (int)w;
   // per leaf the virtual patches its ghost faces read
   std::vector<int> lidx(ns, -1), rptr{0}, rsrc;
   for (int k = 0; k < nl; ++k) lidx[a->leaves[k]] = k;
@@ -1363,7 +1287,6 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   CHK(amr_upload(&a->lts.itn, std::vector<int>(1, 1)));
   CHK(amr_upload(&a->lts.need, std::vector<int>(ns, 0)));
   CHK(amr_upload(&a->d_vidx, vidx));
-  CHK(amr_upload(&a->d_widx, widx));
   CHK(amr_upload(&a->d_vptr, vptr));
   CHK(amr_upload(&a->d_vleaf, vleaf));
   CHK(amr_upload(&a->d_nptr, np));
@@ -1385,11 +1308,10 @@ int pc_amr_lts_step(pc_amr* a, int k, double end_time, long long* leaf_steps) {
   mark_state_changed(p);
   a->shared_clock = false;
   Fields F = fields_of(p);
-  CHK(amr_lts_graph(a, F, cur));
   HIPCHK(hipMemcpyAsync(&a->d_clock->end_time, &end_time, sizeof(double),
                         hipMemcpyHostToDevice, p->stream));
   HIPCHK(hipMemsetAsync(a->lts.steps, 0, sizeof(unsigned long long), p->stream));
-  for (int it = 0; it < k; ++it) HIPCHK(hipGraphLaunch(a->lgexec, p->stream));
+  for (int it = 0; it < k; ++it) CHK(amr_launch_lts(a, F, cur));
   unsigned long long n = 0;
   const size_t ns = a->lts_ns;
   std::vector<double> t(ns), dt(ns);
@@ -1421,10 +1343,9 @@ int pc_amr_step(pc_amr* a, int k, double end_time, double* last_dt) {
   CHK(amr_cur(a, &cur));
   mark_state_changed(p);
   Fields F = fields_of(p);
-  CHK(amr_graph(a, F, cur));
   HIPCHK(hipMemcpyAsync(&a->d_clock->end_time, &end_time, sizeof(double),
                         hipMemcpyHostToDevice, p->stream));
-  for (int it = 0; it < k; ++it) HIPCHK(hipGraphLaunch(a->gexec, p->stream));
+  for (int it = 0; it < k; ++it) CHK(amr_launch_step(a, F, cur));
   AmrClock c;
   HIPCHK(hipMemcpyAsync(&c, a->d_clock, sizeof(c), hipMemcpyDeviceToHost, p->stream));
   HIPCHK(hipStreamSynchronize(p->stream));

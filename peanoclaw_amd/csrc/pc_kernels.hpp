@@ -32,8 +32,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
 #include "swe_device.hpp"
 
 namespace pcamd {
@@ -187,11 +185,9 @@ struct GhostStrip {
   int length, negate;
 };
 
-// kUpdateFromOld: the reads and writes of kUpdateSwap without its uOld
-// store, for callers that copied uNew -> uOld before the update (the store
-// would write the values already there); with nothing written into the tile
-// it reads, row segments of one patch may run in parallel.
-enum MarchMode { kSpeed = 0, kUpdate = 1, kUpdateSwap = 2, kUpdateFromOld = 3 };
+// kUpdateFromOld: reads uOld (the other state) and writes uNew (the current
+// one), for the one-patch solve, whose uNew has been saved before.
+enum MarchMode { kSpeed = 0, kUpdate = 1, kUpdateFromOld = 2 };
 
 __device__ __forceinline__ int pow2ceil(int v) {
   int w = 1;
@@ -264,10 +260,6 @@ struct MarchArgs {
   double* smax;       // kSpeed: full per-patch max; fused: next-state interior max
   const ScnDev* scn;  // pruned mode: the scenario's last CFL step (threshold)
   double slack;       // pruned mode: threshold slack
-  // per-patch steps (PERSEG): the step of patch p is seg_dt[p], and only
-  // patches with seg_adv[p] != 0 are updated (local time stepping)
-  const double* seg_dt = nullptr;
-  const int* seg_adv = nullptr;
   // slots per patch of `smax` (kMaxRowSeg for the update's interior maxima
   // of row segments; a whole-patch kSpeed pass fills slot 0 and clears the
   // others)
@@ -298,9 +290,8 @@ struct TileMem<true> {
 
 // FUSE: 0 = no next-state speeds, 1 = exact speeds of every interior edge of
 // the new state, 2 = pruned (exact speeds only for bound candidates).
-// PERSEG: every patch of the task has its own step and advance flag.
 // O32: 32-bit tile offsets (TileMem).
-template <int MODE, bool SIDES, int FUSE, int SOLVER, bool PERSEG = false, bool O32 = false>
+template <int MODE, bool SIDES, int FUSE, int SOLVER, bool O32 = false>
 __device__ __forceinline__ void march_task(const Task& t, const MarchArgs& A, MarchLds& L) {
   using M = TileMem<O32>;
   using I = typename M::I;
@@ -321,31 +312,24 @@ __device__ __forceinline__ void march_task(const Task& t, const MarchArgs& A, Ma
   // the update's y-edges on col-1 lanes are dummies (see the y-sweep)
   const unsigned long long col1_lanes = __builtin_amdgcn_ballot_w64(col == 1);
   const int p = gl(A.plist + t.first + (segok ? seg : 0));
-  const bool active = segok && (col <= ny) && (!PERSEG || gl(A.seg_adv + p) != 0);
+  const bool active = segok && (col <= ny);
   // lane masks for the pruned mode's candidate votes
   const unsigned long long act_lanes = __builtin_amdgcn_ballot_w64(active);
   const PatchDev P = gl(A.pd + p);
   const int stride = P.stride;  // the same for every patch of the task
   const int par = A.par;
-  constexpr bool FROM_OLD = MODE == kUpdateSwap || MODE == kUpdateFromOld;
+  constexpr bool FROM_OLD = MODE == kUpdateFromOld;
   const int src = FROM_OLD ? 1 - par : par;
   const int dst = FROM_OLD ? par : 1 - par;
   const Fields& F = A.F;
-  // kUpdateSwap writes into the tile it reads (rows already consumed), so
-  // its source pointers must not be declared non-aliasing.
-  using SrcPtr = typename std::conditional<MODE == kUpdateSwap, const double*,
-                                           const double* __restrict__>::type;
   // state pointers picked with selects (a run-time index into the argument
   // arrays would place them in scratch memory)
-  double* const Hsrc = src ? F.h[1] : F.h[0];
-  double* const HUsrc = src ? F.hu[1] : F.hu[0];
-  double* const HVsrc = src ? F.hv[1] : F.hv[0];
+  const double* __restrict__ Hs = src ? F.h[1] : F.h[0];
+  const double* __restrict__ HUs = src ? F.hu[1] : F.hu[0];
+  const double* __restrict__ HVs = src ? F.hv[1] : F.hv[0];
   double* const Hdst = dst ? F.h[1] : F.h[0];
   double* const HUdst = dst ? F.hu[1] : F.hu[0];
   double* const HVdst = dst ? F.hv[1] : F.hv[0];
-  SrcPtr Hs = Hsrc;
-  SrcPtr HUs = HUsrc;
-  SrcPtr HVs = HVsrc;
   const double* __restrict__ Bs = F.b;
   const double* Ecur = SIDES ? (par ? A.E.e[1] : A.E.e[0]) : nullptr;
   double* const Edst = SIDES ? (dst ? A.E.e[1] : A.E.e[0]) : nullptr;
@@ -416,7 +400,7 @@ __device__ __forceinline__ void march_task(const Task& t, const MarchArgs& A, Ma
 
   const I base = (I)(P.off + col);
   const double dxinv = P.dxinv, dyinv = P.dyinv;
-  const double dt = PERSEG ? gl(A.seg_dt + p) : A.dt;
+  const double dt = A.dt;
   double smaxl = 0.0;
   // pruned mode: speed threshold of this lane's patch (0 = every edge exact)
   float thr = 0.0f;
@@ -521,12 +505,6 @@ __device__ __forceinline__ void march_task(const Task& t, const MarchArgs& A, Ma
           if (h1 < 0.0) h1 = 0.0;
           if (active) {
             const I o = base + (I)(r - 1) * (I)stride;
-            if (MODE == kUpdateSwap) {
-              // uOld interior <- old uNew, uNew <- new values
-              M::st(Hsrc, o, M::ld(Hdst, o));
-              M::st(HUsrc, o, M::ld(HUdst, o));
-              M::st(HVsrc, o, M::ld(HVdst, o));
-            }
             M::st(Hdst, o, h1);
             M::st(HUdst, o, hu1);
             M::st(HVdst, o, hv1);
@@ -755,7 +733,7 @@ k_update(const Task* __restrict__ tasks, int ntasks, const int* __restrict__ pli
       MarchArgs A{plist, pd, F, sides, E, (gl(&S->stepc) - 1) & 1, gl(&S->dt_applied),
                   smax_next, scn, slack};
       A.smax_stride = kMaxRowSeg;
-      march_task<kUpdate, SIDES, SIDES ? FUSE : 0, SOLVER, false, O32>(t, A, L);
+      march_task<kUpdate, SIDES, SIDES ? FUSE : 0, SOLVER, O32>(t, A, L);
     }
     if (!persistent) return;
   }

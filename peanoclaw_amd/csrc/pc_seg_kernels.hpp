@@ -124,44 +124,61 @@ __device__ __forceinline__ SegLane seg_lane(const Task& t) {
   return g;
 }
 
-// Cells of rows ra-1 .. ra+R of the lane's column (rows past rb+1 and lanes
+// h, hu, hv of one state.
+struct State {
+  const double *h, *hu, *hv;
+};
+__device__ __forceinline__ State state_of(const Fields& F, int s) {
+  return State{F.H(s), F.HU(s), F.HV(s)};
+}
+
+// Cells of rows ra-1 .. ra+R of the lane's column (rows past `last` and lanes
 // without a cell: a wet cell at rest).  hv of a ghost row is not used.
+// Interior and ghost rows can be loaded apart, the ghosts from another state.
+enum RowPart { kRowsInterior = 1, kRowsGhost = 2, kRowsAll = 3 };
 template <int R, bool B>
 struct SegRows {
   double h[R + 2], hu[R + 2], hv[R + 2], b[R + 2];
-  __device__ __forceinline__ void load(const SegDesc& D, const SegLane& g, const double* H,
-                                       const double* HU, const double* HV, const double* Bf,
-                                       int last) {
+  template <int PART>
+  __device__ __forceinline__ void load(const SegDesc& D, const SegLane& g, const State& S,
+                                       const double* Bf, int last) {
 #pragma unroll
     for (int k = 0; k < R + 2; ++k) {
-      h[k] = 1.0; hu[k] = 0.0; hv[k] = 0.0; b[k] = 0.0;
       const int r = g.ra - 1 + k;
+      const bool ghost = r == 0 || r == D.nx + 1;
+      if (PART & kRowsInterior) {
+        h[k] = 1.0; hu[k] = 0.0; hv[k] = 0.0; b[k] = 0.0;
+      }
       if (!g.active || r > last) continue;
       const long long i = D.off + (long long)r * D.stride + g.col;
       const long long j = r == 0 ? D.gx[0] + g.col : (r == D.nx + 1 ? D.gx[1] + g.col : i);
-      h[k] = gl(H + j);
-      hu[k] = gl(HU + j);
-      hv[k] = gl(HV + j);
-      if (B) b[k] = gl(Bf + i);
+      if ((PART & kRowsInterior) && B) b[k] = gl(Bf + i);
+      if (PART == kRowsInterior && ghost) continue;
+      if (PART == kRowsGhost && !ghost) continue;
+      h[k] = gl(S.h + j);
+      hu[k] = gl(S.hu + j);
+      hv[k] = gl(S.hv + j);
     }
+    if (PART & kRowsGhost) {
 #pragma unroll
-    for (int k = 0; k < R + 2; ++k) {
-      const int r = g.ra - 1 + k;
-      if ((r == 0 && (D.neg & 1)) || (r == D.nx + 1 && (D.neg & 2))) hu[k] = -hu[k];
+      for (int k = 0; k < R + 2; ++k) {
+        const int r = g.ra - 1 + k;
+        if ((r == 0 && (D.neg & 1)) || (r == D.nx + 1 && (D.neg & 2))) hu[k] = -hu[k];
+      }
     }
   }
 };
 
 // The y-edges that touch the ghost columns, two per row and patch, one per
 // lane: entry e is side e & 1 of row ra + (e >> 1) % rows of patch
-// (e >> 1) / rows.
+// (e >> 1) / rows.  Own cells and ghosts may come from two states.
 struct SegSide {
   int slot, side;
   double hL, hvL, bL, hR, hvR, bR, dyinv;
   template <bool B>
   __device__ __forceinline__ void load(const SegDesc* __restrict__ desc, const Task& t,
-                                       const SegLane& g, int e, const double* H,
-                                       const double* HV, const double* Bf) {
+                                       const SegLane& g, int e, const State& S,
+                                       const State& G, const double* Bf) {
     side = e & 1;
     const int s = (e >> 1) / g.rows;
     const int row = g.ra + (e >> 1) - s * g.rows;
@@ -171,8 +188,8 @@ struct SegSide {
     const long long at = Q.off + (long long)row * Q.stride;
     const long long io = at + (side ? Q.ny : 1);
     const long long ig = (side ? Q.gy[1] : Q.gy[0]) + (long long)row * Q.stride;
-    const double ho = gl(H + io), hvo = gl(HV + io);
-    double hg = gl(H + ig), hvg = gl(HV + ig);
+    const double ho = gl(S.h + io), hvo = gl(S.hv + io);
+    double hg = gl(G.h + ig), hvg = gl(G.hv + ig);
     if (Q.neg & (side ? 8 : 4)) hvg = -hvg;
     const double bo = B ? gl(Bf + io) : 0.0;
     const double bg = B ? gl(Bf + at + (side ? Q.ny + 1 : 0)) : 0.0;
@@ -181,46 +198,24 @@ struct SegSide {
   }
 };
 
-// Minimum of v over the workgroup (every thread calls it), in thread 0.
-__device__ __forceinline__ double block_min(double v, double* red) {
-  for (int o = 32; o >= 1; o >>= 1) v = dmin(v, __shfl_xor(v, o));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int k = 1; k < (int)blockDim.x / 64; ++k) v = dmin(v, red[k]);
-  return v;
-}
-
-// Exact edge speeds of the current state: one maximum per row segment in
-// smax_seg[slot * kSegSlots + segment] (for the patches' own estimates), and
-// per workgroup the smallest CFL step of its segments.  The CFL step falls
-// with the speed, so the minimum over segments is the minimum over patches.
+// Largest speed of the segment's edges per patch, in every lane of the
+// patch.  `pre`: this wavefront's LDS.  The edge below the last row belongs
+// to the next segment (`last`: the last row loaded).
 template <int R, int SOLVER>
-__global__ void __launch_bounds__(64 * kSegWaves)
-k_seg_speed(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
-            const ScnDev* __restrict__ scn, double* __restrict__ smax_seg,
-            double* __restrict__ cfl_block) {
+__device__ __forceinline__ double seg_speeds(const Task& t, const SegLane& g,
+                                             const SegDesc* __restrict__ desc,
+                                             const SegRows<R, SOLVER != 0>& q, int last,
+                                             const State& S, const State& G, const double* Bf,
+                                             double (*pre)[64]) {
   using ES = EdgeSolver<SOLVER>;
   constexpr bool B = SOLVER != 0;  // the f-wave's speeds do not depend on b
-  __shared__ double pre[kSegWaves][2][64];
-  __shared__ double red[kSegWaves];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
-  const SegLane g = seg_lane(t);
-  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
-  const int par = gl(&scn[t.scn].stepc) & 1;
-  const double *H = F.H(par), *HU = F.HU(par), *HV = F.HV(par);
-  // the edge below the last row belongs to the next segment
-  const int last = g.rb == t.nx ? g.rb + 1 : g.rb;
-  SegRows<R, B> q;
-  q.load(D, g, H, HU, HV, F.b, last);
   const int npre = t.nseg * g.rows * 2;
-  for (int e = lane; e < npre; e += 64) {
+  for (int e = threadIdx.x & 63; e < npre; e += 64) {
     SegSide s;
-    s.load<B>(desc, t, g, e, H, HV, F.b);
+    s.load<B>(desc, t, g, e, S, G, Bf);
     const CellQ cl = cell_dir(cell_base(s.hL, s.bL), s.hvL);
     const CellQ cr = cell_dir(cell_base(s.hR, s.bR), s.hvR);
-    pre[w][s.side][s.slot] = ES::speed(cl, cr);
+    pre[s.side][s.slot] = ES::speed(cl, cr);
   }
   CellBase cb[R + 2];
   CellQ cx[R + 2];
@@ -255,110 +250,51 @@ k_seg_speed(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fi
   wave_sync();
   if (g.active && (g.col == 1 || g.col == t.ny))
     for (int k = 0; k < g.rows; ++k) {
-      if (g.col == 1) sm = dmax(sm, pre[w][0][g.seg * g.rows + k]);
-      if (g.col == t.ny) sm = dmax(sm, pre[w][1][g.seg * g.rows + k]);
+      if (g.col == 1) sm = dmax(sm, pre[0][g.seg * g.rows + k]);
+      if (g.col == t.ny) sm = dmax(sm, pre[1][g.seg * g.rows + k]);
     }
   double v = g.active ? sm : 0.0;
   for (int m = pow2ceil(t.ny) >> 1; m >= 1; m >>= 1) v = dmax(v, __shfl_xor(v, m));
-  if (g.segok && g.col == 1) gs(smax_seg + (long long)D.slot * kSegSlots + t.sidx, v);
-  const double c = block_min(g.segok ? max_timestep(v, D.dx, D.dy) : kNoLimit, red);
-  if (threadIdx.x == 0) gs(cfl_block + blockIdx.x, c);
-}
-
-// Every patch's own CFL step from its segments' speed maxima.
-__global__ void __launch_bounds__(64)
-k_seg_estimates(const SegDesc* __restrict__ desc, int n, int R,
-                const double* __restrict__ smax_seg, double* __restrict__ est) {
-  const int k = blockIdx.x * 64 + threadIdx.x;
-  if (k >= n) return;
-  const SegDesc D = gl(desc + k);
-  double s = 0.0;
-  for (int j = 0; j < seg_count(D.nx, R); ++j)
-    s = dmax(s, gl(smax_seg + (long long)D.slot * kSegSlots + j));
-  est[D.slot] = max_timestep(s, D.dx, D.dy);
-}
-
-// Blocks [first, last) of the segment kernels hold the tasks of a scenario.
-struct SegRange {
-  int first, last;
-};
-
-// This thread's share of a scenario's CFL step: the minimum over every
-// `stride`-th of its blocks from the `at`-th on.
-__device__ __forceinline__ double cfl_share(const SegRange& r,
-                                            const double* __restrict__ cfl_block, int at,
-                                            int stride) {
-  double v = kNoLimit;
-  for (int k = r.first + at; k < r.last; k += stride) v = dmin(v, gl(cfl_block + k));
-  for (int o = 32; o >= 1; o >>= 1) v = dmin(v, __shfl_xor(v, o));
   return v;
 }
 
-// The update of the same segments, current state -> other state.  Every
-// workgroup takes its scenario's step from the blocks' minima and the clock
-// `in`; the last workgroup advances the clocks of all scenarios into `out`
-// (the next step's `in`), so no launch is needed between the speeds and the
-// update.
-template <int R, int SOLVER>
-__global__ void __launch_bounds__(64 * kSegWaves)
-__attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
-k_seg_update(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
-             const ScnDev* __restrict__ in, ScnDev* __restrict__ out, int nscn,
-             const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block) {
-  using ES = EdgeSolver<SOLVER>;
-  __shared__ double pre[kSegWaves][4][64];
-  __shared__ double red[kSegWaves];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (blockIdx.x == gridDim.x - 1) {
-    for (int s = w; s < nscn; s += kSegWaves) {
-      const double cfl = cfl_share(gl(ranges + s), cfl_block, lane, 64);
-      if (lane == 0) {
-        ScnDev S = in[s];
-        dt_final_one(S, cfl, 0, nullptr, 1.0);
-        out[s] = S;
-      }
-    }
-    return;
-  }
-  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
-  const SegLane g = seg_lane(t);
-  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
-  const ScnDev* S = in + t.scn;  // one scenario per workgroup
-  const double max_dt = gl(&S->end_time) - (gl(&S->time) + gl(&S->dt));
-  if (!(max_dt - 0.0 > kLaEps)) return;
-  const int par = gl(&S->stepc) & 1;
-  const double *H = F.H(par), *HU = F.HU(par), *HV = F.HV(par);
-  SegRows<R, true> q;
-  q.load(D, g, H, HU, HV, F.b, g.rb + 1);
-  const double share = cfl_share(gl(ranges + t.scn), cfl_block, (int)threadIdx.x,
-                                 64 * kSegWaves);
-  if (lane == 0) red[w] = share;
+// Shares of the segment's ghost-column y-edges, into this wavefront's LDS.
+template <int SOLVER>
+__device__ __forceinline__ void seg_side_shares(const Task& t, const SegLane& g,
+                                                const SegDesc* __restrict__ desc,
+                                                const State& S, const double* Bf,
+                                                double (*pre)[64]) {
   const int npre = t.nseg * g.rows * 2;
-  for (int e = lane; e < npre; e += 64) {
+  for (int e = threadIdx.x & 63; e < npre; e += 64) {
     SegSide s;
-    s.load<true>(desc, t, g, e, H, HV, F.b);
+    s.load<true>(desc, t, g, e, S, S, Bf);
     const CellQ cl = cell_dir(cell_base(s.hL, s.bL), s.hvL);
     const CellQ cr = cell_dir(cell_base(s.hR, s.bR), s.hvR);
     double dhL, dhR, dqL, dqR;
-    ES::solve(cl, cr, dhL, dhR, dqL, dqR);
+    EdgeSolver<SOLVER>::solve(cl, cr, dhL, dhR, dqL, dqR);
     // side 0: the right cell (row,1) takes the "upwards" part;
     // side 1: the left cell (row,ny) takes the "downwards" part.
-    pre[w][s.side * 2 + 0][s.slot] = s.dyinv * (s.side ? dhL : dhR);
-    pre[w][s.side * 2 + 1][s.slot] = s.dyinv * (s.side ? dqL : dqR);
+    pre[s.side * 2 + 0][s.slot] = s.dyinv * (s.side ? dhL : dhR);
+    pre[s.side * 2 + 1][s.slot] = s.dyinv * (s.side ? dqL : dqR);
   }
-  __syncthreads();
-  double dt = max_dt;
-  for (int k = 0; k < kSegWaves; ++k) dt = fmin(red[k], dt);
-  if (t.nseg == 0) return;
+}
+
+// Update of the segment's rows by dt, written to (Hd, HUd, HVd); `pre` holds
+// seg_side_shares.
+template <int R, int SOLVER>
+__device__ __forceinline__ void seg_update_rows(const Task& t, const SegLane& g,
+                                                const SegDesc& D, const SegRows<R, true>& q,
+                                                double dt, double (*pre)[64],
+                                                double* __restrict__ Hd,
+                                                double* __restrict__ HUd,
+                                                double* __restrict__ HVd) {
+  using ES = EdgeSolver<SOLVER>;
   bool wet = true;
 #pragma unroll
   for (int k = 0; k < R + 2; ++k) wet = wet && q.h[k] >= kDryTol;
   const bool fast = SOLVER == 0 && wave_all(wet);
   const unsigned long long col1 = __builtin_amdgcn_ballot_w64(g.col == 1);
   const double dxinv = D.dxinv, dyinv = D.dyinv;
-  double* const Hd = F.H(1 - par);
-  double* const HUd = F.HU(1 - par);
-  double* const HVd = F.HV(1 - par);
   // Chunks of rows: the edges below the chunk's rows (x-edge k | k+1, y-edges
   // of row k+1) in straight-line code, one vote, then the rows they complete.
   // Few rows go in one chunk (most overlap); with more, two by two, for the
@@ -448,16 +384,127 @@ k_seg_update(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, F
         dnq = from_right(dyinv * yqL[c]);
         const int slot = g.seg * g.rows + k;
         if (k < g.rows && g.active && g.col == 1) {
-          uph = pre[w][0][slot];
-          upq = pre[w][1][slot];
+          uph = pre[0][slot];
+          upq = pre[1][slot];
         }
         if (k < g.rows && g.active && g.col == t.ny) {
-          dnh = pre[w][2][slot];
-          dnq = pre[w][3][slot];
+          dnh = pre[2][slot];
+          dnq = pre[3][slot];
         }
       }
     }
   }
+}
+
+// Minimum of v over the workgroup (every thread calls it), in thread 0.
+__device__ __forceinline__ double block_min(double v, double* red) {
+  for (int o = 32; o >= 1; o >>= 1) v = dmin(v, __shfl_xor(v, o));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int k = 1; k < (int)blockDim.x / 64; ++k) v = dmin(v, red[k]);
+  return v;
+}
+
+// Exact edge speeds of the current state: one maximum per row segment in
+// smax_seg[slot * kSegSlots + segment] (for the patches' own estimates), and
+// per workgroup the smallest CFL step of its segments.  The CFL step falls
+// with the speed, so the minimum over segments is the minimum over patches.
+template <int R, int SOLVER>
+__global__ void __launch_bounds__(64 * kSegWaves)
+k_seg_speed(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
+            const ScnDev* __restrict__ scn, double* __restrict__ smax_seg,
+            double* __restrict__ cfl_block) {
+  __shared__ double pre[kSegWaves][2][64];
+  __shared__ double red[kSegWaves];
+  const int w = threadIdx.x >> 6;
+  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
+  const SegLane g = seg_lane(t);
+  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
+  const State S = state_of(F, gl(&scn[t.scn].stepc) & 1);
+  const int last = g.rb == t.nx ? g.rb + 1 : g.rb;
+  SegRows<R, SOLVER != 0> q;
+  q.template load<kRowsAll>(D, g, S, F.b, last);
+  const double v = seg_speeds<R, SOLVER>(t, g, desc, q, last, S, S, F.b, pre[w]);
+  if (g.segok && g.col == 1) gs(smax_seg + (long long)D.slot * kSegSlots + t.sidx, v);
+  const double c = block_min(g.segok ? max_timestep(v, D.dx, D.dy) : kNoLimit, red);
+  if (threadIdx.x == 0) gs(cfl_block + blockIdx.x, c);
+}
+
+// Every patch's own CFL step from its segments' speed maxima.
+__global__ void __launch_bounds__(64)
+k_seg_estimates(const SegDesc* __restrict__ desc, int n, int R,
+                const double* __restrict__ smax_seg, double* __restrict__ est) {
+  const int k = blockIdx.x * 64 + threadIdx.x;
+  if (k >= n) return;
+  const SegDesc D = gl(desc + k);
+  double s = 0.0;
+  for (int j = 0; j < seg_count(D.nx, R); ++j)
+    s = dmax(s, gl(smax_seg + (long long)D.slot * kSegSlots + j));
+  est[D.slot] = max_timestep(s, D.dx, D.dy);
+}
+
+// Blocks [first, last) of the segment kernels hold the tasks of a scenario.
+struct SegRange {
+  int first, last;
+};
+
+// This thread's share of a scenario's CFL step: the minimum over every
+// `stride`-th of its blocks from the `at`-th on.
+__device__ __forceinline__ double cfl_share(const SegRange& r,
+                                            const double* __restrict__ cfl_block, int at,
+                                            int stride) {
+  double v = kNoLimit;
+  for (int k = r.first + at; k < r.last; k += stride) v = dmin(v, gl(cfl_block + k));
+  for (int o = 32; o >= 1; o >>= 1) v = dmin(v, __shfl_xor(v, o));
+  return v;
+}
+
+// The update of the same segments, current state -> other state.  Every
+// workgroup takes its scenario's step from the blocks' minima and the clock
+// `in`; the last workgroup advances the clocks of all scenarios into `out`
+// (the next step's `in`), so no launch is needed between the speeds and the
+// update.
+template <int R, int SOLVER>
+__global__ void __launch_bounds__(64 * kSegWaves)
+__attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
+k_seg_update(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
+             const ScnDev* __restrict__ in, ScnDev* __restrict__ out, int nscn,
+             const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block) {
+  __shared__ double pre[kSegWaves][4][64];
+  __shared__ double red[kSegWaves];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (blockIdx.x == gridDim.x - 1) {
+    for (int s = w; s < nscn; s += kSegWaves) {
+      const double cfl = cfl_share(gl(ranges + s), cfl_block, lane, 64);
+      if (lane == 0) {
+        ScnDev S = in[s];
+        dt_final_one(S, cfl, 0, nullptr, 1.0);
+        out[s] = S;
+      }
+    }
+    return;
+  }
+  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
+  const SegLane g = seg_lane(t);
+  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
+  const ScnDev* C = in + t.scn;  // one scenario per workgroup
+  const double max_dt = gl(&C->end_time) - (gl(&C->time) + gl(&C->dt));
+  if (!(max_dt - 0.0 > kLaEps)) return;
+  const int par = gl(&C->stepc) & 1;
+  const State S = state_of(F, par);
+  SegRows<R, true> q;
+  q.template load<kRowsAll>(D, g, S, F.b, g.rb + 1);
+  const double share = cfl_share(gl(ranges + t.scn), cfl_block, (int)threadIdx.x,
+                                 64 * kSegWaves);
+  if (lane == 0) red[w] = share;
+  seg_side_shares<SOLVER>(t, g, desc, S, F.b, pre[w]);
+  __syncthreads();
+  double dt = max_dt;
+  for (int k = 0; k < kSegWaves; ++k) dt = fmin(red[k], dt);
+  if (t.nseg == 0) return;
+  seg_update_rows<R, SOLVER>(t, g, D, q, dt, pre[w], F.H(1 - par), F.HU(1 - par),
+                             F.HV(1 - par));
 }
 
 }  // namespace pcamd
