@@ -81,26 +81,37 @@ __device__ __forceinline__ bool amr_phase_runs(const AmrClock* clock, const AmrL
   return amr_advance(*clock);
 }
 
-// 64 consecutive cells of one virtual patch
-// the restriction kernel's lanes per virtual-patch cell, and cells per
-// wavefront (one AmrVBlock)
-constexpr int kRestrictLanes = 8;
-constexpr int kRestrictCells = 64 / kRestrictLanes;
+// The restriction kernel's lanes per virtual-patch cell, cells per workgroup
+// (one AmrVBlock) and contributions per cell held in LDS at a time.
+constexpr int kRestrictLanes = 16;
+constexpr int kRestrictCells = 256 / kRestrictLanes;
+constexpr int kRestrictChunk = 2 * kRestrictLanes;
 
+// kRestrictCells consecutive cells of one virtual patch
 struct AmrVBlock {
-  int slot;   // the virtual patch
+  long long off;     // its tile
+  double dstRegion;  // area of its cells
+  int slot;
   int cell0;  // first cell (x * ny + y)
   int base;   // index of cell 0 of this patch in the per-cell lists
-  int pad;
+  int nx, ny, stride;
+};
+
+// One fine cell of a leaf inside a virtual-patch cell: where it is
+// (kContribBits bits: index in the field arrays; above: the leaf's place in
+// the plan) and the area they share.
+constexpr int kContribBits = 40;
+struct AmrContrib {
+  unsigned long long at;
+  double region;
 };
 
 // Restriction of the whole leaf `src` into one virtual patch
 // (DefaultRestriction.cpph:16-106 over region (0, n)).
 struct AmrRestrict {
-  int src;
+  int src, leaf;  // slot, place in the plan's leaves
   int rSize[2];
   int dOff[2], dSize[2];
-  int pad;
   double srcSub[2], dstSub[2], dstRegion;
   double spos[2], dpos[2];
 };
@@ -144,71 +155,50 @@ __device__ __forceinline__ void amr_restrict_factors(const AmrClock& c, double& 
   }
 }
 
-// One virtual-patch cell per group of kRestrictLanes lanes (kRestrictCells
-// cells per wavefront): the contributions of its fine cells are computed
-// kRestrictLanes at a time in parallel and summed by the group's first lane
-// in the order of the per-call sequence (pairs in plan order, fine cells x
-// outer, y inner), so the sums equal the sequential ones bit for bit.
-// `cptr`/`cpairs` list, per cell, the restriction pairs whose destination
-// region holds it, in plan order.
-template <bool LTS>
-__global__ void __launch_bounds__(64)
-k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ cptr,
-               const int* __restrict__ cpairs, const AmrRestrict* __restrict__ pairs,
-               const PatchDev* __restrict__ pd, Fields F, int cur, const AmrClock* clock,
-               AmrLts L) {
-  constexpr int K = kRestrictLanes;
-  __shared__ double con[kRestrictCells][6][K];
-  const AmrClock c = *clock;
-  if (!amr_phase_runs<LTS>(clock, L)) return;
-  const AmrVBlock B = blocks[blockIdx.x];
-  // local time stepping: only the virtual patches an advancing leaf reads
-  if (LTS && L.need[B.slot] != *L.itn) return;
-  const PatchDev D = pd[B.slot];
-  const int g = (int)threadIdx.x / K, sub = (int)threadIdx.x - g * K;
-  const int k = B.cell0 + g;
-  const bool cellok = k < D.nx * D.ny;
-  double tfOld, tfNew;
-  amr_restrict_factors(c, tfOld, tfNew);
+// Fine cells of a leaf under row (d = 0) or column (d = 1) `di` of a virtual
+// patch: [o, o + n) (DefaultRestriction.cpph:60-83).
+__host__ __device__ __forceinline__ void amr_fine_span(const AmrRestrict& a, int d, int di,
+                                                       int& o, int& n) {
   const double eps = 1e-12;
-  const int oldSt = 1 - cur;
-  const int di0 = cellok ? k / D.ny : 0, di1 = cellok ? k - di0 * D.ny : 0;
-  double accO[3] = {0.0, 0.0, 0.0};
-  double accN[3] = {0.0, 0.0, 0.0};
-  const int jb = cellok ? cptr[B.base + k] : 0, je = cellok ? cptr[B.base + k + 1] : 0;
-  for (int j = jb; j < je; ++j) {  // uniform within the group
-    const AmrRestrict a = pairs[cpairs[j]];
+  const double dp = a.dpos[d] + (double)di * a.dstSub[d];
+  double ot = (dp - a.spos[d] + eps);
+  ot /= a.srcSub[d];
+  const int first = (int)ot;
+  double st = dp + a.dstSub[d] - a.spos[d] - eps;
+  st /= a.srcSub[d];
+  st -= ot;
+  st += 1.0;
+  const int upper = first + (int)st, rUpper = a.rSize[d];
+  o = first > 0 ? first : 0;
+  n = (upper < rUpper ? upper : rUpper) - o;
+  if (n < 0) n = 0;
+}
+
+// The plan's contributions, one thread per virtual-patch cell, in the order
+// of the per-call sequence (pairs in plan order, fine cells x outer, y
+// inner): contribs[xptr[cell] ..].  Runs once per plan.  `cptr`/`cpairs`
+// list, per cell, the restriction pairs whose destination region holds it.
+__global__ void __launch_bounds__(256)
+k_amr_contribs(const AmrVBlock* __restrict__ blocks, const int* __restrict__ cptr,
+               const int* __restrict__ cpairs, const int* __restrict__ xptr,
+               const AmrRestrict* __restrict__ pairs, const PatchDev* __restrict__ pd,
+               AmrContrib* __restrict__ contribs) {
+  const AmrVBlock B = blocks[blockIdx.x * (256 / kRestrictCells) + threadIdx.x / kRestrictCells];
+  const int k = B.cell0 + (int)threadIdx.x % kRestrictCells;
+  if (k >= B.nx * B.ny) return;
+  const int d0 = k / B.ny, d1 = k - d0 * B.ny;
+  AmrContrib* out = contribs + xptr[B.base + k];
+  for (int j = cptr[B.base + k]; j < cptr[B.base + k + 1]; ++j) {
+    const AmrRestrict& a = pairs[cpairs[j]];
     const PatchDev S = pd[a.src];
-    if (LTS) {
-      // each leaf restricts on its own interval
-      AmrClock cs = c;
-      cs.time = L.t[a.src];
-      cs.dt = L.dt[a.src];
-      amr_restrict_factors(cs, tfOld, tfNew);
-    }
-    const double dp[2] = {a.dpos[0] + (double)di0 * a.dstSub[0],
-                          a.dpos[1] + (double)di1 * a.dstSub[1]};
-    int cOff[2], cSize[2];
-    for (int d = 0; d < 2; ++d) {
-      double ot = (dp[d] - a.spos[d] + eps);
-      ot /= a.srcSub[d];
-      const int o = (int)ot;
-      double st = dp[d] + a.dstSub[d] - a.spos[d] - eps;
-      st /= a.srcSub[d];
-      st -= ot;
-      st += 1.0;
-      const int s = (int)st;
-      const int upper = o + s, rUpper = a.rSize[d];
-      cOff[d] = o > 0 ? o : 0;
-      cSize[d] = (upper < rUpper ? upper : rUpper) - cOff[d];
-    }
-    const int nfine = cSize[0] > 0 && cSize[1] > 0 ? cSize[0] * cSize[1] : 0;
-    for (int r0 = 0; r0 < nfine; r0 += K) {  // uniform within the group
-      const int m = r0 + sub;
-      double dO[3] = {0.0, 0.0, 0.0}, dN[3] = {0.0, 0.0, 0.0};
-      if (m < nfine) {
-        const int sx = m / cSize[1];
-        const int s0 = cOff[0] + sx, s1 = cOff[1] + (m - sx * cSize[1]);
+    const double dp[2] = {a.dpos[0] + (double)d0 * a.dstSub[0],
+                          a.dpos[1] + (double)d1 * a.dstSub[1]};
+    int o[2], n[2];
+    amr_fine_span(a, 0, d0, o[0], n[0]);
+    amr_fine_span(a, 1, d1, o[1], n[1]);
+    for (int x = 0; x < n[0]; ++x)
+      for (int y = 0; y < n[1]; ++y) {
+        const int s0 = o[0] + x, s1 = o[1] + y;
         const double sp[2] = {a.spos[0] + (double)s0 * a.srcSub[0],
                               a.spos[1] + (double)s1 * a.srcSub[1]};
         double region = 1.0;
@@ -218,42 +208,89 @@ k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ cpt
           region *= hi - lo;
           region = dmax(region, 0.0);
         }
-        const long long si = tile_index(S, s0, s1);
-        const double bv = F.b[si];
-        const double vo[3] = {F.H(oldSt)[si] + 1.0 * bv, F.HU(oldSt)[si], F.HV(oldSt)[si]};
-        const double vn[3] = {F.H(cur)[si] + 1.0 * bv, F.HU(cur)[si], F.HV(cur)[si]};
-        for (int q = 0; q < 3; ++q) {
-          dO[q] = (vo[q] * (1.0 - tfOld) + vn[q] * tfOld) * region / a.dstRegion;
-          dN[q] = (vo[q] * (1.0 - tfNew) + vn[q] * tfNew) * region / a.dstRegion;
-        }
+        out->at = (unsigned long long)tile_index(S, s0, s1) |
+                  ((unsigned long long)a.leaf << kContribBits);
+        out->region = region;
+        ++out;
       }
+  }
+}
+
+// Restriction (DefaultRestriction.cpph:16-106, SWEKernel::
+// postProcessRestriction): kRestrictLanes lanes per virtual-patch cell take
+// its contributions in turn; lane q < 6 sums one of the six quantities (h +
+// b, hu, hv in both states) in the order of the per-call sequence, so the
+// sums equal the sequential ones bit for bit.
+//
+// Bound by latency: geometry, source cells and shared areas come from the
+// plan's contribution list (16 bytes each), so a cell's chain is block ->
+// list bounds -> list -> cells; deriving them per step, behind four
+// divisions and five more dependent loads, took 15.7 us on the 2-level grid
+// of 1129 16^2 leaves and 24.8 us on the 3-level grid of 729 27^2 leaves.
+template <bool LTS>
+__global__ void __launch_bounds__(256)
+k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ xptr,
+               const AmrContrib* __restrict__ contribs, const int* __restrict__ leaves,
+               Fields F, int cur, const AmrClock* clock, AmrLts L) {
+  constexpr int K = kRestrictLanes, N = kRestrictChunk;
+  __shared__ double con[kRestrictCells][6][N + 1];
+  const AmrClock c = *clock;
+  const AmrVBlock B = blocks[blockIdx.x];
+  const int g = (int)threadIdx.x / K, sub = (int)threadIdx.x - g * K;
+  const int k = B.cell0 + g;
+  const bool cellok = k < B.nx * B.ny;
+  const int beg = cellok ? gl(xptr + B.base + k) : 0;
+  const int n = cellok ? gl(xptr + B.base + k + 1) - beg : 0;
+  if (!amr_phase_runs<LTS>(clock, L)) return;
+  // local time stepping: only the virtual patches an advancing leaf reads
+  if (LTS && L.need[B.slot] != *L.itn) return;
+  double tfOld, tfNew;
+  amr_restrict_factors(c, tfOld, tfNew);
+  const State O = state_of(F, 1 - cur), W = state_of(F, cur);
+  int most = n;  // of the wavefront's cells
+  for (int o = 32; o >= K; o >>= 1) most = max(most, __shfl_xor(most, o));
+  double acc = 0.0;
+  for (int r0 = 0; r0 < most; r0 += N) {
+#pragma unroll
+    for (int half = 0; half < N; half += K) {
+      const int m = r0 + half + sub;
+      if (m >= n) continue;
+      const AmrContrib a = gl(contribs + beg + m);
+      const long long i = (long long)(a.at & ((1ull << kContribBits) - 1));
+      if (LTS) {
+        // each leaf restricts on its own interval
+        const int s = gl(leaves + (a.at >> kContribBits));
+        AmrClock cs = c;
+        cs.time = L.t[s];
+        cs.dt = L.dt[s];
+        amr_restrict_factors(cs, tfOld, tfNew);
+      }
+      const double bv = gl(F.b + i);
+      const double vo[3] = {gl(O.h + i) + 1.0 * bv, gl(O.hu + i), gl(O.hv + i)};
+      const double vn[3] = {gl(W.h + i) + 1.0 * bv, gl(W.hu + i), gl(W.hv + i)};
       for (int q = 0; q < 3; ++q) {
-        con[g][q][sub] = dO[q];
-        con[g][3 + q][sub] = dN[q];
+        con[g][q][half + sub] =
+            (vo[q] * (1.0 - tfOld) + vn[q] * tfOld) * a.region / B.dstRegion;
+        con[g][3 + q][half + sub] =
+            (vo[q] * (1.0 - tfNew) + vn[q] * tfNew) * a.region / B.dstRegion;
       }
-      wave_sync();
-      if (sub == 0) {
-        const int cnt = nfine - r0 < K ? nfine - r0 : K;
-        for (int i = 0; i < cnt; ++i)
-          for (int q = 0; q < 3; ++q) {
-            accO[q] = accO[q] + con[g][q][i];
-            accN[q] = accN[q] + con[g][3 + q][i];
-          }
-      }
-      wave_sync();
     }
+    wave_sync();
+    if (sub < 6) {
+      const int cnt = n - r0 < N ? n - r0 : N;
+      for (int i = 0; i < cnt; ++i) acc = acc + con[g][sub][i];
+    }
+    wave_sync();
   }
-  if (cellok && sub == 0) {
-    // SWEKernel::postProcessRestriction: h + b -> h with the virtual's b
-    const long long di = tile_index(D, di0, di1);
-    const double bd = F.b[di];
-    F.H(oldSt)[di] = accO[0] + (-1.0) * bd;
-    F.HU(oldSt)[di] = accO[1];
-    F.HV(oldSt)[di] = accO[2];
-    F.H(cur)[di] = accN[0] + (-1.0) * bd;
-    F.HU(cur)[di] = accN[1];
-    F.HV(cur)[di] = accN[2];
-  }
+  if (!cellok || sub >= 6) return;
+  const int x = k / B.ny, y = k - x * B.ny;
+  const long long di = B.off + (long long)(x + 1) * B.stride + (y + 1);
+  const int q = sub % 3, st = sub < 3 ? 1 - cur : cur;
+  // h + b -> h with the virtual patch's b
+  if (q == 0)
+    gs(F.H(st) + di, acc + (-1.0) * gl(F.b + di));
+  else
+    gs((q == 1 ? F.HU(st) : F.HV(st)) + di, acc);
 }
 
 // Cell k of a ghost entry.  LTS: every leaf runs on its own clock.  Else all
@@ -651,6 +688,7 @@ struct pc_amr {
   pc_pool* pool = nullptr;
   std::vector<int> leaves, virtuals, plan_slots;
   std::vector<int> leaf_nx, leaf_ny;
+  std::vector<long long> plan_off;  // tile of every plan slot: the tables hold places in it
   int nvblocks = 0, nghosts = 0;
   // tasks of leaves, their row segments (at most seg_rows rows), and what
   // the fill reads (AmrPlanDev)
@@ -663,9 +701,8 @@ struct pc_amr {
   double* d_cfl = nullptr;  // per block, then the folded one
   int* d_leaves = nullptr;
   AmrVBlock* d_vblocks = nullptr;
-  int* d_cptr = nullptr;
-  int* d_cpairs = nullptr;
-  AmrRestrict* d_pairs = nullptr;
+  int* d_xptr = nullptr;  // per virtual cell: its contributions
+  AmrContrib* d_contribs = nullptr;
   AmrGhost* d_ghosts = nullptr;
   AmrWalls* d_walls = nullptr;  // per leaf in task order
   int* d_wall_dims = nullptr;
@@ -740,11 +777,13 @@ int amr_check_slots(pc_amr* a) {
     const int s = a->leaves[i];
     if (!valid_slot(p, s) || p->slots[s].desc.is_virtual ||
         p->slots[s].desc.subdivision_factor[0] != a->leaf_nx[i] ||
-        p->slots[s].desc.subdivision_factor[1] != a->leaf_ny[i])
+        p->slots[s].desc.subdivision_factor[1] != a->leaf_ny[i] ||
+        p->slots[s].off != a->plan_off[i])
       return fail(PC_E_INVALID, "a leaf of the AMR plan changed or was released");
   }
-  for (int s : a->virtuals)
-    if (!valid_slot(p, s) || !p->slots[s].desc.is_virtual)
+  for (size_t i = 0; i < a->virtuals.size(); ++i)
+    if (!valid_slot(p, a->virtuals[i]) || !p->slots[a->virtuals[i]].desc.is_virtual ||
+        p->slots[a->virtuals[i]].off != a->plan_off[a->leaves.size() + i])
       return fail(PC_E_INVALID, "a virtual patch of the AMR plan changed or was released");
   return PC_OK;
 }
@@ -792,6 +831,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->virtuals.assign(virtuals, virtuals + nvirtuals);
   a->plan_slots = a->leaves;
   a->plan_slots.insert(a->plan_slots.end(), a->virtuals.begin(), a->virtuals.end());
+  for (int s : a->plan_slots) a->plan_off.push_back(p->slots[s].off);
   // leaf clock: every leaf on one clock
   double t0, dt0;
   slot_clock(p, leaves[0], &t0, &dt0);
@@ -877,8 +917,10 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   // restriction pairs grouped by virtual patch, in the given order; per
   // virtual cell the list of pairs covering it
   std::vector<AmrVBlock> vblocks;
-  std::vector<int> cptr{0}, cpairs;
+  std::vector<int> cptr{0}, cpairs, xptr{0};
   std::vector<AmrRestrict> pairs;
+  std::vector<int> leaf_at(role.size(), -1);
+  for (int k = 0; k < nleaves; ++k) leaf_at[leaves[k]] = k;
   // the restrictions of each destination slot, in the given order
   std::vector<int> rbeg(role.size() + 1, 0), rlist(nrestrictions);
   for (int r = 0; r < nrestrictions; ++r) {
@@ -893,7 +935,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
       if (v >= 0 && v < (int)role.size()) rlist[fill[v]++] = r;
     }
   }
-  std::vector<int> ccount;
+  std::vector<int> ccount, xcount, span0, span1;
   for (int vi = 0; vi < nvirtuals; ++vi) {
     const int v = virtuals[vi];
     const int pbeg = (int)pairs.size();
@@ -908,6 +950,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
       const PatchDev S = make_patchdev(p->slots[s]);
       AmrRestrict R{};
       R.src = s;
+      R.leaf = leaf_at[s];
       const int z[2] = {0, 0};
       const int sn[2] = {sd.subdivision_factor[0], sd.subdivision_factor[1]};
       const int dn[2] = {dd.subdivision_factor[0], dd.subdivision_factor[1]};
@@ -928,18 +971,31 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     for (int pi = pbeg; pi < (int)pairs.size(); ++pi) a->vleaves.back().push_back(pairs[pi].src);
     const int nx = dd.subdivision_factor[0], ny = dd.subdivision_factor[1];
     const int base = (int)cptr.size() - 1;
+    const double area = (dd.size[0] * (1.0 / (double)nx)) * (dd.size[1] * (1.0 / (double)ny));
     for (int c0 = 0; c0 < nx * ny; c0 += kRestrictCells)
-      vblocks.push_back(AmrVBlock{v, c0, base, 0});
+      vblocks.push_back(AmrVBlock{D.off, area, v, c0, base, nx, ny, D.stride});
     // per cell the pairs whose region covers it, in pair order: count, then
     // fill pair by pair (each pair marks its region's cells)
     ccount.assign((size_t)nx * ny, 0);
+    xcount.assign((size_t)nx * ny, 0);
     for (int pi = pbeg; pi < (int)pairs.size(); ++pi) {
       const AmrRestrict& R = pairs[pi];
+      int o;
+      span0.resize(R.dSize[0] > 0 ? R.dSize[0] : 0);
+      span1.resize(R.dSize[1] > 0 ? R.dSize[1] : 0);
+      for (size_t k = 0; k < span0.size(); ++k) amr_fine_span(R, 0, R.dOff[0] + (int)k, o, span0[k]);
+      for (size_t k = 0; k < span1.size(); ++k) amr_fine_span(R, 1, R.dOff[1] + (int)k, o, span1[k]);
       for (int x = R.dOff[0]; x < R.dOff[0] + R.dSize[0]; ++x)
-        for (int y = R.dOff[1]; y < R.dOff[1] + R.dSize[1]; ++y) ++ccount[(size_t)x * ny + y];
+        for (int y = R.dOff[1]; y < R.dOff[1] + R.dSize[1]; ++y) {
+          ++ccount[(size_t)x * ny + y];
+          xcount[(size_t)x * ny + y] += span0[x - R.dOff[0]] * span1[y - R.dOff[1]];
+        }
     }
     const size_t cbeg = cpairs.size();
-    for (int c = 0; c < nx * ny; ++c) cptr.push_back(cptr.back() + ccount[c]);
+    for (int c = 0; c < nx * ny; ++c) {
+      cptr.push_back(cptr.back() + ccount[c]);
+      xptr.push_back(xptr.back() + xcount[c]);
+    }
     cpairs.resize(cptr.back());
     for (int c = 0; c < nx * ny; ++c) ccount[c] = cptr[base + c] - (int)cbeg;  // cursors
     for (int pi = pbeg; pi < (int)pairs.size(); ++pi) {
@@ -1086,19 +1142,28 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   const size_t o_gmap = st.add(gmap), o_gcell0 = st.add(gcell0);
   const size_t o_cfl = st.add(nullptr, (blocks.size() + 1) * sizeof(double));
   const size_t o_leaves = st.add(a->leaves);
+  // (whole workgroups of the kernel that lists the contributions)
+  while (vblocks.size() % (256 / kRestrictCells)) {
+    vblocks.push_back(vblocks.back());
+    vblocks.back().nx = 0;
+  }
   const size_t o_vblocks = st.add(vblocks), o_cptr = st.add(cptr), o_cpairs = st.add(cpairs);
+  const size_t o_xptr = st.add(xptr);
   const size_t o_pairs = st.add(pairs), o_ghosts = st.add(gh), o_walls = st.add(wl);
   const size_t o_wall_dims = st.add(wdims);
   const std::vector<AmrClock> clk{c};
   const size_t o_clock = st.add(clk), o_next = st.add(clk);
+  // the contributions follow, listed on the device
+  const size_t o_contribs = (st.total + 255) / 256 * 256;
+  const size_t bytes = o_contribs + (size_t)xptr.back() * sizeof(AmrContrib) + 16;
   hipError_t e = hipSuccess;
-  if (p->amr_tables && p->amr_tables_cap >= st.total) {
+  if (p->amr_tables && p->amr_tables_cap >= bytes) {
     a->d_tables = p->amr_tables;  // idle: its plan was destroyed after a sync
     a->tables_cap = p->amr_tables_cap;
     p->amr_tables = nullptr;
     p->amr_tables_cap = 0;
   } else {
-    a->tables_cap = 2 * st.total;  // room for a grown grid
+    a->tables_cap = 2 * bytes;  // room for a grown grid
     e = hipMalloc(&a->d_tables, a->tables_cap);
   }
   if (e != hipSuccess) {
@@ -1121,14 +1186,24 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->d_cfl = reinterpret_cast<double*>(base + o_cfl);
   a->d_leaves = reinterpret_cast<int*>(base + o_leaves);
   a->d_vblocks = reinterpret_cast<AmrVBlock*>(base + o_vblocks);
-  a->d_cptr = reinterpret_cast<int*>(base + o_cptr);
-  a->d_cpairs = reinterpret_cast<int*>(base + o_cpairs);
-  a->d_pairs = reinterpret_cast<AmrRestrict*>(base + o_pairs);
+  a->d_xptr = reinterpret_cast<int*>(base + o_xptr);
+  a->d_contribs = reinterpret_cast<AmrContrib*>(base + o_contribs);
   a->d_ghosts = reinterpret_cast<AmrGhost*>(base + o_ghosts);
   a->d_walls = reinterpret_cast<AmrWalls*>(base + o_walls);
   a->d_wall_dims = reinterpret_cast<int*>(base + o_wall_dims);
   a->d_clock = reinterpret_cast<AmrClock*>(base + o_clock);
   a->d_clock_next = reinterpret_cast<AmrClock*>(base + o_next);
+  if (!vblocks.empty())
+    hipLaunchKernelGGL(k_amr_contribs, dim3((unsigned)(vblocks.size() * kRestrictCells / 256)),
+                       dim3(256), 0, p->stream, a->d_vblocks,
+                       reinterpret_cast<int*>(base + o_cptr),
+                       reinterpret_cast<int*>(base + o_cpairs), a->d_xptr,
+                       reinterpret_cast<AmrRestrict*>(base + o_pairs), p->d_pd, a->d_contribs);
+  if (hipGetLastError() != hipSuccess) {
+    amr_free(a);
+    delete a;
+    return fail(PC_E_HIP, "plan contributions");
+  }
   *out = a;
   return PC_OK;
 }
@@ -1184,9 +1259,9 @@ void amr_launch_leaves(pc_amr* a, Fields F, int cur) {
 int amr_launch_step(pc_amr* a, Fields F, int cur) {
   pc_pool* p = a->pool;
   if (a->nvblocks > 0)
-    hipLaunchKernelGGL(k_amr_restrict<false>, dim3(a->nvblocks), dim3(64), 0, p->stream,
-                       a->d_vblocks, a->d_cptr, a->d_cpairs, a->d_pairs, p->d_pd, F, cur,
-                       a->d_clock, a->lts);
+    hipLaunchKernelGGL(k_amr_restrict<false>, dim3(a->nvblocks), dim3(256), 0, p->stream,
+                       a->d_vblocks, a->d_xptr, a->d_contribs, a->d_leaves, F, cur, a->d_clock,
+                       a->lts);
   amr_launch_leaves<false>(a, F, cur);
   HIPCHK(hipGetLastError());
   std::swap(a->d_clock, a->d_clock_next);
@@ -1211,9 +1286,9 @@ int amr_launch_lts(pc_amr* a, Fields F, int cur) {
                        a->d_leaves, nl, a->d_nptr, a->d_nbr, a->d_vptr, a->d_vleaf, a->d_vidx,
                        a->d_rptr, a->d_rsrc, a->d_clock, L);
   if (a->nvblocks > 0)
-    hipLaunchKernelGGL(k_amr_restrict<true>, dim3(a->nvblocks), dim3(64), 0, p->stream,
-                       a->d_vblocks, a->d_cptr, a->d_cpairs, a->d_pairs, p->d_pd, F, cur,
-                       a->d_clock, L);
+    hipLaunchKernelGGL(k_amr_restrict<true>, dim3(a->nvblocks), dim3(256), 0, p->stream,
+                       a->d_vblocks, a->d_xptr, a->d_contribs, a->d_leaves, F, cur, a->d_clock,
+                       L);
   if (a->nseg_cells > 0)
     hipLaunchKernelGGL(k_lts_ghosts, dim3((a->nseg_cells + 255) / 256), dim3(256), 0, p->stream,
                        a->d_gmap, a->d_gcell0, a->nseg_cells, a->d_ghosts, p->d_pd, F, cur,
