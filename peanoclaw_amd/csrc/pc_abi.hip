@@ -110,6 +110,9 @@ struct pc_pool {
   Task* d_stasks = nullptr;
   int nstasks = 0;
   size_t stasks_cap = 0;
+  SegRec* d_segrecs = nullptr;  // per wavefront, seg_list.group each
+  size_t segrecs_cap = 0;
+  SegList seg_list{};
   SegDesc* d_segdesc = nullptr;  // per entry of the task patch list
   size_t segdesc_cap = 0;
   int nsegdesc = 0;
@@ -547,6 +550,22 @@ int build_segments(pc_pool* p) {
                         hipMemcpyHostToDevice, p->stream));
   HIPCHK(hipMemcpyAsync(p->d_ranges, ranges.data(), ranges.size() * sizeof(SegRange),
                         hipMemcpyHostToDevice, p->stream));
+  SegList& A = p->seg_list;
+  A = SegList{nullptr, 1, 0, st[0].scn};
+  int lanes = 1;
+  while (lanes < st[0].ny) lanes <<= 1;
+  A.lanes = lanes;
+  for (const Task& t : st) {
+    A.group = std::max(A.group, t.nseg);
+    if (t.ny > lanes || 2 * t.ny <= lanes) A.lanes = 0;
+    if (t.scn != A.scn) A.scn = -1;
+  }
+  const int nrec = (int)st.size() * A.group;
+  CHK(ensure_dev(&p->d_segrecs, &p->segrecs_cap, nrec));
+  A.recs = p->d_segrecs;
+  hipLaunchKernelGGL(k_seg_records, dim3((nrec + 255) / 256), dim3(256), 0, p->stream,
+                     p->d_stasks, p->d_segdesc, nrec, A.group, p->d_segrecs);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(p->stream));  // the host vectors end here
   return PC_OK;
 }
@@ -860,10 +879,10 @@ template <int R, int SOLVER>
 void launch_segments(pc_pool* p, Fields F, hipEvent_t eb, hipEvent_t ee) {
   const unsigned g = (unsigned)(p->nstasks / kSegWaves);
   hipLaunchKernelGGL((k_seg_speed<R, SOLVER>), dim3(g), dim3(64 * kSegWaves), 0, p->stream,
-                     p->d_stasks, p->d_segdesc, F, p->d_scn, p->d_smax_seg, p->d_cfl_block);
+                     p->seg_list, F, p->d_scn, p->d_smax_seg, p->d_cfl_block);
   if (eb) hipEventRecord(eb, p->stream);
   hipLaunchKernelGGL((k_seg_update<R, SOLVER>), dim3(g + 1), dim3(64 * kSegWaves), 0,
-                     p->stream, p->d_stasks, p->d_segdesc, F, p->d_scn, p->d_scn_alt,
+                     p->stream, p->seg_list, F, p->d_scn, p->d_scn_alt,
                      (int)p->scn.size(), p->d_ranges, p->d_cfl_block);
   if (ee) hipEventRecord(ee, p->stream);
   std::swap(p->d_scn, p->d_scn_alt);
@@ -1080,7 +1099,7 @@ int pc_pool_destroy(pc_pool* p) {
                   p->d_counter, p->d_iota, p->d_segmax, p->d_keep, p->d_result, p->d_aux, p->d_flags, p->d_ebuf[0],
                   p->d_ebuf[1], p->d_bcol, p->d_sides, p->d_single, p->d_single_slot,
                   p->d_edge_io, p->d_flux, p->d_batch, p->amr_tables, p->d_stasks,
-                  p->d_segdesc, p->d_smax_seg, p->d_cfl_block, p->d_ranges,
+                  p->d_segdesc, p->d_segrecs, p->d_smax_seg, p->d_cfl_block, p->d_ranges,
                   p->d_scn_alt};
   for (void* q : ptrs)
     if (q) hipFree(q);

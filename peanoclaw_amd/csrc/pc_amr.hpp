@@ -123,6 +123,10 @@ struct AmrGhost {
   int sx, sy, sox, soy, dox, doy;
   int sn[2];
   int cell0;  // its first cell among the ghost cells of its task's leaves
+  // tile rows: first cell of the source region (interpolation: cell (0, 0)
+  // of the source), first cell of the destination region
+  long long sbase, dbase;
+  int sstride, dstride;
   double spos[2], ssub[2], sinv[2], dpos[2], dsub[2];
 };
 
@@ -131,13 +135,13 @@ struct AmrWalls {
   int first, count;
 };
 
-// One task of leaves in the fill: its row segments tasks[first .. first +
-// nwaves), its leaves at plist positions [leaf0, leaf0 + nseg), its ghost
-// cells (entry of each in gmap[cell0 .. cell0 + ncells)).
+// One task of leaves in the fill (workgroup b): its row segments are
+// wavefronts [b max_waves, + nwaves) of the plan's records, its ghost cells'
+// entries gmap[b max_cells .. + ncells).
 struct AmrBlock {
-  int first, nwaves, leaf0, nseg;
+  int nwaves, leaf0, nseg;  // leaf0: place of its first leaf in task order
   int nx, ny;
-  int cell0, ncells;
+  int ncells;
   int nwalls;  // most walls of one of its leaves
   int pad;
 };
@@ -298,9 +302,8 @@ k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ xpt
 // launch, so not read here).
 template <bool LTS>
 __device__ __forceinline__ void amr_ghost_cell(const AmrGhost& g, int k,
-                                               const PatchDev* __restrict__ pd, const Fields& F,
-                                               int cur, const AmrClock& c, const AmrLts& L) {
-  const PatchDev S = pd[g.src], D = pd[g.dst];
+                                               const Fields& F, int cur, const AmrClock& c,
+                                               const AmrLts& L) {
   const int oldSt = 1 - cur;
   const int kind = g.kind;
   const double dTime = LTS ? L.t[g.dst] : c.time, dDt = LTS ? L.dt[g.dst] : c.dt;
@@ -308,7 +311,7 @@ __device__ __forceinline__ void amr_ghost_cell(const AmrGhost& g, int k,
   const double sDt = (LTS && kind != kAmrTransferVirtual) ? L.dt[g.src] : c.dt;
   const double dstTimeUNew = dTime + dDt;
   const int x = k / g.sy, y = k - (k / g.sy) * g.sy;
-  const long long di = tile_index(D, g.dox + x, g.doy + y);
+  const long long di = g.dbase + (long long)x * g.dstride + y;
   const int srcOld = LTS || kind == kAmrTransferVirtual ? oldSt : cur;
   if (kind != kAmrInterpolate) {
     // DefaultTransfer.cpph:27-51
@@ -320,7 +323,7 @@ __device__ __forceinline__ void amr_ghost_cell(const AmrGhost& g, int k,
       tf = (sNew - sOld - 0.0 > kLaEps) ? (dstTimeUNew - sOld) / (sNew - sOld) : 1.0;
     }
     const double inv = 1.0 - tf;
-    const long long si = tile_index(S, g.sox + x, g.soy + y);
+    const long long si = g.sbase + (long long)x * g.sstride + y;
     F.H(oldSt)[di] = F.H(cur)[si] * tf + F.H(srcOld)[si] * inv;
     F.HU(oldSt)[di] = F.HU(cur)[si] * tf + F.HU(srcOld)[si] * inv;
     F.HV(oldSt)[di] = F.HV(cur)[si] * tf + F.HV(srcOld)[si] * inv;
@@ -359,7 +362,7 @@ __device__ __forceinline__ void amr_ghost_cell(const AmrGhost& g, int k,
       const double sign = (double)(1 - 2 * off[d]);
       sf *= 1.0 - (sign * (cc[d] - np[d])) * g.sinv[d];
     }
-    const long long sidx = tile_index(S, nb[0], nb[1]);
+    const long long sidx = g.sbase + (long long)nb[0] * g.sstride + nb[1];
     const double bv = F.b[sidx];
     const double vo[3] = {F.H(srcOld)[sidx] + 1.0 * bv, F.HU(srcOld)[sidx], F.HV(srcOld)[sidx]};
     const double vn[3] = {F.H(cur)[sidx] + 1.0 * bv, F.HU(cur)[sidx], F.HV(cur)[sidx]};
@@ -373,25 +376,25 @@ __device__ __forceinline__ void amr_ghost_cell(const AmrGhost& g, int k,
 // Local time stepping: the ghost cells of the advancing leaves, before any
 // leaf changes (one thread per ghost cell of the plan).
 __global__ void __launch_bounds__(256)
-k_lts_ghosts(const unsigned* __restrict__ gmap, const int* __restrict__ gcell0, int ncells,
-             const AmrGhost* __restrict__ ghosts, const PatchDev* __restrict__ pd, Fields F,
-             int cur, const AmrClock* clock, AmrLts L) {
+k_lts_ghosts(const int* __restrict__ gmap, int max_cells, int ncells,
+             const AmrGhost* __restrict__ ghosts, Fields F, int cur, const AmrClock* clock,
+             AmrLts L) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= ncells || *L.iter == 0) return;
-  const unsigned e = gmap[c];
+  const int e = gmap[c];
+  if (e < 0) return;
   const AmrGhost& g = ghosts[e];
   if (!L.adv[g.dst]) return;
-  amr_ghost_cell<true>(g, c - gcell0[e], pd, F, cur, *clock, L);
+  amr_ghost_cell<true>(g, c % max_cells - g.cell0, F, cur, *clock, L);
 }
 
 // SWEKernel::fillBoundaryLayer (SWEKernel.cpp:176-237) of the leaves of a
 // task, their walls in call order (corner cells read what the previous wall
 // wrote); `adv` null: all of them.
-__device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegDesc* __restrict__ desc,
+__device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegRec* __restrict__ recs,
                                           const AmrWalls* __restrict__ walls,
-                                          const int* __restrict__ dims,
-                                          const PatchDev* __restrict__ pd, const Fields& F,
-                                          int st, const int* adv) {
+                                          const int* __restrict__ dims, const Fields& F, int st,
+                                          const int* adv) {
   const int len = (K.nx > K.ny ? K.nx : K.ny) + 2;
   for (int w = 0; w < K.nwalls; ++w) {
     for (int i = threadIdx.x; i < K.nseg * len; i += blockDim.x) {
@@ -399,9 +402,8 @@ __device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegDesc* __re
       const AmrWalls W = walls[K.leaf0 + s];
       if (w >= W.count) continue;
       const int dim = dims[2 * (W.first + w)], upper = dims[2 * (W.first + w) + 1];
-      const int slot = desc[K.leaf0 + s].slot;
-      const PatchDev P = pd[slot];
-      if (k >= (dim == 0 ? P.ny : P.nx) + 1 || (adv && !adv[slot])) continue;
+      const SegDesc P = recs[s].d;
+      if (k >= (dim == 0 ? P.ny : P.nx) + 1 || (adv && !adv[P.slot])) continue;
       int dx, dy, sx, sy;
       if (dim == 0) {
         dx = upper ? P.nx : -1;
@@ -412,7 +414,8 @@ __device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegDesc* __re
         sy = dy + (upper ? -1 : 1);
         dx = sx = k;
       }
-      const long long d = tile_index(P, dx, dy), q = tile_index(P, sx, sy);
+      const long long d = P.off + (long long)(dx + 1) * P.stride + (dy + 1);
+      const long long q = P.off + (long long)(sx + 1) * P.stride + (sy + 1);
       const double h = F.H(st)[q], hu = F.HU(st)[q], hv = F.HV(st)[q];
       F.H(st)[d] = h;
       F.HU(st)[d] = dim == 0 ? -hu : hu;
@@ -424,10 +427,10 @@ __device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegDesc* __re
 
 // What the fill and the update read of the plan.
 struct AmrPlanDev {
+  SegList list;  // ghosts in the own tile
+  int max_waves, max_cells;
   const AmrBlock* blocks;
-  const Task* tasks;
-  const SegDesc* desc;  // per leaf in task order, ghosts in the own tile
-  const unsigned* gmap;
+  const int* gmap;
   const AmrGhost* ghosts;
   const AmrWalls* walls;  // per leaf in task order
   const int* dims;
@@ -441,8 +444,9 @@ struct AmrPlanDev {
 // MAXT: most threads of a workgroup (the register budget).
 template <int R, int SOLVER, bool LTS, int MAXT>
 __global__ void __launch_bounds__(MAXT)
-k_amr_fill(AmrPlanDev A, const PatchDev* __restrict__ pd, Fields F, int cur,
-           const AmrClock* clock, double* __restrict__ cfl_block, AmrLts L) {
+__attribute__((amdgpu_waves_per_eu(4, 8)))
+k_amr_fill(AmrPlanDev A, Fields F, int cur, const AmrClock* clock,
+           double* __restrict__ cfl_block, AmrLts L) {
   __shared__ double pre[MAXT / 64][2][64];
   __shared__ double red[MAXT / 64];
   __shared__ double leaf_max[LTS ? MAXT / 64 : 1][64];
@@ -450,23 +454,24 @@ k_amr_fill(AmrPlanDev A, const PatchDev* __restrict__ pd, Fields F, int cur,
   if (!amr_phase_runs<LTS>(clock, L)) return;
   const AmrBlock K = A.blocks[blockIdx.x];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const SegRec* const recs = A.list.recs + (long long)blockIdx.x * A.max_waves * A.list.group;
   if (LTS) {
-    const bool go = lane < K.nseg && L.adv[A.desc[K.leaf0 + lane].slot] != 0;
+    const bool go = lane < K.nseg && L.adv[recs[lane].d.slot] != 0;
     if (__builtin_amdgcn_ballot_w64(go) == 0) return;  // the same in every wavefront
   }
-  Task t = gl(A.tasks + K.first + (w < K.nwaves ? w : 0));
-  if (w >= K.nwaves) t.nseg = 0;
-  SegLane g = seg_lane(t);
-  const SegDesc D = gl(A.desc + t.first + (g.segok ? g.seg : 0));
+  SegLane g = seg_lane(A.list, seg_wave(A.max_waves));
+  const SegDesc D = seg_desc(A.list, g);
   if (LTS && g.segok && !L.adv[D.slot]) g.active = false;
   const State N = state_of(F, cur), O = state_of(F, 1 - cur);
-  const int last = g.rb == t.nx ? g.rb + 1 : g.rb;
+  const int last = g.rb == g.nx ? g.rb + 1 : g.rb;
   SegRows<R, SOLVER != 0> q;
   q.template load<kRowsInterior>(D, g, N, F.b, last);
   if (!LTS)
-    for (int i = threadIdx.x; i < K.ncells; i += blockDim.x) {
-      const AmrGhost& e = A.ghosts[A.gmap[K.cell0 + i]];
-      amr_ghost_cell<false>(e, i - e.cell0, pd, F, cur, c, L);
+    for (int i = threadIdx.x; i < A.max_cells; i += blockDim.x) {
+      const int k = gl(A.gmap + (long long)blockIdx.x * A.max_cells + i);
+      if (k < 0) continue;
+      const AmrGhost& e = A.ghosts[k];
+      amr_ghost_cell<false>(e, i - e.cell0, F, cur, c, L);
     }
   // uNew -> uOld (DefaultTransfer::copyUNewToUOld)
 #pragma unroll
@@ -478,9 +483,9 @@ k_amr_fill(AmrPlanDev A, const PatchDev* __restrict__ pd, Fields F, int cur,
     gs(F.HV(1 - cur) + o, q.hv[k]);
   }
   __syncthreads();
-  amr_walls(K, A.desc, A.walls, A.dims, pd, F, 1 - cur, LTS ? L.adv : nullptr);
+  amr_walls(K, recs, A.walls, A.dims, F, 1 - cur, LTS ? L.adv : nullptr);
   q.template load<kRowsGhost>(D, g, O, F.b, last);
-  const double v = seg_speeds<R, SOLVER>(t, g, A.desc, q, last, N, O, F.b, pre[w]);
+  const double v = seg_speeds<R, SOLVER>(g, q, last, N, O, F.b, pre[w]);
   if (!LTS) {
     const double m = block_min(g.segok ? max_timestep(v, D.dx, D.dy) : kNoLimit, red);
     if (threadIdx.x == 0) gs(cfl_block + blockIdx.x, m);
@@ -489,7 +494,7 @@ k_amr_fill(AmrPlanDev A, const PatchDev* __restrict__ pd, Fields F, int cur,
   if (g.segok && g.col == 1) leaf_max[w][g.seg] = v;
   __syncthreads();
   if ((int)threadIdx.x < K.nseg) {
-    const SegDesc P = gl(A.desc + K.leaf0 + threadIdx.x);
+    const SegDesc P = gl(&(recs + threadIdx.x)->d);
     if (L.adv[P.slot]) {
       double m = leaf_max[0][threadIdx.x];
       for (int k = 1; k < K.nwaves; ++k) m = dmax(m, leaf_max[k][threadIdx.x]);
@@ -563,9 +568,8 @@ k_amr_update(AmrPlanDev A, Fields F, int cur, const AmrClock* in, AmrClock* out,
     const double m = cfl_share(all, cfl, (int)threadIdx.x, 64 * kSegWaves);
     if (lane == 0) red[w] = m;
   }
-  const Task t = gl(A.tasks + blockIdx.x * kSegWaves + w);
-  SegLane g = seg_lane(t);
-  const SegDesc D = gl(A.desc + t.first + (g.segok ? g.seg : 0));
+  SegLane g = seg_lane(A.list, seg_wave(kSegWaves));
+  const SegDesc D = seg_desc(A.list, g);
   const State O = state_of(F, 1 - cur);
   if (LTS) {
     const bool go = g.segok && L.adv[D.slot] != 0;
@@ -575,16 +579,16 @@ k_amr_update(AmrPlanDev A, Fields F, int cur, const AmrClock* in, AmrClock* out,
   }
   SegRows<R, true> q;
   q.template load<kRowsAll>(D, g, O, F.b, g.rb + 1);
-  seg_side_shares<SOLVER>(t, g, A.desc, O, F.b, pre[w]);
+  seg_side_shares<SOLVER>(g, O, F.b, pre[w]);
   if (LTS) {
     wave_sync();
   } else {
     __syncthreads();
     for (int k = 0; k < kSegWaves; ++k) dt = red[k] < dt ? red[k] : dt;
-    if (t.nseg == 0) return;
+    if (g.nseg == 0) return;
   }
-  seg_update_rows<R, SOLVER>(t, g, D, q, dt, pre[w], F.H(cur), F.HU(cur), F.HV(cur));
-  if (LTS && g.active && g.col == 1 && t.sidx == 0) {
+  seg_update_rows<R, SOLVER>(g, D, q, dt, pre[w], F.H(cur), F.HU(cur), F.HV(cur));
+  if (LTS && g.active && g.col == 1 && g.sidx == 0) {
     if (dt - 0.0 > kLaEps) {
       L.t[D.slot] = L.t[D.slot] + L.dt[D.slot];
       L.dt[D.slot] = dt;
@@ -692,12 +696,10 @@ struct pc_amr {
   int nvblocks = 0, nghosts = 0;
   // tasks of leaves, their row segments (at most seg_rows rows), and what
   // the fill reads (AmrPlanDev)
-  int seg_rows = 4, nblocks = 0, nsegs = 0, nseg_cells = 0, max_waves = 1;
+  int seg_rows = 4, nblocks = 0, nsegs = 0, max_waves = 1, max_cells = 0;
   AmrBlock* d_blocks = nullptr;
-  Task* d_tasks = nullptr;
-  SegDesc* d_desc = nullptr;
-  unsigned* d_gmap = nullptr;
-  int* d_gcell0 = nullptr;  // per ghost entry: its first cell in gmap
+  SegList list{};
+  int* d_gmap = nullptr;
   double* d_cfl = nullptr;  // per block, then the folded one
   int* d_leaves = nullptr;
   AmrVBlock* d_vblocks = nullptr;
@@ -891,26 +893,35 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   }
   for (const Task& t : tasks) {
     AmrBlock B{};
-    B.first = (int)segs.size();
     B.nwaves = seg_count(t.nx, a->seg_rows);
     B.leaf0 = t.first;
     B.nseg = t.nseg;
     B.nx = t.nx;
     B.ny = t.ny;
-    for (int k = 0; k < B.nwaves; ++k) {
-      Task u = t;
-      u.r0 = seg_first_row(k, t.nx, B.nwaves);
-      u.r1 = seg_first_row(k + 1, t.nx, B.nwaves) - 1;
-      u.sidx = k;
-      segs.push_back(u);
-    }
     a->max_waves = std::max(a->max_waves, B.nwaves);
     blocks.push_back(B);
   }
+  for (size_t b = 0; b < blocks.size(); ++b)
+    for (int k = 0; k < a->max_waves; ++k) {
+      Task u = tasks[b];
+      const int n = blocks[b].nwaves;
+      u.r0 = k < n ? seg_first_row(k, u.nx, n) : 1;
+      u.r1 = k < n ? seg_first_row(k + 1, u.nx, n) - 1 : 1;
+      u.sidx = k;
+      if (k >= n) u.nseg = 0;
+      segs.push_back(u);
+    }
   while (segs.size() % kSegWaves) {
     Task u = segs.back();
     u.nseg = 0;
     segs.push_back(u);
+  }
+  a->list.lanes = 1;
+  while (a->list.lanes < tasks[0].ny) a->list.lanes <<= 1;
+  a->list.group = 1;
+  for (const Task& t : tasks) {
+    a->list.group = std::max(a->list.group, t.nseg);
+    if (a->list.lanes && (t.ny > a->list.lanes || 2 * t.ny <= a->list.lanes)) a->list.lanes = 0;
   }
   a->nblocks = (int)blocks.size();
   a->nsegs = (int)segs.size();
@@ -1079,6 +1090,11 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     } else {
       return bail("ghost kind must be 0 (transfer) or 1 (interpolation)");
     }
+    const Slot &ss = p->slots[s], &ds = p->slots[d];
+    g.sbase = ss.off + (long long)(g.sox + 1) * ss.stride + (g.soy + 1);
+    g.dbase = ds.off + (long long)(g.dox + 1) * ds.stride + (g.doy + 1);
+    g.sstride = ss.stride;
+    g.dstride = ds.stride;
     gh.push_back(g);
   }
   a->nghosts = (int)gh.size();
@@ -1087,8 +1103,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   std::vector<int> block_of(plist.size());
   for (size_t b = 0; b < blocks.size(); ++b)
     for (int k = 0; k < blocks[b].nseg; ++k) block_of[blocks[b].leaf0 + k] = (int)b;
-  std::vector<int> gcell0(gh.size());
-  std::vector<unsigned> gmap;
+  std::vector<int> gmap;
   {
     std::vector<int> b_of(gh.size());
     for (size_t e = 0; e < gh.size(); ++e) {
@@ -1096,19 +1111,13 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
       AmrBlock& B = blocks[b_of[e]];
       gh[e].cell0 = B.ncells;
       B.ncells += gh[e].sx * gh[e].sy;
+      a->max_cells = std::max(a->max_cells, B.ncells);
     }
-    int top = 0;
-    for (AmrBlock& B : blocks) {
-      B.cell0 = top;
-      top += B.ncells;
-    }
-    gmap.resize(top);
-    for (size_t e = 0; e < gh.size(); ++e) {
-      gcell0[e] = blocks[b_of[e]].cell0 + gh[e].cell0;
-      std::fill_n(gmap.begin() + gcell0[e], gh[e].sx * gh[e].sy, (unsigned)e);
-    }
+    gmap.assign(blocks.size() * (size_t)a->max_cells, -1);
+    for (size_t e = 0; e < gh.size(); ++e)
+      std::fill_n(gmap.begin() + (size_t)b_of[e] * a->max_cells + gh[e].cell0,
+                  gh[e].sx * gh[e].sy, (int)e);
   }
-  a->nseg_cells = (int)gmap.size();
   // walls grouped per leaf in call order
   std::vector<AmrWalls> wl(plist.size(), AmrWalls{0, 0});
   for (int i = 0; i < nwalls; ++i) {
@@ -1139,7 +1148,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   // DMA instead of fifteen of each)
   PinnedTables st;
   const size_t o_blocks = st.add(blocks), o_tasks = st.add(segs), o_desc = st.add(desc);
-  const size_t o_gmap = st.add(gmap), o_gcell0 = st.add(gcell0);
+  const size_t o_gmap = st.add(gmap);
   const size_t o_cfl = st.add(nullptr, (blocks.size() + 1) * sizeof(double));
   const size_t o_leaves = st.add(a->leaves);
   // (whole workgroups of the kernel that lists the contributions)
@@ -1153,8 +1162,10 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   const size_t o_wall_dims = st.add(wdims);
   const std::vector<AmrClock> clk{c};
   const size_t o_clock = st.add(clk), o_next = st.add(clk);
-  // the contributions follow, listed on the device
-  const size_t o_contribs = (st.total + 255) / 256 * 256;
+  // the records and contributions follow, made on the device
+  const int nrec = (int)segs.size() * a->list.group;
+  const size_t o_recs = (st.total + 255) / 256 * 256;
+  const size_t o_contribs = o_recs + (size_t)nrec * sizeof(SegRec);
   const size_t bytes = o_contribs + (size_t)xptr.back() * sizeof(AmrContrib) + 16;
   hipError_t e = hipSuccess;
   if (p->amr_tables && p->amr_tables_cap >= bytes) {
@@ -1179,10 +1190,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   }
   char* const base = a->d_tables;
   a->d_blocks = reinterpret_cast<AmrBlock*>(base + o_blocks);
-  a->d_tasks = reinterpret_cast<Task*>(base + o_tasks);
-  a->d_desc = reinterpret_cast<SegDesc*>(base + o_desc);
-  a->d_gmap = reinterpret_cast<unsigned*>(base + o_gmap);
-  a->d_gcell0 = reinterpret_cast<int*>(base + o_gcell0);
+  a->d_gmap = reinterpret_cast<int*>(base + o_gmap);
   a->d_cfl = reinterpret_cast<double*>(base + o_cfl);
   a->d_leaves = reinterpret_cast<int*>(base + o_leaves);
   a->d_vblocks = reinterpret_cast<AmrVBlock*>(base + o_vblocks);
@@ -1193,6 +1201,12 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->d_wall_dims = reinterpret_cast<int*>(base + o_wall_dims);
   a->d_clock = reinterpret_cast<AmrClock*>(base + o_clock);
   a->d_clock_next = reinterpret_cast<AmrClock*>(base + o_next);
+  a->list.recs = reinterpret_cast<SegRec*>(base + o_recs);
+  a->list.scn = 0;  // the plan has its own clock
+  hipLaunchKernelGGL(k_seg_records, dim3((nrec + 255) / 256), dim3(256), 0, p->stream,
+                     reinterpret_cast<Task*>(base + o_tasks),
+                     reinterpret_cast<SegDesc*>(base + o_desc), nrec, a->list.group,
+                     reinterpret_cast<SegRec*>(base + o_recs));
   if (!vblocks.empty())
     hipLaunchKernelGGL(k_amr_contribs, dim3((unsigned)(vblocks.size() * kRestrictCells / 256)),
                        dim3(256), 0, p->stream, a->d_vblocks,
@@ -1213,8 +1227,8 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
 namespace {
 
 AmrPlanDev amr_plan(const pc_amr* a) {
-  return AmrPlanDev{a->d_blocks, a->d_tasks, a->d_desc,     a->d_gmap,
-                    a->d_ghosts, a->d_walls, a->d_wall_dims};
+  return AmrPlanDev{a->list,   a->max_waves, a->max_cells, a->d_blocks,
+                    a->d_gmap, a->d_ghosts,  a->d_walls,   a->d_wall_dims};
 }
 
 template <int R, int SOLVER, bool LTS>
@@ -1224,10 +1238,10 @@ void amr_launch_segments(pc_amr* a, Fields F, int cur) {
   const dim3 b(64 * a->max_waves);
   if (a->max_waves <= 8)
     hipLaunchKernelGGL((k_amr_fill<R, SOLVER, LTS, 512>), dim3(a->nblocks), b, 0, p->stream, A,
-                       p->d_pd, F, cur, a->d_clock, a->d_cfl, a->lts);
+                       F, cur, a->d_clock, a->d_cfl, a->lts);
   else
     hipLaunchKernelGGL((k_amr_fill<R, SOLVER, LTS, 1024>), dim3(a->nblocks), b, 0, p->stream, A,
-                       p->d_pd, F, cur, a->d_clock, a->d_cfl, a->lts);
+                       F, cur, a->d_clock, a->d_cfl, a->lts);
   const double* cfl = a->d_cfl;
   int ncfl = a->nblocks;
   if (!LTS && ncfl > kCflFold) {
@@ -1289,10 +1303,10 @@ int amr_launch_lts(pc_amr* a, Fields F, int cur) {
     hipLaunchKernelGGL(k_amr_restrict<true>, dim3(a->nvblocks), dim3(256), 0, p->stream,
                        a->d_vblocks, a->d_xptr, a->d_contribs, a->d_leaves, F, cur, a->d_clock,
                        L);
-  if (a->nseg_cells > 0)
-    hipLaunchKernelGGL(k_lts_ghosts, dim3((a->nseg_cells + 255) / 256), dim3(256), 0, p->stream,
-                       a->d_gmap, a->d_gcell0, a->nseg_cells, a->d_ghosts, p->d_pd, F, cur,
-                       a->d_clock, L);
+  const int ncells = a->nblocks * a->max_cells;
+  if (ncells > 0)
+    hipLaunchKernelGGL(k_lts_ghosts, dim3((ncells + 255) / 256), dim3(256), 0, p->stream,
+                       a->d_gmap, a->max_cells, ncells, a->d_ghosts, F, cur, a->d_clock, L);
   amr_launch_leaves<true>(a, F, cur);
   HIPCHK(hipGetLastError());
   return PC_OK;

@@ -40,6 +40,41 @@ struct SegDesc {
   double dx, dy, dxinv, dyinv;
 };
 
+// What one wavefront reads first: records recs[wave * group .. + nseg) of the
+// patches of its task with the rows it takes.  A kernel starts on cold caches
+// (another XCD wrote what it reads), every dependent load costs 0.7-0.9 us,
+// and a record's place follows from the wavefront's number alone, so cells
+// are one load away instead of three (task -> patch list -> patch).
+struct alignas(128) SegRec {
+  SegDesc d;
+  int r0, r1, sidx, nseg;
+};
+
+// The records of a launch.  lanes: lanes per patch (columns rounded up to a
+// power of two) where it is the same for all, else 0; scn: likewise the
+// scenario, else -1.
+struct SegList {
+  const SegRec* recs;
+  int group, lanes, scn;
+};
+
+// Records from tasks and patch descriptions, one thread per record.
+__global__ void __launch_bounds__(256)
+k_seg_records(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, int n, int group,
+              SegRec* __restrict__ recs) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= n) return;
+  const Task t = tasks[k / group];
+  const int s = k % group;
+  SegRec r;
+  r.d = desc[t.first + (s < t.nseg ? s : 0)];
+  r.r0 = t.r0;
+  r.r1 = t.r1;
+  r.sidx = t.sidx;
+  r.nseg = t.nseg;
+  recs[k] = r;
+}
+
 // Slots per patch of the segments' speed maxima (nx <= 64 rows).
 constexpr int kSegSlots = 64;
 constexpr int kSegWaves = 4;  // wavefronts (independent tasks) per workgroup
@@ -105,23 +140,42 @@ __device__ __forceinline__ CellQ left_cell(const CellQ& c) {
 
 // The rows of one wavefront and the lanes' places in them.
 struct SegLane {
+  const SegRec* recs;    // of this wavefront
   int ra, rb, rows;      // interior rows ra..rb of the patch
+  int nx, ny, nseg, sidx;
+  int lanes;             // per patch
   int seg, col;          // patch of the task, 1-based interior column
   bool segok, active;
 };
 
-__device__ __forceinline__ SegLane seg_lane(const Task& t) {
+__device__ __forceinline__ SegLane seg_lane(const SegList& A, int wave) {
   SegLane g;
   const int lane = threadIdx.x & 63;
-  const int W = pow2ceil(t.ny);
-  g.ra = t.r0;
-  g.rb = t.r1;
-  g.rows = t.r1 - t.r0 + 1;
-  g.seg = lane / W;
-  g.col = lane - g.seg * W + 1;
-  g.segok = g.seg < t.nseg;
-  g.active = g.segok && g.col <= t.ny;
+  g.recs = A.recs + (long long)wave * A.group;
+  g.ra = gl(&g.recs->r0);
+  g.rb = gl(&g.recs->r1);
+  g.sidx = gl(&g.recs->sidx);
+  g.nseg = gl(&g.recs->nseg);
+  g.nx = gl(&g.recs->d.nx);
+  g.ny = gl(&g.recs->d.ny);
+  g.rows = g.rb - g.ra + 1;
+  g.lanes = A.lanes ? A.lanes : pow2ceil(g.ny);
+  g.seg = lane / g.lanes;
+  g.col = lane - g.seg * g.lanes + 1;
+  g.segok = g.seg < g.nseg;
+  g.active = g.segok && g.col <= g.ny;
   return g;
+}
+
+// The lane's patch (read without waiting for the wavefront's record: its
+// place needs the number of lanes only).
+__device__ __forceinline__ SegDesc seg_desc(const SegList& A, const SegLane& g) {
+  return gl(&(g.recs + (g.seg < A.group ? g.seg : 0))->d);
+}
+
+// This thread's wavefront among those of the launch's workgroups, uniform.
+__device__ __forceinline__ int seg_wave(int waves) {
+  return __builtin_amdgcn_readfirstlane((int)blockIdx.x * waves + (int)(threadIdx.x >> 6));
 }
 
 // h, hu, hv of one state.
@@ -176,14 +230,13 @@ struct SegSide {
   int slot, side;
   double hL, hvL, bL, hR, hvR, bR, dyinv;
   template <bool B>
-  __device__ __forceinline__ void load(const SegDesc* __restrict__ desc, const Task& t,
-                                       const SegLane& g, int e, const State& S,
+  __device__ __forceinline__ void load(const SegLane& g, int e, const State& S,
                                        const State& G, const double* Bf) {
     side = e & 1;
     const int s = (e >> 1) / g.rows;
     const int row = g.ra + (e >> 1) - s * g.rows;
     slot = e >> 1;
-    const SegDesc Q = gl(desc + t.first + s);
+    const SegDesc Q = gl(&(g.recs + s)->d);
     dyinv = Q.dyinv;
     const long long at = Q.off + (long long)row * Q.stride;
     const long long io = at + (side ? Q.ny : 1);
@@ -202,17 +255,16 @@ struct SegSide {
 // patch.  `pre`: this wavefront's LDS.  The edge below the last row belongs
 // to the next segment (`last`: the last row loaded).
 template <int R, int SOLVER>
-__device__ __forceinline__ double seg_speeds(const Task& t, const SegLane& g,
-                                             const SegDesc* __restrict__ desc,
+__device__ __forceinline__ double seg_speeds(const SegLane& g,
                                              const SegRows<R, SOLVER != 0>& q, int last,
                                              const State& S, const State& G, const double* Bf,
                                              double (*pre)[64]) {
   using ES = EdgeSolver<SOLVER>;
   constexpr bool B = SOLVER != 0;  // the f-wave's speeds do not depend on b
-  const int npre = t.nseg * g.rows * 2;
+  const int npre = g.nseg * g.rows * 2;
   for (int e = threadIdx.x & 63; e < npre; e += 64) {
     SegSide s;
-    s.load<B>(desc, t, g, e, S, G, Bf);
+    s.load<B>(g, e, S, G, Bf);
     const CellQ cl = cell_dir(cell_base(s.hL, s.bL), s.hvL);
     const CellQ cr = cell_dir(cell_base(s.hR, s.bR), s.hvR);
     pre[s.side][s.slot] = ES::speed(cl, cr);
@@ -248,26 +300,24 @@ __device__ __forceinline__ double seg_speeds(const Task& t, const SegLane& g,
     }
   }
   wave_sync();
-  if (g.active && (g.col == 1 || g.col == t.ny))
+  if (g.active && (g.col == 1 || g.col == g.ny))
     for (int k = 0; k < g.rows; ++k) {
       if (g.col == 1) sm = dmax(sm, pre[0][g.seg * g.rows + k]);
-      if (g.col == t.ny) sm = dmax(sm, pre[1][g.seg * g.rows + k]);
+      if (g.col == g.ny) sm = dmax(sm, pre[1][g.seg * g.rows + k]);
     }
   double v = g.active ? sm : 0.0;
-  for (int m = pow2ceil(t.ny) >> 1; m >= 1; m >>= 1) v = dmax(v, __shfl_xor(v, m));
+  for (int m = g.lanes >> 1; m >= 1; m >>= 1) v = dmax(v, __shfl_xor(v, m));
   return v;
 }
 
 // Shares of the segment's ghost-column y-edges, into this wavefront's LDS.
 template <int SOLVER>
-__device__ __forceinline__ void seg_side_shares(const Task& t, const SegLane& g,
-                                                const SegDesc* __restrict__ desc,
-                                                const State& S, const double* Bf,
-                                                double (*pre)[64]) {
-  const int npre = t.nseg * g.rows * 2;
+__device__ __forceinline__ void seg_side_shares(const SegLane& g, const State& S,
+                                                const double* Bf, double (*pre)[64]) {
+  const int npre = g.nseg * g.rows * 2;
   for (int e = threadIdx.x & 63; e < npre; e += 64) {
     SegSide s;
-    s.load<true>(desc, t, g, e, S, S, Bf);
+    s.load<true>(g, e, S, S, Bf);
     const CellQ cl = cell_dir(cell_base(s.hL, s.bL), s.hvL);
     const CellQ cr = cell_dir(cell_base(s.hR, s.bR), s.hvR);
     double dhL, dhR, dqL, dqR;
@@ -282,8 +332,8 @@ __device__ __forceinline__ void seg_side_shares(const Task& t, const SegLane& g,
 // Update of the segment's rows by dt, written to (Hd, HUd, HVd); `pre` holds
 // seg_side_shares.
 template <int R, int SOLVER>
-__device__ __forceinline__ void seg_update_rows(const Task& t, const SegLane& g,
-                                                const SegDesc& D, const SegRows<R, true>& q,
+__device__ __forceinline__ void seg_update_rows(const SegLane& g, const SegDesc& D,
+                                                const SegRows<R, true>& q,
                                                 double dt, double (*pre)[64],
                                                 double* __restrict__ Hd,
                                                 double* __restrict__ HUd,
@@ -387,7 +437,7 @@ __device__ __forceinline__ void seg_update_rows(const Task& t, const SegLane& g,
           uph = pre[0][slot];
           upq = pre[1][slot];
         }
-        if (k < g.rows && g.active && g.col == t.ny) {
+        if (k < g.rows && g.active && g.col == g.ny) {
           dnh = pre[2][slot];
           dnq = pre[3][slot];
         }
@@ -412,21 +462,20 @@ __device__ __forceinline__ double block_min(double v, double* red) {
 // with the speed, so the minimum over segments is the minimum over patches.
 template <int R, int SOLVER>
 __global__ void __launch_bounds__(64 * kSegWaves)
-k_seg_speed(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
-            const ScnDev* __restrict__ scn, double* __restrict__ smax_seg,
+k_seg_speed(SegList A, Fields F, const ScnDev* __restrict__ scn, double* __restrict__ smax_seg,
             double* __restrict__ cfl_block) {
   __shared__ double pre[kSegWaves][2][64];
   __shared__ double red[kSegWaves];
   const int w = threadIdx.x >> 6;
-  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
-  const SegLane g = seg_lane(t);
-  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
-  const State S = state_of(F, gl(&scn[t.scn].stepc) & 1);
-  const int last = g.rb == t.nx ? g.rb + 1 : g.rb;
+  const SegLane g = seg_lane(A, seg_wave(kSegWaves));
+  const SegDesc D = seg_desc(A, g);
+  const int s = A.scn >= 0 ? A.scn : gl(&g.recs->d.scn);
+  const State S = state_of(F, gl(&scn[s].stepc) & 1);
+  const int last = g.rb == g.nx ? g.rb + 1 : g.rb;
   SegRows<R, SOLVER != 0> q;
   q.template load<kRowsAll>(D, g, S, F.b, last);
-  const double v = seg_speeds<R, SOLVER>(t, g, desc, q, last, S, S, F.b, pre[w]);
-  if (g.segok && g.col == 1) gs(smax_seg + (long long)D.slot * kSegSlots + t.sidx, v);
+  const double v = seg_speeds<R, SOLVER>(g, q, last, S, S, F.b, pre[w]);
+  if (g.segok && g.col == 1) gs(smax_seg + (long long)D.slot * kSegSlots + g.sidx, v);
   const double c = block_min(g.segok ? max_timestep(v, D.dx, D.dy) : kNoLimit, red);
   if (threadIdx.x == 0) gs(cfl_block + blockIdx.x, c);
 }
@@ -468,9 +517,9 @@ __device__ __forceinline__ double cfl_share(const SegRange& r,
 template <int R, int SOLVER>
 __global__ void __launch_bounds__(64 * kSegWaves)
 __attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
-k_seg_update(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, Fields F,
-             const ScnDev* __restrict__ in, ScnDev* __restrict__ out, int nscn,
-             const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block) {
+k_seg_update(SegList A, Fields F, const ScnDev* __restrict__ in, ScnDev* __restrict__ out,
+             int nscn, const SegRange* __restrict__ ranges,
+             const double* __restrict__ cfl_block) {
   __shared__ double pre[kSegWaves][4][64];
   __shared__ double red[kSegWaves];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -485,25 +534,25 @@ k_seg_update(const Task* __restrict__ tasks, const SegDesc* __restrict__ desc, F
     }
     return;
   }
-  const Task t = gl(tasks + blockIdx.x * kSegWaves + w);
-  const SegLane g = seg_lane(t);
-  const SegDesc D = gl(desc + t.first + (g.segok ? g.seg : 0));
-  const ScnDev* C = in + t.scn;  // one scenario per workgroup
+  const SegLane g = seg_lane(A, seg_wave(kSegWaves));
+  const SegDesc D = seg_desc(A, g);
+  const int s = A.scn >= 0 ? A.scn : gl(&g.recs->d.scn);  // one per workgroup
+  const ScnDev* C = in + s;
   const double max_dt = gl(&C->end_time) - (gl(&C->time) + gl(&C->dt));
   if (!(max_dt - 0.0 > kLaEps)) return;
   const int par = gl(&C->stepc) & 1;
   const State S = state_of(F, par);
   SegRows<R, true> q;
   q.template load<kRowsAll>(D, g, S, F.b, g.rb + 1);
-  const double share = cfl_share(gl(ranges + t.scn), cfl_block, (int)threadIdx.x,
+  const double share = cfl_share(gl(ranges + s), cfl_block, (int)threadIdx.x,
                                  64 * kSegWaves);
   if (lane == 0) red[w] = share;
-  seg_side_shares<SOLVER>(t, g, desc, S, F.b, pre[w]);
+  seg_side_shares<SOLVER>(g, S, F.b, pre[w]);
   __syncthreads();
   double dt = max_dt;
   for (int k = 0; k < kSegWaves; ++k) dt = fmin(red[k], dt);
-  if (t.nseg == 0) return;
-  seg_update_rows<R, SOLVER>(t, g, D, q, dt, pre[w], F.H(1 - par), F.HU(1 - par),
+  if (g.nseg == 0) return;
+  seg_update_rows<R, SOLVER>(g, D, q, dt, pre[w], F.H(1 - par), F.HU(1 - par),
                              F.HV(1 - par));
 }
 
