@@ -1525,23 +1525,6 @@ static int plan_transform(pc_pool* p, int slot, const int off[2], const int size
   return PC_OK;
 }
 
-static int launch_transform(pc_pool* p, const TransformItem& it) {
-  const int n = it.sx * it.sy;
-  if (n <= 0) return PC_OK;
-  hipLaunchKernelGGL(k_transform, dim3((n + 255) / 256), dim3(256), 0, p->stream, p->d_pd,
-                     it.slot, fields_of(p), it.st, it.ox, it.oy, it.sx, it.sy, it.sign,
-                     it.unew_layout);
-  HIPCHK(hipGetLastError());
-  return PC_OK;
-}
-
-static int transform(pc_pool* p, int slot, const int off[2], const int size[2], int uold,
-                     int to_above_sea_floor) {
-  TransformItem it;
-  CHK(plan_transform(p, slot, off, size, uold, to_above_sea_floor, it));
-  return launch_transform(p, it);
-}
-
 // Region::mapToPatch (Region.cpp:174-206)
 static void map_to_patch(const int off[2], const int size[2], const PatchDev& src,
                          const pc_cell_description& sd, const PatchDev& dst,
@@ -1567,15 +1550,10 @@ static void map_to_patch(const int off[2], const int size[2], const PatchDev& sr
 // DefaultInterpolation.cpph:29-270), planned and checked before anything
 // runs: the source region (grown by one cell) to h + b in both states, the
 // interpolation, both back to h, the destination region back to h.
-struct InterpPlan {
-  InterpArgs a;
-  int n;  // destination cells
-  TransformItem fwd[2], back[3];
-};
-
 static int plan_interpolation(pc_pool* p, const int dsize[2], const int doff[2], int src,
                               int dst, int toUOld, int toCurrentTime, int useTimeUNewOrUOld,
-                              InterpPlan& out) {
+                              InterpCall& out) {
+  out = InterpCall{};
   if (!valid_slot(p, src) || !valid_slot(p, dst) || !dsize || !doff)
     return fail(PC_E_INVALID, "invalid argument");
   const auto& sd = p->slots[src].desc;
@@ -1633,6 +1611,8 @@ static int plan_interpolation(pc_pool* p, const int dsize[2], const int doff[2],
   a.dpos[0] = dd.position[0]; a.dpos[1] = dd.position[1];
   a.dsub[0] = D.dx; a.dsub[1] = D.dy;
   a.sn[0] = sn[0]; a.sn[1] = sn[1];
+  out.S = S;
+  out.D = D;
   out.n = dsize[0] * dsize[1];
   return PC_OK;
 }
@@ -1643,18 +1623,12 @@ int pc_interpolate_solution(pc_pool* p, const int dsize[2], const int doff[2], i
     return fail(PC_E_INVALID, "invalid argument");
   hipSetDevice(p->device);
   CHK(prepare(p));
-  InterpPlan pl;
-  CHK(plan_interpolation(p, dsize, doff, src, dst, toUOld, toCurrentTime, useTimeUNewOrUOld,
-                         pl));
+  InterpCall c;
+  CHK(plan_interpolation(p, dsize, doff, src, dst, toUOld, toCurrentTime, useTimeUNewOrUOld, c));
   mark_state_changed(p);
-  CHK(launch_transform(p, pl.fwd[0]));
-  CHK(launch_transform(p, pl.fwd[1]));
-  if (pl.n > 0) {
-    hipLaunchKernelGGL(k_interpolate, dim3((pl.n + 127) / 128), dim3(128), 0, p->stream,
-                       p->d_pd, fields_of(p), pl.a);
-    HIPCHK(hipGetLastError());
-  }
-  for (const TransformItem& it : pl.back) CHK(launch_transform(p, it));
+  hipLaunchKernelGGL(k_level_call<InterpCall>, dim3(1), dim3(kCallThreads), 0, p->stream,
+                     fields_of(p), c);
+  HIPCHK(hipGetLastError());
   return PC_OK;
 }
 
@@ -1710,14 +1684,9 @@ static int overlapped_regions(const double lower[2], const double upper[2],
 // DefaultRestriction.cpph:16-142), planned and checked before anything runs:
 // the source to h + b in both states, its (up to four) regions accumulated
 // into the destination in order, the source back to h.
-struct RestrictPlan {
-  TransformItem fwd[2], back[2];
-  RestrictArgs r[4];
-  int nr;  // non-empty regions, in the reference's order
-};
-
 static int plan_restriction(pc_pool* p, int src, int dst, int onlyOverlapped,
-                            RestrictPlan& out) {
+                            RestrictCall& out) {
+  out = RestrictCall{};
   if (!valid_slot(p, src) || !valid_slot(p, dst))
     return fail(PC_E_INVALID, "invalid slot");
   const auto& sd = p->slots[src].desc;
@@ -1778,6 +1747,8 @@ static int plan_restriction(pc_pool* p, int src, int dst, int onlyOverlapped,
         return fail(PC_E_INVALID, "restriction source is not inside the destination");
     if (a.dSize[0] * a.dSize[1] > 0) out.r[out.nr++] = a;
   }
+  out.S = S;
+  out.D = D;
   return PC_OK;
 }
 
@@ -1786,19 +1757,12 @@ int pc_restrict_solution(pc_pool* p, int src, int dst, int onlyOverlapped) {
     return fail(PC_E_INVALID, "invalid slot");
   hipSetDevice(p->device);
   CHK(prepare(p));
-  RestrictPlan pl;
-  CHK(plan_restriction(p, src, dst, onlyOverlapped, pl));
+  RestrictCall c;
+  CHK(plan_restriction(p, src, dst, onlyOverlapped, c));
   mark_state_changed(p);
-  CHK(launch_transform(p, pl.fwd[0]));
-  CHK(launch_transform(p, pl.fwd[1]));
-  for (int r = 0; r < pl.nr; ++r) {
-    const int n = pl.r[r].dSize[0] * pl.r[r].dSize[1];
-    hipLaunchKernelGGL(k_restrict, dim3((n + 63) / 64), dim3(64), 0, p->stream, p->d_pd,
-                       fields_of(p), pl.r[r]);
-    HIPCHK(hipGetLastError());
-  }
-  CHK(launch_transform(p, pl.back[0]));
-  CHK(launch_transform(p, pl.back[1]));
+  hipLaunchKernelGGL(k_level_call<RestrictCall>, dim3(1), dim3(kCallThreads), 0, p->stream,
+                     fields_of(p), c);
+  HIPCHK(hipGetLastError());
   return PC_OK;
 }
 
@@ -1807,10 +1771,50 @@ int pc_restrict_solution(pc_pool* p, int src, int dst, int onlyOverlapped) {
 // ---- batched level transfers ----
 //
 // A batch is exactly the sequence of its per-call entry points.  Calls that
-// share no patch commute, so each call goes to the first wave after every
-// earlier call it shares a source or destination with; a wave runs as a few
-// launches with one item per call (blockIdx.y).  Everything is checked
+// share no patch commute.  Calls linked by shared patches form a sequence;
+// all sequences run in one launch, a workgroup each (k_level_calls).  Where
+// few links join many calls (a sequence over four times as long as the
+// longest chain of conflicts; a call takes a workgroup about 3 us, a wave's
+// launches about 12 us), each call goes to the first wave after every
+// earlier call it shares a source or destination with, and a wave runs as a
+// few launches with one item per call (blockIdx.y).  Everything is checked
 // before anything runs.
+
+// Calls grouped by shared patches, each group in the given order: order[]
+// holds the calls, first[g] .. first[g + 1] those of group g.
+struct CallGroups {
+  std::vector<int> order, first;
+  int longest = 0;
+};
+static CallGroups call_groups(int count, const int* a, const int* b, int nslots) {
+  std::vector<int> root(nslots);
+  for (int i = 0; i < nslots; ++i) root[i] = i;
+  auto find = [&](int s) {
+    while (root[s] != s) s = root[s] = root[root[s]];
+    return s;
+  };
+  for (int i = 0; i < count; ++i) root[find(a[i])] = find(b[i]);
+  CallGroups g;
+  std::vector<int> id(nslots, -1), of(count), size;
+  for (int i = 0; i < count; ++i) {
+    int& k = id[find(a[i])];
+    if (k < 0) {
+      k = (int)size.size();
+      size.push_back(0);
+    }
+    of[i] = k;
+    ++size[k];
+  }
+  g.first.assign(size.size() + 1, 0);
+  for (size_t k = 0; k < size.size(); ++k) {
+    g.first[k + 1] = g.first[k] + size[k];
+    g.longest = std::max(g.longest, size[k]);
+  }
+  std::vector<int> at(g.first.begin(), g.first.end() - 1);
+  g.order.resize(count);
+  for (int i = 0; i < count; ++i) g.order[at[of[i]]++] = i;
+  return g;
+}
 
 // Wave of every call: one more than the latest wave of an earlier call that
 // touches either of its two patches.
@@ -1898,6 +1902,25 @@ static int upload_staging(pc_pool* p, const Staging& st) {
 
 constexpr int kMaxBatchY = 65535;  // grid y limit: items per launch
 
+// The groups' calls as sequences, one launch.
+template <class Call>
+static int launch_call_groups(pc_pool* p, const std::vector<Call>& calls, const CallGroups& g) {
+  std::vector<Call> v;
+  v.reserve(calls.size());
+  for (int i : g.order) v.push_back(calls[i]);
+  Staging st;
+  const size_t oc = st.add(v), of = st.add(g.first);
+  CHK(upload_staging(p, st));
+  hipLaunchKernelGGL(k_level_calls<Call>, dim3((unsigned)g.first.size() - 1),
+                     dim3(kCallThreads), 0, p->stream, fields_of(p),
+                     reinterpret_cast<const Call*>(p->d_batch + oc),
+                     reinterpret_cast<const int*>(p->d_batch + of));
+  HIPCHK(hipGetLastError());
+  // the host image of the calls lives until the copy has been consumed
+  HIPCHK(hipStreamSynchronize(p->stream));
+  return PC_OK;
+}
+
 static int launch_transform_batch(pc_pool* p, size_t off, const std::vector<TransformItem>& v) {
   int most = 0;
   for (const auto& it : v) most = std::max(most, it.sx * it.sy);
@@ -1934,12 +1957,17 @@ int pc_interpolate_batch(pc_pool* p, int count, const int* dsize, const int* dof
   if (count == 0) return PC_OK;
   hipSetDevice(p->device);
   CHK(prepare(p));
-  std::vector<InterpPlan> pl(count);
+  std::vector<InterpCall> pl(count);
   for (int i = 0; i < count; ++i)
     CHK(plan_interpolation(p, dsize + 2 * i, doff + 2 * i, src[i], dst[i], opts[3 * i],
                            opts[3 * i + 1], opts[3 * i + 2], pl[i]));
   int nw = 0;
   const std::vector<int> wave = conflict_waves(count, src, dst, &nw);
+  const CallGroups groups = call_groups(count, src, dst, (int)p->slots.size());
+  if (groups.longest <= 4 * nw) {
+    mark_state_changed(p);
+    return launch_call_groups(p, pl, groups);
+  }
   std::vector<std::vector<TransformItem>> fwd(nw), back(nw);
   std::vector<std::vector<InterpArgs>> interp(nw);
   std::vector<int> most(nw, 0);
@@ -1986,10 +2014,15 @@ int pc_restrict_batch(pc_pool* p, int count, const int* src, const int* dst,
   if (count == 0) return PC_OK;
   hipSetDevice(p->device);
   CHK(prepare(p));
-  std::vector<RestrictPlan> pl(count);
+  std::vector<RestrictCall> pl(count);
   for (int i = 0; i < count; ++i) CHK(plan_restriction(p, src[i], dst[i], onlyOverlapped, pl[i]));
   int nw = 0;
   const std::vector<int> wave = conflict_waves(count, src, dst, &nw);
+  const CallGroups groups = call_groups(count, src, dst, (int)p->slots.size());
+  if (groups.longest <= 4 * nw) {
+    mark_state_changed(p);
+    return launch_call_groups(p, pl, groups);
+  }
   // per wave: forward transforms, region k of every call (k = 0..3, in the
   // order of each call's regions), back transforms
   std::vector<std::vector<TransformItem>> fwd(nw), back(nw);
@@ -2246,8 +2279,12 @@ int pc_post_process_restriction(pc_pool* p, int dst, int onlyOverlapped) {
   const int z[2] = {0, 0};
   const int dn[2] = {p->slots[dst].desc.subdivision_factor[0],
                      p->slots[dst].desc.subdivision_factor[1]};
-  CHK(transform(p, dst, z, dn, 1, 1));
-  CHK(transform(p, dst, z, dn, 0, 1));
+  TransformPair t;
+  CHK(plan_transform(p, dst, z, dn, 1, 1, t.item[0]));
+  CHK(plan_transform(p, dst, z, dn, 0, 1, t.item[1]));
+  hipLaunchKernelGGL(k_transform_pair, dim3((dn[0] * dn[1] + 255) / 256, 2), dim3(256), 0,
+                     p->stream, p->d_pd, fields_of(p), t);
+  HIPCHK(hipGetLastError());
   return PC_OK;
 }
 

@@ -196,13 +196,10 @@ __global__ void k_copy_swap(const PatchDev* __restrict__ pd, int slot, Fields F,
 // addresses element x*ny + y of that array: unknown q = idx / (nx ny) at
 // (x', y') = ((idx mod nx ny) / ny, idx mod ny).  With unew_layout set the
 // kernel writes that element, as the reference does; b is read at (x, y).
-__device__ __forceinline__ void transform_cell(const PatchDev& P, const Fields& F, int st,
-                                               int ox, int oy, int sy, double sign,
-                                               int unew_layout, int k) {
-  const int x = ox + k / sy, y = oy + (k - (k / sy) * sy);
-  const long long ib = tile_index(P, x, y);
+__device__ __forceinline__ double* transform_target(const PatchDev& P, const Fields& F, int st,
+                                                    int x, int y, int unew_layout) {
   double* f = F.H(st);
-  long long i = ib;
+  long long i = tile_index(P, x, y);
   if (unew_layout && (x >= P.nx || y >= P.ny)) {
     const int lin = x * P.ny + y;
     const int area = P.nx * P.ny;
@@ -210,29 +207,40 @@ __device__ __forceinline__ void transform_cell(const PatchDev& P, const Fields& 
     f = q == 0 ? F.H(st) : (q == 1 ? F.HU(st) : F.HV(st));
     i = tile_index(P, r / P.ny, r - (r / P.ny) * P.ny);
   }
-  f[i] = f[i] + sign * F.b[ib];
+  return f + i;
+}
+__device__ __forceinline__ void transform_cell(const PatchDev& P, const Fields& F, int st,
+                                               int ox, int oy, int sy, double sign,
+                                               int unew_layout, int k) {
+  const int x = ox + k / sy, y = oy + (k - (k / sy) * sy);
+  double* const f = transform_target(P, F, st, x, y, unew_layout);
+  *f = *f + sign * F.b[tile_index(P, x, y)];
 }
 
-__global__ void k_transform(const PatchDev* __restrict__ pd, int slot, Fields F,
-                            int st, int ox, int oy, int sx, int sy, double sign,
-                            int unew_layout) {
-  const PatchDev P = pd[slot];
-  for (int k = threadIdx.x + blockIdx.x * blockDim.x; k < sx * sy;
-       k += blockDim.x * gridDim.x)
-    transform_cell(P, F, st, ox, oy, sy, sign, unew_layout, k);
-}
-
-// One region transform of a batch (the arguments of one k_transform launch).
+// One region transform.
 struct TransformItem {
   int slot, st, ox, oy, sx, sy, unew_layout, pad;
   double sign;
 };
 
-// Batched k_transform: item blockIdx.y, its region cells over blockIdx.x.
+// Independent transforms: item blockIdx.y, its region cells over blockIdx.x.
 // The items of one launch touch disjoint memory.
 __global__ void k_transform_batch(const PatchDev* __restrict__ pd, Fields F,
                                   const TransformItem* __restrict__ items) {
   const TransformItem it = items[blockIdx.y];
+  const PatchDev P = pd[it.slot];
+  for (int k = threadIdx.x + blockIdx.x * blockDim.x; k < it.sx * it.sy;
+       k += blockDim.x * gridDim.x)
+    transform_cell(P, F, it.st, it.ox, it.oy, it.sy, it.sign, it.unew_layout, k);
+}
+
+// The two transforms of a postProcessRestriction (uOld and uNew of a patch).
+struct TransformPair {
+  TransformItem item[2];
+};
+__global__ void __launch_bounds__(256)
+k_transform_pair(const PatchDev* __restrict__ pd, Fields F, TransformPair t) {
+  const TransformItem it = t.item[blockIdx.y];
   const PatchDev P = pd[it.slot];
   for (int k = threadIdx.x + blockIdx.x * blockDim.x; k < it.sx * it.sy;
        k += blockDim.x * gridDim.x)
@@ -261,9 +269,7 @@ __device__ __forceinline__ void interp_cell(const PatchDev& S, const PatchDev& D
   } else {
     dq[0] = F.H(a.dstCur); dq[1] = F.HU(a.dstCur); dq[2] = F.HV(a.dstCur);
   }
-  F.H(dOld)[di] = 0.0;
-  F.HU(dOld)[di] = 0.0;
-  F.HV(dOld)[di] = 0.0;
+  double* const old[3] = {F.H(dOld), F.HU(dOld), F.HV(dOld)};  // zeroed in any case
   double c[2];
   c[0] = a.dpos[0] + a.dsub[0] * (double)x + a.dsub[0] * 0.5;
   c[1] = a.dpos[1] + a.dsub[1] * (double)y + a.dsub[1] * 0.5;
@@ -277,6 +283,11 @@ __device__ __forceinline__ void interp_cell(const PatchDev& S, const PatchDev& D
     si[d] = v;
   }
   const double tf = a.tf;
+  // sums in registers, so that all loads are in flight together: uOld starts
+  // from zero, uNew from its own value
+  double acc[3] = {0.0, 0.0, 0.0};
+  if (!a.toUOld)
+    for (int q = 0; q < 3; ++q) acc[q] = dq[q][di];
   for (int o = 0; o < 4; ++o) {
     const int off[2] = {o & 1, (o >> 1) & 1};
     const int nb[2] = {si[0] + off[0], si[1] + off[1]};
@@ -294,23 +305,18 @@ __device__ __forceinline__ void interp_cell(const PatchDev& S, const PatchDev& D
     for (int q = 0; q < 3; ++q) {
       const double vo = so[q][si_], vn = sn[q][si_];
       if (a.toUOld)
-        dq[q][di] = dq[q][di] + sf * (vo * (1.0 - tf) + vn * tf);
+        acc[q] = acc[q] + sf * (vo * (1.0 - tf) + vn * tf);
       else
-        dq[q][di] = dq[q][di] + sf * vo * (1.0 - tf) + sf * vn * tf;
+        acc[q] = acc[q] + sf * vo * (1.0 - tf) + sf * vn * tf;
     }
   }
+  if (!a.toUOld)
+    for (int q = 0; q < 3; ++q) old[q][di] = 0.0;
+  for (int q = 0; q < 3; ++q) dq[q][di] = acc[q];
 }
 
-// One thread per destination cell.
-__global__ void k_interpolate(const PatchDev* __restrict__ pd, Fields F, InterpArgs a) {
-  const PatchDev S = pd[a.srcSlot], D = pd[a.dstSlot];
-  for (int k = threadIdx.x + blockIdx.x * blockDim.x; k < a.sx * a.sy;
-       k += blockDim.x * gridDim.x)
-    interp_cell(S, D, F, a, k);
-}
-
-// Batched k_interpolate: call blockIdx.y, its destination cells over
-// blockIdx.x; the calls of one launch touch disjoint patches.
+// Independent interpolations (no shared patch): call blockIdx.y, its
+// destination cells over blockIdx.x.
 __global__ void k_interpolate_batch(const PatchDev* __restrict__ pd, Fields F,
                                     const InterpArgs* __restrict__ items) {
   const InterpArgs a = items[blockIdx.y];
@@ -356,41 +362,51 @@ __device__ __forceinline__ void restrict_cell(const PatchDev& S, const PatchDev&
   const int dOldSt = 1 - a.dstCur, sOldSt = 1 - a.srcCur;
   double accO[3] = {F.H(dOldSt)[di], F.HU(dOldSt)[di], F.HV(dOldSt)[di]};
   double accN[3] = {F.H(a.dstCur)[di], F.HU(a.dstCur)[di], F.HV(a.dstCur)[di]};
+  // kAhead fine cells' loads at a time, summed in order
+  constexpr int kAhead = 3;
+  const double *so[3] = {F.H(sOldSt), F.HU(sOldSt), F.HV(sOldSt)};
+  const double *sn[3] = {F.H(a.srcCur), F.HU(a.srcCur), F.HV(a.srcCur)};
   for (int sx = 0; sx < cSize[0]; ++sx)
-    for (int sy = 0; sy < cSize[1]; ++sy) {
-      const int s0 = cOff[0] + sx, s1 = cOff[1] + sy;
-      const double sp[2] = {a.spos[0] + (double)s0 * a.srcSub[0],
-                            a.spos[1] + (double)s1 * a.srcSub[1]};
-      double region = 1.0;
-      for (int d = 0; d < 2; ++d) {
-        const double hi = dmin(dp[d] + a.dstSub[d], sp[d] + a.srcSub[d]);
-        const double lo = dmax(dp[d], sp[d]);
-        region *= hi - lo;
-        region = dmax(region, 0.0);
+    for (int y0 = 0; y0 < cSize[1]; y0 += kAhead) {
+      double vo[kAhead][3], vn[kAhead][3];
+#pragma unroll
+      for (int m = 0; m < kAhead; ++m) {
+        // (past the end: the last cell again, not used)
+        const int sy = y0 + m < cSize[1] ? y0 + m : cSize[1] - 1;
+        const long long si = tile_index(S, cOff[0] + sx, cOff[1] + sy);
+        for (int q = 0; q < 3; ++q) {
+          vo[m][q] = gl(so[q] + si);
+          vn[m][q] = gl(sn[q] + si);
+        }
       }
-      const long long si = tile_index(S, s0, s1);
-      const double vo[3] = {F.H(sOldSt)[si], F.HU(sOldSt)[si], F.HV(sOldSt)[si]};
-      const double vn[3] = {F.H(a.srcCur)[si], F.HU(a.srcCur)[si], F.HV(a.srcCur)[si]};
-      for (int q = 0; q < 3; ++q) {
-        const double dO = (vo[q] * (1.0 - a.tfOld) + vn[q] * a.tfOld) * region / a.dstRegion;
-        const double dN = (vo[q] * (1.0 - a.tfNew) + vn[q] * a.tfNew) * region / a.dstRegion;
-        accO[q] = accO[q] + dO;
-        accN[q] = accN[q] + dN;
+#pragma unroll
+      for (int m = 0; m < kAhead; ++m) {
+        if (y0 + m >= cSize[1]) break;
+        const int s0 = cOff[0] + sx, s1 = cOff[1] + y0 + m;
+        const double sp[2] = {a.spos[0] + (double)s0 * a.srcSub[0],
+                              a.spos[1] + (double)s1 * a.srcSub[1]};
+        double region = 1.0;
+        for (int d = 0; d < 2; ++d) {
+          const double hi = dmin(dp[d] + a.dstSub[d], sp[d] + a.srcSub[d]);
+          const double lo = dmax(dp[d], sp[d]);
+          region *= hi - lo;
+          region = dmax(region, 0.0);
+        }
+        for (int q = 0; q < 3; ++q) {
+          const double dO =
+              (vo[m][q] * (1.0 - a.tfOld) + vn[m][q] * a.tfOld) * region / a.dstRegion;
+          const double dN =
+              (vo[m][q] * (1.0 - a.tfNew) + vn[m][q] * a.tfNew) * region / a.dstRegion;
+          accO[q] = accO[q] + dO;
+          accN[q] = accN[q] + dN;
+        }
       }
     }
   F.H(dOldSt)[di] = accO[0]; F.HU(dOldSt)[di] = accO[1]; F.HV(dOldSt)[di] = accO[2];
   F.H(a.dstCur)[di] = accN[0]; F.HU(a.dstCur)[di] = accN[1]; F.HV(a.dstCur)[di] = accN[2];
 }
 
-// One thread per destination cell.
-__global__ void k_restrict(const PatchDev* __restrict__ pd, Fields F, RestrictArgs a) {
-  const PatchDev S = pd[a.srcSlot], D = pd[a.dstSlot];
-  const int n = a.dSize[0] * a.dSize[1];
-  for (int k = threadIdx.x + blockIdx.x * blockDim.x; k < n; k += blockDim.x * gridDim.x)
-    restrict_cell(S, D, F, a, k);
-}
-
-// Batched k_restrict: region blockIdx.y, its destination cells over
+// Independent restrictions: region blockIdx.y, its destination cells over
 // blockIdx.x; the regions of one launch write disjoint destination patches.
 __global__ void k_restrict_batch(const PatchDev* __restrict__ pd, Fields F,
                                  const RestrictArgs* __restrict__ items) {
@@ -401,10 +417,107 @@ __global__ void k_restrict_batch(const PatchDev* __restrict__ pd, Fields F,
     restrict_cell(S, D, F, a, k);
 }
 
+// ---- whole level-transfer calls, one workgroup each ----
+//
+// interpolateSolution is three dependent phases (source to h + b in both
+// states, the interpolation, source and destination back to h),
+// restrictSolution two around its up to four regions.  A launch per phase
+// made a call five or six launches of 2-8 us for a few hundred cells; here a
+// workgroup runs a call's phases with barriers between them, and a sequence
+// of calls that share patches one after another.  The calls' descriptions
+// are read ahead into LDS, so a phase waits for its cells only.  A regrid's
+// 432 interpolations and 216 restrictions (24 patches of 16^2 refined and 24
+// coarsened) went from 81 launches, 0.72 ms of kernels, to two.
+constexpr int kCallThreads = 512;
+
+struct InterpCall {
+  PatchDev S, D;
+  InterpArgs a;
+  int n;  // destination cells
+  int pad;
+  TransformItem fwd[2], back[3];
+};
+
+struct RestrictCall {
+  PatchDev S, D;
+  TransformItem fwd[2], back[2];
+  RestrictArgs r[4];
+  int nr;  // non-empty regions, in the reference's order
+  int pad;
+};
+
+__device__ __forceinline__ void run_transform(const PatchDev& P, const Fields& F,
+                                              const TransformItem& it) {
+  for (int k = threadIdx.x; k < it.sx * it.sy; k += blockDim.x)
+    transform_cell(P, F, it.st, it.ox, it.oy, it.sy, it.sign, it.unew_layout, k);
+}
+
+// The transforms of one region in uOld and uNew (two states, so disjoint),
+// their loads together.
+__device__ __forceinline__ void run_transforms(const PatchDev& P, const Fields& F,
+                                               const TransformItem* it) {
+  const int n = it[0].sx * it[0].sy;
+  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    const int x = it[0].ox + k / it[0].sy, y = it[0].oy + (k - (k / it[0].sy) * it[0].sy);
+    double* const f0 = transform_target(P, F, it[0].st, x, y, it[0].unew_layout);
+    double* const f1 = transform_target(P, F, it[1].st, x, y, it[1].unew_layout);
+    const double b = gl(F.b + tile_index(P, x, y)), h0 = gl(f0), h1 = gl(f1);
+    gs(f0, h0 + it[0].sign * b);
+    gs(f1, h1 + it[1].sign * b);
+  }
+}
+
+__device__ __forceinline__ void run_call(const InterpCall& c, const Fields& F) {
+  run_transforms(c.S, F, c.fwd);
+  __syncthreads();
+  for (int k = threadIdx.x; k < c.n; k += blockDim.x) interp_cell(c.S, c.D, F, c.a, k);
+  __syncthreads();
+  run_transforms(c.S, F, c.back);
+  if (c.a.srcSlot == c.a.dstSlot) __syncthreads();
+  run_transform(c.D, F, c.back[2]);
+}
+
+__device__ __forceinline__ void run_call(const RestrictCall& c, const Fields& F) {
+  run_transforms(c.S, F, c.fwd);
+  for (int r = 0; r < c.nr; ++r) {
+    __syncthreads();
+    const int n = c.r[r].dSize[0] * c.r[r].dSize[1];
+    for (int k = threadIdx.x; k < n; k += blockDim.x) restrict_cell(c.S, c.D, F, c.r[r], k);
+  }
+  __syncthreads();
+  run_transforms(c.S, F, c.back);
+}
+
+// One call (its description in the kernel arguments).
+template <class Call>
+__global__ void __launch_bounds__(kCallThreads)
+k_level_call(Fields F, Call c) {
+  run_call(c, F);
+}
+
+// Sequences of calls, one per workgroup: calls[first[b] .. first[b + 1]) in
+// order; no patch belongs to two sequences.
+template <class Call>
+__global__ void __launch_bounds__(kCallThreads)
+k_level_calls(Fields F, const Call* __restrict__ calls, const int* __restrict__ first) {
+  static_assert(sizeof(Call) % sizeof(double) == 0, "copied in doubles");
+  constexpr int N = sizeof(Call) / sizeof(double);
+  __shared__ double buf[2][N];
+  const int b = first[blockIdx.x], e = first[blockIdx.x + 1];
+  auto fetch = [&](int c) {
+    for (int k = threadIdx.x; k < N; k += blockDim.x)
+      buf[(c - b) & 1][k] = reinterpret_cast<const double*>(calls + c)[k];
+  };
+  fetch(b);
+  __syncthreads();
+  for (int c = b; c < e; ++c) {
+    if (c + 1 < e) fetch(c + 1);
+    run_call(*reinterpret_cast<const Call*>(buf[(c - b) & 1]), F);
+    __syncthreads();
+  }
+}
+
 // Patch::switchToLeaf (Patch.cpp:793-830) of a batch of patches (patch
-// blockIdx.y): the [0, 1]-basis values of the restriction evaluated at the
-// leaf's interval, uOld = vo (1 - fOld) + vn fOld and uNew = vo (1 - fNew)
-// + vn fNew over the interior cells.
 struct LeafSwitch {
   int slot, cur;
   double fOld, fNew;
