@@ -302,9 +302,9 @@ int pc_set_wave_propagation_solver(pc_pool *pool, int solver);
  * not depend on slack; slack < 1 makes every step take the fallback. */
 int pc_set_prune_slack(pc_pool *pool, double slack);
 /* Row segments of the batched update (no reference counterpart): 0 =
- * automatic (a step with fewer tasks than the GPU holds splits the rows of
- * each patch into 2 or 4 segments of at least 8 rows, each marched by its
- * own wavefront; with still fewer, into segments of at most 4 rows whose
+ * automatic (a step whose tasks would leave part of the GPU idle splits the
+ * rows of each patch into 2 or 4 segments of at least 8 rows, each marched by
+ * its own wavefront; with few tasks, into segments of at most 4 rows whose
  * speeds are exact in every launch mode), 1 = whole patches, 2 or 4 = that many segments where the
  * patch has at least 8 rows per segment.  Results do not depend on it. */
 int pc_set_row_segments(pc_pool *pool, int segments);
@@ -331,9 +331,10 @@ int pc_pool_slot_capacity(pc_pool *pool, int *n);
 int pc_scenario_mass(pc_pool *pool, int scenario, double *out);
 /* Device time (ms) of the last pc_step_all / pc_graph_replay call measured
  * with HIP events on the pool stream, and (pc_step_all only) the mean
- * duration of one update-kernel launch over that call's steps, from an
- * event pair recorded around every update launch (steps of so few patches
- * that they run on short row segments: around the last one). */
+ * duration of one update-kernel launch over that call's steps, from event
+ * pairs recorded around every eighth update launch and the last one (steps
+ * of so few patches that they run on short row segments: the last one; a
+ * pair leaves the GPU idle for some microseconds). */
 int pc_last_timing(pc_pool *pool, double *total_ms, double *update_ms);
 
 /* Diagnostic: run the pool's device edge solver on n host edges

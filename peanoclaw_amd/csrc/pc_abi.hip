@@ -570,6 +570,51 @@ int build_segments(pc_pool* p) {
   return PC_OK;
 }
 
+// Row segments the march gives a patch of nx rows: at most `want`, of at
+// least 8 rows each.
+int segments_of(int nx, int want) {
+  int r = want;
+  while (r > 1 && nx / r < 8) r /= 2;
+  return r;
+}
+
+// Row segments of the march's update.  A SIMD runs up to 3 of its wavefronts
+// together; measured on 64-row patches, 1, 2 and 3 together take 96, 123 and
+// 138 us, so a last round that is nearly empty costs most of a full one.
+// With n wavefronts a SIMD, a list takes floor(n / 3) rounds of 3 and one of
+// the rest; a segment of m rows reads two more.  The count is the smallest
+// that this model does not put 5% above another.  Us of the update for 1, 2,
+// 4 segments (the model takes 4, 4, 2, 2, 1, 4, 2):
+//   40 x 40 patches of 64^2: 123 116 102   56 x 56: 222 188 180
+//   80 x 80 of 64^2: 366 334 340           90 x 90 of 32^2: 139 123 141
+//   100 x 100 of 48^2: 338 344 401         24 x 24 of 64^2: 96 57 46
+//   32 x 32 of 64^2: 97 73 73
+int march_split(const std::vector<Task>& tasks) {
+  constexpr double kSimds = 1024, kTogether[4] = {0.0, 96.0, 123.0, 138.0};
+  if (tasks.empty()) return 1;
+  auto cost = [&](int s) {
+    double rows = 0.0, longest = 0.0;
+    for (const Task& t : tasks) {
+      const int r = segments_of(t.nx, s);
+      rows += t.nx + 2.0 * r;
+      longest = std::max(longest, (double)t.nx / r + 2.0);
+    }
+    const double n = rows / longest / kSimds;  // equal wavefronts a SIMD
+    const double full = std::floor(n / 3.0);
+    return (full * kTogether[3] + kTogether[(int)std::ceil(n - 3.0 * full)]) * longest;
+  };
+  int want = 1;
+  double best = cost(1);
+  for (int s = 2; s <= kMaxRowSeg; s *= 2) {
+    const double c = cost(s);
+    if (c < 0.95 * best) {
+      best = c;
+      want = s;
+    }
+  }
+  return want;
+}
+
 // Work list: tasks of same-size patches of one scenario, large sizes first.
 int rebuild_topology(pc_pool* p) {
   if (!p->topo_dirty) return PC_OK;
@@ -677,23 +722,14 @@ int rebuild_topology(pc_pool* p) {
     p->h_tasks.push_back(t);
   }
   p->ntasks = (int)p->h_tasks.size();
-  // the update's tasks: below the number of wavefronts the GPU holds at the
-  // update's occupancy, the rows of each patch are split into row segments
-  // (at least 8 rows each), so a small step is not bound by the march of
-  // whole patches
+  // the update's tasks: the rows of each patch split into row segments where
+  // whole patches would leave SIMDs idle
   std::vector<Task> utasks;
   std::vector<int> rseg_of(ns, 1);
   {
-    constexpr int kFill = 3 * 1024;  // 3 waves on each of the 1024 SIMDs
-    int want = 1;
-    if (p->row_segments == 0) {
-      while (want < kMaxRowSeg && (long long)p->ntasks * want * 2 <= kFill) want *= 2;
-    } else {
-      want = p->row_segments;
-    }
+    const int want = p->row_segments ? p->row_segments : march_split(p->h_tasks);
     for (const Task& t : p->h_tasks) {
-      int r = want;
-      while (r > 1 && t.nx / r < 8) r /= 2;
+      const int r = segments_of(t.nx, want);
       for (int k = 0; k < r; ++k) {
         Task u = t;
         u.r0 = seg_first_row(k, t.nx, r);
@@ -2676,32 +2712,40 @@ int pc_step_all(pc_pool* p, int k) {
   if (!p || k < 0) return fail(PC_E_INVALID, "invalid argument");
   hipSetDevice(p->device);
   CHK(prepare_batched(p));
-  // one event pair around every update launch: the update kernel's mean
-  // duration over exactly these k steps.  On short row segments around the
-  // last one only: a pair leaves the GPU idle for about 8 us, half of such a
-  // step.
-  const int first = p->seg_rows && k > 0 ? k - 1 : 0;
-  while (p->upd_ev.size() < 2 * (size_t)(k - first)) {
-    hipEvent_t e;
-    HIPCHK(hipEventCreate(&e));
-    p->upd_ev.push_back(e);
-  }
+  // an event pair around every kTimedEvery-th update launch and the last one
+  // (short row segments: the last one only): a pair leaves the GPU idle for 5
+  // to 8 us
+  constexpr int kTimedEvery = 8;
+  auto timed = [&](int i) {
+    return i == k - 1 || (!p->seg_rows && (k - 1 - i) % kTimedEvery == 0);
+  };
+  int ntimed = 0;
   HIPCHK(hipEventRecord(p->ev0, p->stream));
-  for (int i = 0; i < first; ++i) CHK(launch_step(p, false));
-  for (int i = 0; i < k - first; ++i)
-    CHK(launch_step(p, true, p->upd_ev[2 * i], p->upd_ev[2 * i + 1]));
+  for (int i = 0; i < k; ++i) {
+    if (!timed(i)) {
+      CHK(launch_step(p, false));
+      continue;
+    }
+    while (p->upd_ev.size() < 2 * (size_t)(ntimed + 1)) {
+      hipEvent_t e;
+      HIPCHK(hipEventCreate(&e));
+      p->upd_ev.push_back(e);
+    }
+    CHK(launch_step(p, true, p->upd_ev[2 * ntimed], p->upd_ev[2 * ntimed + 1]));
+    ++ntimed;
+  }
   HIPCHK(hipEventRecord(p->ev1, p->stream));
   HIPCHK(hipEventSynchronize(p->ev1));
   HIPCHK(hipEventElapsedTime(&p->last_total_ms, p->ev0, p->ev1));
   p->last_update_ms = 0.f;
   if (k > 0 && p->ntasks > 0) {
     double sum = 0.0;
-    for (int i = 0; i < k - first; ++i) {
+    for (int i = 0; i < ntimed; ++i) {
       float ms = 0.f;
       HIPCHK(hipEventElapsedTime(&ms, p->upd_ev[2 * i], p->upd_ev[2 * i + 1]));
       sum += ms;
     }
-    p->last_update_ms = (float)(sum / (k - first));
+    p->last_update_ms = (float)(sum / ntimed);
   }
   p->scn_host_stale = true;
   mark_batched_clock(p);

@@ -1097,6 +1097,27 @@ k_dt_block(ScnDev* __restrict__ scn, int nscn, const int* __restrict__ plist_scn
   if (mode == 2 && gl(redo) == 0) return;
   if (mode == 1 && threadIdx.x == 0) *redo = 0;
   const int lane = threadIdx.x & 63;
+  if (nscn == 1) {
+    // one scenario: its minimum through LDS, no atomics (1600 patches: 8.1
+    // us with them)
+    __shared__ double red[16];
+    double m = 1.7976931348623157e308;
+    for (int k = threadIdx.x; k < nentries; k += blockDim.x) {
+      const int p = gl(plist_scn + k);
+      const double v = max_timestep(gl(smax + p), gl(&pd[p].dx), gl(&pd[p].dy));
+      gs(est_patch + p, v);
+      m = dmin(m, v);
+    }
+    for (int o = 32; o >= 1; o >>= 1) m = dmin(m, __shfl_xor(m, o));
+    if (lane == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int k = 1; k < (int)blockDim.x / 64; ++k) m = dmin(m, red[k]);
+      if (counter) *counter = 0;
+      dt_final_one(scn[0], m, mode, redo, slack);
+    }
+    return;
+  }
   for (int k0 = threadIdx.x - lane; k0 < nentries; k0 += blockDim.x) {
     const int k = k0 + lane;
     const bool ok = k < nentries;

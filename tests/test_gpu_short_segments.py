@@ -90,3 +90,39 @@ def test_tile_ghosts(solver):
 @pytest.mark.parametrize("solver", [1, 2])
 def test_longer_segments(solver):
     _equal([(63, 40, 8, 7)], solver, 2, True, False, 4)
+
+
+# march steps whose whole patches would leave SIMDs idle are split (here into
+# four): the same bits as whole patches
+def test_split_march():
+    def run(segments):
+        with PatchPool(0) as pool:
+            layouts = []
+            rng = np.random.default_rng(3)
+            px = py = 42
+            grid = -np.ones((px, py), dtype=np.int32)
+            tile = 66 * 80
+            pool.reserve(px * py * (tile + 16))
+            for k in range(px * py):
+                i, j = divmod(k, py)
+                grid[i, j] = pool.register(make_description((i, j), 1.0, 64))
+            o = [pool.offset(int(s)) for s in grid.ravel()]
+            cells = o[-1] + tile - o[0]
+            f = [rng.uniform(0.5, 2.0, cells) * a for a in (1.0, 0.3, 0.3, 0.1)]
+            pool.copy_fields(True, 0, o[0], *f)
+            layouts.append(GridLayout(64, grid))
+            wl = Workload(pool, layouts, 0, 0, [])
+            wl.build_ghost_table()
+            pool.scenario_set(0, 0.0, 0.0, math.inf)
+            pool.launch_config(fused=2)
+            pool.row_segments(segments)
+            pool.step(3)
+            out = [np.empty(cells) for _ in range(3)]
+            pool.copy_fields(False, 1, o[0], *out)
+            out = [a[:px * py * tile - 80].reshape(-1)[:(px * py - 1) * tile]
+                   .reshape(-1, 66, 80)[:, 1:-1, 1:65] for a in out]
+            return out, pool.scenario_get(0)
+    (a, ta), (b, tb) = run(0), run(1)
+    assert ta == tb
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
