@@ -176,6 +176,10 @@ struct pc_pool {
   // pinned host staging for large synchronous uploads (plan tables)
   char* h_stage = nullptr;
   size_t h_stage_cap = 0;
+  // one patch's arrays in pinned host memory (pc_patch_upload / download) and
+  // their device address
+  double* h_patch_io = nullptr;
+  double* d_patch_io = nullptr;
   // graph
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -1141,6 +1145,7 @@ int pc_pool_destroy(pc_pool* p) {
     if (q) hipFree(q);
   if (p->h_result) hipHostFree(p->h_result);
   if (p->h_stage) hipHostFree(p->h_stage);
+  if (p->h_patch_io) hipHostFree(p->h_patch_io);
   for (hipEvent_t e : p->upd_ev) hipEventDestroy(e);
   hipEventDestroy(p->ev0);
   hipEventDestroy(p->ev1);
@@ -1293,33 +1298,44 @@ int pc_patch_set_description(pc_pool* p, int slot, const pc_cell_description* d)
   return PC_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// The pinned buffer of one patch's arrays (the largest patch's; the calls
+// that use it wait for the GPU before they return).
+int patch_io_buffer(pc_pool* p, double** host) {
+  if (!p->h_patch_io) {
+    HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&p->h_patch_io),
+                         (size_t)patch_io_size(64, 64) * sizeof(double),
+                         hipHostMallocMapped | hipHostMallocCoherent));
+    HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void**>(&p->d_patch_io), p->h_patch_io, 0));
+  }
+  *host = p->h_patch_io;
+  return PC_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int pc_patch_upload(pc_pool* p, int slot, const double* unew, const double* uold,
                     const double* b) {
   if (!valid_slot(p, slot)) return fail(PC_E_INVALID, "invalid slot");
   hipSetDevice(p->device);
   CHK(sync_scn_host(p));
-  const Slot& s = p->slots[slot];
-  const int nx = s.desc.subdivision_factor[0], ny = s.desc.subdivision_factor[1];
-  const int cur = cur_of(p, slot);
-  // host arrays in the reference layout (rows of ny, or ny + 2 with the
-  // ghost ring), tile rows of s.stride
-  const size_t w = (size_t)(ny + 2), area = (size_t)(nx + 2) * w, pitch = s.stride * sizeof(double);
-  if (unew) {
-    for (int q = 0; q < 3; ++q) {
-      double* dst = p->f[2 * q + cur] + s.off + s.stride + 1;
-      HIPCHK(hipMemcpy2DAsync(dst, pitch, unew + (size_t)q * nx * ny, ny * sizeof(double),
-                              ny * sizeof(double), nx, hipMemcpyHostToDevice, p->stream));
-    }
+  double* host;
+  CHK(patch_io_buffer(p, &host));
+  const PatchDev P = make_patchdev(p->slots[slot]);
+  const size_t n3 = 3 * (size_t)P.nx * P.ny, a = (size_t)(P.nx + 2) * (P.ny + 2);
+  if (unew) std::memcpy(host, unew, n3 * sizeof(double));
+  if (uold) std::memcpy(host + n3, uold, 3 * a * sizeof(double));
+  if (b) std::memcpy(host + n3 + 3 * a, b, a * sizeof(double));
+  const int what = (unew ? kIoNew : 0) | (uold ? kIoOld : 0) | (b ? kIoB : 0);
+  if (what) {
+    hipLaunchKernelGGL(k_patch_io<true>, dim3((patch_io_size(P.nx, P.ny) + 255) / 256),
+                       dim3(256), 0, p->stream, P, fields_of(p), cur_of(p, slot),
+                       p->d_patch_io, what);
+    HIPCHK(hipGetLastError());
   }
-  if (uold) {
-    for (int q = 0; q < 3; ++q)
-      HIPCHK(hipMemcpy2DAsync(p->f[2 * q + 1 - cur] + s.off, pitch, uold + q * area,
-                              w * sizeof(double), w * sizeof(double), nx + 2,
-                              hipMemcpyHostToDevice, p->stream));
-  }
-  if (b)
-    HIPCHK(hipMemcpy2DAsync(p->f[6] + s.off, pitch, b, w * sizeof(double), w * sizeof(double),
-                            nx + 2, hipMemcpyHostToDevice, p->stream));
   HIPCHK(hipStreamSynchronize(p->stream));
   mark_state_changed(p);
   return PC_OK;
@@ -1329,27 +1345,21 @@ int pc_patch_download(pc_pool* p, int slot, double* unew, double* uold, double* 
   if (!valid_slot(p, slot)) return fail(PC_E_INVALID, "invalid slot");
   hipSetDevice(p->device);
   CHK(sync_scn_host(p));
-  const Slot& s = p->slots[slot];
-  const int nx = s.desc.subdivision_factor[0], ny = s.desc.subdivision_factor[1];
-  const int cur = cur_of(p, slot);
-  const size_t w = (size_t)(ny + 2), area = (size_t)(nx + 2) * w, pitch = s.stride * sizeof(double);
-  if (unew) {
-    for (int q = 0; q < 3; ++q) {
-      const double* src = p->f[2 * q + cur] + s.off + s.stride + 1;
-      HIPCHK(hipMemcpy2DAsync(unew + (size_t)q * nx * ny, ny * sizeof(double), src, pitch,
-                              ny * sizeof(double), nx, hipMemcpyDeviceToHost, p->stream));
-    }
+  double* host;
+  CHK(patch_io_buffer(p, &host));
+  const PatchDev P = make_patchdev(p->slots[slot]);
+  const size_t n3 = 3 * (size_t)P.nx * P.ny, a = (size_t)(P.nx + 2) * (P.ny + 2);
+  const int what = (unew ? kIoNew : 0) | (uold ? kIoOld : 0) | (b ? kIoB : 0);
+  if (what) {
+    hipLaunchKernelGGL(k_patch_io<false>, dim3((patch_io_size(P.nx, P.ny) + 255) / 256),
+                       dim3(256), 0, p->stream, P, fields_of(p), cur_of(p, slot),
+                       p->d_patch_io, what);
+    HIPCHK(hipGetLastError());
   }
-  if (uold) {
-    for (int q = 0; q < 3; ++q)
-      HIPCHK(hipMemcpy2DAsync(uold + q * area, w * sizeof(double), p->f[2 * q + 1 - cur] + s.off,
-                              pitch, w * sizeof(double), nx + 2, hipMemcpyDeviceToHost,
-                              p->stream));
-  }
-  if (b)
-    HIPCHK(hipMemcpy2DAsync(b, w * sizeof(double), p->f[6] + s.off, pitch, w * sizeof(double),
-                            nx + 2, hipMemcpyDeviceToHost, p->stream));
   HIPCHK(hipStreamSynchronize(p->stream));
+  if (unew) std::memcpy(unew, host, n3 * sizeof(double));
+  if (uold) std::memcpy(uold, host + n3, 3 * a * sizeof(double));
+  if (b) std::memcpy(b, host + n3 + 3 * a, a * sizeof(double));
   return PC_OK;
 }
 

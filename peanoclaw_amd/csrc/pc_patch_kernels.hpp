@@ -38,6 +38,44 @@ __device__ __forceinline__ void signal_done(double* out, unsigned long long seq)
                      __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A patch's arrays between its tile and a buffer in pinned host memory that
+// holds them as the reference lays them out: uNew (3 nx ny), uOld (3 (nx + 2)
+// (ny + 2)), b ((nx + 2) (ny + 2)); `what`: which of the three move (bits
+// kIoNew, kIoOld, kIoB).  The GPU reads or writes the host buffer itself: one
+// launch for up to seven strided arrays.  As seven pitched copies from and to
+// pageable memory an upload of a 16^2 patch took 1.05 ms.
+enum PatchIo { kIoNew = 1, kIoOld = 2, kIoB = 4 };
+__host__ __device__ __forceinline__ int patch_io_size(int nx, int ny) {
+  return 3 * nx * ny + 4 * (nx + 2) * (ny + 2);
+}
+template <bool UPLOAD>
+__global__ void __launch_bounds__(256)
+k_patch_io(PatchDev P, Fields F, int cur, double* __restrict__ host, int what) {
+  const int n = P.nx * P.ny, w = P.ny + 2, a = (P.nx + 2) * w;
+  int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= patch_io_size(P.nx, P.ny)) return;
+  double* const hp = host + k;
+  double* tile;
+  if (k < 3 * n) {
+    if (!(what & kIoNew)) return;
+    const int q = k / n;
+    k -= q * n;
+    tile = q == 0 ? F.H(cur) : (q == 1 ? F.HU(cur) : F.HV(cur));
+    tile += tile_index(P, k / P.ny, k % P.ny);
+  } else {
+    k -= 3 * n;
+    const int q = k / a;
+    if (!(what & (q < 3 ? kIoOld : kIoB))) return;
+    k -= q * a;
+    tile = q == 0 ? F.H(1 - cur) : (q == 1 ? F.HU(1 - cur) : (q == 2 ? F.HV(1 - cur) : F.b));
+    tile += tile_index(P, k / w - 1, k % w - 1);
+  }
+  if (UPLOAD)
+    *tile = *hp;
+  else
+    *hp = *tile;
+}
+
 // SWEKernel::solveTimestep on one patch (SWEKernel.cpp:50-88): speed of
 // every edge of uOld, dt = fmin(CFL, maxDt), update, swap.  Both the speeds
 // and the update run in blockDim/64 row segments, one wavefront each: the
