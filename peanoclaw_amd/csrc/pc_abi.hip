@@ -180,6 +180,10 @@ struct pc_pool {
   // their device address
   double* h_patch_io = nullptr;
   double* d_patch_io = nullptr;
+  // pinned host memory for the results of the AMR step calls
+  double* h_amr = nullptr;
+  double* d_amr_host = nullptr;
+  size_t amr_host_cap = 0;
   // graph
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -1146,6 +1150,7 @@ int pc_pool_destroy(pc_pool* p) {
   if (p->h_result) hipHostFree(p->h_result);
   if (p->h_stage) hipHostFree(p->h_stage);
   if (p->h_patch_io) hipHostFree(p->h_patch_io);
+  if (p->h_amr) hipHostFree(p->h_amr);
   for (hipEvent_t e : p->upd_ev) hipEventDestroy(e);
   hipEventDestroy(p->ev0);
   hipEventDestroy(p->ev1);

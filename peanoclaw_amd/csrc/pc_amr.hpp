@@ -425,6 +425,21 @@ __device__ __forceinline__ void amr_walls(const AmrBlock& K, const SegRec* __res
   }
 }
 
+// After a call's iterations of local time stepping: the leaves' clocks and
+// the leaf steps taken, into pinned host memory (time and step of leaf k at
+// host[2 k + 1]; the count, reset here, at host[0]).
+__global__ void __launch_bounds__(256)
+k_lts_report(const int* __restrict__ leaves, int nleaves, AmrLts L, double* host) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k == 0) {
+    *reinterpret_cast<unsigned long long*>(host) = *L.steps;
+    *L.steps = 0;
+  }
+  if (k >= nleaves) return;
+  host[2 * k + 1] = L.t[leaves[k]];
+  host[2 * k + 2] = L.dt[leaves[k]];
+}
+
 // What the fill and the update read of the plan.
 struct AmrPlanDev {
   SegList list;  // ghosts in the own tile
@@ -519,14 +534,15 @@ k_cfl_fold(const double* __restrict__ cfl_block, int n, double* __restrict__ out
 // The update of every leaf, uOld -> uNew, after the fill; the last workgroup
 // does the clocks.  Global steps: the step is the smallest of cfl[0 .. ncfl)
 // bounded by the step left to the end time (every leaf's fmin(own CFL step,
-// bound) equals it), the clock goes from `in` to `out`.  Local time stepping:
+// bound) equals it), the clock goes from `in` to `out` and, with the last
+// step of a call, to pinned host memory (`host`).  Local time stepping:
 // the advancing leaves by their own steps, their clocks (SWEKernel.cpp:83-87)
 // by their first segment.
 template <int R, int SOLVER, bool LTS>
 __global__ void __launch_bounds__(64 * kSegWaves)
 __attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
 k_amr_update(AmrPlanDev A, Fields F, int cur, const AmrClock* in, AmrClock* out,
-             const double* __restrict__ cfl, int ncfl, AmrLts L) {
+             AmrClock* host, const double* __restrict__ cfl, int ncfl, AmrLts L) {
   __shared__ double pre[kSegWaves][4][64];
   __shared__ double red[kSegWaves];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -562,6 +578,7 @@ k_amr_update(AmrPlanDev A, Fields F, int cur, const AmrClock* in, AmrClock* out,
         n.steps = c.steps + 1;
       }
       *out = n;
+      if (host) *host = n;
       return;
     }
     dt = c.end_time - (c.time + c.dt);
@@ -710,6 +727,7 @@ struct pc_amr {
   int* d_wall_dims = nullptr;
   AmrClock* d_clock = nullptr;
   AmrClock* d_clock_next = nullptr;  // the clock a global step writes
+  AmrClock h_clock{};                // as after the last call
   char* d_tables = nullptr;  // one allocation holding every d_* table above
   size_t tables_cap = 0;
   double last_dt = 0.0;
@@ -718,7 +736,6 @@ struct pc_amr {
   // leaves, leaves below each virtual patch
   std::vector<std::vector<int>> vleaves;  // per virtual patch, plan order
   bool lts_ready = false;
-  size_t lts_ns = 0;  // slots covered by the per-slot arrays
   AmrLts lts{};
   int* d_vidx = nullptr;   // per slot: index of the virtual patch, -1 otherwise
   int* d_rptr = nullptr;   // per leaf (plan order): the virtual patches its faces read
@@ -1160,6 +1177,8 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   const size_t o_xptr = st.add(xptr);
   const size_t o_pairs = st.add(pairs), o_ghosts = st.add(gh), o_walls = st.add(wl);
   const size_t o_wall_dims = st.add(wdims);
+  c.end_time = INFINITY;
+  a->h_clock = c;
   const std::vector<AmrClock> clk{c};
   const size_t o_clock = st.add(clk), o_next = st.add(clk);
   // the records and contributions follow, made on the device
@@ -1231,8 +1250,33 @@ AmrPlanDev amr_plan(const pc_amr* a) {
                     a->d_gmap, a->d_ghosts,  a->d_walls,   a->d_wall_dims};
 }
 
+// Pinned host memory of at least n doubles for a call's results, and its
+// device address; the call waits for the GPU before it reads them.
+int amr_host_buffer(pc_pool* p, size_t n) {
+  if (n <= p->amr_host_cap) return PC_OK;
+  if (p->h_amr) HIPCHK(hipHostFree(p->h_amr));
+  p->h_amr = nullptr;
+  p->amr_host_cap = 0;
+  const size_t cap = std::max<size_t>(2 * n, 4096);
+  HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&p->h_amr), cap * sizeof(double),
+                       hipHostMallocMapped | hipHostMallocCoherent));
+  HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void**>(&p->d_amr_host), p->h_amr, 0));
+  p->amr_host_cap = cap;
+  return PC_OK;
+}
+
+// The end time of the steps to come, on the device (it stays from call to
+// call).
+int amr_set_end(pc_amr* a, double end_time) {
+  if (std::memcmp(&a->h_clock.end_time, &end_time, sizeof(double)) == 0) return PC_OK;
+  HIPCHK(hipMemcpyAsync(&a->d_clock->end_time, &end_time, sizeof(double),
+                        hipMemcpyHostToDevice, a->pool->stream));
+  a->h_clock.end_time = end_time;
+  return PC_OK;
+}
+
 template <int R, int SOLVER, bool LTS>
-void amr_launch_segments(pc_amr* a, Fields F, int cur) {
+void amr_launch_segments(pc_amr* a, Fields F, int cur, AmrClock* host) {
   pc_pool* p = a->pool;
   const AmrPlanDev A = amr_plan(a);
   const dim3 b(64 * a->max_waves);
@@ -1252,31 +1296,31 @@ void amr_launch_segments(pc_amr* a, Fields F, int cur) {
   }
   hipLaunchKernelGGL((k_amr_update<R, SOLVER, LTS>), dim3(a->nsegs / kSegWaves + 1),
                      dim3(64 * kSegWaves), 0, p->stream, A, F, cur, a->d_clock, a->d_clock_next,
-                     cfl, ncfl, a->lts);
+                     host, cfl, ncfl, a->lts);
 }
 
 template <bool LTS>
-void amr_launch_leaves(pc_amr* a, Fields F, int cur) {
+void amr_launch_leaves(pc_amr* a, Fields F, int cur, AmrClock* host = nullptr) {
   if (a->pool->solver) {
     if (a->seg_rows == 2)
-      amr_launch_segments<2, 1, LTS>(a, F, cur);
+      amr_launch_segments<2, 1, LTS>(a, F, cur, host);
     else
-      amr_launch_segments<4, 1, LTS>(a, F, cur);
+      amr_launch_segments<4, 1, LTS>(a, F, cur, host);
   } else {
     if (a->seg_rows == 2)
-      amr_launch_segments<2, 0, LTS>(a, F, cur);
+      amr_launch_segments<2, 0, LTS>(a, F, cur, host);
     else
-      amr_launch_segments<4, 0, LTS>(a, F, cur);
+      amr_launch_segments<4, 0, LTS>(a, F, cur, host);
   }
 }
 
-int amr_launch_step(pc_amr* a, Fields F, int cur) {
+int amr_launch_step(pc_amr* a, Fields F, int cur, AmrClock* host) {
   pc_pool* p = a->pool;
   if (a->nvblocks > 0)
     hipLaunchKernelGGL(k_amr_restrict<false>, dim3(a->nvblocks), dim3(256), 0, p->stream,
                        a->d_vblocks, a->d_xptr, a->d_contribs, a->d_leaves, F, cur, a->d_clock,
                        a->lts);
-  amr_launch_leaves<false>(a, F, cur);
+  amr_launch_leaves<false>(a, F, cur, host);
   HIPCHK(hipGetLastError());
   std::swap(a->d_clock, a->d_clock_next);
   return PC_OK;
@@ -1380,7 +1424,6 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   CHK(amr_upload(&a->d_vleaf, vleaf));
   CHK(amr_upload(&a->d_nptr, np));
   CHK(amr_upload(&a->d_nbr, nb));
-  a->lts_ns = ns;
   a->lts_ready = true;
   return PC_OK;
 }
@@ -1397,25 +1440,23 @@ int pc_amr_lts_step(pc_amr* a, int k, double end_time, long long* leaf_steps) {
   mark_state_changed(p);
   a->shared_clock = false;
   Fields F = fields_of(p);
-  HIPCHK(hipMemcpyAsync(&a->d_clock->end_time, &end_time, sizeof(double),
-                        hipMemcpyHostToDevice, p->stream));
-  HIPCHK(hipMemsetAsync(a->lts.steps, 0, sizeof(unsigned long long), p->stream));
+  const int nl = (int)a->leaves.size();
+  CHK(amr_host_buffer(p, 2 * (size_t)nl + 1));
+  CHK(amr_set_end(a, end_time));
   for (int it = 0; it < k; ++it) CHK(amr_launch_lts(a, F, cur));
-  unsigned long long n = 0;
-  const size_t ns = a->lts_ns;
-  std::vector<double> t(ns), dt(ns);
-  HIPCHK(hipMemcpyAsync(&n, a->lts.steps, sizeof(n), hipMemcpyDeviceToHost, p->stream));
-  HIPCHK(hipMemcpyAsync(t.data(), a->lts.t, ns * sizeof(double), hipMemcpyDeviceToHost,
-                        p->stream));
-  HIPCHK(hipMemcpyAsync(dt.data(), a->lts.dt, ns * sizeof(double), hipMemcpyDeviceToHost,
-                        p->stream));
+  hipLaunchKernelGGL(k_lts_report, dim3((nl + 255) / 256), dim3(256), 0, p->stream, a->d_leaves,
+                     nl, a->lts, p->d_amr_host);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(p->stream));
   // the leaves' descriptors follow their device clocks
-  for (int s : a->leaves) {
-    p->slots[s].desc.time = t[s];
-    p->slots[s].desc.timestep_size = dt[s];
-    p->slots[s].clock_from_scenario = false;
+  for (int i = 0; i < nl; ++i) {
+    Slot& s = p->slots[a->leaves[i]];
+    s.desc.time = p->h_amr[2 * i + 1];
+    s.desc.timestep_size = p->h_amr[2 * i + 2];
+    s.clock_from_scenario = false;
   }
+  unsigned long long n;
+  std::memcpy(&n, p->h_amr, sizeof(n));
   if (leaf_steps) *leaf_steps = (long long)n;
   return PC_OK;
 }
@@ -1432,12 +1473,14 @@ int pc_amr_step(pc_amr* a, int k, double end_time, double* last_dt) {
   CHK(amr_cur(a, &cur));
   mark_state_changed(p);
   Fields F = fields_of(p);
-  HIPCHK(hipMemcpyAsync(&a->d_clock->end_time, &end_time, sizeof(double),
-                        hipMemcpyHostToDevice, p->stream));
-  for (int it = 0; it < k; ++it) CHK(amr_launch_step(a, F, cur));
-  AmrClock c;
-  HIPCHK(hipMemcpyAsync(&c, a->d_clock, sizeof(c), hipMemcpyDeviceToHost, p->stream));
+  CHK(amr_host_buffer(p, sizeof(AmrClock) / sizeof(double)));
+  CHK(amr_set_end(a, end_time));
+  for (int it = 0; it < k; ++it)
+    CHK(amr_launch_step(a, F, cur,
+                        it == k - 1 ? reinterpret_cast<AmrClock*>(p->d_amr_host) : nullptr));
   HIPCHK(hipStreamSynchronize(p->stream));
+  if (k > 0) std::memcpy(&a->h_clock, p->h_amr, sizeof(AmrClock));
+  const AmrClock& c = a->h_clock;
   // the leaves' descriptors follow the device clock (as pc_solve_timestep
   // would have left them)
   for (int s : a->leaves) {
@@ -1452,10 +1495,7 @@ int pc_amr_step(pc_amr* a, int k, double end_time, double* last_dt) {
 
 int pc_amr_clock(pc_amr* a, double* time, double* timestep_size, long long* steps) {
   if (!a) return fail(PC_E_INVALID, "invalid argument");
-  hipSetDevice(a->pool->device);
-  AmrClock c;
-  HIPCHK(hipMemcpyAsync(&c, a->d_clock, sizeof(c), hipMemcpyDeviceToHost, a->pool->stream));
-  HIPCHK(hipStreamSynchronize(a->pool->stream));
+  const AmrClock& c = a->h_clock;  // every step call has brought it back
   if (time) *time = c.time;
   if (timestep_size) *timestep_size = c.dt;
   if (steps) *steps = c.steps;
