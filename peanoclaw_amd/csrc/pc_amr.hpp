@@ -519,6 +519,72 @@ k_amr_fill(AmrPlanDev A, Fields F, int cur, const AmrClock* clock,
   }
 }
 
+// Local time stepping of one task of leaves in one launch, where its row
+// segments are at most 8 wavefronts (the register budget holds a wavefront's
+// rows from the speeds to the update): the fill of the advancing leaves, each
+// leaf's step, its update and clock.  No workgroup reads what another writes:
+// the ghost cells were filled before.  As two launches, fill and update took
+// 11.1 + 8.0 us an iteration on the 2-level grid of 1129 16^2 leaves.
+template <int R, int SOLVER>
+__global__ void __launch_bounds__(512)
+k_lts_leaves(AmrPlanDev A, Fields F, int cur, const AmrClock* clock, AmrLts L) {
+  constexpr int kWaves = 8;
+  __shared__ double pre[kWaves][4][64];
+  __shared__ double leaf_max[kWaves][64];
+  __shared__ double leaf_dt[64];
+  const AmrBlock K = A.blocks[blockIdx.x];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const SegRec* const recs = A.list.recs + (long long)blockIdx.x * A.max_waves * A.list.group;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // not read in this launch
+    *L.iter = 0;
+    *L.itn = *L.itn + 1;
+  }
+  const int leaf_slot = recs[lane < K.nseg ? lane : 0].d.slot;
+  const bool go = lane < K.nseg && L.adv[leaf_slot] != 0;
+  const unsigned long long advancing = __builtin_amdgcn_ballot_w64(go);
+  if (advancing == 0) return;  // the same in every wavefront
+  SegLane g = seg_lane(A.list, seg_wave(A.max_waves));
+  const SegDesc D = seg_desc(A.list, g);
+  if (g.segok && !L.adv[D.slot]) g.active = false;
+  const State N = state_of(F, cur), O = state_of(F, 1 - cur);
+  SegRows<R, true> q;
+  q.template load<kRowsInterior>(D, g, N, F.b, g.rb + 1);
+  // uNew -> uOld (DefaultTransfer::copyUNewToUOld)
+#pragma unroll
+  for (int k = 1; k <= R; ++k) {
+    if (!g.active || k > g.rows) continue;
+    const long long o = D.off + (long long)(g.ra - 1 + k) * D.stride + g.col;
+    gs(F.H(1 - cur) + o, q.h[k]);
+    gs(F.HU(1 - cur) + o, q.hu[k]);
+    gs(F.HV(1 - cur) + o, q.hv[k]);
+  }
+  __syncthreads();
+  amr_walls(K, recs, A.walls, A.dims, F, 1 - cur, L.adv);
+  q.template load<kRowsGhost>(D, g, O, F.b, g.rb + 1);
+  const double v = seg_speeds<R, SOLVER>(g, q, g.rb == g.nx ? g.rb + 1 : g.rb, N, O, F.b, pre[w]);
+  if (g.segok && g.col == 1) leaf_max[w][g.seg] = v;
+  wave_sync();
+  seg_side_shares<SOLVER>(g, O, F.b, pre[w]);
+  __syncthreads();
+  if (w == 0 && go) {
+    const SegDesc P = gl(&(recs + lane)->d);
+    double m = leaf_max[0][lane];
+    for (int k = 1; k < K.nwaves; ++k) m = dmax(m, leaf_max[k][lane]);
+    const double t = L.t[leaf_slot], dt0 = L.dt[leaf_slot];
+    const double md = clock->end_time - (t + dt0);
+    const double dt = fmin(max_timestep(m, P.dx, P.dy), md);  // SWEKernel.cpp:60-68
+    leaf_dt[lane] = dt;
+    if (dt - 0.0 > kLaEps) {  // SWEKernel.cpp:83-87
+      L.t[leaf_slot] = t + dt0;
+      L.dt[leaf_slot] = dt;
+    }
+  }
+  if (threadIdx.x == 0) atomicAdd(L.steps, (unsigned long long)__popcll(advancing));
+  __syncthreads();
+  seg_update_rows<R, SOLVER>(g, D, q, g.active ? leaf_dt[g.seg] : 0.0, pre[w], F.H(cur),
+                             F.HU(cur), F.HV(cur));
+}
+
 // The smallest of many workgroups' CFL steps, where the update's workgroups
 // would otherwise each read more than kCflFold of them.
 constexpr int kCflFold = 1024;
@@ -658,48 +724,70 @@ k_lts_flags(const int* __restrict__ leaves, int nleaves, const int* __restrict__
   }
 }
 
-// The same decision in one workgroup of 1024 threads for plans of up to
-// kLtsBlockLeaves leaves and kLtsBlockVirtuals virtual patches: first the end time of every
-// virtual patch (one wavefront per virtual patch, its leaves over the lanes,
-// an exact minimum), kept in LDS, then the leaves' flags reading it, so no
-// thread walks the leaves below a virtual neighbour itself.
-constexpr int kLtsBlockLeaves = 8192;
+// A double as an unsigned integer of the same order, and back.
+__device__ __forceinline__ unsigned long long order_key(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  return b ^ ((unsigned long long)((long long)b >> 63) | 0x8000000000000000ull);
+}
+__device__ __forceinline__ double from_order_key(unsigned long long k) {
+  return __longlong_as_double(
+      (long long)(k ^ ((k >> 63) ? 0x8000000000000000ull : 0xFFFFFFFFFFFFFFFFull)));
+}
+
+// The same decision for plans of up to kLtsBlockVirtuals virtual patches and
+// kLtsBlockPairs leaves below them whose leaves have at most kLtsNeighbours
+// neighbours: every workgroup first takes the virtual patches' end times in
+// LDS (a thread per leaf below one, LDS minima), while its own leaves' data
+// is on the way, then decides one leaf per thread.  neighbours[k *
+// kLtsNeighbours ..]: leaf slots, -1 - v for the virtual patch of index v,
+// the leaf itself in free places.
+//
+// Latency-bound: about four dependent loads.  One workgroup of 1024 threads
+// with offset lists (eight dependent loads, two rounds of 1129 leaves, an
+// atomic per advancing leaf) took 12.7 us an iteration.
 constexpr int kLtsBlockVirtuals = 4096;  // 32 KiB of LDS
-__global__ void __launch_bounds__(1024)
-k_lts_flags_block(const int* __restrict__ leaves, int nleaves, const int* __restrict__ nptr,
-                  const int* __restrict__ nbr, const int* __restrict__ vptr, int nvirt,
-                  const int* __restrict__ vleaf, const int* __restrict__ vidx,
+constexpr int kLtsBlockPairs = 16384;
+constexpr int kLtsNeighbours = 8;
+__global__ void __launch_bounds__(256)
+k_lts_flags_block(const int* __restrict__ leaves, int nleaves,
+                  const int* __restrict__ neighbours, const int* __restrict__ vleaf,
+                  const int* __restrict__ vowner, int npairs, int nvirt,
                   const int* __restrict__ rptr, const int* __restrict__ rsrc,
                   const AmrClock* clock, AmrLts L) {
-  extern __shared__ double vend[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-  for (int v = wave; v < nvirt; v += nwaves) {
-    double m = 1.7976931348623157e308;
-    for (int i = vptr[v] + lane; i < vptr[v + 1]; i += 64) {
-      const int x = vleaf[i];
-      m = dmin(m, L.t[x] + L.dt[x]);
-    }
-    for (int o = 32; o >= 1; o >>= 1) m = dmin(m, __shfl_xor(m, o));
-    if (lane == 0) vend[v] = m;
+  extern __shared__ unsigned long long vend[];
+  for (int v = threadIdx.x; v < nvirt; v += 256) vend[v] = order_key(kNoLimit);
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  const bool ok = k < nleaves;
+  const int s = ok ? leaves[k] : 0;
+  int q[kLtsNeighbours];
+#pragma unroll
+  for (int j = 0; j < kLtsNeighbours; ++j)
+    q[j] = ok ? gl(neighbours + k * kLtsNeighbours + j) : -1;
+  const int r0 = ok ? rptr[k] : 0, r1 = ok ? rptr[k + 1] : 0;
+  double c = kNoLimit, e = 0.0;
+  if (ok) {
+    e = gl(L.t + s) + gl(L.dt + s);
+#pragma unroll
+    for (int j = 0; j < kLtsNeighbours; ++j)
+      if (q[j] >= 0) c = dmin(c, gl(L.t + q[j]) + gl(L.dt + q[j]));
   }
   __syncthreads();
-  const double end_time = clock->end_time;
-  const int stamp = *L.itn;
-  for (int k = threadIdx.x; k < nleaves; k += blockDim.x) {
-    const int s = leaves[k];
-    const double e = L.t[s] + L.dt[s];
-    const double md = end_time - e;
-    double c = 1.7976931348623157e308;
-    for (int j = nptr[k]; j < nptr[k + 1]; ++j) {
-      const int q = nbr[j];
-      c = dmin(c, q >= 0 ? L.t[q] + L.dt[q] : vend[vidx[-1 - q]]);
-    }
-    const int adv = (md - 0.0 > kLaEps) && !(e - c > kLaEps);
-    L.adv[s] = adv;
-    if (adv) {
-      atomicAdd(L.iter, 1);
-      for (int j = rptr[k]; j < rptr[k + 1]; ++j) L.need[rsrc[j]] = stamp;
-    }
+  for (int i = threadIdx.x; i < npairs; i += 256) {
+    const int x = vleaf[i];
+    atomicMin(&vend[vowner[i]], order_key(gl(L.t + x) + gl(L.dt + x)));
+  }
+  __syncthreads();
+  const double md = clock->end_time - e;
+#pragma unroll
+  for (int j = 0; j < kLtsNeighbours; ++j)
+    if (ok && q[j] < 0) c = dmin(c, from_order_key(vend[-1 - q[j]]));
+  const bool adv = ok && (md - 0.0 > kLaEps) && !(e - c > kLaEps);
+  if (ok) L.adv[s] = adv ? 1 : 0;
+  const unsigned long long m = __builtin_amdgcn_ballot_w64(adv);
+  if (m && (threadIdx.x & 63) == 0) atomicAdd(L.iter, (int)__popcll(m));
+  if (adv && r1 > r0) {
+    const int stamp = *L.itn;
+    for (int j = r0; j < r1; ++j) L.need[rsrc[j]] = stamp;
   }
 }
 
@@ -745,6 +833,9 @@ struct pc_amr {
   int* d_vleaf = nullptr;
   int* d_nptr = nullptr;
   int* d_nbr = nullptr;
+  int* d_vowner = nullptr;      // per entry of d_vleaf: its virtual patch's index
+  int* d_neighbours = nullptr;  // k_lts_flags_block's table, where the plan fits it
+  int npairs = 0;
 };
 
 namespace {
@@ -768,7 +859,7 @@ void amr_free(pc_amr* a) {
   a->d_tables = nullptr;
   void* lts[] = {a->lts.t,   a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
                  a->lts.itn, a->lts.need, a->d_vidx,  a->d_vptr,     a->d_vleaf,  a->d_nptr,
-                 a->d_nbr,   a->d_rptr,   a->d_rsrc};
+                 a->d_nbr,   a->d_rptr,   a->d_rsrc, a->d_vowner, a->d_neighbours};
   for (void* q : lts) hipFree(q);
 }
 
@@ -1280,8 +1371,13 @@ void amr_launch_segments(pc_amr* a, Fields F, int cur, AmrClock* host) {
   pc_pool* p = a->pool;
   const AmrPlanDev A = amr_plan(a);
   const dim3 b(64 * a->max_waves);
-  if (a->max_waves <= 8)
-    hipLaunchKernelGGL((k_amr_fill<R, SOLVER, LTS, 512>), dim3(a->nblocks), b, 0, p->stream, A,
+  if (LTS && a->max_waves <= 8) {
+    hipLaunchKernelGGL((k_lts_leaves<R, SOLVER>), dim3(a->nblocks), b, 0, p->stream, A, F, cur,
+                       a->d_clock, a->lts);
+    return;
+  }
+  if (!LTS && a->max_waves <= 8)
+    hipLaunchKernelGGL((k_amr_fill<R, SOLVER, false, 512>), dim3(a->nblocks), b, 0, p->stream, A,
                        F, cur, a->d_clock, a->d_cfl, a->lts);
   else
     hipLaunchKernelGGL((k_amr_fill<R, SOLVER, LTS, 1024>), dim3(a->nblocks), b, 0, p->stream, A,
@@ -1335,10 +1431,11 @@ int amr_launch_lts(pc_amr* a, Fields F, int cur) {
   const int nl = (int)a->leaves.size();
   const AmrLts& L = a->lts;
   const int nv = (int)a->vleaves.size();
-  if (nl <= kLtsBlockLeaves && nv <= kLtsBlockVirtuals)
-    hipLaunchKernelGGL(k_lts_flags_block, dim3(1), dim3(1024), nv * sizeof(double), p->stream,
-                       a->d_leaves, nl, a->d_nptr, a->d_nbr, a->d_vptr, nv, a->d_vleaf,
-                       a->d_vidx, a->d_rptr, a->d_rsrc, a->d_clock, L);
+  if (a->d_neighbours)
+    hipLaunchKernelGGL(k_lts_flags_block, dim3((nl + 255) / 256), dim3(256),
+                       std::max(nv, 1) * sizeof(double), p->stream, a->d_leaves, nl,
+                       a->d_neighbours, a->d_vleaf, a->d_vowner, a->npairs, nv, a->d_rptr,
+                       a->d_rsrc, a->d_clock, L);
   else
     hipLaunchKernelGGL(k_lts_flags, dim3((nl + 255) / 256), dim3(256), 0, p->stream,
                        a->d_leaves, nl, a->d_nptr, a->d_nbr, a->d_vptr, a->d_vleaf, a->d_vidx,
@@ -1392,11 +1489,11 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   for (int s : a->leaves) slot_clock(p, s, &t[s], &dt[s]);
   void* old[] = {a->lts.t,   a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
                  a->lts.itn, a->lts.need, a->d_vidx,  a->d_vptr,     a->d_vleaf,  a->d_nptr,
-                 a->d_nbr,   a->d_rptr,   a->d_rsrc};
+                 a->d_nbr,   a->d_rptr,   a->d_rsrc, a->d_vowner, a->d_neighbours};
   for (void* q : old) hipFree(q);
   a->lts = AmrLts{};
   a->d_vidx = a->d_vptr = a->d_vleaf = a->d_nptr = a->d_nbr = nullptr;
-  a->d_rptr = a->d_rsrc = nullptr;
+  a->d_rptr = a->d_rsrc = a->d_vowner = a->d_neighbours = nullptr;
   CHK(amr_upload(&a->lts.t, t));
   CHK(amr_upload(&a->lts.dt, dt));
   CHK(amr_upload(&a->lts.adv, std::vector<int>(ns, 0)));
@@ -1424,6 +1521,23 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   CHK(amr_upload(&a->d_vleaf, vleaf));
   CHK(amr_upload(&a->d_nptr, np));
   CHK(amr_upload(&a->d_nbr, nb));
+  std::vector<int> vowner(vleaf.size());
+  for (size_t v = 0; v + 1 < vptr.size(); ++v)
+    std::fill(vowner.begin() + vptr[v], vowner.begin() + vptr[v + 1], (int)v);
+  CHK(amr_upload(&a->d_vowner, vowner));
+  a->npairs = (int)vleaf.size();
+  int most = 0;
+  for (int k = 0; k < nl; ++k) most = std::max(most, np[k + 1] - np[k]);
+  if (most <= kLtsNeighbours && a->virtuals.size() <= kLtsBlockVirtuals &&
+      a->npairs <= kLtsBlockPairs) {
+    std::vector<int> t8((size_t)nl * kLtsNeighbours);
+    for (int k = 0; k < nl; ++k)
+      for (int j = 0; j < kLtsNeighbours; ++j) {
+        const int e = np[k] + j < np[k + 1] ? nb[np[k] + j] : a->leaves[k];
+        t8[(size_t)k * kLtsNeighbours + j] = e >= 0 ? e : -1 - vidx[-1 - e];
+      }
+    CHK(amr_upload(&a->d_neighbours, t8));
+  }
   a->lts_ready = true;
   return PC_OK;
 }

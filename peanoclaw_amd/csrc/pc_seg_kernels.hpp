@@ -254,9 +254,9 @@ struct SegSide {
 // Largest speed of the segment's edges per patch, in every lane of the
 // patch.  `pre`: this wavefront's LDS.  The edge below the last row belongs
 // to the next segment (`last`: the last row loaded).
-template <int R, int SOLVER>
+template <int R, int SOLVER, class Rows>
 __device__ __forceinline__ double seg_speeds(const SegLane& g,
-                                             const SegRows<R, SOLVER != 0>& q, int last,
+                                             const Rows& q, int last,
                                              const State& S, const State& G, const double* Bf,
                                              double (*pre)[64]) {
   using ES = EdgeSolver<SOLVER>;

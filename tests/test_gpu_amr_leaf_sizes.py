@@ -62,3 +62,29 @@ def test_local_time_stepping(n, solver):
             assert np.array_equal(dev.b.pool.download(p.handle)[0],
                                   one.b.pool.download(q.handle)[0])
         amr.close()
+
+
+def test_neighbour_lists_of_any_length():
+    """Neighbour lists longer than the usual eight (here every neighbour three
+    times) give the same flags."""
+    from peanoclaw_amd.amr import BatchedAmr, iarr_list
+    from peanoclaw_amd.pool import PatchPool
+    with PatchPool(0) as pa, PatchPool(0) as pb:
+        amrs = []
+        for pool in (pa, pb):
+            dev, _ = _grids(8, 1, pool)
+            amrs.append(BatchedAmr(dev))
+            amrs[-1].lts_init()
+        g = amrs[1].grid
+        ptr, idx = [0], []
+        for p in g.leaves:
+            idx += [q.handle for q in g._lts[2][p.handle]] * 3
+            ptr.append(len(idx))
+        assert amrs[1].lib.pc_amr_lts_init(amrs[1].h, iarr_list(ptr), iarr_list(idx)) == 0
+        for _ in range(20):
+            assert amrs[0].lts_iterations(1, 1.0) == amrs[1].lts_iterations(1, 1.0)
+        for p in g.leaves:
+            q = amrs[0].grid.levels[p.level][p.ij]
+            assert np.array_equal(pb.download(p.handle)[0], pa.download(q.handle)[0])
+        for a in amrs:
+            a.close()
