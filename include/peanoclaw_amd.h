@@ -313,9 +313,10 @@ int pc_step_all(pc_pool *pool, int k);
 /* Plain per-patch-launch form of the same step (reference call pattern:
  * ghost fill, per-patch CFL estimate, per-patch update, one launch each). */
 int pc_step_all_per_patch(pc_pool *pool, int k);
-/* Capture one step as a hipGraph and replay it k times (steps of so few
- * patches that they run on short row segments: their two kernels are
- * launched again instead, which leaves no gap between steps). */
+/* Prepare one step and replay it k times without looking at the grid again.
+ * The step's two to seven kernels are launched each time rather than a
+ * recorded graph: between two graph launches the GPU idles 5 to 8 us, between
+ * kernel launches it does not. */
 int pc_graph_capture(pc_pool *pool);
 int pc_graph_replay(pc_pool *pool, int k);
 /* Refinement flags of all patches (1 refine, 0 coarsening allowed, 2 keep),

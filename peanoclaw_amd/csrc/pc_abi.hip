@@ -47,6 +47,11 @@ int fail(int code, const std::string& msg) {
 
 constexpr int kNumFields = 7;  // h0 h1 hu0 hu1 hv0 hv1 b
 constexpr size_t kBytesPerCell = kNumFields * sizeof(double);
+// Wavefronts of the boundary pass the GPU holds at once (4 a SIMD).  Up to
+// that many, a lane takes half the edges it can hold (1600 patches of 64^2:
+// 10.0 us, 12.9 with all); beyond, all of them and wider workgroups, whose
+// fewer minima the dt stage reads faster.
+constexpr int kBoundaryWide = 4096;
 constexpr int kFallbackWgs = 2048;  // grid of the (usually idle) exact fallback pass
 
 struct Slot {
@@ -88,6 +93,7 @@ struct pc_pool {
   std::vector<SideDev> h_sides;
   bool sides_any = false;
   bool edges_dirty = true;
+  bool fused_exact = false;  // they are exact (no step since k_speed), not pruned
   bool fused_ready = false;
   bool uploaded = true;  // state changed from outside since the last batched step
   int* d_scn_of = nullptr;
@@ -132,6 +138,11 @@ struct pc_pool {
   std::vector<int> h_live;  // live slots (for flags / sums)
   int* d_live = nullptr;
   BoundaryDesc* d_bdesc = nullptr;  // ghost-edge sources of the live slots
+  // in the same allocation: their wavefronts in the boundary speed pass, and
+  // the smallest CFL step of each of its workgroups
+  BoundaryWave* d_bwaves = nullptr;
+  double* d_bcfl = nullptr;
+  int nbwaves = 0;
   size_t bdesc_cap = 0;
   size_t live_cap = 0;
   GhostStrip* d_strips = nullptr;
@@ -139,7 +150,9 @@ struct pc_pool {
   size_t strips_cap = 0;
   std::vector<GhostStrip> h_strips;
   std::vector<int> strip_begin;  // per slot (for the per-patch form)
-  int* d_counter = nullptr;  // [0] persistent task counter, [1] pruned-mode redo flag
+  // [0] persistent task counter, [1] pruned-mode redo flag (0 between steps:
+  // the finished workgroups of k_march_dt's fallback are counted there too)
+  int* d_counter = nullptr;
   int* d_redo = nullptr;     // = d_counter + 1
   int* d_iota = nullptr;   // d_iota[i] = i for every slot (per-patch kernels' lists)
   double* d_segmax = nullptr;  // row-segment speed maxima of the one-patch kernels
@@ -184,10 +197,7 @@ struct pc_pool {
   double* h_amr = nullptr;
   double* d_amr_host = nullptr;
   size_t amr_host_cap = 0;
-  // graph
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
-  bool graph_valid = false;
+  bool graph_valid = false;  // pc_graph_replay may run (pc_graph_capture)
   // launch config
   int persistent_wgs = 0;
   int fused = 0;
@@ -276,14 +286,7 @@ int ensure_dev(T** ptr, size_t* cap, size_t need) {
   return PC_OK;
 }
 
-int invalidate_graph(pc_pool* p) {
-  if (p->gexec) HIPCHK(hipGraphExecDestroy(p->gexec));
-  if (p->graph) HIPCHK(hipGraphDestroy(p->graph));
-  p->gexec = nullptr;
-  p->graph = nullptr;
-  p->graph_valid = false;
-  return PC_OK;
-}
+void invalidate_graph(pc_pool* p) { p->graph_valid = false; }
 
 int grow_fields(pc_pool* p, long long need_cells) {
   if (need_cells <= p->cap_cells) return PC_OK;
@@ -307,7 +310,7 @@ int grow_fields(pc_pool* p, long long need_cells) {
     p->f[k] = nf;
   }
   p->cap_cells = ncap;
-  CHK(invalidate_graph(p));
+  invalidate_graph(p);
   return PC_OK;
 }
 
@@ -801,14 +804,64 @@ int rebuild_topology(pc_pool* p) {
     HIPCHK(hipMemcpyAsync(p->d_utasks, utasks.data(), utasks.size() * sizeof(Task),
                           hipMemcpyHostToDevice, p->stream));
   {
-    // ghost-edge sources of every live patch for the boundary speed pass
-    std::vector<BoundaryDesc> bdv(live.size());
-    for (size_t k = 0; k < live.size(); ++k) {
+    // ghost-edge sources of every live patch for the boundary speed pass, by
+    // scenario and number of edges
+    const size_t n = live.size();
+    std::vector<unsigned char> shared(n);  // bit d: lower side d shared with a
+                                           // same-size neighbour that sees this
+                                           // patch across its upper side
+    std::vector<int> edges(n);
+    long long lanes = 0;
+    // lanes of a patch: enough to hold its edges per_lane at a time
+    auto lane_class = [](int e, int per_lane) {
+      int c = 0;
+      while (c < kEdgeLaneClasses - 1 && (kMinEdgeLanes << c) * per_lane < e) ++c;
+      return c;
+    };
+    for (size_t k = 0; k < n; ++k) {
+      const int i = live[k];
+      const PatchDev& P = pd[i];
+      const SideDev& sd = p->h_sides[i];
+      for (int d = 0; d < 2; ++d) {
+        if (sd.kind[2 * d] != kSideNeighbour) continue;
+        const int q = sd.src[2 * d];
+        const SideDev& sq = p->h_sides[q];
+        const PatchDev& Q = pd[q];
+        if (sq.kind[2 * d + 1] == kSideNeighbour && sq.src[2 * d + 1] == i && Q.dx == P.dx &&
+            Q.dy == P.dy && Q.nx == P.nx && Q.ny == P.ny && Q.scn == P.scn && p->slots[q].live)
+          shared[k] |= 1 << d;
+      }
+      edges[k] = ((shared[k] & 1 ? 1 : 2) + rseg_of[i] - 1) * P.ny +
+                 (shared[k] & 2 ? 1 : 2) * P.nx;
+      lanes += kMinEdgeLanes << lane_class(edges[k], kEdgesPerLane / 2);
+    }
+    // half of what a lane can hold where that still fits the GPU at once
+    const int per_lane =
+        lanes / 64 <= kBoundaryWide ? kEdgesPerLane / 2 : kEdgesPerLane;
+    std::vector<int> first((size_t)nscn * kEdgeLaneClasses + 1);
+    for (size_t k = 0; k < n; ++k)
+      ++first[(size_t)pd[live[k]].scn * kEdgeLaneClasses + lane_class(edges[k], per_lane) + 1];
+    for (size_t k = 1; k < first.size(); ++k) first[k] += first[k - 1];
+    // wavefronts: patches of one scenario with equally many lanes
+    std::vector<BoundaryWave> waves;
+    for (size_t k = 0; k + 1 < first.size(); ++k) {
+      const int ln = kMinEdgeLanes << (k % kEdgeLaneClasses);
+      for (int at = first[k]; at < first[k + 1]; at += 64 / ln)
+        waves.push_back(BoundaryWave{at, std::min(64 / ln, first[k + 1] - at), ln,
+                                     (int)(k / kEdgeLaneClasses)});
+    }
+    p->nbwaves = (int)waves.size();
+    // the lists as they lie on the device
+    std::vector<char> lists(n * sizeof(BoundaryDesc) + waves.size() * sizeof(BoundaryWave));
+    BoundaryDesc* const bdv = reinterpret_cast<BoundaryDesc*>(lists.data());
+    if (n) std::memcpy(bdv + n, waves.data(), waves.size() * sizeof(BoundaryWave));
+    for (size_t k = 0; k < n; ++k) {
       const int i = live[k];
       const PatchDev& P = pd[i];
       const SideDev& sd = p->h_sides[i];
       const long long stride = P.stride;  // a same-size neighbour's too
-      BoundaryDesc& D = bdv[k];
+      BoundaryDesc& D = bdv[first[(size_t)P.scn * kEdgeLaneClasses +
+                                  lane_class(edges[k], per_lane)]++];
       D.off = P.off;
       D.stride = P.stride;
       D.nx = P.nx;
@@ -836,27 +889,22 @@ int rebuild_topology(pc_pool* p) {
         else
           D.ebg[side] = ky == kSideWall ? -1 : -2;
       }
-      for (int d = 0; d < 2; ++d) {
-        // lower side d shared with a same-size neighbour that sees this patch
-        // across its upper side
-        D.shared[d] = 0;
-        if (sd.kind[2 * d] != kSideNeighbour) continue;
-        const int q = sd.src[2 * d];
-        const SideDev& sq = p->h_sides[q];
-        const PatchDev& Q = pd[q];
-        D.shared[d] = sq.kind[2 * d + 1] == kSideNeighbour && sq.src[2 * d + 1] == i &&
-                      Q.dx == P.dx && Q.dy == P.dy && Q.nx == P.nx && Q.ny == P.ny &&
-                      Q.scn == P.scn && p->slots[q].live;
-      }
+      for (int d = 0; d < 2; ++d) D.shared[d] = shared[k] >> d & 1;
     }
-    if (bdv.size() > p->bdesc_cap) {
+    if (n > p->bdesc_cap) {
+      // at most one wavefront and less than one workgroup per patch
       if (p->d_bdesc) HIPCHK(hipFree(p->d_bdesc));
-      p->bdesc_cap = bdv.size() * 2;
-      HIPCHK(hipMalloc(&p->d_bdesc, p->bdesc_cap * sizeof(BoundaryDesc)));
+      p->d_bdesc = nullptr;
+      p->bdesc_cap = n * 2;
+      HIPCHK(hipMalloc(&p->d_bdesc, p->bdesc_cap * (sizeof(BoundaryDesc) + sizeof(BoundaryWave) +
+                                                    sizeof(double))));
     }
-    if (!bdv.empty())
-      HIPCHK(hipMemcpyAsync(p->d_bdesc, bdv.data(), bdv.size() * sizeof(BoundaryDesc),
-                            hipMemcpyHostToDevice, p->stream));
+    if (n) {
+      p->d_bwaves = reinterpret_cast<BoundaryWave*>(p->d_bdesc + n);
+      p->d_bcfl = reinterpret_cast<double*>(p->d_bwaves + n);
+      HIPCHK(hipMemcpyAsync(p->d_bdesc, lists.data(), lists.size(), hipMemcpyHostToDevice,
+                            p->stream));
+    }
   }
   CHK(build_segments(p));
   CHK(ensure_dev(&p->d_live, &p->live_cap, std::max<size_t>(live.size(), 1)));
@@ -866,11 +914,12 @@ int rebuild_topology(pc_pool* p) {
   CHK(upload_scn(p));
   HIPCHK(hipStreamSynchronize(p->stream));
   p->topo_dirty = false;
+  p->fused_exact = false;
   // The interior speed maxima of unchanged patches stay valid; the pruned
   // mode re-derives those of scenarios whose patch set changed through its
   // exact fallback (their estimate is reset on register / release).
   if (fused_mode(p) != 2 || realloc || resplit) p->fused_ready = false;
-  CHK(invalidate_graph(p));
+  invalidate_graph(p);
   return PC_OK;
 }
 
@@ -915,6 +964,7 @@ int prepare_batched(pc_pool* p, bool march = false) {
                  kMaxRowSeg);
     HIPCHK(hipGetLastError());
     p->fused_ready = true;
+    p->fused_exact = true;
   }
   return PC_OK;
 }
@@ -969,11 +1019,16 @@ int launch_step(pc_pool* p, bool timed_update, hipEvent_t eb = nullptr,
     return launch_seg_step(p, timed_update ? (eb ? eb : p->ev2) : nullptr,
                            timed_update ? (ee ? ee : p->ev3) : nullptr);
   p->est_in_segments = false;
+  const bool exact = p->fused_exact;
+  p->fused_exact = false;
   Fields F = fields_of(p);
   EdgeBufs E = edges_of(p);
   const SideDev* sides = p->sides_any ? p->d_sides : nullptr;
   const bool fused = fused_mode(p) && p->sides_any;
   const bool prune = fused && fused_mode(p) == 2;
+  // exact interior maxima (a fresh state's): the boundary pass is exact too,
+  // so the minimum needs no proof and no fallback
+  const bool check = prune && !exact;
   if (p->nstrips > 0) {
     hipLaunchKernelGGL(k_gather, dim3((p->nstrips + 3) / 4), dim3(256), 0, p->stream,
                        p->d_strips, p->nstrips, p->d_pd, F, p->d_scn);
@@ -982,32 +1037,46 @@ int launch_step(pc_pool* p, bool timed_update, hipEvent_t eb = nullptr,
     launch_speed(p, dim3(p->ntasks), p->d_tasks, p->ntasks, p->d_plist, F, sides, E,
                  p->d_smax, nullptr);
   const int nscn = (int)p->scn.size();
+  // pruned speeds of one scenario: the boundary pass folds the CFL steps per
+  // workgroup, k_march_dt does the rest
+  const bool one = prune && nscn == 1 && p->nentries > 0 && p->ntasks > 0;
+  // wavefronts a workgroup of the boundary pass
+  const int nbw = p->nbwaves > kBoundaryWide ? 8 : 4;
   if (nscn > 0) {
     if (p->nentries > 0 && fused) {
-      const int nl = (int)p->h_live.size();
-      const dim3 g((nl + 3) / 4);
+      const int wgs = (p->nbwaves + nbw - 1) / nbw;
       if (prune)
-        hipLaunchKernelGGL(k_boundary_speed<true>, g, dim3(256), 0, p->stream, p->d_scn,
-                           p->d_bdesc, nl, F, E, p->d_smax_int, p->d_smax, p->prune_slack);
+        hipLaunchKernelGGL(k_boundary_speed<true>, dim3(wgs), dim3(64 * nbw), 0, p->stream,
+                           p->d_scn, p->d_bwaves, p->nbwaves, p->d_bdesc, F, E, p->d_smax_int,
+                           p->d_smax, p->d_est, one ? p->d_bcfl : nullptr,
+                           p->prune_slack, exact);
       else
-        hipLaunchKernelGGL(k_boundary_speed<false>, g, dim3(256), 0, p->stream, p->d_scn,
-                           p->d_bdesc, nl, F, E, p->d_smax_int, p->d_smax, 1.0);
+        hipLaunchKernelGGL(k_boundary_speed<false>, dim3(wgs), dim3(64 * nbw), 0, p->stream,
+                           p->d_scn, p->d_bwaves, p->nbwaves, p->d_bdesc, F, E, p->d_smax_int,
+                           p->d_smax, p->d_est, nullptr, 1.0, true);
     }
     // few patch entries: both dt stages in one workgroup
     const bool block = p->nentries <= kDtBlockEntries;
-    if (block) {
+    if (one) {
+      hipLaunchKernelGGL(k_march_dt, dim3(std::min(p->ntasks, kFallbackWgs)), dim3(64), 0,
+                         p->stream, p->d_tasks, p->ntasks, p->d_plist, p->d_pd, F, p->d_scn,
+                         p->d_scn_alt, sides, E, p->d_smax, p->d_est, p->d_bcfl,
+                         (p->nbwaves + nbw - 1) / nbw, p->d_counter, p->d_redo, p->prune_slack, exact);
+      std::swap(p->d_scn, p->d_scn_alt);
+      std::swap(p->scn_cap, p->scn_alt_cap);
+    } else if (block) {
       hipLaunchKernelGGL(k_dt_block, dim3(1), dim3(1024), 0, p->stream, p->d_scn, nscn,
                          p->d_plist_scn, p->d_scn_of, p->nentries, p->d_pd, p->d_smax, p->d_est,
-                         p->d_counter, prune ? 1 : 0, p->d_redo, p->prune_slack);
+                         p->d_counter, check ? 1 : 0, p->d_redo, p->prune_slack);
     } else {
       if (p->nentries > 0)
         hipLaunchKernelGGL(k_dt_partial, dim3((p->nentries + 1023) / 1024), dim3(256), 0,
                            p->stream, p->d_scn, p->d_plist_scn, p->d_scn_of, p->nentries,
-                           p->d_pd, p->d_smax, p->d_est, prune ? p->d_redo : nullptr, nullptr);
+                           p->d_pd, p->d_smax, p->d_est, check ? p->d_redo : nullptr, nullptr);
       hipLaunchKernelGGL(k_dt_final, dim3((nscn + 63) / 64), dim3(64), 0, p->stream, p->d_scn,
-                         nscn, p->d_counter, prune ? 1 : 0, p->d_redo, p->prune_slack);
+                         nscn, p->d_counter, check ? 1 : 0, p->d_redo, p->prune_slack);
     }
-    if (prune) {
+    if (check && !one) {
       // exact fallback, a no-op unless the pruned minimum was not proven exact
       if (p->ntasks > 0)
         hipLaunchKernelGGL((k_speed<true, 0>), dim3(std::min(p->ntasks, kFallbackWgs)),
@@ -1135,7 +1204,6 @@ int pc_pool_destroy(pc_pool* p) {
   if (!p) return fail(PC_E_INVALID, "pool is NULL");
   hipSetDevice(p->device);
   hipStreamSynchronize(p->stream);
-  invalidate_graph(p);
   for (int k = 0; k < kNumFields; ++k)
     if (p->f[k]) hipFree(p->f[k]);
   void* ptrs[] = {p->d_pd, p->d_smax, p->d_smax_int, p->d_est, p->d_scn, p->d_tasks, p->d_utasks,
@@ -2494,7 +2562,7 @@ int pc_set_ghost_strips(pc_pool* p, const pc_ghost_strip* strips, int n) {
                           hipMemcpyHostToDevice, p->stream));
   HIPCHK(hipStreamSynchronize(p->stream));
   p->nstrips = n;
-  CHK(invalidate_graph(p));
+  invalidate_graph(p);
   return PC_OK;
 }
 
@@ -2667,7 +2735,7 @@ int pc_scenario_get(pc_pool* p, int scenario, double* time, double* dt, double* 
 int pc_set_prune_slack(pc_pool* p, double slack) {
   if (!p || !(slack > 0.0) || !(slack < 1e3)) return fail(PC_E_INVALID, "slack must be in (0, 1e3)");
   p->prune_slack = slack;
-  CHK(invalidate_graph(p));
+  invalidate_graph(p);
   return PC_OK;
 }
 
@@ -2683,7 +2751,7 @@ int pc_set_wave_propagation_solver(pc_pool* p, int solver) {
     p->fused_ready = false;
     for (auto& S : p->scn) S.est = 0.0;  // pruning thresholds came from the other solver
     p->scn_dev_dirty = true;
-    CHK(invalidate_graph(p));
+    invalidate_graph(p);
   }
   return PC_OK;
 }
@@ -2696,7 +2764,7 @@ int pc_set_launch_config(pc_pool* p, int persistent_wgs, int fused, int cap) {
   p->fused = fused;
   if (cap != p->task_cap) p->topo_dirty = true;
   p->task_cap = cap;
-  CHK(invalidate_graph(p));
+  invalidate_graph(p);
   return PC_OK;
 }
 
@@ -2706,7 +2774,7 @@ int pc_set_row_segments(pc_pool* p, int segments) {
     return fail(PC_E_INVALID, "row segments must be 0 (automatic), 1, 2 or 4");
   if (segments != p->row_segments) p->topo_dirty = true;
   p->row_segments = segments;
-  CHK(invalidate_graph(p));
+  invalidate_graph(p);
   return PC_OK;
 }
 
@@ -2882,23 +2950,11 @@ int pc_graph_capture(pc_pool* p) {
   if (!p) return fail(PC_E_INVALID, "pool is NULL");
   hipSetDevice(p->device);
   CHK(prepare_batched(p));
-  CHK(invalidate_graph(p));
-  if (p->seg_rows) {
-    // nothing to capture: the two kernels of such a step are launched again
-    // by the replay.  Between two graph launches the GPU idles 5-8 us, more
-    // than half of a small step; between two kernel launches it does not.
-    p->graph_valid = true;
-    return PC_OK;
-  }
-  HIPCHK(hipStreamSynchronize(p->stream));
-  HIPCHK(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
-  int rc = launch_step(p, false);
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(p->stream, &g);
-  if (rc != PC_OK) return rc;
-  if (e != hipSuccess) return fail(PC_E_HIP, std::string("capture: ") + hipGetErrorString(e));
-  p->graph = g;
-  HIPCHK(hipGraphInstantiate(&p->gexec, g, nullptr, nullptr, 0));
+  invalidate_graph(p);
+  // Nothing is recorded: the replay launches the step's two to seven kernels
+  // again.  Between two graph launches the GPU idles 5 to 8 us, more than half
+  // of a small step; between kernel launches it does not, and they are issued
+  // faster than any step runs.
   p->graph_valid = true;
   return PC_OK;
 }
@@ -2910,10 +2966,7 @@ int pc_graph_replay(pc_pool* p, int k) {
     return fail(PC_E_INVALID, "no valid captured graph (grid, scenarios or state changed)");
   CHK(sync_scn_host(p));
   HIPCHK(hipEventRecord(p->ev0, p->stream));
-  if (p->seg_rows)
-    for (int i = 0; i < k; ++i) CHK(launch_step(p, false));
-  else
-    for (int i = 0; i < k; ++i) HIPCHK(hipGraphLaunch(p->gexec, p->stream));
+  for (int i = 0; i < k; ++i) CHK(launch_step(p, false));
   HIPCHK(hipEventRecord(p->ev1, p->stream));
   HIPCHK(hipEventSynchronize(p->ev1));
   HIPCHK(hipEventElapsedTime(&p->last_total_ms, p->ev0, p->ev1));

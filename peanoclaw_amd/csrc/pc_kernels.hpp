@@ -123,6 +123,17 @@ struct BoundaryDesc {
   int stride;  // row stride of the tile
   double dx, dy;
 };
+static_assert(sizeof(BoundaryDesc) % 16 == 0, "the wavefront list follows the descriptors");
+
+// One wavefront of the boundary speed pass: `count` patches from descriptor
+// `first` on, `lanes` lanes (a power of two) each, all of scenario `scn`.
+struct BoundaryWave {
+  int first, count, lanes, scn;
+};
+// Edges a lane of that pass holds at a time; a patch gets 8, 16, 32 or 64 lanes.
+constexpr int kEdgesPerLane = 4;
+constexpr int kMinEdgeLanes = 8;
+constexpr int kEdgeLaneClasses = 4;
 
 // Edge buffers: h and hv of the first (side 0) and last (side 1) interior
 // column of every patch, per state: e[s][((p*2 + side)*2 + q)*kERows + row-1]
@@ -740,150 +751,146 @@ k_update(const Task* __restrict__ tasks, int ntasks, const int* __restrict__ pli
 }
 
 // Ghost-edge speeds of every patch folded with the interior maximum of the
-// same state (left by the fused update): smax[p] = max(smax_int[p],
-// ghost-edge maximum).  One wavefront per patch (4 per workgroup) walks the
-// 2 (nx + ny) ghost edges of its patch as one list (x sides: ghost row 0|1
-// and nx|nx+1 along the columns; y sides: columns 0|1 and ny|ny+1 along the
-// rows, the own column from the edge buffer).  PRUNE: exact speeds only
-// where the bound may reach the scenario's last CFL limit, as in the update.
+// same state (left by the fused update).  The 2 (nx + ny) ghost edges of a
+// patch are one list (x sides: ghost row 0|1 and nx|nx+1 along the columns;
+// y sides: columns 0|1 and ny|ny+1 along the rows, the own column from the
+// edge buffer), walked by the patch's share of a wavefront
+// (BoundaryWave::lanes).  PRUNE: exact speeds only where the bound may reach
+// the scenario's last CFL limit, as in the update, or (`exact`) everywhere.
+// Results: with `cfl_block` (a step of one scenario with pruned speeds) the
+// minimum of the patches' CFL steps per workgroup and the patches' own steps
+// in est; without it smax[p] = max(interior, ghost edges).
+//
+// Bound by latency, not by its bytes: a wavefront is one chain of dependent
+// loads (list -> descriptor and clock -> cells), so what counts is how many
+// chains there are.  A patch gets just enough lanes to hold its edges
+// kEdgesPerLane at a time: an n x n patch inside a grid has 2 n edges in
+// pruned mode, half a wavefront at 64^2 and an eighth at 16^2.  50,000 patches
+// of 8^2 to 64^2: 56 us with a wavefront each, 37 us so (110 MB, 20 us at the
+// memory's rate).
 template <bool PRUNE>
-__global__ void __launch_bounds__(256)
-k_boundary_speed(const ScnDev* __restrict__ scn, const BoundaryDesc* __restrict__ bd, int nslots,
-                 Fields F, EdgeBufs E, const double* __restrict__ smax_int,
-                 double* __restrict__ smax, double slack) {
-  constexpr int kIt = 4;  // 2 (nx + ny) <= 4 * 64 edges (nx, ny <= kERows)
+__global__ void __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(4, 8)))
+k_boundary_speed(const ScnDev* __restrict__ scn, const BoundaryWave* __restrict__ bw, int nwaves,
+                 const BoundaryDesc* __restrict__ bd, Fields F, EdgeBufs E,
+                 const double* __restrict__ smax_int, double* __restrict__ smax,
+                 double* __restrict__ est, double* __restrict__ cfl_block, double slack,
+                 bool exact) {
+  constexpr int kIt = kEdgesPerLane;
+  __shared__ double red[8];
   const int lane = threadIdx.x & 63;
-  const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (k >= nslots) return;
-  const BoundaryDesc D = gl(bd + k);
-  const int par = gl(&scn[D.scn].stepc) & 1;
-  float thr = 0.0f;
-  if (PRUNE) {
-    const double est = gl(&scn[D.scn].est);
-    if (est > 0.0) thr = (float)(kCfl * dmin(D.dx, D.dy) / (est * slack));
-  }
-  const int nx = D.nx, ny = D.ny, stride = D.stride;
-  // edge list: x-lower (ny), x-upper (ny), y-lower (nx), y-upper (nx).  In
-  // pruned mode only the scenario minimum of the CFL steps is used, so an
-  // edge shared with a same-size neighbour is evaluated once, by the patch
-  // below it; each patch keeps its upper sides, walls and tile ghosts.
-  const int l0 = (PRUNE && D.shared[0]) ? 0 : ny;
-  const int l2 = (PRUNE && D.shared[1]) ? 0 : nx;
-  const int b1 = l0, b2 = l0 + ny, b3 = b2 + l2;
-  const int ne = b3 + nx;
-  const double* H = F.H(par);
-  const double* HU = F.HU(par);
-  const double* HV = F.HV(par);
-  const double* Ecur = par ? E.e[1] : E.e[0];
-  // all loads first: own boundary cell (ho, qo) and the cell across the
-  // edge (hg, qg) of every edge this lane owns
-  double ho[kIt], qo[kIt], hg[kIt], qg[kIt];
-  bool up[kIt];
-#pragma unroll
-  for (int it = 0; it < kIt; ++it) {
-    const int e = it * 64 + lane;
-    ho[it] = 1.0; qo[it] = 0.0; hg[it] = 1.0; qg[it] = 0.0; up[it] = false;
-    if (e < b2) {
-      // x side: edge (row 0 | 1) or (nx | nx+1) at column c
-      const bool upper = e >= b1;
-      const int c = (upper ? e - b1 : e) + 1;
-      const long long io = D.off + (long long)(upper ? nx : 1) * stride + c;
-      const long long ig = (upper ? D.xrow[1] : D.xrow[0]) + c;
-      ho[it] = gl(H + io);
-      qo[it] = gl(HU + io);
-      hg[it] = gl(H + ig);
-      qg[it] = gl(HU + ig);
-      up[it] = upper;
-    } else if (e < ne) {
-      // y side: edge (col 0 | 1) or (ny | ny+1) at row r
-      const bool upper = e >= b3;
-      const int r = (upper ? e - b3 : e - b2) + 1;
-      const long long eo = (upper ? D.ebo[1] : D.ebo[0]) + r - 1;
-      const long long eg = upper ? D.ebg[1] : D.ebg[0];
-      ho[it] = gl(Ecur + eo);
-      qo[it] = gl(Ecur + eo + kERows);
-      if (eg >= 0) {
-        hg[it] = gl(Ecur + eg + r - 1);
-        qg[it] = gl(Ecur + eg + r - 1 + kERows);
-      } else if (eg == -2) {
-        const long long j = D.off + (long long)r * stride + (upper ? ny + 1 : 0);
-        hg[it] = gl(H + j);
-        qg[it] = gl(HV + j);
-      }
-      up[it] = upper;
-    }
-  }
-  double sm = 0.0;
-#pragma unroll
-  for (int it = 0; it < kIt; ++it) {
-    if (it * 64 >= ne) break;  // wave-uniform
-    const int e = it * 64 + lane;
-    const bool valid = e < ne;
-    const bool upper = up[it];
-    // walls mirror the own boundary cell with the normal momentum negated
-    bool wall;
-    if (e < b2)
-      wall = upper ? D.xwall[1] != 0 : D.xwall[0] != 0;
-    else
-      wall = (upper ? D.ebg[1] : D.ebg[0]) == -1;
-    double hgv = hg[it], qgv = qg[it];
-    if (e < b2) {
-      if (wall) qgv = -qgv;  // the own boundary row, read as the ghost source
-    } else if (wall) {
-      hgv = ho[it];
-      qgv = -qo[it];
-    }
-    // orientation: the lower side's ghost is the left cell of its edge
-    const double hL = upper ? ho[it] : hgv, qL = upper ? qo[it] : qgv;
-    const double hR = upper ? hgv : ho[it], qR = upper ? qgv : qo[it];
-    bool need = valid;
-    if (PRUNE) {
-      const BoundTerms bl = bound_terms(hL, qL, 0.0), br = bound_terms(hR, qR, 0.0);
-      need = valid && bound_candidate(bl.ax, bl.c, br.ax, br.c, thr);
-    }
-    if (wave_any(need)) {
-      const CellQ cl = cell_dir(cell_base(hL, 0.0), qL);
-      const CellQ cr = cell_dir(cell_base(hR, 0.0), qR);
-      const double sp = edge_speed_any(cl, cr);
-      if (valid) sm = dmax(sm, sp);
-    }
-  }
-  // seams of the update's row segments: the x-edges (a-1 | a) of the new
-  // state at the first row a of every segment after the first (each segment
-  // of the update saw only one side of them)
-  if (D.rseg > 1) {
-    const int nse = (D.rseg - 1) * ny;
-    for (int e = lane; e - lane < nse; e += 64) {  // wave-uniform trip count
-      const bool valid = e < nse;
-      double hL = 1.0, qL = 0.0, hR = 1.0, qR = 0.0;
-      if (valid) {
-        const int k = e / ny + 1;
-        const int c = e - (k - 1) * ny + 1;
-        const long long i = D.off + (long long)seg_first_row(k, nx, D.rseg) * stride + c;
-        hL = gl(H + i - stride);
-        qL = gl(HU + i - stride);
-        hR = gl(H + i);
-        qR = gl(HU + i);
-      }
-      bool need = valid;
-      if (PRUNE) {
-        const BoundTerms bl = bound_terms(hL, qL, 0.0), br = bound_terms(hR, qR, 0.0);
-        need = valid && bound_candidate(bl.ax, bl.c, br.ax, br.c, thr);
-      }
-      if (wave_any(need)) {
-        const CellQ cl = cell_dir(cell_base(hL, 0.0), qL);
-        const CellQ cr = cell_dir(cell_base(hR, 0.0), qR);
-        const double sp = edge_speed_any(cl, cr);
-        if (valid) sm = dmax(sm, sp);
-      }
-    }
-  }
-  for (int o = 32; o >= 1; o >>= 1) sm = dmax(sm, __shfl_xor(sm, o));
-  if (lane == 0) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int k = blockIdx.x * (blockDim.x >> 6) + w;
+  double cfl = 1.7976931348623157e308;
+  if (k < nwaves) {
+    const BoundaryWave W = gl(bw + k);
+    const int sub = lane & (W.lanes - 1);
+    const bool have = lane / W.lanes < W.count;
+    const BoundaryDesc D = gl(bd + W.first + (have ? lane / W.lanes : 0));
+    const int par = gl(&scn[W.scn].stepc) & 1;
+    double est_scn = 0.0;
+    if (PRUNE && !exact) est_scn = gl(&scn[W.scn].est);
+    float thr = 0.0f;
+    if (PRUNE && est_scn > 0.0) thr = (float)(kCfl * dmin(D.dx, D.dy) / (est_scn * slack));
+    const int nx = D.nx, ny = D.ny, stride = D.stride;
+    // edge list: x-lower (ny), x-upper (ny), y-lower (nx), y-upper (nx), then
+    // the seams of the update's row segments: the x-edges (a-1 | a) of the new
+    // state at the first row a of every segment after the first (each segment
+    // of the update saw only one side of them).  In pruned mode only the scenario minimum of the CFL steps is used, so an
+    // edge shared with a same-size neighbour is evaluated once, by the patch
+    // below it; each patch keeps its upper sides, walls and tile ghosts.
+    const int l0 = (PRUNE && D.shared[0]) ? 0 : ny;
+    const int l2 = (PRUNE && D.shared[1]) ? 0 : nx;
+    const int b1 = l0, b2 = l0 + ny, b3 = b2 + l2;
+    const int b4 = b3 + nx, nlist = b4 + (D.rseg - 1) * ny, ne = have ? nlist : 0;
+    // the segments' interior maxima
     const double* si = smax_int + (long long)D.slot * kMaxRowSeg;
-    double m = gl(si);
-    for (int k = 1; k < D.rseg; ++k) m = dmax(m, gl(si + k));
-    smax[D.slot] = dmax(m, sm);
+    double sm = gl(si);
+    for (int j = 1; wave_any(j < D.rseg); ++j)
+      if (j < D.rseg) sm = dmax(sm, gl(si + j));
+    const double* H = F.H(par);
+    const double* HU = F.HU(par);
+    const double* HV = F.HV(par);
+    const double* Ecur = par ? E.e[1] : E.e[0];
+    // mostly once; 64 lanes may take more rounds (all four sides, seams)
+    for (int e0 = sub; wave_any(e0 < ne); e0 += kIt * W.lanes) {
+      // all loads first, at addresses picked without branches: own boundary
+      // cell (ho, qo) and the cell across the edge (hg, qg) of every edge
+      // this lane owns (lanes past the list repeat its last edge)
+      double ho[kIt], qo[kIt], hg[kIt], qg[kIt];
+#pragma unroll
+      for (int it = 0; it < kIt; ++it) {
+        const int e = min(e0 + it * W.lanes, nlist - 1);
+        const bool seam = e >= b4, xs = e < b2 || seam;
+        const bool upper = e < b2 ? e >= b1 : e >= b3 && !seam;
+        // column of an x side, row of a y side
+        const int c = e - (e < b2 ? (upper ? b1 : 0) : (upper ? b3 : b2)) + 1;
+        // x side: edge (row 0 | 1) or (nx | nx+1) at column c
+        long long io = D.off + (upper ? nx * stride : stride) + c;
+        long long ig = (upper ? D.xrow[1] : D.xrow[0]) + c;
+        if (wave_any(seam)) {
+          const int j = (e - b4) / ny;
+          const long long is =
+              D.off + (long long)seg_first_row(j + 1, nx, D.rseg) * stride + (e - b4 - j * ny) + 1;
+          io = seam ? is : io;
+          ig = seam ? is - stride : ig;
+        }
+        // y side: edge (col 0 | 1) or (ny | ny+1) at row c; a wall's ghost is
+        // the own column again, a tile ghost comes from the tile
+        const long long eo = (upper ? D.ebo[1] : D.ebo[0]) + c - 1;
+        const long long eg = upper ? D.ebg[1] : D.ebg[0];
+        const long long jt = D.off + c * stride + (upper ? ny + 1 : 0);
+        const double* const yo = Ecur + eo;
+        const double* const yg = eg >= 0 ? Ecur + eg + c - 1 : yo;
+        const bool tile = !xs && eg == -2;
+        ho[it] = gl(xs ? H + io : yo);
+        qo[it] = gl(xs ? HU + io : yo + kERows);
+        hg[it] = gl(xs ? H + ig : tile ? H + jt : yg);
+        qg[it] = gl(xs ? HU + ig : tile ? HV + jt : yg + kERows);
+      }
+#pragma unroll
+      for (int it = 0; it < kIt; ++it) {
+        const int e = e0 + it * W.lanes;
+        const bool valid = e < ne;
+        if (!wave_any(valid)) break;
+        const bool upper = e < b2 ? e >= b1 : e >= b3 && e < b4;
+        // walls mirror the own boundary cell with the normal momentum negated
+        const bool wall = e < b2 ? (upper ? D.xwall[1] : D.xwall[0]) != 0
+                                 : e < b4 && (upper ? D.ebg[1] : D.ebg[0]) == -1;
+        const double hgv = hg[it], qgv = wall ? -qg[it] : qg[it];
+        // orientation: the lower side's ghost is the left cell of its edge
+        const double hL = upper ? ho[it] : hgv, qL = upper ? qo[it] : qgv;
+        const double hR = upper ? hgv : ho[it], qR = upper ? qgv : qo[it];
+        bool need = valid;
+        if (PRUNE) {
+          const BoundTerms bl = bound_terms(hL, qL, 0.0), br = bound_terms(hR, qR, 0.0);
+          need = valid && bound_candidate(bl.ax, bl.c, br.ax, br.c, thr);
+        }
+        if (wave_any(need)) {
+          const CellQ cl = cell_dir(cell_base(hL, 0.0), qL);
+          const CellQ cr = cell_dir(cell_base(hR, 0.0), qR);
+          const double sp = edge_speed_any(cl, cr);
+          if (valid) sm = dmax(sm, sp);
+        }
+      }
+    }
+    for (int o = W.lanes >> 1; o >= 1; o >>= 1) sm = dmax(sm, __shfl_xor(sm, o));
+    if (have && sub == 0) {
+      if (cfl_block) {
+        cfl = max_timestep(sm, D.dx, D.dy);
+        gs(est + D.slot, cfl);
+      } else {
+        gs(smax + D.slot, sm);
+      }
+    }
+  }
+  if (!cfl_block) return;
+  for (int o = 32; o >= 1; o >>= 1) cfl = dmin(cfl, __shfl_xor(cfl, o));
+  if (lane == 0) red[w] = cfl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int j = 1; j < (int)(blockDim.x >> 6); ++j) cfl = dmin(cfl, red[j]);
+    gs(cfl_block + blockIdx.x, cfl);
   }
 }
 
@@ -1147,6 +1154,76 @@ k_dt_block(ScnDev* __restrict__ scn, int nscn, const int* __restrict__ plist_scn
         &S.minbits, (unsigned long long)__double_as_longlong(1.7976931348623157e308));
     dt_final_one(S, __longlong_as_double((long long)bits), mode, redo, slack);
   }
+}
+
+// The dt stage of a march step of one scenario with pruned speeds: the
+// scenario's minimum over the boundary pass's workgroups, the decision
+// (dt_final_one) and, where the minimum is not proven exact, the exact speed
+// pass, in one launch.  Every workgroup takes the minimum and the clock `in`
+// by itself, so all agree without waiting for each other; workgroup 0 writes
+// the advanced clock to `out` (the next kernels' `in`).  On the fallback all
+// workgroups march their share of the tasks, fold their patches' steps into
+// in->minbits, and the last to finish (`ticket`, 0 between launches) decides.
+// `exact`: the minimum is exact as it is.
+//
+// What it replaces is launches that mostly did nothing, 4 to 5 us each: dt
+// and, for the fallback, speeds and dt once more (two dt launches each time
+// beyond kDtBlockEntries patches).  A step of 50,000 patches spent 26 us on
+// them, one of 1600 patches 14 us; this launch takes 6 and 5 us.
+__global__ void __launch_bounds__(64)
+k_march_dt(const Task* __restrict__ tasks, int ntasks, const int* __restrict__ plist,
+           const PatchDev* __restrict__ pd, Fields F, ScnDev* in, ScnDev* __restrict__ out,
+           const SideDev* __restrict__ sides, EdgeBufs E, double* smax,
+           double* __restrict__ est, const double* __restrict__ cfl_block, int nblocks,
+           int* __restrict__ counter, int* __restrict__ ticket, double slack, bool exact) {
+  __shared__ MarchLds L;
+  constexpr double kNone = 1.7976931348623157e308;
+  const int lane = threadIdx.x;
+  const double end_time = gl(&in->end_time), time = gl(&in->time), dt = gl(&in->dt);
+  const double last = gl(&in->est);
+  const int pbeg = gl(&in->pbeg), pend = gl(&in->pend);
+  double cfl = kNone;
+#pragma unroll 16
+  for (int k = lane; k < nblocks; k += 64) cfl = dmin(cfl, gl(cfl_block + k));
+  for (int o = 32; o >= 1; o >>= 1) cfl = dmin(cfl, __shfl_xor(cfl, o));
+  const bool can_advance = pend > pbeg && end_time - (time + dt) - 0.0 > kLaEps;
+  if (exact || !can_advance || cfl <= last * (slack * kPruneCheckFrac)) {
+    if (blockIdx.x == 0 && lane == 0) {
+      ScnDev S = *in;
+      dt_final_one(S, cfl, 0, nullptr, 1.0);
+      *out = S;
+      *counter = 0;
+    }
+    return;
+  }
+  const int par = gl(&in->stepc) & 1;
+  double m = kNone;
+  for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
+    const Task t = gl(tasks + ti);
+    MarchArgs A{plist, pd, F, sides, E, par, 0.0, smax, in, 1.0};
+    A.smax_stride = 1;
+    march_task<kSpeed, true, 0, 0>(t, A, L);
+    __syncthreads();  // the task's smax, for all lanes
+    if (lane < t.nseg) {
+      const int p = gl(plist + t.first + lane);
+      const double v = max_timestep(smax[p], gl(&pd[p].dx), gl(&pd[p].dy));
+      gs(est + p, v);
+      m = dmin(m, v);
+    }
+  }
+  for (int o = 32; o >= 1; o >>= 1) m = dmin(m, __shfl_xor(m, o));
+  if (lane != 0) return;
+  atomicMin(&in->minbits, (unsigned long long)__double_as_longlong(m));
+  __threadfence();
+  if (atomicAdd(ticket, 1) != (int)gridDim.x - 1) return;
+  __threadfence();
+  ScnDev S = *in;
+  S.minbits = (unsigned long long)__double_as_longlong(kNone);
+  const unsigned long long bits = atomicExch(&in->minbits, S.minbits);
+  dt_final_one(S, __longlong_as_double((long long)bits), 0, nullptr, 1.0);
+  *out = S;
+  *counter = 0;
+  *ticket = 0;
 }
 
 // Ghost fill of the current state's tile ghost cells: one wavefront per strip.

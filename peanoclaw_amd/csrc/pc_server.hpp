@@ -7,7 +7,7 @@
 // (first fit in arrival order), registers its N/n x N/n patches in one
 // contiguous tile range, writes its initial state on the device, then
 // advances all active requests by `steps` shared batched steps (each
-// scenario with its own CFL dt; replayed from a captured graph while the
+// scenario with its own CFL dt; replayed (pc_graph_replay) while the
 // set of requests is unchanged), and retires the requests that reached
 // their end time: digest of the final state, mass, step count, patches
 // released.  The reference has no counterpart (it runs one simulation per
@@ -227,6 +227,7 @@ int server_admit(pc_server* s, int id) {
     HIPCHK(hipGetLastError());
   }
   if (fused_mode(p) != 2) p->fused_ready = false;  // exact modes recompute all speeds
+  p->fused_exact = false;
   HIPCHK(hipStreamSynchronize(p->stream));
   q.status = 1;
   q.admitted_round = s->round;
@@ -338,9 +339,8 @@ int pc_server_round(pc_server* s, int steps, int* active_out, int* queued_out) {
   }
   if (!s->active.empty() && steps > 0) {
     // Between admissions and completions the step is the same launch
-    // sequence: replay it as a captured graph (state read on the device);
-    // after a change, one plain step applies it and the graph is captured
-    // again.
+    // sequence: replay it (state read on the device); after a change, one
+    // plain step applies it and prepares the next replay.
     if (graph_usable(p)) {
       CHK(pc_graph_replay(p, steps));
     } else {
