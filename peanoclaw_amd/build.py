@@ -34,6 +34,9 @@ def flags():
         f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
         "-ffp-contract=off", "-fno-fast-math",
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        # leading scalar and pointer arguments arrive in registers: one cold
+        # load less at the head of every kernel (0.1 to 0.2 us of each launch)
+        "-mllvm", "-amdgpu-kernarg-preload-count=14",
         "-Wall", "-Wno-unused-result",
     ]
 

@@ -462,8 +462,9 @@ __device__ __forceinline__ double block_min(double v, double* red) {
 // with the speed, so the minimum over segments is the minimum over patches.
 template <int R, int SOLVER>
 __global__ void __launch_bounds__(64 * kSegWaves)
-k_seg_speed(SegList A, Fields F, const ScnDev* __restrict__ scn, double* __restrict__ smax_seg,
-            double* __restrict__ cfl_block) {
+k_seg_speed(const SegRec* recs, const ScnDev* __restrict__ scn, int group, int lanes, int one,
+            double* __restrict__ cfl_block, double* __restrict__ smax_seg, Fields F) {
+  const SegList A{recs, group, lanes, one};
   __shared__ double pre[kSegWaves][2][64];
   __shared__ double red[kSegWaves];
   const int w = threadIdx.x >> 6;
@@ -517,9 +518,10 @@ __device__ __forceinline__ double cfl_share(const SegRange& r,
 template <int R, int SOLVER>
 __global__ void __launch_bounds__(64 * kSegWaves)
 __attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
-k_seg_update(SegList A, Fields F, const ScnDev* __restrict__ in, ScnDev* __restrict__ out,
-             int nscn, const SegRange* __restrict__ ranges,
-             const double* __restrict__ cfl_block) {
+k_seg_update(const SegRec* recs, const ScnDev* __restrict__ in, int group, int lanes, int one,
+             int nscn, const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block,
+             ScnDev* __restrict__ out, Fields F) {
+  const SegList A{recs, group, lanes, one};
   __shared__ double pre[kSegWaves][4][64];
   __shared__ double red[kSegWaves];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
