@@ -112,7 +112,7 @@ struct pc_pool {
   // steps with too few patches to fill the GPU run on short row segments
   // (pc_seg_kernels.hpp) of at most seg_rows rows; 0: the row march
   int seg_rows = 0;
-  int seg_solver = -1;  // the solver seg_rows was chosen for
+  int seg_mode = -1;  // the speed mode seg_rows was chosen for (speed_mode)
   Task* d_stasks = nullptr;
   int nstasks = 0;
   size_t stasks_cap = 0;
@@ -215,6 +215,9 @@ namespace {
 // Next-step speeds are fused into the update for the f-wave only; the
 // augmented solver runs the separate exact speed pass.
 inline int fused_mode(const pc_pool* p) { return p->solver ? 0 : p->fused; }
+
+// How a step finds its speeds: the f-wave's launch mode, 3 augmented.
+inline int speed_mode(const pc_pool* p) { return p->solver ? 3 : p->fused; }
 
 // Exact CFL speed pass over `ntasks` tasks (grid `g`), picking the kernel
 // instance for the ghost-source mode and the edge solver.
@@ -453,8 +456,7 @@ int segment_estimates(pc_pool* p) {
 // read R + 2 and solve R + 1 x-edges per column).  The lines are where the
 // measured times cross, us a step of n x n grids of 32^2 patches (9, 16, 24,
 // 32, 40 a side; wavefronts at R = 2: 656, 2048, 4608, 8192, 12800):
-//   f-wave    R = 2: 14.9 19.7 35.7 52.6  83.2   R = 4: 17.0 19.2 30.3 41.4 63.1
-//             row march (pruned speeds): 35.0 36.3 40.6 44.6 57.1
+//   f-wave    R = 2: 14.9 19.7 35.7 52.6  83.2   R = 4: 17.0 19.2 28.0 38.6  61.6
 //   augmented R = 1: 41 66 129 220 343   R = 2: 43 57 108 165 250
 //             R = 4: 62 63 107 149 227   row march: 180 182 202 215 283
 // and 9 x 9 patches of 16^2: f-wave 14.1 (R = 2), 17.0 (R = 4), 34.7 (march);
@@ -462,6 +464,19 @@ int segment_estimates(pc_pool* p) {
 // edges cost about six times the f-wave's, so its lines lie further out; at
 // 40 x 40 patches of 64^2 (25,600 wavefronts) R = 4 still takes 794 us, the
 // march 923 us.
+// The march's time depends on its speeds (f-wave launch mode 2 pruned, 1
+// exact in the update, 0 a pass of their own), and so does the line; R = 4
+// against the best split of the march in modes 2 / 1 / 0, us a step:
+//   wavefronts  2304 (24 x 24 of 32^2)   28.0   31.6   35.8   50.9
+//               4096 (32 x 32 of 32^2)   38.6   35.8    -      -
+//               4096 (16 x 16 of 64^2)   37.9   39.9    -      -
+//               4356 (33 x 33 of 32^2)   43.9   38.9    -      -
+//               4624 (34 x 34 of 32^2)   46.0   40.8   45.3   57.7
+//               5184 (18 x 18 of 64^2)   52.2   46.6   54.3   80.2
+//               6400 (40 x 40 of 32^2)   61.6   51.0   54.5   63.5
+//               6400 (80 x 80 of 16^2)   63.4   53.8   61.4   62.6
+//               9216 (48 x 48 of 32^2)   81.1   60.0   66.3   79.2
+// Beyond 4096 wavefronts (4 a SIMD) the segments' time rises by a step.
 int choose_seg_rows(const pc_pool* p) {
   if (p->row_segments != 0 || p->h_tasks.empty()) return 0;
   auto waves = [&](int R) {
@@ -475,13 +490,14 @@ int choose_seg_rows(const pc_pool* p) {
     return waves(4) <= 32768 ? 4 : 0;
   }
   if (waves(2) <= 1536) return 2;
-  return waves(4) <= 4608 ? 4 : 0;
+  const int most = p->fused == 2 ? 4096 : p->fused == 1 ? 4608 : 6144;
+  return waves(4) <= most ? 4 : 0;
 }
 
 // The work list and patch records of a step on short row segments.
 int build_segments(pc_pool* p) {
   CHK(segment_estimates(p));
-  p->seg_solver = p->solver;
+  p->seg_mode = speed_mode(p);
   p->seg_rows = choose_seg_rows(p);
   p->nstasks = 0;
   if (!p->seg_rows) return PC_OK;
@@ -926,7 +942,7 @@ int rebuild_topology(pc_pool* p) {
 int prepare(pc_pool* p) {
   CHK(sync_scn_host(p));
   CHK(rebuild_topology(p));
-  if (p->seg_solver != p->solver) CHK(build_segments(p));  // its line is the solver's
+  if (p->seg_mode != speed_mode(p)) CHK(build_segments(p));  // its line is the mode's
   if (p->scn_dev_dirty) CHK(upload_scn(p));
   return PC_OK;
 }
@@ -942,11 +958,11 @@ EdgeBufs edges_of(pc_pool* p) {
 // Everything the batched step needs that is derived from the current
 // state: edge buffers (after uploads / per-patch calls), and in fused mode
 // the interior speed maxima of the current state.
-int prepare_batched(pc_pool* p, bool march = false) {
+int prepare_batched(pc_pool* p, bool plain = false) {
   CHK(prepare(p));
   p->uploaded = false;
   // a step on short row segments reads the tiles alone
-  if (p->seg_rows && !march) return PC_OK;
+  if (p->seg_rows && !plain) return PC_OK;
   if (p->sides_any && p->edges_dirty && !p->h_live.empty()) {
     hipLaunchKernelGGL(k_edges_init, dim3((unsigned)p->h_live.size()), dim3(64), 0, p->stream,
                        p->d_live, (int)p->h_live.size(), p->d_pd, fields_of(p), p->d_scn,
@@ -955,7 +971,8 @@ int prepare_batched(pc_pool* p, bool march = false) {
     p->edges_dirty = false;
     p->fused_ready = false;
   }
-  if (fused_mode(p) && !p->fused_ready && p->ntasks > 0) {
+  // (the plain form computes every patch's CFL step separately)
+  if (!plain && fused_mode(p) && !p->fused_ready && p->ntasks > 0) {
     if (p->nstrips > 0)
       hipLaunchKernelGGL(k_gather, dim3((p->nstrips + 3) / 4), dim3(256), 0, p->stream,
                          p->d_strips, p->nstrips, p->d_pd, fields_of(p), p->d_scn);
@@ -2839,11 +2856,7 @@ int pc_step_all(pc_pool* p, int k) {
 int pc_step_all_per_patch(pc_pool* p, int k) {
   if (!p || k < 0) return fail(PC_E_INVALID, "invalid argument");
   hipSetDevice(p->device);
-  const int fused = p->fused;
-  p->fused = 0;  // the plain form computes every patch's CFL step separately
-  int rc = prepare_batched(p, true);
-  p->fused = fused;
-  if (rc != PC_OK) return rc;
+  CHK(prepare_batched(p, true));
   // per-patch tasks (one patch per launch)
   std::vector<Task> single;
   for (int s : p->h_live) {

@@ -91,3 +91,32 @@ def test_many_patches(slack):
     assert ta == tb
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+# 4356 row segments: on segments with fused = 0 and 1, marched with fused = 2;
+# changing the mode between steps changes the path, not the bits
+def test_mode_changes_the_path():
+    def run(segments):
+        with PatchPool(0) as pool:
+            rng = np.random.default_rng(9)
+            p, n = 33, 32
+            slots = [pool.register(make_description(divmod(k, p), 1.0, n)) for k in range(p * p)]
+            o = [pool.offset(s) for s in slots]
+            cells = o[-1] + (n + 2) * tile_stride(n) - o[0]
+            pool.copy_fields(True, 0, o[0], *[rng.uniform(0.5, 2.0, cells) * a
+                                              for a in (1.0, 0.3, 0.3, 0.1)])
+            wl = Workload(pool, [GridLayout(n, np.array(slots, np.int32).reshape(p, p))], 0, 0, [])
+            wl.build_ghost_table()
+            pool.scenario_set(0, 0.0, 0.0, math.inf)
+            pool.row_segments(segments)
+            clocks = []
+            for fused in (0, 2, 1, 2, 0):
+                pool.launch_config(fused=fused)
+                pool.step(2)
+                clocks.append(pool.scenario_get(0))
+                pool.step_per_patch(1) if fused == 2 else pool.step(1)
+            return clocks, [pool.download(s)[0] for s in slots[::31]]
+    (ta, a), (tb, b) = run(0), run(1)
+    assert ta == tb
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
