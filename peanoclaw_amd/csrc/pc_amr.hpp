@@ -235,7 +235,9 @@ k_amr_contribs(const AmrVBlock* __restrict__ blocks, const int* __restrict__ cpt
 // plan's contribution list (16 bytes each), so a cell's chain is block ->
 // list bounds -> list -> cells; deriving them per step, behind four
 // divisions and five more dependent loads, took 15.7 us on the 2-level grid
-// of 1129 16^2 leaves and 24.8 us on the 3-level grid of 729 27^2 leaves.
+// of 1129 16^2 leaves and 24.8 us on the 3-level grid of 729 27^2 leaves, so
+// 6.3 and 18.0 us.  On the latter its bytes bound it (about 0.95 M
+// contributions of 72 bytes): loading them two rounds ahead gave nothing.
 template <bool LTS>
 __global__ void __launch_bounds__(256)
 k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ xptr,
@@ -542,7 +544,7 @@ k_amr_fill(AmrPlanDev A, Fields F, int cur, const AmrClock* clock,
 // rows from the speeds to the update): the fill of the advancing leaves, each
 // leaf's step, its update and clock.  No workgroup reads what another writes:
 // the ghost cells were filled before.  As two launches, fill and update took
-// 11.1 + 8.0 us an iteration on the 2-level grid of 1129 16^2 leaves.
+// 11.1 + 8.0 us an iteration on the 2-level grid of 1129 16^2 leaves, so 14.2.
 template <int R, int SOLVER>
 __global__ void __launch_bounds__(512)
 k_lts_leaves(AmrPlanDev A, Fields F, int cur, const AmrClock* clock, AmrLts L) {
@@ -764,7 +766,7 @@ __device__ __forceinline__ double from_order_key(unsigned long long k) {
 //
 // Latency-bound: about four dependent loads.  One workgroup of 1024 threads
 // with offset lists (eight dependent loads, two rounds of 1129 leaves, an
-// atomic per advancing leaf) took 12.7 us an iteration.
+// atomic per advancing leaf) took 12.7 us an iteration, this form 5.2.
 constexpr int kLtsBlockVirtuals = 4096;  // 32 KiB of LDS
 constexpr int kLtsBlockPairs = 16384;
 constexpr int kLtsNeighbours = 8;
@@ -888,9 +890,9 @@ void amr_free(pc_amr* a) {
 constexpr int kAmrTaskLeaves = 16;
 
 // Rows per segment of the plan's leaves: 2 while that gives at most 2.5
-// wavefronts a SIMD (2-level grid of 1129 16^2 leaves, 2264 wavefronts: 63 us
-// a step against 65 with 4 rows), else 4 (3-level grid of 729 27^2 leaves,
-// 5110 wavefronts: 92 us against 94).
+// wavefronts a SIMD (2-level grid of 1129 16^2 leaves, 2264 wavefronts: 44.3
+// us a step against 45.1 with 4 rows), else 4 (3-level grid of 729 27^2
+// leaves, 5110 wavefronts: 66.7 us against 74.5).
 int amr_seg_rows(const std::vector<Task>& tasks) {
   long long n = 0;
   for (const Task& t : tasks) {

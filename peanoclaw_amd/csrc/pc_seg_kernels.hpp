@@ -12,9 +12,9 @@
 // (the same operands, so the same bits).  The step is two launches, exact
 // speeds and update; the update takes its dt from the speed pass's block
 // minima itself, so there is no reduction launch and none for a fallback.
-// 9 x 9 patches of 16^2, f-wave: 34.7 -> 14.1 us a step (speeds 5.4, update
+// 9 x 9 patches of 16^2, f-wave: 34.7 -> 13.9 us a step (speeds 5.4, update
 // 5.6, the rest launches; five launches before, update 16.9); 24 x 24 of
-// 32^2: 40.6 -> 30.3 us; 16 x 16 of 32^2, augmented: 182 -> 57 us.
+// 32^2: 40.6 -> 28.0 us; 16 x 16 of 32^2, augmented: 182 -> 57 us.
 //
 // Results are those of the row march bit for bit: the same operations per
 // edge and the same order of accumulation per cell (x-left, x-right, y-up,
