@@ -480,8 +480,11 @@ int pc_server_release(pc_server *srv, int id);
  * results agree with the per-call form to ~1e-14 relative).  No reference
  * counterpart as one entry point: it replaces the traversal's calls for a
  * grid whose leaves share one clock.  The plan stays valid while its
- * patches stay registered; the patches must belong to one scenario, which
- * pc_step_all must not advance meanwhile. */
+ * slots hold patches of the same kind (leaf or virtual) and numbers of cells;
+ * a step call fails (PC_E_INVALID) once one does not.  Speeds and updates take
+ * the patches' sizes as they are at the call; the transfers between patches
+ * keep the geometry of pc_amr_create.  The patches must belong to one
+ * scenario, which pc_step_all must not advance meanwhile. */
 typedef struct pc_amr pc_amr;
 /* kind 0: transferGhostlayer of size at src_offset of src to dst_offset of
  * dst (src a leaf or virtual patch of the same level); kind 1:

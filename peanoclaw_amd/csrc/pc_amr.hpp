@@ -815,12 +815,30 @@ k_lts_flags_block(const int* __restrict__ leaves, int nleaves,
 
 }  // namespace
 
+// A slot as the plan's tables know it.
+struct AmrPlace {
+  long long off;   // its tile
+  double size[2];  // of the patch
+  int nx, ny;
+};
+
 struct pc_amr {
   pc_pool* pool = nullptr;
   std::vector<int> leaves, virtuals, plan_slots;
   std::vector<int> leaf_nx, leaf_ny;
-  std::vector<long long> plan_off;  // tile of every plan slot: the tables hold places in it
   int nvblocks = 0, nghosts = 0;
+  // what the tables hold of the plan's slots (amr_refresh), and the tables
+  // themselves where they depend on it
+  std::vector<AmrPlace> places;  // per plan slot
+  std::vector<SegDesc> h_desc;   // per leaf in task order
+  std::vector<AmrVBlock> h_vblocks;
+  std::vector<AmrGhost> h_ghosts;
+  Task* d_tasks = nullptr;  // row segments of the tasks
+  SegDesc* d_desc = nullptr;
+  int nrec = 0;  // records made of them
+  int* d_cptr = nullptr;
+  int* d_cpairs = nullptr;
+  AmrRestrict* d_pairs = nullptr;
   // tasks of leaves, their row segments (at most seg_rows rows), and what
   // the fill reads (AmrPlanDev)
   int seg_rows = 4, nblocks = 0, nsegs = 0, max_waves = 1, max_cells = 0;
@@ -850,7 +868,6 @@ struct pc_amr {
   int* d_vidx = nullptr;   // per slot: index of the virtual patch, -1 otherwise
   int* d_rptr = nullptr;   // per leaf (plan order): the virtual patches its faces read
   int* d_rsrc = nullptr;
-  std::vector<AmrGhost> h_ghosts;
   int* d_vptr = nullptr;
   int* d_vleaf = nullptr;
   int* d_nptr = nullptr;
@@ -902,21 +919,103 @@ int amr_seg_rows(const std::vector<Task>& tasks) {
   return n <= 2560 ? 2 : 4;
 }
 
-// The plan's slots must still be live with the same role and size.
+// The plan's slots must still be live with the same role and numbers of cells.
 int amr_check_slots(pc_amr* a) {
   pc_pool* p = a->pool;
-  for (size_t i = 0; i < a->leaves.size(); ++i) {
-    const int s = a->leaves[i];
-    if (!valid_slot(p, s) || p->slots[s].desc.is_virtual ||
-        p->slots[s].desc.subdivision_factor[0] != a->leaf_nx[i] ||
-        p->slots[s].desc.subdivision_factor[1] != a->leaf_ny[i] ||
-        p->slots[s].off != a->plan_off[i])
-      return fail(PC_E_INVALID, "a leaf of the AMR plan changed or was released");
+  for (size_t i = 0; i < a->plan_slots.size(); ++i) {
+    const bool virt = i >= a->leaves.size();
+    const int s = a->plan_slots[i];
+    if (!valid_slot(p, s) || (p->slots[s].desc.is_virtual != 0) != virt ||
+        p->slots[s].desc.subdivision_factor[0] != a->places[i].nx ||
+        p->slots[s].desc.subdivision_factor[1] != a->places[i].ny)
+      return fail(PC_E_INVALID,
+                  virt ? "a virtual patch of the AMR plan changed or was released"
+                       : "a leaf of the AMR plan changed or was released");
   }
-  for (size_t i = 0; i < a->virtuals.size(); ++i)
-    if (!valid_slot(p, a->virtuals[i]) || !p->slots[a->virtuals[i]].desc.is_virtual ||
-        p->slots[a->virtuals[i]].off != a->plan_off[a->leaves.size() + i])
-      return fail(PC_E_INVALID, "a virtual patch of the AMR plan changed or was released");
+  return PC_OK;
+}
+
+AmrPlace amr_place(const Slot& s) {
+  return AmrPlace{s.off, {s.desc.size[0], s.desc.size[1]}, s.desc.subdivision_factor[0],
+                  s.desc.subdivision_factor[1]};
+}
+
+// A leaf as the fill and the update read it: ghosts in its own tile.
+SegDesc amr_seg_desc(const pc_pool* p, int slot) {
+  const PatchDev P = make_patchdev(p->slots[slot]);
+  SegDesc d{};
+  d.off = P.off;
+  d.gx[0] = P.off;
+  d.gx[1] = P.off + (long long)(P.nx + 1) * P.stride;
+  d.gy[0] = P.off;
+  d.gy[1] = P.off + P.ny + 1;
+  d.nx = P.nx; d.ny = P.ny; d.stride = P.stride;
+  d.slot = slot;
+  d.scn = P.scn;
+  d.dx = P.dx; d.dy = P.dy; d.dxinv = P.dxinv; d.dyinv = P.dyinv;
+  return d;
+}
+
+// Where a ghost entry's source and destination regions begin.
+void amr_ghost_places(const pc_pool* p, AmrGhost& g) {
+  const Slot &ss = p->slots[g.src], &ds = p->slots[g.dst];
+  g.sbase = ss.off + (long long)(g.sox + 1) * ss.stride + (g.soy + 1);
+  g.dbase = ds.off + (long long)(g.dox + 1) * ds.stride + (g.doy + 1);
+  g.sstride = ss.stride;
+  g.dstride = ds.stride;
+}
+
+// The tables the device makes itself: the leaves' records and, with
+// `places`, the restriction's contributions (their cells' places).
+int amr_device_tables(pc_amr* a, bool places) {
+  pc_pool* p = a->pool;
+  hipLaunchKernelGGL(k_seg_records, dim3((a->nrec + 255) / 256), dim3(256), 0, p->stream,
+                     a->d_tasks, a->d_desc, a->nrec, a->list.group,
+                     const_cast<SegRec*>(a->list.recs));
+  if (places && !a->h_vblocks.empty())
+    hipLaunchKernelGGL(k_amr_contribs,
+                       dim3((unsigned)(a->h_vblocks.size() * kRestrictCells / 256)), dim3(256), 0,
+                       p->stream, a->d_vblocks, a->d_cptr, a->d_cpairs, a->d_xptr, a->d_pairs,
+                       p->d_pd, a->d_contribs);
+  HIPCHK(hipGetLastError());
+  return PC_OK;
+}
+
+// The plan's tables follow its slots: the tile of a slot moves when it is
+// released and registered again, and pc_patch_set_description may give a live
+// patch another size.  Steps and speeds take the cells' size as it is now; the
+// transfers between patches keep the geometry they were created with.  Called
+// ahead of every step call, after prepare (the slots' tiles on the device) and
+// amr_check_slots.
+int amr_refresh(pc_amr* a) {
+  pc_pool* p = a->pool;
+  bool moved = false, sized = false;
+  for (size_t i = 0; i < a->plan_slots.size(); ++i) {
+    const Slot& s = p->slots[a->plan_slots[i]];
+    const AmrPlace& q = a->places[i];
+    moved = moved || s.off != q.off;
+    sized = sized || s.desc.size[0] != q.size[0] || s.desc.size[1] != q.size[1];
+  }
+  if (!moved && !sized) return PC_OK;
+  for (SegDesc& d : a->h_desc) d = amr_seg_desc(p, d.slot);
+  HIPCHK(hipMemcpyAsync(a->d_desc, a->h_desc.data(), a->h_desc.size() * sizeof(SegDesc),
+                        hipMemcpyHostToDevice, p->stream));
+  if (moved) {
+    for (AmrVBlock& B : a->h_vblocks) B.off = p->slots[B.slot].off;
+    for (AmrGhost& g : a->h_ghosts) amr_ghost_places(p, g);
+    if (!a->h_vblocks.empty())
+      HIPCHK(hipMemcpyAsync(a->d_vblocks, a->h_vblocks.data(),
+                            a->h_vblocks.size() * sizeof(AmrVBlock), hipMemcpyHostToDevice,
+                            p->stream));
+    if (!a->h_ghosts.empty())
+      HIPCHK(hipMemcpyAsync(a->d_ghosts, a->h_ghosts.data(),
+                            a->h_ghosts.size() * sizeof(AmrGhost), hipMemcpyHostToDevice,
+                            p->stream));
+  }
+  CHK(amr_device_tables(a, moved));
+  HIPCHK(hipStreamSynchronize(p->stream));
+  for (size_t i = 0; i < a->plan_slots.size(); ++i)
+    a->places[i] = amr_place(p->slots[a->plan_slots[i]]);
   return PC_OK;
 }
 
@@ -963,7 +1062,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->virtuals.assign(virtuals, virtuals + nvirtuals);
   a->plan_slots = a->leaves;
   a->plan_slots.insert(a->plan_slots.end(), a->virtuals.begin(), a->virtuals.end());
-  for (int s : a->plan_slots) a->plan_off.push_back(p->slots[s].off);
+  for (int s : a->plan_slots) a->places.push_back(amr_place(p->slots[s]));
   // leaf clock: every leaf on one clock
   double t0, dt0;
   slot_clock(p, leaves[0], &t0, &dt0);
@@ -1007,18 +1106,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   std::vector<SegDesc> desc;
   std::vector<int> pos(p->slots.size(), -1);  // place of a leaf in plist
   for (size_t k = 0; k < plist.size(); ++k) {
-    const PatchDev P = make_patchdev(p->slots[plist[k]]);
-    SegDesc d{};
-    d.off = P.off;
-    d.gx[0] = P.off;
-    d.gx[1] = P.off + (long long)(P.nx + 1) * P.stride;
-    d.gy[0] = P.off;
-    d.gy[1] = P.off + P.ny + 1;
-    d.nx = P.nx; d.ny = P.ny; d.stride = P.stride;
-    d.slot = plist[k];
-    d.scn = P.scn;
-    d.dx = P.dx; d.dy = P.dy; d.dxinv = P.dxinv; d.dyinv = P.dyinv;
-    desc.push_back(d);
+    desc.push_back(amr_seg_desc(p, plist[k]));
     pos[plist[k]] = (int)k;
   }
   for (const Task& t : tasks) {
@@ -1220,15 +1308,10 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     } else {
       return bail("ghost kind must be 0 (transfer) or 1 (interpolation)");
     }
-    const Slot &ss = p->slots[s], &ds = p->slots[d];
-    g.sbase = ss.off + (long long)(g.sox + 1) * ss.stride + (g.soy + 1);
-    g.dbase = ds.off + (long long)(g.dox + 1) * ds.stride + (g.doy + 1);
-    g.sstride = ss.stride;
-    g.dstride = ds.stride;
+    amr_ghost_places(p, g);
     gh.push_back(g);
   }
   a->nghosts = (int)gh.size();
-  a->h_ghosts = gh;
   // the ghost cells of every task, one after another
   std::vector<int> block_of(plist.size());
   for (size_t b = 0; b < blocks.size(); ++b)
@@ -1295,9 +1378,9 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   const std::vector<AmrClock> clk{c};
   const size_t o_clock = st.add(clk), o_next = st.add(clk);
   // the records and contributions follow, made on the device
-  const int nrec = (int)segs.size() * a->list.group;
+  a->nrec = (int)segs.size() * a->list.group;
   const size_t o_recs = (st.total + 255) / 256 * 256;
-  const size_t o_contribs = o_recs + (size_t)nrec * sizeof(SegRec);
+  const size_t o_contribs = o_recs + (size_t)a->nrec * sizeof(SegRec);
   const size_t bytes = o_contribs + (size_t)xptr.back() * sizeof(AmrContrib) + 16;
   hipError_t e = hipSuccess;
   if (p->amr_tables && p->amr_tables_cap >= bytes) {
@@ -1335,20 +1418,19 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->d_clock_next = reinterpret_cast<AmrClock*>(base + o_next);
   a->list.recs = reinterpret_cast<SegRec*>(base + o_recs);
   a->list.scn = 0;  // the plan has its own clock
-  hipLaunchKernelGGL(k_seg_records, dim3((nrec + 255) / 256), dim3(256), 0, p->stream,
-                     reinterpret_cast<Task*>(base + o_tasks),
-                     reinterpret_cast<SegDesc*>(base + o_desc), nrec, a->list.group,
-                     reinterpret_cast<SegRec*>(base + o_recs));
-  if (!vblocks.empty())
-    hipLaunchKernelGGL(k_amr_contribs, dim3((unsigned)(vblocks.size() * kRestrictCells / 256)),
-                       dim3(256), 0, p->stream, a->d_vblocks,
-                       reinterpret_cast<int*>(base + o_cptr),
-                       reinterpret_cast<int*>(base + o_cpairs), a->d_xptr,
-                       reinterpret_cast<AmrRestrict*>(base + o_pairs), p->d_pd, a->d_contribs);
-  if (hipGetLastError() != hipSuccess) {
+  a->d_tasks = reinterpret_cast<Task*>(base + o_tasks);
+  a->d_desc = reinterpret_cast<SegDesc*>(base + o_desc);
+  a->d_cptr = reinterpret_cast<int*>(base + o_cptr);
+  a->d_cpairs = reinterpret_cast<int*>(base + o_cpairs);
+  a->d_pairs = reinterpret_cast<AmrRestrict*>(base + o_pairs);
+  a->h_desc = std::move(desc);
+  a->h_vblocks = std::move(vblocks);
+  a->h_ghosts = std::move(gh);
+  const int rc = amr_device_tables(a, true);
+  if (rc != PC_OK) {
     amr_free(a);
     delete a;
-    return fail(PC_E_HIP, "plan contributions");
+    return rc;
   }
   *out = a;
   return PC_OK;
@@ -1571,6 +1653,7 @@ int pc_amr_lts_step(pc_amr* a, int k, double end_time, long long* leaf_steps) {
   hipSetDevice(p->device);
   CHK(prepare(p));
   CHK(amr_check_slots(a));
+  CHK(amr_refresh(a));
   int cur;
   CHK(amr_cur(a, &cur));
   mark_state_changed(p);
@@ -1605,6 +1688,7 @@ int pc_amr_step(pc_amr* a, int k, double end_time, double* last_dt) {
   hipSetDevice(p->device);
   CHK(prepare(p));
   CHK(amr_check_slots(a));
+  CHK(amr_refresh(a));
   int cur;
   CHK(amr_cur(a, &cur));
   mark_state_changed(p);
