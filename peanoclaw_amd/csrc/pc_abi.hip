@@ -2778,7 +2778,9 @@ int pc_set_launch_config(pc_pool* p, int persistent_wgs, int fused, int cap) {
   if (!p || persistent_wgs < 0 || cap < 0) return fail(PC_E_INVALID, "invalid config");
   p->persistent_wgs = persistent_wgs;
   if (fused > 2) return fail(PC_E_INVALID, "fused must be 0, 1 or 2");
-  if ((fused != 0) != (p->fused != 0)) p->fused_ready = false;
+  // (the interior maxima of the pruned mode are lower bounds: no other mode may
+  // take them for exact)
+  if (fused != p->fused) p->fused_ready = false;
   p->fused = fused;
   if (cap != p->task_cap) p->topo_dirty = true;
   p->task_cap = cap;
