@@ -2881,7 +2881,7 @@ int pc_step_all_per_patch(pc_pool* p, int k) {
   EdgeBufs E = edges_of(p);
   const SideDev* sides = p->sides_any ? p->d_sides : nullptr;
   const int nscn = (int)p->scn.size();
-  p->est_in_segments = false;
+  if (k > 0) p->est_in_segments = false;  // every step writes them to d_est
   HIPCHK(hipEventRecord(p->ev0, p->stream));
   for (int it = 0; it < k; ++it) {
     // ghost fill of tile-side patches, one launch per destination patch

@@ -1,5 +1,6 @@
-"""Changes of launch mode between batched steps, bitwise against one mode
-throughout: the modes differ in how they find the same speeds."""
+"""Changes of launch mode and calls without a step between batched steps,
+bitwise against one mode throughout: the modes differ in how they find the
+same speeds."""
 import math
 
 import numpy as np
@@ -46,3 +47,17 @@ def test_pruned_to_exact(n, slack):
             return out + [pool.download(s)[0] for s in slots]
     for x, y in zip(run((2, 1, 2, 1)), run((0, 0, 0, 0))):
         assert np.array_equal(x, y)
+
+
+# a call of no steps leaves the patches' estimates of the step before
+@pytest.mark.parametrize("form", ["step", "step_per_patch"])
+def test_no_steps_keep_the_estimates(form):
+    def run(call):
+        pool, slots = _pool(16, 3, 3)
+        with pool:
+            pool.step(3)
+            if call:
+                getattr(pool, form)(0)
+            return [pool.description(s).estimated_next_timestep_size for s in slots]
+    a, b = run(True), run(False)
+    assert a == b and min(b) > 0.0
