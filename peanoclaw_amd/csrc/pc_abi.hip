@@ -993,9 +993,10 @@ void launch_segments(pc_pool* p, Fields F, hipEvent_t eb, hipEvent_t ee) {
   hipLaunchKernelGGL((k_seg_speed<R, SOLVER>), dim3(g), dim3(64 * kSegWaves), 0, p->stream,
                      A.recs, p->d_scn, A.group, A.lanes, A.scn, p->d_cfl_block, p->d_smax_seg, F);
   if (eb) hipEventRecord(eb, p->stream);
-  hipLaunchKernelGGL((k_seg_update<R, SOLVER>), dim3(g + 1), dim3(64 * kSegWaves), 0,
-                     p->stream, A.recs, p->d_scn, A.group, A.lanes, A.scn, (int)p->scn.size(),
-                     p->d_ranges, p->d_cfl_block, p->d_scn_alt, F);
+  const int nscn = (int)p->scn.size();
+  hipLaunchKernelGGL((k_seg_update<R, SOLVER>), dim3(g + seg_clock_groups(nscn)),
+                     dim3(64 * kSegWaves), 0, p->stream, A.recs, p->d_scn, A.group, A.lanes,
+                     A.scn, nscn, p->d_ranges, p->d_cfl_block, p->d_scn_alt, F);
   if (ee) hipEventRecord(ee, p->stream);
   std::swap(p->d_scn, p->d_scn_alt);
   std::swap(p->scn_cap, p->scn_alt_cap);
