@@ -1690,8 +1690,7 @@ static void map_to_patch(const int off[2], const int size[2], const PatchDev& sr
 // interpolation, both back to h, the destination region back to h.
 static int plan_interpolation(pc_pool* p, const int dsize[2], const int doff[2], int src,
                               int dst, int toUOld, int toCurrentTime, int useTimeUNewOrUOld,
-                              InterpCall& out) {
-  out = InterpCall{};
+                              InterpCall& out) {  // zeroed by the caller
   if (!valid_slot(p, src) || !valid_slot(p, dst) || !dsize || !doff)
     return fail(PC_E_INVALID, "invalid argument");
   const auto& sd = p->slots[src].desc;
@@ -1737,7 +1736,6 @@ static int plan_interpolation(pc_pool* p, const int dsize[2], const int doff[2],
   CHK(plan_transform(p, src, so, ss, 0, 1, out.back[1]));
   CHK(plan_transform(p, dst, doff, dsize, toUOld, 1, out.back[2]));
   InterpArgs& a = out.a;
-  a = InterpArgs{};
   a.srcSlot = src; a.dstSlot = dst;
   a.srcCur = cur_of(p, src); a.dstCur = cur_of(p, dst);
   a.sx = dsize[0]; a.sy = dsize[1]; a.ox = doff[0]; a.oy = doff[1];
@@ -1761,7 +1759,7 @@ int pc_interpolate_solution(pc_pool* p, const int dsize[2], const int doff[2], i
     return fail(PC_E_INVALID, "invalid argument");
   hipSetDevice(p->device);
   CHK(prepare(p));
-  InterpCall c;
+  InterpCall c{};
   CHK(plan_interpolation(p, dsize, doff, src, dst, toUOld, toCurrentTime, useTimeUNewOrUOld, c));
   mark_state_changed(p);
   hipLaunchKernelGGL(k_level_call<InterpCall>, dim3(1), dim3(kCallThreads), 0, p->stream,
@@ -1823,8 +1821,7 @@ static int overlapped_regions(const double lower[2], const double upper[2],
 // the source to h + b in both states, its (up to four) regions accumulated
 // into the destination in order, the source back to h.
 static int plan_restriction(pc_pool* p, int src, int dst, int onlyOverlapped,
-                            RestrictCall& out) {
-  out = RestrictCall{};
+                            RestrictCall& out) {  // zeroed by the caller
   if (!valid_slot(p, src) || !valid_slot(p, dst))
     return fail(PC_E_INVALID, "invalid slot");
   const auto& sd = p->slots[src].desc;
@@ -1895,7 +1892,7 @@ int pc_restrict_solution(pc_pool* p, int src, int dst, int onlyOverlapped) {
     return fail(PC_E_INVALID, "invalid slot");
   hipSetDevice(p->device);
   CHK(prepare(p));
-  RestrictCall c;
+  RestrictCall c{};
   CHK(plan_restriction(p, src, dst, onlyOverlapped, c));
   mark_state_changed(p);
   hipLaunchKernelGGL(k_level_call<RestrictCall>, dim3(1), dim3(kCallThreads), 0, p->stream,
@@ -1911,20 +1908,45 @@ int pc_restrict_solution(pc_pool* p, int src, int dst, int onlyOverlapped) {
 // A batch is exactly the sequence of its per-call entry points.  Calls that
 // share no patch commute.  Calls linked by shared patches form a sequence;
 // all sequences run in one launch, a workgroup each (k_level_calls).  Where
-// few links join many calls (a sequence over four times as long as the
-// longest chain of conflicts; a call takes a workgroup about 3 us, a wave's
-// launches about 12 us), each call goes to the first wave after every
-// earlier call it shares a source or destination with, and a wave runs as a
-// few launches with one item per call (blockIdx.y).  Everything is checked
-// before anything runs.
+// the longest sequence outlasts that (few links join many calls, or large
+// calls), each call goes to the first wave after every earlier call it shares
+// a source or destination with, and a wave runs as a few launches with one
+// item per call (blockIdx.y).  Everything is checked before anything runs.
+
+// Us a call takes on one workgroup, by its cells, and us it adds to a wave,
+// whose launches take kWaveUs and spread it over the GPU.  Measured us of a
+// batch, sequences / waves: one patch of n^2 cells interpolated twice into
+// each of its nine children (18 calls, 18 waves) and they restricted back (9
+// calls, 9 waves), and 24 such patches at once:
+//   n                      16         32         48         64
+//   interpolation, 1   82 / 228  129 / 232  237 / 232  360 / 207
+//                  24 148 / 332  194 / 345  317 / 387  513 / 378
+//   restriction, 1     63 / 114   73 / 123   96 / 130  135 / 125
+//                24   109 / 198  116 / 205  146 / 217  199 / 232
+constexpr double kWaveUs = 12.0;
+struct CallUs {
+  double alone, in_wave;
+};
+static CallUs call_us(const InterpCall& c) {
+  const double cells = std::max(c.n, c.fwd[0].sx * c.fwd[0].sy);
+  return CallUs{2.5 + cells / 250.0, cells / 80000.0};
+}
+static CallUs call_us(const RestrictCall& c) {
+  const double cells = c.fwd[0].sx * c.fwd[0].sy;
+  return CallUs{3.0 + cells / 400.0, cells / 20000.0};
+}
 
 // Calls grouped by shared patches, each group in the given order: order[]
 // holds the calls, first[g] .. first[g + 1] those of group g.
 struct CallGroups {
   std::vector<int> order, first;
-  int longest = 0;
+  double longest = 0.0;  // us of the longest group
+  double in_waves = 0.0;  // us the calls add to the waves' launches
 };
-static CallGroups call_groups(int count, const int* a, const int* b, int nslots) {
+template <class Call>
+static CallGroups call_groups(const std::vector<Call>& calls, const int* a, const int* b,
+                              int nslots) {
+  const int count = (int)calls.size();
   std::vector<int> root(nslots);
   for (int i = 0; i < nslots; ++i) root[i] = i;
   auto find = [&](int s) {
@@ -1934,19 +1956,24 @@ static CallGroups call_groups(int count, const int* a, const int* b, int nslots)
   for (int i = 0; i < count; ++i) root[find(a[i])] = find(b[i]);
   CallGroups g;
   std::vector<int> id(nslots, -1), of(count), size;
+  std::vector<double> us;
   for (int i = 0; i < count; ++i) {
     int& k = id[find(a[i])];
     if (k < 0) {
       k = (int)size.size();
       size.push_back(0);
+      us.push_back(0.0);
     }
     of[i] = k;
     ++size[k];
+    const CallUs u = call_us(calls[i]);
+    us[k] += u.alone;
+    g.in_waves += u.in_wave;
   }
   g.first.assign(size.size() + 1, 0);
   for (size_t k = 0; k < size.size(); ++k) {
     g.first[k + 1] = g.first[k] + size[k];
-    g.longest = std::max(g.longest, size[k]);
+    g.longest = std::max(g.longest, us[k]);
   }
   std::vector<int> at(g.first.begin(), g.first.end() - 1);
   g.order.resize(count);
@@ -2101,8 +2128,8 @@ int pc_interpolate_batch(pc_pool* p, int count, const int* dsize, const int* dof
                            opts[3 * i + 1], opts[3 * i + 2], pl[i]));
   int nw = 0;
   const std::vector<int> wave = conflict_waves(count, src, dst, &nw);
-  const CallGroups groups = call_groups(count, src, dst, (int)p->slots.size());
-  if (groups.longest <= 4 * nw) {
+  const CallGroups groups = call_groups(pl, src, dst, (int)p->slots.size());
+  if (groups.longest <= nw * kWaveUs + groups.in_waves) {
     mark_state_changed(p);
     return launch_call_groups(p, pl, groups);
   }
@@ -2156,8 +2183,8 @@ int pc_restrict_batch(pc_pool* p, int count, const int* src, const int* dst,
   for (int i = 0; i < count; ++i) CHK(plan_restriction(p, src[i], dst[i], onlyOverlapped, pl[i]));
   int nw = 0;
   const std::vector<int> wave = conflict_waves(count, src, dst, &nw);
-  const CallGroups groups = call_groups(count, src, dst, (int)p->slots.size());
-  if (groups.longest <= 4 * nw) {
+  const CallGroups groups = call_groups(pl, src, dst, (int)p->slots.size());
+  if (groups.longest <= nw * kWaveUs + groups.in_waves) {
     mark_state_changed(p);
     return launch_call_groups(p, pl, groups);
   }
