@@ -150,10 +150,11 @@ struct pc_pool {
   size_t strips_cap = 0;
   std::vector<GhostStrip> h_strips;
   std::vector<int> strip_begin;  // per slot (for the per-patch form)
-  // [0] persistent task counter, [1] pruned-mode redo flag (0 between steps:
-  // the finished workgroups of k_march_dt's fallback are counted there too)
+  // [0] persistent task counter, [1] pruned-mode redo flag, [2] finished
+  // workgroups of k_march_dt's fallback (0 between launches)
   int* d_counter = nullptr;
   int* d_redo = nullptr;     // = d_counter + 1
+  int* d_ticket = nullptr;   // = d_counter + 2
   int* d_iota = nullptr;   // d_iota[i] = i for every slot (per-patch kernels' lists)
   double* d_segmax = nullptr;  // row-segment speed maxima of the one-patch kernels
   double* d_keep = nullptr;    // k_patch_solve: uNew of the patch while it is updated
@@ -1080,7 +1081,8 @@ int launch_step(pc_pool* p, bool timed_update, hipEvent_t eb = nullptr,
       hipLaunchKernelGGL(k_march_dt, dim3(std::min(p->ntasks, kFallbackWgs)), dim3(64), 0,
                          p->stream, p->d_tasks, p->ntasks, p->d_plist, p->d_pd, F, p->d_scn,
                          p->d_scn_alt, sides, E, p->d_smax, p->d_est, p->d_bcfl,
-                         (p->nbwaves + nbw - 1) / nbw, p->d_counter, p->d_redo, p->prune_slack, exact);
+                         (p->nbwaves + nbw - 1) / nbw, p->d_counter, p->d_ticket, p->prune_slack,
+                         exact);
       std::swap(p->d_scn, p->d_scn_alt);
       std::swap(p->scn_cap, p->scn_alt_cap);
     } else if (block) {
@@ -1200,9 +1202,10 @@ int pc_pool_create(int device, size_t hbm_budget_bytes, pc_pool** out) {
     delete p;
     return fail(PC_E_HIP, "hipStreamCreate failed");
   }
-  HIPCHK(hipMalloc(&p->d_counter, 2 * sizeof(int)));
-  HIPCHK(hipMemsetAsync(p->d_counter, 0, 2 * sizeof(int), p->stream));
+  HIPCHK(hipMalloc(&p->d_counter, 3 * sizeof(int)));
+  HIPCHK(hipMemsetAsync(p->d_counter, 0, 3 * sizeof(int), p->stream));
   p->d_redo = p->d_counter + 1;
+  p->d_ticket = p->d_counter + 2;
   HIPCHK(hipMalloc(&p->d_result, 8 * sizeof(double)));
   // fine-grained (coherent), so a kernel's stores are visible while it runs
   HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&p->h_result), 8 * sizeof(double),
