@@ -498,10 +498,15 @@ int choose_seg_rows(const pc_pool* p) {
 // The work list and patch records of a step on short row segments.
 int build_segments(pc_pool* p) {
   CHK(segment_estimates(p));
-  p->seg_mode = speed_mode(p);
-  p->seg_rows = choose_seg_rows(p);
+  // (a list whose making fails is made again by the next call: seg_mode is set
+  // at the end)
+  p->seg_mode = -1;
   p->nstasks = 0;
-  if (!p->seg_rows) return PC_OK;
+  p->seg_rows = choose_seg_rows(p);
+  if (!p->seg_rows) {
+    p->seg_mode = speed_mode(p);
+    return PC_OK;
+  }
   std::vector<PatchDev> pd(p->slots.size());
   for (int i : p->h_live) pd[i] = make_patchdev(p->slots[i]);
   // segments by scenario, each scenario's list padded to whole workgroups
@@ -595,6 +600,7 @@ int build_segments(pc_pool* p) {
                      p->d_stasks, p->d_segdesc, nrec, A.group, p->d_segrecs);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(p->stream));  // the host vectors end here
+  p->seg_mode = speed_mode(p);
   return PC_OK;
 }
 
@@ -912,9 +918,10 @@ int rebuild_topology(pc_pool* p) {
       // at most one wavefront and less than one workgroup per patch
       if (p->d_bdesc) HIPCHK(hipFree(p->d_bdesc));
       p->d_bdesc = nullptr;
-      p->bdesc_cap = n * 2;
-      HIPCHK(hipMalloc(&p->d_bdesc, p->bdesc_cap * (sizeof(BoundaryDesc) + sizeof(BoundaryWave) +
-                                                    sizeof(double))));
+      p->bdesc_cap = 0;
+      HIPCHK(hipMalloc(&p->d_bdesc, 2 * n * (sizeof(BoundaryDesc) + sizeof(BoundaryWave) +
+                                             sizeof(double))));
+      p->bdesc_cap = 2 * n;
     }
     if (n) {
       p->d_bwaves = reinterpret_cast<BoundaryWave*>(p->d_bdesc + n);
@@ -1399,12 +1406,12 @@ namespace {
 // The pinned buffer of one patch's arrays (the largest patch's; the calls
 // that use it wait for the GPU before they return).
 int patch_io_buffer(pc_pool* p, double** host) {
-  if (!p->h_patch_io) {
+  if (!p->h_patch_io)
     HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&p->h_patch_io),
                          (size_t)patch_io_size(64, 64) * sizeof(double),
                          hipHostMallocMapped | hipHostMallocCoherent));
+  if (!p->d_patch_io)
     HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void**>(&p->d_patch_io), p->h_patch_io, 0));
-  }
   *host = p->h_patch_io;
   return PC_OK;
 }
