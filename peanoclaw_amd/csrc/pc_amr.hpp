@@ -778,39 +778,48 @@ k_amr_update(AmrPlanDev A, Fields F, int cur, const AmrClock* in, AmrClock* out,
   }
 }
 
+// End time of every virtual patch: the minimum over the leaves below it
+// (vleaf[vptr[v] .. vptr[v + 1])), a wavefront each.
+__global__ void __launch_bounds__(256)
+k_lts_virtual_ends(const int* __restrict__ vptr, const int* __restrict__ vleaf, int nvirt,
+                   AmrLts L, double* __restrict__ vend) {
+  const int v = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (v >= nvirt) return;
+  double m = kNoLimit;
+  for (int i = vptr[v] + lane; i < vptr[v + 1]; i += 64) {
+    const int x = vleaf[i];
+    m = dmin(m, L.t[x] + L.dt[x]);
+  }
+  for (int o = 32; o >= 1; o >>= 1) m = dmin(m, __shfl_xor(m, o));
+  if (lane == 0) vend[v] = m;
+}
+
 // TimeIntervals::isAllowedToAdvanceInTime (TimeIntervals.cpp:24-84) of each
 // leaf: the step bound end - (t + dt) > 1e-8 and t + dt - constraint <= 1e-8,
 // the constraint being the minimal end time over the neighbours listed in
 // nptr/nbr (>= 0: a leaf slot; < 0: -1 - the slot of a virtual patch, whose
-// end time is the minimum over the leaves below it: vleaf[vptr[v]..vptr[v+1])
-// with v = vidx[slot]).  Counts the advancing leaves into *iter (zeroed by
-// the last launch of the previous iteration) and stamps the virtual patches
-// they read with the iteration number.
+// end time is vend[vidx[slot]], from k_lts_virtual_ends).  Counts the
+// advancing leaves into *iter (zeroed by the last launch of the previous
+// iteration) and stamps the virtual patches they read with the iteration
+// number.
+//
+// For plans past the limits of k_lts_flags_block: an iteration of 4681 8^2
+// leaves on five levels (16,407 leaves below virtual patches) takes 34.1 us;
+// with every leaf walking the leaves below its virtual neighbours it took 582.
 __global__ void __launch_bounds__(256)
 k_lts_flags(const int* __restrict__ leaves, int nleaves, const int* __restrict__ nptr,
-            const int* __restrict__ nbr, const int* __restrict__ vptr,
-            const int* __restrict__ vleaf, const int* __restrict__ vidx,
-            const int* __restrict__ rptr, const int* __restrict__ rsrc,
-            const AmrClock* clock, AmrLts L) {
+            const int* __restrict__ nbr, const double* __restrict__ vend,
+            const int* __restrict__ vidx, const int* __restrict__ rptr,
+            const int* __restrict__ rsrc, const AmrClock* clock, AmrLts L) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= nleaves) return;
   const int s = leaves[k];
   const double e = L.t[s] + L.dt[s];
   const double md = clock->end_time - e;
-  double c = 1.7976931348623157e308;
+  double c = kNoLimit;
   for (int j = nptr[k]; j < nptr[k + 1]; ++j) {
     const int q = nbr[j];
-    if (q >= 0) {
-      c = dmin(c, L.t[q] + L.dt[q]);
-    } else {
-      const int v = vidx[-1 - q];
-      double m = 1.7976931348623157e308;
-      for (int i = vptr[v]; i < vptr[v + 1]; ++i) {
-        const int x = vleaf[i];
-        m = dmin(m, L.t[x] + L.dt[x]);
-      }
-      c = dmin(c, m);
-    }
+    c = dmin(c, q >= 0 ? L.t[q] + L.dt[q] : vend[vidx[-1 - q]]);
   }
   const int adv = (md - 0.0 > kLaEps) && !(e - c > kLaEps);
   L.adv[s] = adv;
@@ -844,7 +853,10 @@ __device__ __forceinline__ double from_order_key(unsigned long long k) {
 // with offset lists (eight dependent loads, two rounds of 1129 leaves, an
 // atomic per advancing leaf) took 12.7 us an iteration, this form 5.2.
 constexpr int kLtsBlockVirtuals = 4096;  // 32 KiB of LDS
-constexpr int kLtsBlockPairs = 16384;
+// Every workgroup walks all pairs: us an iteration, this form / two launches,
+// 1157 pairs 22.3 / 25.2, 3158: 26.4 / 28.3, 4857: 28.2 / 28.6, 12,358: 54.6 /
+// 36.2, 48,229: 145 / 58.6.
+constexpr int kLtsBlockPairs = 4096;
 constexpr int kLtsNeighbours = 8;
 __global__ void __launch_bounds__(256)
 k_lts_flags_block(const int* __restrict__ leaves, int nleaves,
@@ -948,6 +960,7 @@ struct pc_amr {
   int* d_vleaf = nullptr;
   int* d_nptr = nullptr;
   int* d_nbr = nullptr;
+  double* d_vend = nullptr;     // end times of the virtual patches (k_lts_virtual_ends)
   int* d_vowner = nullptr;      // per entry of d_vleaf: its virtual patch's index
   int* d_neighbours = nullptr;  // k_lts_flags_block's table, where the plan fits it
   int npairs = 0;
@@ -974,7 +987,7 @@ void amr_free(pc_amr* a) {
   a->d_tables = nullptr;
   void* lts[] = {a->lts.t,   a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
                  a->lts.itn, a->lts.need, a->d_vidx,  a->d_vptr,     a->d_vleaf,  a->d_nptr,
-                 a->d_nbr,   a->d_rptr,   a->d_rsrc, a->d_vowner, a->d_neighbours};
+                 a->d_nbr,   a->d_rptr,   a->d_rsrc, a->d_vowner, a->d_neighbours, a->d_vend};
   for (void* q : lts) hipFree(q);
 }
 
@@ -1646,15 +1659,19 @@ int amr_launch_lts(pc_amr* a, Fields F, int cur) {
   const int nl = (int)a->leaves.size();
   const AmrLts& L = a->lts;
   const int nv = (int)a->vleaves.size();
-  if (a->d_neighbours)
+  if (a->d_neighbours) {
     hipLaunchKernelGGL(k_lts_flags_block, dim3((nl + 255) / 256), dim3(256),
                        std::max(nv, 1) * sizeof(double), p->stream, a->d_leaves, nl,
                        a->d_neighbours, a->d_vleaf, a->d_vowner, a->npairs, nv, a->d_rptr,
                        a->d_rsrc, a->d_clock, L);
-  else
+  } else {
+    if (nv > 0)
+      hipLaunchKernelGGL(k_lts_virtual_ends, dim3((nv + 3) / 4), dim3(256), 0, p->stream,
+                         a->d_vptr, a->d_vleaf, nv, L, a->d_vend);
     hipLaunchKernelGGL(k_lts_flags, dim3((nl + 255) / 256), dim3(256), 0, p->stream,
-                       a->d_leaves, nl, a->d_nptr, a->d_nbr, a->d_vptr, a->d_vleaf, a->d_vidx,
-                       a->d_rptr, a->d_rsrc, a->d_clock, L);
+                       a->d_leaves, nl, a->d_nptr, a->d_nbr, a->d_vend, a->d_vidx, a->d_rptr,
+                       a->d_rsrc, a->d_clock, L);
+  }
   amr_launch_restrict<true>(a, F, cur);
   const int ncells = a->nblocks * a->max_cells;
   if (ncells > 0)
@@ -1701,11 +1718,12 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   for (int s : a->leaves) slot_clock(p, s, &t[s], &dt[s]);
   void* old[] = {a->lts.t,   a->lts.dt,   a->lts.adv, a->lts.stepdt, a->lts.iter, a->lts.steps,
                  a->lts.itn, a->lts.need, a->d_vidx,  a->d_vptr,     a->d_vleaf,  a->d_nptr,
-                 a->d_nbr,   a->d_rptr,   a->d_rsrc, a->d_vowner, a->d_neighbours};
+                 a->d_nbr,   a->d_rptr,   a->d_rsrc, a->d_vowner, a->d_neighbours, a->d_vend};
   for (void* q : old) hipFree(q);
   a->lts = AmrLts{};
   a->d_vidx = a->d_vptr = a->d_vleaf = a->d_nptr = a->d_nbr = nullptr;
   a->d_rptr = a->d_rsrc = a->d_vowner = a->d_neighbours = nullptr;
+  a->d_vend = nullptr;
   CHK(amr_upload(&a->lts.t, t));
   CHK(amr_upload(&a->lts.dt, dt));
   CHK(amr_upload(&a->lts.adv, std::vector<int>(ns, 0)));
@@ -1749,6 +1767,8 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
         t8[(size_t)k * kLtsNeighbours + j] = e >= 0 ? e : -1 - vidx[-1 - e];
       }
     CHK(amr_upload(&a->d_neighbours, t8));
+  } else {
+    CHK(amr_upload(&a->d_vend, std::vector<double>(a->virtuals.size(), 0.0)));
   }
   a->lts_ready = true;
   return PC_OK;
