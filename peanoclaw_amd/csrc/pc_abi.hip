@@ -102,18 +102,21 @@ struct pc_pool {
   ScnDev* d_scn = nullptr;
   size_t scn_cap = 0;
   Task* d_tasks = nullptr;
+  size_t tasks_cap = 0;
   int ntasks = 0;
   std::vector<Task> h_tasks;
   // the update's work list: h_tasks, with the rows of every patch split into
   // row segments when the step has fewer tasks than the GPU holds
   Task* d_utasks = nullptr;
+  size_t utasks_cap = 0;
   int nutasks = 0;
   int row_segments = 0;  // 0 automatic, 1 off, 2 or 4 forced
   std::vector<int> h_rseg;  // row segments per slot of the current list
+  std::vector<PatchDev> h_pd;  // d_pd's rows
   // steps with too few patches to fill the GPU run on short row segments
   // (pc_seg_kernels.hpp) of at most seg_rows rows; 0: the row march
   int seg_rows = 0;
-  int seg_mode = -1;  // the speed mode seg_rows was chosen for (speed_mode)
+  int seg_mode = -1;  // the speed mode seg_rows was chosen for (speed_mode), -1 none
   Task* d_stasks = nullptr;
   int nstasks = 0;
   size_t stasks_cap = 0;
@@ -123,6 +126,7 @@ struct pc_pool {
   SegDesc* d_segdesc = nullptr;  // per entry of the task patch list
   size_t segdesc_cap = 0;
   int nsegdesc = 0;
+  std::vector<SegDesc> h_segdesc;
   double* d_smax_seg = nullptr;  // kSegSlots per slot
   size_t smax_seg_cap = 0;
   double* d_cfl_block = nullptr;  // smallest CFL step of every workgroup
@@ -138,12 +142,14 @@ struct pc_pool {
   std::vector<int> h_plist;
   std::vector<int> h_live;  // live slots (for flags / sums)
   int* d_live = nullptr;
+  bool boundary_ready = false;      // the three lists that follow
   BoundaryDesc* d_bdesc = nullptr;  // ghost-edge sources of the live slots
   // in the same allocation: their wavefronts in the boundary speed pass, and
   // the smallest CFL step of each of its workgroups
   BoundaryWave* d_bwaves = nullptr;
   double* d_bcfl = nullptr;
   int nbwaves = 0;
+  std::vector<char> h_boundary;  // their host image, kept: fresh pages cost more than the lists
   size_t bdesc_cap = 0;
   size_t live_cap = 0;
   GhostStrip* d_strips = nullptr;
@@ -508,8 +514,7 @@ int build_segments(pc_pool* p) {
     p->seg_mode = speed_mode(p);
     return PC_OK;
   }
-  std::vector<PatchDev> pd(p->slots.size());
-  for (int i : p->h_live) pd[i] = make_patchdev(p->slots[i]);
+  const std::vector<PatchDev>& pd = p->h_pd;
   // segments by scenario, each scenario's list padded to whole workgroups
   const int nscn = (int)p->scn.size();
   std::vector<std::vector<int>> by_scn(nscn);
@@ -517,7 +522,8 @@ int build_segments(pc_pool* p) {
     by_scn[pd[p->h_plist[p->h_tasks[k].first]].scn].push_back((int)k);
   std::vector<Task> st;
   std::vector<SegRange> ranges(std::max(nscn, 1));
-  std::vector<SegDesc> desc(p->h_plist.size());
+  std::vector<SegDesc>& desc = p->h_segdesc;
+  desc.resize(p->h_plist.size());
   for (int s = 0; s < nscn; ++s) {
     ranges[s].first = (int)st.size() / kSegWaves;
     for (int ti : by_scn[s]) {
@@ -600,7 +606,7 @@ int build_segments(pc_pool* p) {
   hipLaunchKernelGGL(k_seg_records, dim3((nrec + 255) / 256), dim3(256), 0, p->stream,
                      p->d_stasks, p->d_segdesc, nrec, A.group, p->d_segrecs);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(p->stream));  // the host vectors end here
+  HIPCHK(hipStreamSynchronize(p->stream));  // the host vectors end or may change again
   p->seg_mode = speed_mode(p);
   return PC_OK;
 }
@@ -627,12 +633,15 @@ int segments_of(int nx, int want) {
 int march_split(const std::vector<Task>& tasks) {
   constexpr double kSimds = 1024, kTogether[4] = {0.0, 96.0, 123.0, 138.0};
   if (tasks.empty()) return 1;
+  int count[kERows + 1] = {};  // tasks by rows
+  for (const Task& t : tasks) ++count[t.nx];
   auto cost = [&](int s) {
     double rows = 0.0, longest = 0.0;
-    for (const Task& t : tasks) {
-      const int r = segments_of(t.nx, s);
-      rows += t.nx + 2.0 * r;
-      longest = std::max(longest, (double)t.nx / r + 2.0);
+    for (int nx = 1; nx <= kERows; ++nx) {
+      if (!count[nx]) continue;
+      const int r = segments_of(nx, s);
+      rows += count[nx] * (nx + 2.0 * r);
+      longest = std::max(longest, (double)nx / r + 2.0);
     }
     const double n = rows / longest / kSimds;  // equal wavefronts a SIMD
     const double full = std::floor(n / 3.0);
@@ -650,12 +659,137 @@ int march_split(const std::vector<Task>& tasks) {
   return want;
 }
 
+// The lists of the boundary speed pass: ghost-edge sources of every live patch
+// by scenario and number of edges, and their wavefronts.
+int build_boundary(pc_pool* p) {
+  const std::vector<int>& live = p->h_live;
+  const std::vector<int>& rseg_of = p->h_rseg;
+  const std::vector<PatchDev>& pd = p->h_pd;
+  const size_t n = live.size(), nscn = p->scn.size();
+  std::vector<unsigned char> shared(n);  // bit d: lower side d shared with a
+                                         // same-size neighbour that sees this
+                                         // patch across its upper side
+  std::vector<int> edges(n);
+  long long lanes = 0;
+  // lanes of a patch: enough to hold its edges per_lane at a time
+  auto lane_class = [](int e, int per_lane) {
+    int c = 0;
+    while (c < kEdgeLaneClasses - 1 && (kMinEdgeLanes << c) * per_lane < e) ++c;
+    return c;
+  };
+  for (size_t k = 0; k < n; ++k) {
+    const int i = live[k];
+    const PatchDev& P = pd[i];
+    const SideDev& sd = p->h_sides[i];
+    for (int d = 0; d < 2; ++d) {
+      if (sd.kind[2 * d] != kSideNeighbour) continue;
+      const int q = sd.src[2 * d];
+      const SideDev& sq = p->h_sides[q];
+      const PatchDev& Q = pd[q];
+      if (sq.kind[2 * d + 1] == kSideNeighbour && sq.src[2 * d + 1] == i && Q.dx == P.dx &&
+          Q.dy == P.dy && Q.nx == P.nx && Q.ny == P.ny && Q.scn == P.scn && p->slots[q].live)
+        shared[k] |= 1 << d;
+    }
+    edges[k] = ((shared[k] & 1 ? 1 : 2) + rseg_of[i] - 1) * P.ny +
+               (shared[k] & 2 ? 1 : 2) * P.nx;
+    lanes += kMinEdgeLanes << lane_class(edges[k], kEdgesPerLane / 2);
+  }
+  // half of what a lane can hold where that still fits the GPU at once
+  const int per_lane =
+      lanes / 64 <= kBoundaryWide ? kEdgesPerLane / 2 : kEdgesPerLane;
+  std::vector<int> first(nscn * kEdgeLaneClasses + 1);
+  for (size_t k = 0; k < n; ++k)
+    ++first[(size_t)pd[live[k]].scn * kEdgeLaneClasses + lane_class(edges[k], per_lane) + 1];
+  for (size_t k = 1; k < first.size(); ++k) first[k] += first[k - 1];
+  // wavefronts: patches of one scenario with equally many lanes
+  std::vector<BoundaryWave> waves;
+  for (size_t k = 0; k + 1 < first.size(); ++k) {
+    const int ln = kMinEdgeLanes << (k % kEdgeLaneClasses);
+    for (int at = first[k]; at < first[k + 1]; at += 64 / ln)
+      waves.push_back(BoundaryWave{at, std::min(64 / ln, first[k + 1] - at), ln,
+                                   (int)(k / kEdgeLaneClasses)});
+  }
+  p->nbwaves = (int)waves.size();
+  // the lists as they lie on the device
+  std::vector<char>& lists = p->h_boundary;
+  lists.resize(n * sizeof(BoundaryDesc) + waves.size() * sizeof(BoundaryWave));
+  BoundaryDesc* const bdv = reinterpret_cast<BoundaryDesc*>(lists.data());
+  if (n) std::memcpy(bdv + n, waves.data(), waves.size() * sizeof(BoundaryWave));
+  for (size_t k = 0; k < n; ++k) {
+    const int i = live[k];
+    const PatchDev& P = pd[i];
+    const SideDev& sd = p->h_sides[i];
+    const long long stride = P.stride;  // a same-size neighbour's too
+    BoundaryDesc& D = bdv[first[(size_t)P.scn * kEdgeLaneClasses +
+                                lane_class(edges[k], per_lane)]++];
+    D.off = P.off;
+    D.stride = P.stride;
+    D.nx = P.nx;
+    D.ny = P.ny;
+    D.scn = P.scn;
+    D.slot = i;
+    D.dx = P.dx;
+    D.dy = P.dy;
+    D.rseg = rseg_of[i];
+    for (int side = 0; side < 2; ++side) {
+      const int kx = sd.kind[side];
+      D.xwall[side] = kx == kSideWall;
+      if (kx == kSideNeighbour) {
+        const PatchDev& Q = pd[sd.src[side]];
+        D.xrow[side] = Q.off + (side ? 1 : Q.nx) * stride;
+      } else if (kx == kSideWall) {
+        D.xrow[side] = P.off + (side ? P.nx : 1) * stride;
+      } else {
+        D.xrow[side] = P.off + (side ? P.nx + 1 : 0) * stride;
+      }
+      const int ky = sd.kind[2 + side];
+      D.ebo[side] = (long long)((i * 2 + side) * 2) * kERows;
+      if (ky == kSideNeighbour)
+        D.ebg[side] = (long long)((sd.src[2 + side] * 2 + (1 - side)) * 2) * kERows;
+      else
+        D.ebg[side] = ky == kSideWall ? -1 : -2;
+    }
+    for (int d = 0; d < 2; ++d) D.shared[d] = shared[k] >> d & 1;
+  }
+  if (n > p->bdesc_cap) {
+    // at most one wavefront and less than one workgroup per patch
+    if (p->d_bdesc) HIPCHK(hipFree(p->d_bdesc));
+    p->d_bdesc = nullptr;
+    p->bdesc_cap = 0;
+    HIPCHK(hipMalloc(&p->d_bdesc, 2 * n * (sizeof(BoundaryDesc) + sizeof(BoundaryWave) +
+                                           sizeof(double))));
+    p->bdesc_cap = 2 * n;
+  }
+  if (n) {
+    p->d_bwaves = reinterpret_cast<BoundaryWave*>(p->d_bdesc + n);
+    p->d_bcfl = reinterpret_cast<double*>(p->d_bwaves + n);
+    HIPCHK(hipMemcpyAsync(p->d_bdesc, lists.data(), lists.size(), hipMemcpyHostToDevice,
+                          p->stream));
+  }
+  HIPCHK(hipStreamSynchronize(p->stream));  // the host image may change again
+  p->boundary_ready = true;
+  return PC_OK;
+}
+
+// The lists of a batched step of the present patches in the present mode.
+// Made ahead of a step only: a grid that is being built or a request that is
+// being admitted changes the patches many times in between, and neither list
+// serves the other kind of step.
+int step_lists(pc_pool* p) {
+  if (p->seg_mode != speed_mode(p)) CHK(build_segments(p));  // its line is the mode's
+  if (!p->seg_rows && fused_mode(p) && p->sides_any && !p->boundary_ready) CHK(build_boundary(p));
+  return PC_OK;
+}
+
 // Work list: tasks of same-size patches of one scenario, large sizes first.
 int rebuild_topology(pc_pool* p) {
   if (!p->topo_dirty) return PC_OK;
   CHK(segment_estimates(p));  // from the old lists
+  p->seg_mode = -1;           // step_lists
+  p->boundary_ready = false;
   const int ns = (int)p->slots.size();
-  std::vector<PatchDev> pd(std::max(ns, 1));
+  std::vector<PatchDev>& pd = p->h_pd;
+  pd.assign(std::max(ns, 1), PatchDev{});
   for (int i = 0; i < ns; ++i)
     if (p->slots[i].live) pd[i] = make_patchdev(p->slots[i]);
   const size_t old_cap = p->pd_cap;
@@ -817,121 +951,14 @@ int rebuild_topology(pc_pool* p) {
     HIPCHK(hipMemcpyAsync(p->d_scn_of, scn_of.data(), scn_of.size() * sizeof(int),
                           hipMemcpyHostToDevice, p->stream));
   }
-  if (p->d_tasks) HIPCHK(hipFree(p->d_tasks));
-  HIPCHK(hipMalloc(&p->d_tasks, std::max<size_t>(p->h_tasks.size(), 1) * sizeof(Task)));
+  CHK(ensure_dev(&p->d_tasks, &p->tasks_cap, p->h_tasks.size()));
   if (!p->h_tasks.empty())
     HIPCHK(hipMemcpyAsync(p->d_tasks, p->h_tasks.data(), p->h_tasks.size() * sizeof(Task),
                           hipMemcpyHostToDevice, p->stream));
-  if (p->d_utasks) HIPCHK(hipFree(p->d_utasks));
-  HIPCHK(hipMalloc(&p->d_utasks, std::max<size_t>(utasks.size(), 1) * sizeof(Task)));
+  CHK(ensure_dev(&p->d_utasks, &p->utasks_cap, utasks.size()));
   if (!utasks.empty())
     HIPCHK(hipMemcpyAsync(p->d_utasks, utasks.data(), utasks.size() * sizeof(Task),
                           hipMemcpyHostToDevice, p->stream));
-  {
-    // ghost-edge sources of every live patch for the boundary speed pass, by
-    // scenario and number of edges
-    const size_t n = live.size();
-    std::vector<unsigned char> shared(n);  // bit d: lower side d shared with a
-                                           // same-size neighbour that sees this
-                                           // patch across its upper side
-    std::vector<int> edges(n);
-    long long lanes = 0;
-    // lanes of a patch: enough to hold its edges per_lane at a time
-    auto lane_class = [](int e, int per_lane) {
-      int c = 0;
-      while (c < kEdgeLaneClasses - 1 && (kMinEdgeLanes << c) * per_lane < e) ++c;
-      return c;
-    };
-    for (size_t k = 0; k < n; ++k) {
-      const int i = live[k];
-      const PatchDev& P = pd[i];
-      const SideDev& sd = p->h_sides[i];
-      for (int d = 0; d < 2; ++d) {
-        if (sd.kind[2 * d] != kSideNeighbour) continue;
-        const int q = sd.src[2 * d];
-        const SideDev& sq = p->h_sides[q];
-        const PatchDev& Q = pd[q];
-        if (sq.kind[2 * d + 1] == kSideNeighbour && sq.src[2 * d + 1] == i && Q.dx == P.dx &&
-            Q.dy == P.dy && Q.nx == P.nx && Q.ny == P.ny && Q.scn == P.scn && p->slots[q].live)
-          shared[k] |= 1 << d;
-      }
-      edges[k] = ((shared[k] & 1 ? 1 : 2) + rseg_of[i] - 1) * P.ny +
-                 (shared[k] & 2 ? 1 : 2) * P.nx;
-      lanes += kMinEdgeLanes << lane_class(edges[k], kEdgesPerLane / 2);
-    }
-    // half of what a lane can hold where that still fits the GPU at once
-    const int per_lane =
-        lanes / 64 <= kBoundaryWide ? kEdgesPerLane / 2 : kEdgesPerLane;
-    std::vector<int> first((size_t)nscn * kEdgeLaneClasses + 1);
-    for (size_t k = 0; k < n; ++k)
-      ++first[(size_t)pd[live[k]].scn * kEdgeLaneClasses + lane_class(edges[k], per_lane) + 1];
-    for (size_t k = 1; k < first.size(); ++k) first[k] += first[k - 1];
-    // wavefronts: patches of one scenario with equally many lanes
-    std::vector<BoundaryWave> waves;
-    for (size_t k = 0; k + 1 < first.size(); ++k) {
-      const int ln = kMinEdgeLanes << (k % kEdgeLaneClasses);
-      for (int at = first[k]; at < first[k + 1]; at += 64 / ln)
-        waves.push_back(BoundaryWave{at, std::min(64 / ln, first[k + 1] - at), ln,
-                                     (int)(k / kEdgeLaneClasses)});
-    }
-    p->nbwaves = (int)waves.size();
-    // the lists as they lie on the device
-    std::vector<char> lists(n * sizeof(BoundaryDesc) + waves.size() * sizeof(BoundaryWave));
-    BoundaryDesc* const bdv = reinterpret_cast<BoundaryDesc*>(lists.data());
-    if (n) std::memcpy(bdv + n, waves.data(), waves.size() * sizeof(BoundaryWave));
-    for (size_t k = 0; k < n; ++k) {
-      const int i = live[k];
-      const PatchDev& P = pd[i];
-      const SideDev& sd = p->h_sides[i];
-      const long long stride = P.stride;  // a same-size neighbour's too
-      BoundaryDesc& D = bdv[first[(size_t)P.scn * kEdgeLaneClasses +
-                                  lane_class(edges[k], per_lane)]++];
-      D.off = P.off;
-      D.stride = P.stride;
-      D.nx = P.nx;
-      D.ny = P.ny;
-      D.scn = P.scn;
-      D.slot = i;
-      D.dx = P.dx;
-      D.dy = P.dy;
-      D.rseg = rseg_of[i];
-      for (int side = 0; side < 2; ++side) {
-        const int kx = sd.kind[side];
-        D.xwall[side] = kx == kSideWall;
-        if (kx == kSideNeighbour) {
-          const PatchDev& Q = pd[sd.src[side]];
-          D.xrow[side] = Q.off + (side ? 1 : Q.nx) * stride;
-        } else if (kx == kSideWall) {
-          D.xrow[side] = P.off + (side ? P.nx : 1) * stride;
-        } else {
-          D.xrow[side] = P.off + (side ? P.nx + 1 : 0) * stride;
-        }
-        const int ky = sd.kind[2 + side];
-        D.ebo[side] = (long long)((i * 2 + side) * 2) * kERows;
-        if (ky == kSideNeighbour)
-          D.ebg[side] = (long long)((sd.src[2 + side] * 2 + (1 - side)) * 2) * kERows;
-        else
-          D.ebg[side] = ky == kSideWall ? -1 : -2;
-      }
-      for (int d = 0; d < 2; ++d) D.shared[d] = shared[k] >> d & 1;
-    }
-    if (n > p->bdesc_cap) {
-      // at most one wavefront and less than one workgroup per patch
-      if (p->d_bdesc) HIPCHK(hipFree(p->d_bdesc));
-      p->d_bdesc = nullptr;
-      p->bdesc_cap = 0;
-      HIPCHK(hipMalloc(&p->d_bdesc, 2 * n * (sizeof(BoundaryDesc) + sizeof(BoundaryWave) +
-                                             sizeof(double))));
-      p->bdesc_cap = 2 * n;
-    }
-    if (n) {
-      p->d_bwaves = reinterpret_cast<BoundaryWave*>(p->d_bdesc + n);
-      p->d_bcfl = reinterpret_cast<double*>(p->d_bwaves + n);
-      HIPCHK(hipMemcpyAsync(p->d_bdesc, lists.data(), lists.size(), hipMemcpyHostToDevice,
-                            p->stream));
-    }
-  }
-  CHK(build_segments(p));
   CHK(ensure_dev(&p->d_live, &p->live_cap, std::max<size_t>(live.size(), 1)));
   if (!live.empty())
     HIPCHK(hipMemcpyAsync(p->d_live, live.data(), live.size() * sizeof(int),
@@ -951,7 +978,6 @@ int rebuild_topology(pc_pool* p) {
 int prepare(pc_pool* p) {
   CHK(sync_scn_host(p));
   CHK(rebuild_topology(p));
-  if (p->seg_mode != speed_mode(p)) CHK(build_segments(p));  // its line is the mode's
   if (p->scn_dev_dirty) CHK(upload_scn(p));
   return PC_OK;
 }
@@ -969,6 +995,7 @@ EdgeBufs edges_of(pc_pool* p) {
 // the interior speed maxima of the current state.
 int prepare_batched(pc_pool* p, bool plain = false) {
   CHK(prepare(p));
+  if (!plain) CHK(step_lists(p));
   p->uploaded = false;
   // a step on short row segments reads the tiles alone
   if (p->seg_rows && !plain) return PC_OK;
