@@ -1170,6 +1170,9 @@ k_dt_block(ScnDev* __restrict__ scn, int nscn, const int* __restrict__ plist_scn
 // and, for the fallback, speeds and dt once more (two dt launches each time
 // beyond kDtBlockEntries patches).  A step of 50,000 patches spent 26 us on
 // them, one of 1600 patches 14 us; this launch takes 6 and 5 us.
+// The fallback's workgroups pass nothing but atomics on, so their order needs
+// no fence: two agent-scope fences each (an L2 write-back) took 44 us of the
+// 440 us of a step of 14,400 patches of 32^2 that falls back.
 __global__ void __launch_bounds__(64)
 k_march_dt(const Task* __restrict__ tasks, int ntasks, const int* __restrict__ plist,
            const PatchDev* __restrict__ pd, Fields F, ScnDev* in, ScnDev* __restrict__ out,
@@ -1213,10 +1216,11 @@ k_march_dt(const Task* __restrict__ tasks, int ntasks, const int* __restrict__ p
   }
   for (int o = 32; o >= 1; o >>= 1) m = dmin(m, __shfl_xor(m, o));
   if (lane != 0) return;
-  atomicMin(&in->minbits, (unsigned long long)__double_as_longlong(m));
-  __threadfence();
-  if (atomicAdd(ticket, 1) != (int)gridDim.x - 1) return;
-  __threadfence();
+  // counted once its minimum is in (the count waits for what atomicMin returned:
+  // 0 added, the bits being those of a positive number)
+  const unsigned long long before =
+      atomicMin(&in->minbits, (unsigned long long)__double_as_longlong(m));
+  if (atomicAdd(ticket, 1 + (int)(before >> 63)) != (int)gridDim.x - 1) return;
   ScnDev S = *in;
   S.minbits = (unsigned long long)__double_as_longlong(kNone);
   const unsigned long long bits = atomicExch(&in->minbits, S.minbits);
