@@ -630,11 +630,17 @@ int segments_of(int nx, int want) {
 //   80 x 80 of 64^2: 366 334 340           90 x 90 of 32^2: 139 123 141
 //   100 x 100 of 48^2: 338 344 401         24 x 24 of 64^2: 96 57 46
 //   32 x 32 of 64^2: 97 73 73
-int march_split(const std::vector<Task>& tasks) {
+//
+// Without side sources the update holds a fourth wavefront on a SIMD, so three
+// to four of short patches are no round left over: us a step with tile ghosts
+// for 1, 2, 4 segments, 79 x 79 patches of 32^2: 251 259 255, 90 x 90: 325 335
+// 327 (of 64-row patches: 56 x 56, 394 398 380).
+int march_split(const std::vector<Task>& tasks, bool sides) {
   constexpr double kSimds = 1024, kTogether[4] = {0.0, 96.0, 123.0, 138.0};
   if (tasks.empty()) return 1;
   int count[kERows + 1] = {};  // tasks by rows
   for (const Task& t : tasks) ++count[t.nx];
+  double whole = 0.0, most = 0.0;  // wavefronts a SIMD and rows of whole patches
   auto cost = [&](int s) {
     double rows = 0.0, longest = 0.0;
     for (int nx = 1; nx <= kERows; ++nx) {
@@ -644,11 +650,13 @@ int march_split(const std::vector<Task>& tasks) {
       longest = std::max(longest, (double)nx / r + 2.0);
     }
     const double n = rows / longest / kSimds;  // equal wavefronts a SIMD
+    if (s == 1) whole = n, most = longest - 2.0;
     const double full = std::floor(n / 3.0);
     return (full * kTogether[3] + kTogether[(int)std::ceil(n - 3.0 * full)]) * longest;
   };
   int want = 1;
   double best = cost(1);
+  if (!sides && most <= 32.0 && whole > 3.0 && whole <= 4.0) return 1;
   for (int s = 2; s <= kMaxRowSeg; s *= 2) {
     const double c = cost(s);
     if (c < 0.95 * best) {
@@ -896,7 +904,7 @@ int rebuild_topology(pc_pool* p) {
   std::vector<Task> utasks;
   std::vector<int> rseg_of(ns, 1);
   {
-    const int want = p->row_segments ? p->row_segments : march_split(p->h_tasks);
+    const int want = p->row_segments ? p->row_segments : march_split(p->h_tasks, p->sides_any);
     for (const Task& t : p->h_tasks) {
       const int r = segments_of(t.nx, want);
       for (int k = 0; k < r; ++k) {
