@@ -49,3 +49,32 @@ def test_many_scenarios(scenarios, solver, fused):
                           for s in slots]
     for x, y in zip(run(0), run(1)):
         assert np.array_equal(x, y)
+
+
+# the augmented solver on segments of 4 rows: more wavefronts at 2 rows than
+# its limit (33 x 33 patches of 8 x 64: 4356)
+@pytest.mark.parametrize("dry", [False, True])
+def test_augmented_four_rows(dry):
+    def run(segments):
+        with PatchPool(0) as pool:
+            rng = np.random.default_rng(17)
+            p, nx, ny = 33, 8, 64
+            slots = [pool.register(make_description(divmod(k, p), (nx / 64, ny / 64), nx, ny=ny))
+                     for k in range(p * p)]
+            o = [pool.offset(s) for s in slots]
+            cells = o[-1] + (nx + 2) * tile_stride(ny) - o[0]
+            f = [rng.uniform(0.5, 2.0, cells) * a for a in (1.0, 0.3, 0.3, 0.1)]
+            if dry:
+                f[0][rng.uniform(0.0, 1.0, cells) < 0.2] = 0.0
+            pool.copy_fields(True, 0, o[0], *f)
+            grid = np.array(slots, np.int32).reshape(p, p)
+            Workload(pool, [GridLayout(nx, grid, ny)], 0, 0, []).build_ghost_table()
+            pool.scenario_set(0, 0.0, 0.0, math.inf)
+            pool.wave_propagation_solver(2)
+            pool.row_segments(segments)
+            pool.step(3)
+            return ([np.array(pool.scenario_get(0))] + [pool.download(s)[0] for s in slots[::7]] +
+                    [np.array(pool.description(s).estimated_next_timestep_size)
+                     for s in slots[::7]])
+    for x, y in zip(run(0), run(1)):
+        assert np.array_equal(x, y)
