@@ -7,9 +7,9 @@ Gaussian-hill bathymetry; each step = ghost fill + CFL reduction + update
 of every patch with one global dt.  One "step" advances all 68M cells once.
 
 Prints one JSON line: cell-updates/s of the batched path, its HBM roofline
-fraction (update kernel, HIP events around every launch of the timed
-steps), the plain per-patch-launch path on the same pool, the hipGraph
-replay rate, p50/p99 time-to-solution of a served stream of independent
+fraction (update kernel, HIP events around every eighth launch of the timed
+steps and the last), the plain per-patch-launch path on the same pool, the rate of
+replayed steps, p50/p99 time-to-solution of a served stream of independent
 dam-break requests (Poisson arrivals, continuous batching under an HBM
 budget), and the CPU oracle timed on the host cores on a sample.
 
@@ -251,7 +251,7 @@ def main():
     log(f"batched: {ms_per_step:.3f} ms/step (events {ev_total_ms / args.steps:.3f}), "
         f"update kernel {upd_ms:.3f} ms, {value / 1e9:.2f} G cell-updates/s")
 
-    # hipGraph replay of {ghost fill, CFL reduction, dt, update}
+    # replay of {ghost fill, CFL reduction, dt, update} as prepared
     pool.graph_capture()
     pool.graph_replay(2)
     pool.synchronize()

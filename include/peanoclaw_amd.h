@@ -158,8 +158,8 @@ int pc_post_process_restriction(pc_pool *pool, int destination_slot,
  * destroyCell's interpolateSolution and restrictSolution sequences,
  * Remesh.cpp:331-540).  A batch has exactly the effect of its calls made one
  * after another in the order given: calls that share no patch run together,
- * a workgroup each, and calls that share patches one after another.  Every call is checked before any
- * runs; an invalid one fails the batch with nothing changed.
+ * calls that share patches one after another.  Every call is checked before
+ * any runs; an invalid one fails the batch with nothing changed.
  *
  * pc_interpolate_batch: `count` pc_interpolate_solution calls; call i has
  * destination_size {dsize[2i], dsize[2i+1]}, destination_offset
@@ -475,8 +475,11 @@ int pc_server_release(pc_server *srv, int id);
  * interpolation from the coarser leaf, domain walls, global CFL minimum,
  * solveTimestep of every leaf; GridLevelTransfer.cpp:140-198,
  * GhostlayerCompositorFunctors.cpp:59-69, SolveTimestep.cpp:87-142 and
- * 591-751) handed over once as a plan and run as three launches per step.  Level transfers read h + b instead of transforming the source in
- * place and back (the reference's round trip can move a depth by an ulp;
+ * 591-751) handed over once as a plan and run as three launches per step
+ * (four where the leaves make more than 1024 tasks of up to 16 equal leaves
+ * that share a wavefront's columns).  Level transfers read h + b instead of
+ * transforming the source in place and back (the reference's round trip can
+ * move a depth by an ulp;
  * results agree with the per-call form to ~1e-14 relative).  No reference
  * counterpart as one entry point: it replaces the traversal's calls for a
  * grid whose leaves share one clock.  The plan stays valid while its

@@ -2,8 +2,8 @@
 //
 // Host side of the patch pool: HBM allocation of the structure-of-arrays
 // fields, slot registry mirroring CellDescription, scenario clocks, the
-// ghost-strip table, the work list of the batched update, hipGraph capture
-// of one step, and the per-patch Numerics-mirroring calls.
+// ghost-strip table, the work lists of the batched update, the launches of its
+// steps, and the per-patch Numerics-mirroring calls.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -24,6 +24,9 @@
 //   update   of every leaf, uOld -> uNew, with the smallest of those steps
 //            bounded by the end time; one workgroup advances the clock
 //
+// (and a fourth between the last two where there are more than kCflFold
+// workgroups' steps: k_cfl_fold).
+//
 // These grids hold a few hundred thousand cells, so latency bounds them: the
 // fill loads a leaf's cells once for the copy and the speeds, and neither
 // the copy, the walls nor the reduction of dt is a launch of its own.  The
@@ -142,13 +145,12 @@ struct AmrWalls {
 
 // One task of leaves in the fill (workgroup b): its row segments are
 // wavefronts [b max_waves, + nwaves) of the plan's records, its ghost cells'
-// entries gmap[b max_cells .. + ncells).
+// entries gmap[b max_cells .. + max_cells) (-1: none).
 struct AmrBlock {
   int nwaves, leaf0, nseg;  // leaf0: place of its first leaf in task order
   int nx, ny;
-  int ncells;
   int nwalls;  // most walls of one of its leaves
-  int pad;
+  int pad[2];
 };
 
 // Restriction time factors of a leaf source on the [0, 1] basis
@@ -1422,13 +1424,13 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     for (int k = 0; k < blocks[b].nseg; ++k) block_of[blocks[b].leaf0 + k] = (int)b;
   std::vector<int> gmap;
   {
-    std::vector<int> b_of(gh.size());
+    std::vector<int> b_of(gh.size()), ncells(blocks.size(), 0);
     for (size_t e = 0; e < gh.size(); ++e) {
       b_of[e] = block_of[pos[gh[e].dst]];
-      AmrBlock& B = blocks[b_of[e]];
-      gh[e].cell0 = B.ncells;
-      B.ncells += gh[e].sx * gh[e].sy;
-      a->max_cells = std::max(a->max_cells, B.ncells);
+      int& n = ncells[b_of[e]];
+      gh[e].cell0 = n;
+      n += gh[e].sx * gh[e].sy;
+      a->max_cells = std::max(a->max_cells, n);
     }
     gmap.assign(blocks.size() * (size_t)a->max_cells, -1);
     for (size_t e = 0; e < gh.size(); ++e)

@@ -796,9 +796,10 @@ k_boundary_speed(const ScnDev* __restrict__ scn, const BoundaryWave* __restrict_
     // edge list: x-lower (ny), x-upper (ny), y-lower (nx), y-upper (nx), then
     // the seams of the update's row segments: the x-edges (a-1 | a) of the new
     // state at the first row a of every segment after the first (each segment
-    // of the update saw only one side of them).  In pruned mode only the scenario minimum of the CFL steps is used, so an
-    // edge shared with a same-size neighbour is evaluated once, by the patch
-    // below it; each patch keeps its upper sides, walls and tile ghosts.
+    // of the update saw only one side of them).  In pruned mode only the
+    // scenario minimum of the CFL steps is used, so an edge shared with a
+    // same-size neighbour is evaluated once, by the patch below it; each patch
+    // keeps its upper sides, walls and tile ghosts.
     const int l0 = (PRUNE && D.shared[0]) ? 0 : ny;
     const int l2 = (PRUNE && D.shared[1]) ? 0 : nx;
     const int b1 = l0, b2 = l0 + ny, b3 = b2 + l2;

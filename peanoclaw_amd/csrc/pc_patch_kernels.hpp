@@ -556,6 +556,9 @@ k_level_calls(Fields F, const Call* __restrict__ calls, const int* __restrict__ 
 }
 
 // Patch::switchToLeaf (Patch.cpp:793-830) of a batch of patches (patch
+// blockIdx.y): the [0, 1]-basis values of the restriction evaluated at the
+// leaf's interval, uOld = vo (1 - fOld) + vn fOld and uNew = vo (1 - fNew)
+// + vn fNew over the interior cells.
 struct LeafSwitch {
   int slot, cur;
   double fOld, fNew;
