@@ -113,6 +113,9 @@ struct pc_pool {
   int row_segments = 0;  // 0 automatic, 1 off, 2 or 4 forced
   std::vector<int> h_rseg;  // row segments per slot of the current list
   std::vector<PatchDev> h_pd;  // d_pd's rows
+  // counts the changes of the slots' tiles, sizes and roles, as far as prepare
+  // has seen them
+  unsigned long long layout = 0;
   // steps with too few patches to fill the GPU run on short row segments
   // (pc_seg_kernels.hpp) of at most seg_rows rows; 0: the row march
   int seg_rows = 0;
@@ -789,9 +792,11 @@ int step_lists(pc_pool* p) {
   return PC_OK;
 }
 
-// Work list: tasks of same-size patches of one scenario, large sizes first.
-int rebuild_topology(pc_pool* p) {
+// Work list: tasks of same-size patches of one scenario, large sizes first;
+// ahead of a `step` its lists with it (while the copies run).
+int rebuild_topology(pc_pool* p, bool step) {
   if (!p->topo_dirty) return PC_OK;
+  ++p->layout;
   CHK(segment_estimates(p));  // from the old lists
   p->seg_mode = -1;           // step_lists
   p->boundary_ready = false;
@@ -967,6 +972,7 @@ int rebuild_topology(pc_pool* p) {
   if (!utasks.empty())
     HIPCHK(hipMemcpyAsync(p->d_utasks, utasks.data(), utasks.size() * sizeof(Task),
                           hipMemcpyHostToDevice, p->stream));
+  if (step) CHK(step_lists(p));
   CHK(ensure_dev(&p->d_live, &p->live_cap, std::max<size_t>(live.size(), 1)));
   if (!live.empty())
     HIPCHK(hipMemcpyAsync(p->d_live, live.data(), live.size() * sizeof(int),
@@ -983,9 +989,9 @@ int rebuild_topology(pc_pool* p) {
   return PC_OK;
 }
 
-int prepare(pc_pool* p) {
+int prepare(pc_pool* p, bool step = false) {
   CHK(sync_scn_host(p));
-  CHK(rebuild_topology(p));
+  CHK(rebuild_topology(p, step));
   if (p->scn_dev_dirty) CHK(upload_scn(p));
   return PC_OK;
 }
@@ -1002,7 +1008,7 @@ EdgeBufs edges_of(pc_pool* p) {
 // state: edge buffers (after uploads / per-patch calls), and in fused mode
 // the interior speed maxima of the current state.
 int prepare_batched(pc_pool* p, bool plain = false) {
-  CHK(prepare(p));
+  CHK(prepare(p, !plain));
   if (!plain) CHK(step_lists(p));
   p->uploaded = false;
   // a step on short row segments reads the tiles alone
@@ -1040,7 +1046,7 @@ void launch_segments(pc_pool* p, Fields F, hipEvent_t eb, hipEvent_t ee) {
   const int nscn = (int)p->scn.size();
   hipLaunchKernelGGL((k_seg_update<R, SOLVER>), dim3(g + seg_clock_groups(nscn)),
                      dim3(64 * kSegWaves), 0, p->stream, A.recs, p->d_scn, A.group, A.lanes,
-                     A.scn, nscn, p->d_ranges, p->d_cfl_block, p->d_scn_alt, F);
+                     A.scn, nscn, (int)g, p->d_ranges, p->d_cfl_block, p->d_scn_alt, F);
   if (ee) hipEventRecord(ee, p->stream);
   std::swap(p->d_scn, p->d_scn_alt);
   std::swap(p->scn_cap, p->scn_alt_cap);
@@ -1425,6 +1431,7 @@ int pc_patch_set_description(pc_pool* p, int slot, const pc_cell_description* d)
       d->scenario != s.desc.scenario || d->ghostlayer_width != 1)
     return fail(PC_E_INVALID, "size, ghost width and scenario are fixed per slot");
   bool geom = d->size[0] != s.desc.size[0] || d->size[1] != s.desc.size[1];
+  if (d->is_virtual != s.desc.is_virtual) ++p->layout;
   s.desc = *d;
   s.clock_from_scenario = false;
   if (geom) {
@@ -2311,6 +2318,7 @@ int pc_switch_to_leaf(pc_pool* p, int count, const int* slots, const double* tim
   for (int i = 0; i < count; ++i) {
     Slot& s = p->slots[slots[i]];
     s.desc.is_virtual = 0;
+    ++p->layout;
     s.desc.time = time[i];
     s.desc.timestep_size = dt[i];
     s.clock_from_scenario = false;

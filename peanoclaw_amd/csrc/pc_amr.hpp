@@ -917,8 +917,9 @@ struct pc_amr {
   std::vector<int> leaves, virtuals, plan_slots;
   std::vector<int> leaf_nx, leaf_ny;
   int nvblocks = 0, nghosts = 0;
-  // what the tables hold of the plan's slots (amr_refresh), and the tables
+  // what the tables hold of the plan's slots (amr_follow_slots), and the tables
   // themselves where they depend on it
+  unsigned long long layout = 0;  // of the pool, as these follow it
   std::vector<AmrPlace> places;  // per plan slot
   std::vector<SegDesc> h_desc;   // per leaf in task order
   std::vector<AmrVBlock> h_vblocks;
@@ -1089,10 +1090,11 @@ int amr_device_tables(pc_amr* a, bool places) {
 // released and registered again, and pc_patch_set_description may give a live
 // patch another size.  Steps and speeds take the cells' size as it is now; the
 // transfers between patches keep the geometry they were created with.  Called
-// ahead of every step call, after prepare (the slots' tiles on the device) and
-// amr_check_slots.
-int amr_refresh(pc_amr* a) {
+// ahead of every step call, after prepare (the slots' tiles on the device).
+int amr_follow_slots(pc_amr* a) {
   pc_pool* p = a->pool;
+  if (a->layout == p->layout) return PC_OK;
+  CHK(amr_check_slots(a));
   bool moved = false, sized = false;
   for (size_t i = 0; i < a->plan_slots.size(); ++i) {
     const Slot& s = p->slots[a->plan_slots[i]];
@@ -1100,7 +1102,10 @@ int amr_refresh(pc_amr* a) {
     moved = moved || s.off != q.off;
     sized = sized || s.desc.size[0] != q.size[0] || s.desc.size[1] != q.size[1];
   }
-  if (!moved && !sized) return PC_OK;
+  if (!moved && !sized) {
+    a->layout = p->layout;
+    return PC_OK;
+  }
   for (SegDesc& d : a->h_desc) d = amr_seg_desc(p, d.slot);
   HIPCHK(hipMemcpyAsync(a->d_desc, a->h_desc.data(), a->h_desc.size() * sizeof(SegDesc),
                         hipMemcpyHostToDevice, p->stream));
@@ -1120,6 +1125,7 @@ int amr_refresh(pc_amr* a) {
   HIPCHK(hipStreamSynchronize(p->stream));
   for (size_t i = 0; i < a->plan_slots.size(); ++i)
     a->places[i] = amr_place(p->slots[a->plan_slots[i]]);
+  a->layout = p->layout;
   return PC_OK;
 }
 
@@ -1167,6 +1173,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->plan_slots = a->leaves;
   a->plan_slots.insert(a->plan_slots.end(), a->virtuals.begin(), a->virtuals.end());
   for (int s : a->plan_slots) a->places.push_back(amr_place(p->slots[s]));
+  a->layout = p->layout;
   // leaf clock: every leaf on one clock
   double t0, dt0;
   slot_clock(p, leaves[0], &t0, &dt0);
@@ -1694,7 +1701,7 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   pc_pool* p = a->pool;
   hipSetDevice(p->device);
   CHK(prepare(p));
-  CHK(amr_check_slots(a));
+  CHK(amr_follow_slots(a));
   const int nl = (int)a->leaves.size();
   std::vector<char> role(p->slots.size(), 0);
   for (int s : a->leaves) role[s] = 1;
@@ -1782,8 +1789,7 @@ int pc_amr_lts_step(pc_amr* a, int k, double end_time, long long* leaf_steps) {
   pc_pool* p = a->pool;
   hipSetDevice(p->device);
   CHK(prepare(p));
-  CHK(amr_check_slots(a));
-  CHK(amr_refresh(a));
+  CHK(amr_follow_slots(a));
   int cur;
   CHK(amr_cur(a, &cur));
   mark_state_changed(p);
@@ -1817,8 +1823,7 @@ int pc_amr_step(pc_amr* a, int k, double end_time, double* last_dt) {
   pc_pool* p = a->pool;
   hipSetDevice(p->device);
   CHK(prepare(p));
-  CHK(amr_check_slots(a));
-  CHK(amr_refresh(a));
+  CHK(amr_follow_slots(a));
   int cur;
   CHK(amr_cur(a, &cur));
   mark_state_changed(p);

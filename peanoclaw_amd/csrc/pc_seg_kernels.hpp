@@ -521,22 +521,21 @@ __host__ __device__ __forceinline__ int seg_clock_groups(int nscn) {
 
 // The update of the same segments, current state -> other state.  Every
 // workgroup takes its scenario's step from the blocks' minima and the clock
-// `in`; the last workgroups (seg_clock_groups) advance the clocks of the
-// scenarios into `out` (the next step's `in`), so no launch is needed between
+// `in`; the workgroups from `blocks` on (seg_clock_groups) advance the clocks of
+// the scenarios into `out` (the next step's `in`), so no launch is needed between
 // the speeds and the update.
 template <int R, int SOLVER>
 __global__ void __launch_bounds__(64 * kSegWaves)
 __attribute__((amdgpu_waves_per_eu(R == 4 ? 3 : 2, 8)))
 k_seg_update(const SegRec* recs, const ScnDev* __restrict__ in, int group, int lanes, int one,
-             int nscn, const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block,
+             int nscn, int blocks, const SegRange* __restrict__ ranges, const double* __restrict__ cfl_block,
              ScnDev* __restrict__ out, Fields F) {
   const SegList A{recs, group, lanes, one};
   __shared__ double pre[kSegWaves][4][64];
   __shared__ double red[kSegWaves];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int clocks = (int)blockIdx.x - ((int)gridDim.x - seg_clock_groups(nscn));
-  if (clocks >= 0) {
-    const int s = clocks * kSegWaves + w;
+  if ((int)blockIdx.x >= blocks) {
+    const int s = ((int)blockIdx.x - blocks) * kSegWaves + w;
     if (s >= nscn) return;
     const double cfl = cfl_share(gl(ranges + s), cfl_block, lane, 64);
     if (lane == 0) {
