@@ -316,7 +316,8 @@ int pc_step_all_per_patch(pc_pool *pool, int k);
 /* Prepare one step and replay it k times without looking at the grid again.
  * The step's two to seven kernels are launched each time rather than a
  * recorded graph: between two graph launches the GPU idles 5 to 8 us, between
- * kernel launches it does not. */
+ * kernel launches it does not.  The calling thread issues them (about 3 us
+ * each) and has to keep pace with steps shorter than that. */
 int pc_graph_capture(pc_pool *pool);
 int pc_graph_replay(pc_pool *pool, int k);
 /* Refinement flags of all patches (1 refine, 0 coarsening allowed, 2 keep),
