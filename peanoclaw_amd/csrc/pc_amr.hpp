@@ -130,7 +130,7 @@ struct AmrGhost {
   int kind, src, dst;
   int sx, sy, sox, soy, dox, doy;
   int sn[2];
-  int cell0;  // its first cell among the ghost cells of its task's leaves
+  int cell0;  // its first cell in the plan's ghost map
   // tile rows: first cell of the source region (interpolation: cell (0, 0)
   // of the source), first cell of the destination region
   long long sbase, dbase;
@@ -466,19 +466,28 @@ __device__ __forceinline__ void amr_ghost_cell(const AmrGhost g, int k,
   F.HV(oldSt)[di] = acc[2];
 }
 
+// The plan's ghost map (-1 where no entry writes one): every entry's cells, a
+// wavefront per entry.  Runs once per plan.
+__global__ void __launch_bounds__(256)
+k_amr_ghost_map(const AmrGhost* __restrict__ ghosts, int n, int* __restrict__ gmap) {
+  const int e = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  if (e >= n) return;
+  const int cells = ghosts[e].sx * ghosts[e].sy, cell0 = ghosts[e].cell0;
+  for (int k = threadIdx.x & 63; k < cells; k += 64) gmap[cell0 + k] = e;
+}
+
 // Local time stepping: the ghost cells of the advancing leaves, before any
 // leaf changes (one thread per ghost cell of the plan).
 __global__ void __launch_bounds__(256)
-k_lts_ghosts(const int* __restrict__ gmap, int max_cells, int ncells,
-             const AmrGhost* __restrict__ ghosts, Fields F, int cur, const AmrClock* clock,
-             AmrLts L) {
+k_lts_ghosts(const int* __restrict__ gmap, int ncells, const AmrGhost* __restrict__ ghosts,
+             Fields F, int cur, const AmrClock* clock, AmrLts L) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= ncells) return;
   const int e = gl(gmap + c), advancing = gl(L.iter);
   const AmrClock now = gl(clock);
   if (e < 0 || advancing == 0) return;
   const AmrGhost g = gl(ghosts + e);
-  amr_ghost_cell<true>(g, c % max_cells - g.cell0, F, cur, now, L);
+  amr_ghost_cell<true>(g, c - g.cell0, F, cur, now, L);
 }
 
 // SWEKernel::fillBoundaryLayer (SWEKernel.cpp:176-237) of the leaves of a
@@ -584,7 +593,7 @@ k_amr_fill(AmrPlanDev A, Fields F, int cur, const AmrClock* clock,
       const int k = i == (int)threadIdx.x ? ghost : gl(gmap + i);
       if (k < 0) continue;
       const AmrGhost e = gl(A.ghosts + k);
-      amr_ghost_cell<false>(e, i - e.cell0, F, cur, c, L);
+      amr_ghost_cell<false>(e, (int)blockIdx.x * A.max_cells + i - e.cell0, F, cur, c, L);
     }
   // uNew -> uOld (DefaultTransfer::copyUNewToUOld)
 #pragma unroll
@@ -1277,6 +1286,16 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
     }
   }
   std::vector<int> ccount, xcount, span0, span1;
+  {
+    size_t cells = 1;
+    for (int vi = 0; vi < nvirtuals; ++vi)
+      cells += (size_t)p->slots[virtuals[vi]].desc.subdivision_factor[0] *
+               p->slots[virtuals[vi]].desc.subdivision_factor[1];
+    cptr.reserve(cells);
+    xptr.reserve(cells);
+    vblocks.reserve(cells / kRestrictCells + nvirtuals + 256);
+    pairs.reserve(nrestrictions);
+  }
   for (int vi = 0; vi < nvirtuals; ++vi) {
     const int v = virtuals[vi];
     const int pbeg = (int)pairs.size();
@@ -1326,25 +1345,31 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
       span1.resize(R.dSize[1] > 0 ? R.dSize[1] : 0);
       for (size_t k = 0; k < span0.size(); ++k) amr_fine_span(R, 0, R.dOff[0] + (int)k, o, span0[k]);
       for (size_t k = 0; k < span1.size(); ++k) amr_fine_span(R, 1, R.dOff[1] + (int)k, o, span1[k]);
-      for (int x = R.dOff[0]; x < R.dOff[0] + R.dSize[0]; ++x)
-        for (int y = R.dOff[1]; y < R.dOff[1] + R.dSize[1]; ++y) {
-          ++ccount[(size_t)x * ny + y];
-          xcount[(size_t)x * ny + y] += span0[x - R.dOff[0]] * span1[y - R.dOff[1]];
+      for (int x = 0; x < R.dSize[0]; ++x) {
+        const size_t row = (size_t)(R.dOff[0] + x) * ny + R.dOff[1];
+        int *const cc = ccount.data() + row, *const xc = xcount.data() + row, n0 = span0[x];
+        for (int y = 0; y < R.dSize[1]; ++y) {
+          ++cc[y];
+          xc[y] += n0 * span1[y];
         }
+      }
     }
     const size_t cbeg = cpairs.size();
+    cptr.resize(cptr.size() + (size_t)nx * ny);
+    xptr.resize(cptr.size());
     for (int c = 0; c < nx * ny; ++c) {
-      cptr.push_back(cptr.back() + ccount[c]);
+      cptr[base + c + 1] = cptr[base + c] + ccount[c];
       ncontribs += xcount[c];
-      xptr.push_back((int)std::min<long long>(ncontribs, INT_MAX));
+      xptr[base + c + 1] = (int)std::min<long long>(ncontribs, INT_MAX);
     }
     cpairs.resize(cptr.back());
     for (int c = 0; c < nx * ny; ++c) ccount[c] = cptr[base + c] - (int)cbeg;  // cursors
     for (int pi = pbeg; pi < (int)pairs.size(); ++pi) {
       const AmrRestrict& R = pairs[pi];
-      for (int x = R.dOff[0]; x < R.dOff[0] + R.dSize[0]; ++x)
-        for (int y = R.dOff[1]; y < R.dOff[1] + R.dSize[1]; ++y)
-          cpairs[cbeg + ccount[(size_t)x * ny + y]++] = pi;
+      for (int x = 0; x < R.dSize[0]; ++x) {
+        int* const cc = ccount.data() + (size_t)(R.dOff[0] + x) * ny + R.dOff[1];
+        for (int y = 0; y < R.dSize[1]; ++y) cpairs[cbeg + cc[y]++] = pi;
+      }
     }
   }
   for (int r = 0; r < nrestrictions; ++r) {
@@ -1355,6 +1380,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->nvblocks = (int)vblocks.size();
   // ghost faces
   std::vector<AmrGhost> gh;
+  gh.reserve(nghosts);
   for (int i = 0; i < nghosts; ++i) {
     const pc_amr_ghost& G = ghosts[i];
     const int s = G.src, d = G.dst;
@@ -1429,7 +1455,6 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   std::vector<int> block_of(plist.size());
   for (size_t b = 0; b < blocks.size(); ++b)
     for (int k = 0; k < blocks[b].nseg; ++k) block_of[blocks[b].leaf0 + k] = (int)b;
-  std::vector<int> gmap;
   {
     std::vector<int> b_of(gh.size()), ncells(blocks.size(), 0);
     for (size_t e = 0; e < gh.size(); ++e) {
@@ -1439,10 +1464,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
       n += gh[e].sx * gh[e].sy;
       a->max_cells = std::max(a->max_cells, n);
     }
-    gmap.assign(blocks.size() * (size_t)a->max_cells, -1);
-    for (size_t e = 0; e < gh.size(); ++e)
-      std::fill_n(gmap.begin() + (size_t)b_of[e] * a->max_cells + gh[e].cell0,
-                  gh[e].sx * gh[e].sy, (int)e);
+    for (size_t e = 0; e < gh.size(); ++e) gh[e].cell0 += b_of[e] * a->max_cells;
   }
   // walls grouped per leaf in call order
   std::vector<AmrWalls> wl(plist.size(), AmrWalls{0, 0});
@@ -1474,7 +1496,6 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   // DMA instead of fifteen of each)
   PinnedTables st;
   const size_t o_blocks = st.add(blocks), o_tasks = st.add(segs), o_desc = st.add(desc);
-  const size_t o_gmap = st.add(gmap);
   const size_t o_cfl = st.add(nullptr, (blocks.size() + 1) * sizeof(double));
   const size_t o_leaves = st.add(a->leaves);
   // (whole workgroups of the kernel that lists the contributions)
@@ -1490,10 +1511,12 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->h_clock = c;
   const std::vector<AmrClock> clk{c};
   const size_t o_clock = st.add(clk), o_next = st.add(clk);
-  // the records and contributions follow, made on the device
+  // the records, the ghost map and the contributions follow, made on the device
   a->nrec = (int)segs.size() * a->list.group;
   const size_t o_recs = (st.total + 255) / 256 * 256;
-  const size_t o_contribs = o_recs + (size_t)a->nrec * sizeof(SegRec);
+  const size_t o_gmap = o_recs + (size_t)a->nrec * sizeof(SegRec);
+  const size_t gmap_bytes = blocks.size() * (size_t)a->max_cells * sizeof(int);
+  const size_t o_contribs = (o_gmap + gmap_bytes + 255) / 256 * 256;
   bool listed = amr_list_fits(p, ncontribs);
   auto bytes = [&]() {
     return o_contribs + (listed ? (size_t)ncontribs * sizeof(AmrContrib) : 0) + 16;
@@ -1548,7 +1571,13 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   a->h_desc = std::move(desc);
   a->h_vblocks = std::move(vblocks);
   a->h_ghosts = std::move(gh);
-  const int rc = amr_device_tables(a, true);
+  int rc = gmap_bytes && hipMemsetAsync(a->d_gmap, 0xff, gmap_bytes, p->stream) != hipSuccess
+               ? fail(PC_E_HIP, "ghost map")
+               : PC_OK;
+  if (rc == PC_OK && a->nghosts > 0)
+    hipLaunchKernelGGL(k_amr_ghost_map, dim3((a->nghosts + 3) / 4), dim3(256), 0, p->stream,
+                       a->d_ghosts, a->nghosts, a->d_gmap);
+  if (rc == PC_OK) rc = amr_device_tables(a, true);
   if (rc != PC_OK) {
     amr_free(a);
     delete a;
@@ -1685,7 +1714,7 @@ int amr_launch_lts(pc_amr* a, Fields F, int cur) {
   const int ncells = a->nblocks * a->max_cells;
   if (ncells > 0)
     hipLaunchKernelGGL(k_lts_ghosts, dim3((ncells + 255) / 256), dim3(256), 0, p->stream,
-                       a->d_gmap, a->max_cells, ncells, a->d_ghosts, F, cur, a->d_clock, L);
+                       a->d_gmap, ncells, a->d_ghosts, F, cur, a->d_clock, L);
   amr_launch_leaves<true>(a, F, cur);
   HIPCHK(hipGetLastError());
   return PC_OK;
