@@ -130,7 +130,7 @@ struct AmrGhost {
   int kind, src, dst;
   int sx, sy, sox, soy, dox, doy;
   int sn[2];
-  int cell0;  // its first cell in the plan's ghost map
+  int cell0;  // its first cell among the ghost cells of its task's leaves
   // tile rows: first cell of the source region (interpolation: cell (0, 0)
   // of the source), first cell of the destination region
   long long sbase, dbase;
@@ -233,35 +233,6 @@ k_amr_contribs(const AmrVBlock* __restrict__ blocks, const int* __restrict__ cpt
   }
 }
 
-// The six quantities (h + b, hu, hv at the two times) that fine cell i adds to
-// a cell of area dstRegion, into con[0 .. 5][at].
-template <int N>
-__device__ __forceinline__ void amr_contribution(const Fields& F, const State& O, const State& W,
-                                                 long long i, double region, double dstRegion,
-                                                 double tfOld, double tfNew, double (*con)[N],
-                                                 int at) {
-  const double bv = gl(F.b + i);
-  const double vo[3] = {gl(O.h + i) + 1.0 * bv, gl(O.hu + i), gl(O.hv + i)};
-  const double vn[3] = {gl(W.h + i) + 1.0 * bv, gl(W.hu + i), gl(W.hv + i)};
-  for (int q = 0; q < 3; ++q) {
-    con[q][at] = (vo[q] * (1.0 - tfOld) + vn[q] * tfOld) * region / dstRegion;
-    con[3 + q][at] = (vo[q] * (1.0 - tfNew) + vn[q] * tfNew) * region / dstRegion;
-  }
-}
-
-// Sum `sub` (< 6) of virtual-patch cell k into the patch: h + b -> h with its
-// own b (SWEKernel::postProcessRestriction).
-__device__ __forceinline__ void amr_store_restricted(const AmrVBlock& B, const Fields& F, int cur,
-                                                     int k, int sub, double acc) {
-  const int x = k / B.ny, y = k - x * B.ny;
-  const long long di = B.off + (long long)(x + 1) * B.stride + (y + 1);
-  const int q = sub % 3, st = sub < 3 ? 1 - cur : cur;
-  if (q == 0)
-    gs(F.H(st) + di, acc + (-1.0) * gl(F.b + di));
-  else
-    gs((q == 1 ? F.HU(st) : F.HV(st)) + di, acc);
-}
-
 // Restriction (DefaultRestriction.cpph:16-106, SWEKernel::
 // postProcessRestriction): kRestrictLanes lanes per virtual-patch cell take
 // its contributions in turn; lane q < 6 sums one of the six quantities (h +
@@ -313,7 +284,15 @@ k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ xpt
         cs.dt = L.dt[s];
         amr_restrict_factors(cs, tfOld, tfNew);
       }
-      amr_contribution(F, O, W, i, a.region, B.dstRegion, tfOld, tfNew, con[g], half + sub);
+      const double bv = gl(F.b + i);
+      const double vo[3] = {gl(O.h + i) + 1.0 * bv, gl(O.hu + i), gl(O.hv + i)};
+      const double vn[3] = {gl(W.h + i) + 1.0 * bv, gl(W.hu + i), gl(W.hv + i)};
+      for (int q = 0; q < 3; ++q) {
+        con[g][q][half + sub] =
+            (vo[q] * (1.0 - tfOld) + vn[q] * tfOld) * a.region / B.dstRegion;
+        con[g][3 + q][half + sub] =
+            (vo[q] * (1.0 - tfNew) + vn[q] * tfNew) * a.region / B.dstRegion;
+      }
     }
     wave_sync();
     if (sub < 6) {
@@ -322,7 +301,15 @@ k_amr_restrict(const AmrVBlock* __restrict__ blocks, const int* __restrict__ xpt
     }
     wave_sync();
   }
-  if (cellok && sub < 6) amr_store_restricted(B, F, cur, k, sub, acc);
+  if (!cellok || sub >= 6) return;
+  const int x = k / B.ny, y = k - x * B.ny;
+  const long long di = B.off + (long long)(x + 1) * B.stride + (y + 1);
+  const int q = sub % 3, st = sub < 3 ? 1 - cur : cur;
+  // h + b -> h with the virtual patch's b
+  if (q == 0)
+    gs(F.H(st) + di, acc + (-1.0) * gl(F.b + di));
+  else
+    gs((q == 1 ? F.HU(st) : F.HV(st)) + di, acc);
 }
 
 // The same for plans without a contribution list (amr_list_fits): every lane
@@ -368,8 +355,14 @@ k_amr_restrict_pairs(const AmrVBlock* __restrict__ blocks, const int* __restrict
       const int m = r0 + sub;
       if (m < nfine) {
         const int s0 = o[0] + m / n[1], s1 = o[1] + m % n[1];
-        amr_contribution(F, O, W, tile_index(S, s0, s1), amr_shared_area(a, dp, s0, s1),
-                         B.dstRegion, tfOld, tfNew, con[g], sub);
+        const long long i = tile_index(S, s0, s1);
+        const double region = amr_shared_area(a, dp, s0, s1), bv = gl(F.b + i);
+        const double vo[3] = {gl(O.h + i) + 1.0 * bv, gl(O.hu + i), gl(O.hv + i)};
+        const double vn[3] = {gl(W.h + i) + 1.0 * bv, gl(W.hu + i), gl(W.hv + i)};
+        for (int q = 0; q < 3; ++q) {
+          con[g][q][sub] = (vo[q] * (1.0 - tfOld) + vn[q] * tfOld) * region / B.dstRegion;
+          con[g][3 + q][sub] = (vo[q] * (1.0 - tfNew) + vn[q] * tfNew) * region / B.dstRegion;
+        }
       }
       wave_sync();
       if (sub < 6) {
@@ -379,7 +372,13 @@ k_amr_restrict_pairs(const AmrVBlock* __restrict__ blocks, const int* __restrict
       wave_sync();
     }
   }
-  if (cellok && sub < 6) amr_store_restricted(B, F, cur, k, sub, acc);
+  if (!cellok || sub >= 6) return;
+  const long long di = B.off + (long long)(d0 + 1) * B.stride + (d1 + 1);
+  const int q = sub % 3, st = sub < 3 ? 1 - cur : cur;
+  if (q == 0)
+    gs(F.H(st) + di, acc + (-1.0) * gl(F.b + di));
+  else
+    gs((q == 1 ? F.HU(st) : F.HV(st)) + di, acc);
 }
 
 // Cell k of a ghost entry.  LTS: every leaf runs on its own clock, and only
@@ -467,27 +466,30 @@ __device__ __forceinline__ void amr_ghost_cell(const AmrGhost g, int k,
 }
 
 // The plan's ghost map (-1 where no entry writes one): every entry's cells, a
-// wavefront per entry.  Runs once per plan.
+// wavefront per entry; task: the entries' tasks.  Runs once per plan.
 __global__ void __launch_bounds__(256)
-k_amr_ghost_map(const AmrGhost* __restrict__ ghosts, int n, int* __restrict__ gmap) {
+k_amr_ghost_map(const AmrGhost* __restrict__ ghosts, const int* __restrict__ task, int n,
+                int max_cells, int* __restrict__ gmap) {
   const int e = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
   if (e >= n) return;
-  const int cells = ghosts[e].sx * ghosts[e].sy, cell0 = ghosts[e].cell0;
-  for (int k = threadIdx.x & 63; k < cells; k += 64) gmap[cell0 + k] = e;
+  const int cells = ghosts[e].sx * ghosts[e].sy;
+  int* const out = gmap + (long long)task[e] * max_cells + ghosts[e].cell0;
+  for (int k = threadIdx.x & 63; k < cells; k += 64) out[k] = e;
 }
 
 // Local time stepping: the ghost cells of the advancing leaves, before any
 // leaf changes (one thread per ghost cell of the plan).
 __global__ void __launch_bounds__(256)
-k_lts_ghosts(const int* __restrict__ gmap, int ncells, const AmrGhost* __restrict__ ghosts,
-             Fields F, int cur, const AmrClock* clock, AmrLts L) {
+k_lts_ghosts(const int* __restrict__ gmap, int max_cells, int ncells,
+             const AmrGhost* __restrict__ ghosts, Fields F, int cur, const AmrClock* clock,
+             AmrLts L) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= ncells) return;
   const int e = gl(gmap + c), advancing = gl(L.iter);
   const AmrClock now = gl(clock);
   if (e < 0 || advancing == 0) return;
   const AmrGhost g = gl(ghosts + e);
-  amr_ghost_cell<true>(g, c - g.cell0, F, cur, now, L);
+  amr_ghost_cell<true>(g, c % max_cells - g.cell0, F, cur, now, L);
 }
 
 // SWEKernel::fillBoundaryLayer (SWEKernel.cpp:176-237) of the leaves of a
@@ -593,7 +595,7 @@ k_amr_fill(AmrPlanDev A, Fields F, int cur, const AmrClock* clock,
       const int k = i == (int)threadIdx.x ? ghost : gl(gmap + i);
       if (k < 0) continue;
       const AmrGhost e = gl(A.ghosts + k);
-      amr_ghost_cell<false>(e, (int)blockIdx.x * A.max_cells + i - e.cell0, F, cur, c, L);
+      amr_ghost_cell<false>(e, i - e.cell0, F, cur, c, L);
     }
   // uNew -> uOld (DefaultTransfer::copyUNewToUOld)
 #pragma unroll
@@ -1455,8 +1457,9 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   std::vector<int> block_of(plist.size());
   for (size_t b = 0; b < blocks.size(); ++b)
     for (int k = 0; k < blocks[b].nseg; ++k) block_of[blocks[b].leaf0 + k] = (int)b;
+  std::vector<int> b_of(gh.size());
   {
-    std::vector<int> b_of(gh.size()), ncells(blocks.size(), 0);
+    std::vector<int> ncells(blocks.size(), 0);
     for (size_t e = 0; e < gh.size(); ++e) {
       b_of[e] = block_of[pos[gh[e].dst]];
       int& n = ncells[b_of[e]];
@@ -1464,7 +1467,6 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
       n += gh[e].sx * gh[e].sy;
       a->max_cells = std::max(a->max_cells, n);
     }
-    for (size_t e = 0; e < gh.size(); ++e) gh[e].cell0 += b_of[e] * a->max_cells;
   }
   // walls grouped per leaf in call order
   std::vector<AmrWalls> wl(plist.size(), AmrWalls{0, 0});
@@ -1506,7 +1508,7 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
   const size_t o_vblocks = st.add(vblocks), o_cptr = st.add(cptr), o_cpairs = st.add(cpairs);
   const size_t o_xptr = st.add(xptr);
   const size_t o_pairs = st.add(pairs), o_ghosts = st.add(gh), o_walls = st.add(wl);
-  const size_t o_wall_dims = st.add(wdims);
+  const size_t o_wall_dims = st.add(wdims), o_ghost_task = st.add(b_of);
   c.end_time = INFINITY;
   a->h_clock = c;
   const std::vector<AmrClock> clk{c};
@@ -1576,7 +1578,8 @@ int pc_amr_create(pc_pool* p, const int32_t* leaves, int nleaves, const int32_t*
                : PC_OK;
   if (rc == PC_OK && a->nghosts > 0)
     hipLaunchKernelGGL(k_amr_ghost_map, dim3((a->nghosts + 3) / 4), dim3(256), 0, p->stream,
-                       a->d_ghosts, a->nghosts, a->d_gmap);
+                       a->d_ghosts, reinterpret_cast<int*>(base + o_ghost_task), a->nghosts,
+                       a->max_cells, a->d_gmap);
   if (rc == PC_OK) rc = amr_device_tables(a, true);
   if (rc != PC_OK) {
     amr_free(a);
@@ -1714,7 +1717,7 @@ int amr_launch_lts(pc_amr* a, Fields F, int cur) {
   const int ncells = a->nblocks * a->max_cells;
   if (ncells > 0)
     hipLaunchKernelGGL(k_lts_ghosts, dim3((ncells + 255) / 256), dim3(256), 0, p->stream,
-                       a->d_gmap, ncells, a->d_ghosts, F, cur, a->d_clock, L);
+                       a->d_gmap, a->max_cells, ncells, a->d_ghosts, F, cur, a->d_clock, L);
   amr_launch_leaves<true>(a, F, cur);
   HIPCHK(hipGetLastError());
   return PC_OK;
@@ -1784,20 +1787,17 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
   CHK(amr_upload(&a->d_rsrc, rsrc));
   CHK(amr_upload(&a->lts.itn, std::vector<int>(1, 1)));
   CHK(amr_upload(&a->lts.need, std::vector<int>(ns, 0)));
-  CHK(amr_upload(&a->d_vidx, vidx));
-  CHK(amr_upload(&a->d_vptr, vptr));
   CHK(amr_upload(&a->d_vleaf, vleaf));
-  CHK(amr_upload(&a->d_nptr, np));
-  CHK(amr_upload(&a->d_nbr, nb));
-  std::vector<int> vowner(vleaf.size());
-  for (size_t v = 0; v + 1 < vptr.size(); ++v)
-    std::fill(vowner.begin() + vptr[v], vowner.begin() + vptr[v + 1], (int)v);
-  CHK(amr_upload(&a->d_vowner, vowner));
   a->npairs = (int)vleaf.size();
   int most = 0;
   for (int k = 0; k < nl; ++k) most = std::max(most, np[k + 1] - np[k]);
   if (most <= kLtsNeighbours && a->virtuals.size() <= kLtsBlockVirtuals &&
       a->npairs <= kLtsBlockPairs) {
+    // what k_lts_flags_block reads
+    std::vector<int> vowner(vleaf.size());
+    for (size_t v = 0; v + 1 < vptr.size(); ++v)
+      std::fill(vowner.begin() + vptr[v], vowner.begin() + vptr[v + 1], (int)v);
+    CHK(amr_upload(&a->d_vowner, vowner));
     std::vector<int> t8((size_t)nl * kLtsNeighbours);
     for (int k = 0; k < nl; ++k)
       for (int j = 0; j < kLtsNeighbours; ++j) {
@@ -1806,6 +1806,11 @@ int pc_amr_lts_init(pc_amr* a, const int32_t* nptr, const int32_t* nbr) {
       }
     CHK(amr_upload(&a->d_neighbours, t8));
   } else {
+    // what k_lts_virtual_ends and k_lts_flags read
+    CHK(amr_upload(&a->d_vidx, vidx));
+    CHK(amr_upload(&a->d_vptr, vptr));
+    CHK(amr_upload(&a->d_nptr, np));
+    CHK(amr_upload(&a->d_nbr, nb));
     CHK(amr_upload(&a->d_vend, std::vector<double>(a->virtuals.size(), 0.0)));
   }
   a->lts_ready = true;
